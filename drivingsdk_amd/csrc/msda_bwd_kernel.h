@@ -737,7 +737,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                             const int32_t pos =
                                 atomicAdd(&cursor[tile_first[rec_l] + ((rec_key[r] - lvl[rec_l].z) >> a.tile_px_log2)], 1);
                             const uint32_t in_tile = (uint32_t)(rec_key[r] - lvl[rec_l].z) & ((1u << a.tile_px_log2) - 1u);
-                            const u32x4 rec = {in_tile | ((uint32_t)(q - wk.q_begin) << a.tile_px_log2),
+                            const u32x4 rec = {in_tile | ((uint32_t)q << a.tile_px_log2),
                                                __builtin_bit_cast(uint32_t, rec_wa[r]), __builtin_bit_cast(uint32_t, rec_wb[r]), 0u};
                             if (rec_in_lds) {
                                 *rec_lds(pos) = rec;

@@ -48,7 +48,7 @@ namespace mxd {
 struct TileItem {
     int32_t level, H, W, base;   // level geometry
     int32_t p0, p1;              // pixel range of the tile, relative to the batch element
-    int32_t w0, w1;              // range of workgroups of the first kernel whose records are taken
+    int32_t c0, cstep;           // the item takes slabs c0, c0 + cstep, c0 + 2 cstep, ... in the order of KArgs::run_step
     int32_t tile;                // index of the tile within the (batch, head): column of the run table
     int32_t exclusive;           // 1: no other workgroup touches this tile (the item is not split by query range and the
                                  // levels tile the keys, so that no tile of another level holds the same rows)
@@ -62,19 +62,17 @@ struct LevelInfo {
     int32_t px[kMaxLevels];      // pixels of the level inside the value tensor
     int32_t nt[kMaxLevels];      // its tiles (before the run table's room is considered)
     int32_t chunks[kMaxLevels];  // query chunks per tile
-    int32_t wpc[kMaxLevels];     // first-kernel workgroups per chunk
     __device__ void fill(const KArgs& a, int l)
     {
         const i32x4 L = load_level(a, l);
-        int32_t P, w = 0;
+        int32_t P;
         const int32_t n = level_tile_count(L.x, L.y, L.z, a.nk, a.tile_px_log2, &P);
         H[l] = L.x;
         W[l] = L.y;
         base[l] = L.z;
         px[l] = P;
         nt[l] = n;
-        chunks[l] = n > 0 ? level_tile_chunks(a, n, &w) : 0;
-        wpc[l] = w;
+        chunks[l] = n > 0 ? level_tile_chunks(a, n) : 0;
     }
     // levels_tile_the_keys() on the values held here
     __device__ bool tile_the_keys(const KArgs& a) const
@@ -115,7 +113,7 @@ __device__ inline bool decode_tile_item(const KArgs& a, const TileArgs& t, const
         const int32_t nt = lv_nt[l];
         if (nt == 0) continue;
         const int32_t base = lv.base[l], P = lv.px[l];
-        const int32_t wpc = lv.wpc[l], chunks = lv.chunks[l];
+        const int32_t chunks = lv.chunks[l];
         const int32_t n = nt * chunks;
         if (item < first + n) {
             const int32_t ti = (item - first) / chunks, ci = (item - first) % chunks;
@@ -126,8 +124,8 @@ __device__ inline bool decode_tile_item(const KArgs& a, const TileArgs& t, const
             const int32_t tile_px = 1 << a.tile_px_log2;
             out->p0 = base + ti * tile_px;
             out->p1 = (out->p0 + tile_px) < (base + P) ? (out->p0 + tile_px) : (base + P);
-            out->w0 = ci * wpc;
-            out->w1 = (out->w0 + wpc) < a.nwg ? (out->w0 + wpc) : a.nwg;
+            out->c0 = ci;
+            out->cstep = chunks;
             out->tile = lv_first[l] + ti;
             out->exclusive = chunks == 1 && canonical;
             return true;
@@ -267,12 +265,9 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     const int hd = a.hd;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
-    // (float32: read as a scalar -- the compiler cannot know that tid >> 6 is the same in every lane of a wavefront, and
-    //  whatever depends on it, the wavefront's runs and its entry storage, is otherwise a per-lane value steered by exec
-    //  masks: 7 vector registers fewer and no spill, backward at the encoder shape 262.8 -> 260.6 us, BEVFormer shape 997 ->
-    //  989.  The 16-bit instantiations keep the per-lane form: with the scalar one the compiler schedules the walk's row
-    //  requests right in front of their use, encoder backward 270 -> 291 us)
-    const int wave = sizeof(T) == 4 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    // (read as a scalar -- the compiler cannot know that tid >> 6 is the same in every lane of a wavefront, and whatever
+    //  depends on it, the wavefront's runs and its entry storage, is otherwise a per-lane value steered by exec masks)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int npx = it.p1 - it.p0;
     // A tile much smaller than the workgroup is held in several copies (lists and registers),
     // each taking the samples of some queries; the copies meet in the image through atomics.
@@ -300,8 +295,12 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
     const __amdgpu_buffer_rsrc_t rres = make_rsrc(a.rec + bh * a.nwg * a.rec_cap * kRecDwords,
                                                   (uint32_t)a.nwg * (uint32_t)a.rec_cap * (kRecDwords * 4u));
-    // runs of this wavefront: workgroups it.w0 + wave, + NW, + 2 NW, ... of the first kernel
-    const int nruns = (it.w1 - it.w0 - wave + NW - 1) / NW;  // <= 0: none
+    // Runs of this wavefront: number wave, + NW, + 2 NW, ... of the item's.  Every item, and every stretch of an item's
+    // stream, takes slabs from all over the query range: with queries in the raster order of a feature map a stretch of
+    // neighbouring slabs puts its records on a few rows of pixels, and the few lane groups that own those walk long
+    // lists while the others wait.
+    const int item_runs = (a.nwg - it.c0 + it.cstep - 1) / it.cstep;
+    const int nruns = (item_runs - wave + NW - 1) / NW;  // <= 0: none
 
     float* gimg = a.grad_value + (size_t)wk.b * (a.gbatch_bytes / 4);
     const int64_t row_pitch = (int64_t)a.nh * hd;  // floats between neighbouring pixels
@@ -338,7 +337,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         // input state of this wavefront (uniform): next group of runs, records of the current
         // group, next unread record, and the batch fetched ahead
         int rg = 0, N = 0, i0 = 0;
-        u32x4 ahead = {0u, 0u, 0u, 0u};
+        u32x3 ahead = {0u, 0u, 0u};
         auto fetch_ahead = [&](int first) {
             const int i = first + lane;
             if (i < N) {
@@ -349,9 +348,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 // (one 12-byte load, non-temporal: the records are read once)
                 const u32x3 v = __builtin_bit_cast(
                     u32x3, __builtin_amdgcn_raw_buffer_load_b96(rres, (run_src[r] + ((uint32_t)i - run_pre[r])) * (kRecDwords * 4u), 0, 2));
-                // (run r of the current group comes from workgroup it.w0 + wave + NW * (rg - 64 + r) of the first kernel;
-                //  its records name queries relative to that workgroup's first one)
-                ahead = u32x4{v.x, v.y, v.z, (uint32_t)(it.w0 + wave + NW * (rg - kWave + r)) * (uint32_t)a.plan.tile_q};
+                ahead = v;
             }
         };
         bool counted = false;    // this wavefront has reported the end of its work
@@ -366,11 +363,12 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                     const int r = rg + lane;
                     uint32_t len = 0, src = 0;
                     if (r < nruns) {
-                        const int w = it.w0 + wave + NW * r;
+                        const uint32_t i = (uint32_t)(it.c0 + it.cstep * (wave + NW * r));
+                        const uint32_t w = i * a.run_step % (uint32_t)a.nwg;  // (below 2^32: the launcher's choice of the step)
                         const uint32_t* row = tbl + (size_t)w * a.tbl_stride;
                         const uint32_t s = row[0];
                         len = row[1] - s;
-                        src = (uint32_t)w * (uint32_t)a.rec_cap + s;
+                        src = w * (uint32_t)a.rec_cap + s;
                     }
                     uint32_t inc = len;
 #pragma unroll
@@ -392,7 +390,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 }
                 if (count + 2 * kWave > (int)kDummyOfWave) break;  // entry storage full: next round
                 const bool have = i0 + lane < N;
-                const u32x4 rc = ahead;
+                const u32x3 rc = ahead;
                 i0 += kWave;
                 fetch_ahead(i0);
                 // A record is the pair (pixel, pixel + 1).  A pair whose pixels belong to the same
@@ -409,10 +407,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 float wb = 0.f;
                 // (a record that does not belong to this tile or names no query of the batch element is dropped:
                 // the run table and the records are only as good as the workspace the caller hands over)
-                const uint32_t rkey = rc.x, rq0 = rc.w;
-                if (have && (rkey & (uint32_t)(kTilePx - 1)) < (uint32_t)npx && rq0 + (rkey >> kTilePxLog2) < (uint32_t)a.nq) {
+                const uint32_t rkey = rc.x;
+                if (have && (rkey & (uint32_t)(kTilePx - 1)) < (uint32_t)npx && (rkey >> kTilePxLog2) < (uint32_t)a.nq) {
                     const uint32_t ya = rc.y, za = rc.z;
-                    q = rq0 + (rkey >> kTilePxLog2);
+                    q = rkey >> kTilePxLog2;
                     const int pl = (int)(rkey & (uint32_t)(kTilePx - 1));
                     const float wa = __builtin_bit_cast(float, ya);
                     wb = __builtin_bit_cast(float, za);
@@ -513,22 +511,20 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             // The loop body is branch-free: a list that has ended keeps "reading" the dummy entry.
             // kWalk lists are walked together, one entry of each per trip, and two trips are in flight.
             {
-                auto fetch = [&](uint32_t& e, float (&g)[CHL], float& wa, float& wb) {
+                // (a row stays as it was loaded until it is used: what is in flight takes half the registers in the 16-bit
+                //  types, and no conversion waits for its row where the row is requested)
+                typedef typename RowIO<T, VEC>::raw_t raw_t;
+                auto fetch = [&](uint32_t& e, raw_t (&g)[NB][4 / VEC], float& wa, float& wb) {
                     const u32x4 en = ent_at(e);
                     // (a bit cast applied directly to a vector element picks up element 0: copy first)
                     const uint32_t ya = en.y, za = en.z;
                     wa = __builtin_bit_cast(float, ya);
                     wb = __builtin_bit_cast(float, za);
 #pragma unroll
-                    for (int k = 0; k < NB; ++k) {
+                    for (int k = 0; k < NB; ++k)
 #pragma unroll
-                        for (int c = 0; c < 4; c += VEC) {
-                            float g1[VEC];
-                            RowIO<T, VEC>::unpack(RowIO<T, VEC>::load_raw(gres, en.x + lane_off[k] + (uint32_t)(c * sizeof(T))), g1);
-#pragma unroll
-                            for (int v = 0; v < VEC; ++v) g[4 * k + c + v] = g1[v];
-                        }
-                    }
+                        for (int c = 0; c < 4; c += VEC)
+                            g[k][c / VEC] = RowIO<T, VEC>::load_raw(gres, en.x + lane_off[k] + (uint32_t)(c * sizeof(T)));
                     e = en.w;
                 };
 #pragma unroll
@@ -544,17 +540,30 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                     // two sets of rows in flight: the entries and rows of the next trip are requested before the
                     // rows of this trip are used, so that a long list costs its entries' LDS latency per trip
                     // and not the latency of a row load (reads past a list's end land on the dummy entry)
-                    float gA[kWalk][CHL], uA[kWalk], vA[kWalk], gB[kWalk][CHL], uB[kWalk], vB[kWalk];
-                    auto use = [&](float (&g)[kWalk][CHL], float (&u)[kWalk], float (&v)[kWalk]) {
+                    raw_t gA[kWalk][NB][4 / VEC], gB[kWalk][NB][4 / VEC];
+                    float uA[kWalk], vA[kWalk], uB[kWalk], vB[kWalk];
+                    auto use = [&](raw_t (&g)[kWalk][NB][4 / VEC], float (&u)[kWalk], float (&v)[kWalk]) {
 #pragma unroll
                         for (int m = 0; m < kWalk; ++m) {
 #pragma unroll
-                            for (int c = 0; c < CHL; ++c) {
-                                acc[i + m][c] = __builtin_fmaf(u[m], g[m][c], acc[i + m][c]);
-                                if (i + m + 1 < kAccPx)
-                                    acc[(i + m + 1) % kAccPx][c] = __builtin_fmaf(v[m], g[m][c], acc[(i + m + 1) % kAccPx][c]);
+                            for (int k = 0; k < NB * (4 / VEC); ++k) {
+                                float row[VEC];
+                                RowIO<T, VEC>::unpack(g[m][k / (4 / VEC)][k % (4 / VEC)], row);
+#pragma unroll
+                                for (int e = 0; e < VEC; ++e) {
+                                    const int c = k * VEC + e;
+                                    acc[i + m][c] = __builtin_fmaf(u[m], row[e], acc[i + m][c]);
+                                    if (i + m + 1 < kAccPx)
+                                        acc[(i + m + 1) % kAccPx][c] = __builtin_fmaf(v[m], row[e], acc[(i + m + 1) % kAccPx][c]);
+                                }
                             }
                         }
+                    };
+                    // Neither the scheduler nor the optimiser may move the requests behind the use of the other set (left to
+                    // itself the compiler sinks one of the two past the loop's exit test, in some instantiations both).
+                    auto keep_order = []() {
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_sched_barrier(0);
                     };
                     auto any_left = [&]() {
                         bool t = false;
@@ -570,11 +579,13 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                             bool pending = any_left();
 #pragma unroll
                             for (int m = 0; m < kWalk; ++m) fetch(e[m], gB[m], uB[m], vB[m]);
+                            keep_order();
                             use(gA, uA, vA);
                             if (!pending) break;  // (B holds dummy entries only)
                             pending = any_left();
 #pragma unroll
                             for (int m = 0; m < kWalk; ++m) fetch(e[m], gA[m], uA[m], vA[m]);
+                            keep_order();
                             use(gB, uB, vB);
                             if (!pending) break;  // (A holds dummy entries only)
                         }
@@ -722,9 +733,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 template <typename T>
 static hipError_t launch_t(const KArgs& a, const TileArgs& t, hipStream_t stream)
 {
-    // an octet of lanes reads a 32-channel block of a grad_out row, 4 channels per lane: one
-    // load per lane when head_dim and the pointer alignment allow it; the wider forms (tiles of 256 and 128
-    // pixels) are built for that case only
+    // an octet of lanes reads a 32-channel block of a grad_out row, 4 channels per lane: one load per lane, for float32 rows
+    // whatever their length and alignment (16-byte loads need 4-byte addresses only, and the range check at the end of the
+    // buffer zeroes single dwords), for 16-bit rows when head_dim and the pointer alignment allow it; the wider forms
+    // (tiles of 256 and 128 pixels) are built for aligned rows only
     const dim3 grid(t.grid), block(t.block);
     if (a.tile_px_log2 == 8 && t.vec >= 4)
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 8, 4>), grid, block, 0, stream, a, t);
@@ -732,12 +744,14 @@ static hipError_t launch_t(const KArgs& a, const TileArgs& t, hipStream_t stream
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 16, 4>), grid, block, 0, stream, a, t);
     else if (a.tile_px_log2 != kTilePxLog2Max)
         return hipErrorInvalidConfiguration;
-    else if (t.vec >= 4)
+    else if (t.vec >= 4 || sizeof(T) == 4)
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 4>), grid, block, 0, stream, a, t);
-    else if (t.vec == 2)
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 2>), grid, block, 0, stream, a, t);
-    else
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 1>), grid, block, 0, stream, a, t);
+    else if constexpr (sizeof(T) == 2) {
+        if (t.vec == 2)
+            hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 2>), grid, block, 0, stream, a, t);
+        else
+            hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 1>), grid, block, 0, stream, a, t);
+    }
     return hipGetLastError();
 }
 

@@ -363,6 +363,7 @@ BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2)
               lds <= 64 * 1024 &&                          // ... and its strips and counters fit the default limit
               tbl <= (int64_t(1) << 28) &&                 // run table of at most 256 MiB
               L.nwg * L.rec_cap * (mxd::kRecDwords * 4) < (int64_t(1) << 32) &&  // 32-bit byte offsets of the records of a (batch, head)
+              d.nq < (int64_t(1) << (32 - mxd::kTilePxLog2Max)) &&  // a record holds the query above the pixel of its tile
               d.nq * d.nh * d.hd * 4 < (int64_t(1) << 31); // grad_output rows addressed with 32-bit byte offsets
     if (L.tiles) {
         L.tbl_bytes = ((size_t)tbl + 255) & ~(size_t)255;
@@ -381,6 +382,24 @@ BwdLayout bwd_layout(int dtype, const Dims& d, bool wide_rows)
     BwdLayout L = bwd_layout_for(dtype, d, pref);
     if (!L.tiles && pref != mxd::kTilePxLog2Max) L = bwd_layout_for(dtype, d, mxd::kTilePxLog2Max);
     return L;
+}
+
+// Step through the slabs of a (batch, head) in the tile pass: near the golden section of their number, which spreads any
+// stretch of steps evenly over the query range, and without a common divisor with it, so that every slab is met once.
+uint32_t run_step(int64_t nwg)
+{
+    if (nwg < 4 || nwg > 65535) return 1;  // (index times step stays below 2^32)
+    auto gcd = [](uint32_t x, uint32_t y) {
+        while (y != 0) {
+            const uint32_t r = x % y;
+            x = y;
+            y = r;
+        }
+        return x;
+    };
+    uint32_t step = (uint32_t)(0.6180339887 * (double)nwg);
+    while (step > 1 && gcd((uint32_t)nwg, step) != 1) --step;
+    return step;
 }
 
 // Workspace a caller must bring: what the launch may need whichever way its pointers are aligned.
@@ -1045,6 +1064,7 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
     a.tbl = reinterpret_cast<uint32_t*>(ws);
     a.rec = reinterpret_cast<uint32_t*>(ws + L.tbl_bytes);
     a.nwg = (int32_t)L.nwg;
+    a.run_step = run_step(L.nwg);
     a.rec_cap = (int32_t)L.rec_cap;
     a.tbl_stride = (int32_t)L.tbl_stride;
     a.grad_loc = grad_loc;
@@ -1287,6 +1307,7 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
     a.tbl = reinterpret_cast<uint32_t*>(ws);
     a.rec = reinterpret_cast<uint32_t*>(ws + L.tbl_bytes);
     a.nwg = (int32_t)L.nwg;
+    a.run_step = run_step(L.nwg);
     a.rec_cap = (int32_t)L.rec_cap;
     a.tbl_stride = (int32_t)L.tbl_stride;
     a.grad_loc = part;  // per-head partial images, summed below

@@ -61,11 +61,14 @@ struct KArgs {
     // first kernel (tile_q queries of one (batch, head)) owns a slab of rec_cap pair records,
     // which it fills sorted by tile; row [w] of the table holds the start of every tile's run
     // inside slab w (tbl_stride entries, the last used one being the total).
-    // record (12 bytes) = {pixel within its tile | query within the workgroup << tile_px_log2, weight of that pixel,
-    //                      weight of the pixel to its right}
+    // record (12 bytes) = {pixel within its tile | query << tile_px_log2, weight of that pixel, weight of the pixel to its
+    //                      right}
     uint32_t* rec;         // [bs*nh][nwg][rec_cap] records of kRecDwords dwords
     uint32_t* tbl;         // [bs*nh][nwg][tbl_stride]
     int32_t nwg;           // workgroups of the first kernel per (batch, head)
+    uint32_t run_step;     // the tile pass takes the slabs in the order 0, run_step, 2 run_step, ... modulo nwg (a step without a
+                           // common divisor): neighbouring slabs hold neighbouring queries, which in a feature map's raster order
+                           // sample neighbouring pixels
     int32_t rec_cap;       // 2 * tile_q * nl * np
     int32_t tbl_stride;    // upper bound of tiles per (batch, head), plus one
     int32_t tile_px_log2;  // log2 of the pixels per tile of the grad_value pass (9, 8 or 7: see msda_plan.h)
@@ -109,9 +112,9 @@ constexpr int kRowParts = 16;  // pieces a tile's rows are cut into for the zero
 // Pixels per lane group of the tile pass: 8 for tiles of 512 pixels, 4 for 256, 2 for 128 (64 groups per workgroup).
 __device__ inline int32_t tile_group_px(int32_t tile_px_log2) { return 1 << (tile_px_log2 - 6); }
 
-// Query chunks the tiles of a level with `nt` tiles are split into by the tile pass; *wpc: workgroups of the first
-// kernel per chunk.
-__device__ inline int32_t level_tile_chunks(const KArgs& a, int32_t nt, int32_t* wpc)
+// Query chunks the tiles of a level with `nt` tiles are split into by the tile pass (chunk c takes every chunks-th slab of
+// records: see KArgs::run_step).
+__device__ inline int32_t level_tile_chunks(const KArgs& a, int32_t nt)
 {
     // two pair records per sample, spread evenly over the tiles of the level
     // (32-bit divisions wherever the operands allow: a 64-bit one is some 150 instructions, and the workgroups of all
@@ -127,9 +130,7 @@ __device__ inline int32_t level_tile_chunks(const KArgs& a, int32_t nt, int32_t*
     if (chunks < 1) chunks = 1;
     if (chunks > (uint32_t)a.tile_max_chunks) chunks = (uint32_t)a.tile_max_chunks;
     if (chunks > (uint32_t)a.nwg) chunks = (uint32_t)a.nwg;
-    const uint32_t w = ((uint32_t)a.nwg + chunks - 1) / chunks;
-    *wpc = (int32_t)w;
-    return (int32_t)(((uint32_t)a.nwg + w - 1) / w);
+    return (int32_t)chunks;
 }
 
 // A tile of `npx` pixels whose rows its one workgroup of the tile pass stores directly: no other workgroup adds to
@@ -185,8 +186,7 @@ __device__ inline bool atomic_rows_of_part_of(const KArgs& a, GetLevel level, in
             const int32_t ti = tile - first, tile_px = 1 << a.tile_px_log2;
             const int32_t p0 = L.z + ti * tile_px;
             const int32_t npx = (P - ti * tile_px) < tile_px ? (P - ti * tile_px) : tile_px;
-            int32_t wpc;
-            if (tile_stored_directly(level_tile_chunks(a, nt, &wpc), npx, a.tile_px_log2)) {
+            if (tile_stored_directly(level_tile_chunks(a, nt), npx, a.tile_px_log2)) {
                 *r0 = p0;
                 *r1 = part == 0 ? p0 + 1 : p0;
             } else {
