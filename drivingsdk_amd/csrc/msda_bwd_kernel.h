@@ -163,7 +163,12 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
         for (int p = 0; p < NPASS; ++p) {
             const int ch = (c + p * LPR) * VEC;
             if (unit_ok && ch < a.hd) {
-                RowIO<T, VEC>::load_global(grow + ch, gv[p]);
+                const int start = piece_start<VEC>(ch, a.hd);
+                RowIO<T, VEC>::load_global(grow + start, gv[p]);
+                // (channels that the piece before it has as well count there)
+#pragma unroll
+                for (int e = 0; e < VEC - 1; ++e)
+                    if (start + e < ch) gv[p][e] = 0.0f;
             } else {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) gv[p][e] = 0.0f;
@@ -187,7 +192,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 const int ch = (c + p * LPR) * VEC;
                 if (unit_ok && ch < a.hd) {
                     float ov[VEC];
-                    RowIO<T, VEC>::load_global(orow + ch, ov);
+                    RowIO<T, VEC>::load_global(orow + piece_start<VEC>(ch, a.hd), ov);
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) dsum = __builtin_fmaf(ov[e], gv[p][e], dsum);
                 }
@@ -403,7 +408,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
 #pragma unroll
     for (int p = 0; p < NPASS; ++p) {
         const int ch = (c + p * LPR) * VEC;
-        choff[p] = head_off + (ch < a.hd ? ch * (uint32_t)sizeof(T) : 0u);
+        choff[p] = head_off + (ch < a.hd ? piece_start<VEC>(ch, a.hd) * (uint32_t)sizeof(T) : 0u);
     }
 
     // A workgroup that passes through one iteration of one chunk (all samples of the plain operator and of the fused

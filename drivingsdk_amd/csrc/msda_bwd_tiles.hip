@@ -320,6 +320,12 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     // lane j of group g = tid / 8 keeps channels 32k + 4j .. 32k + 4j + 3 (k < NB) of the pixels g*PPG .. g*PPG + PPG - 1
     const int grp = tid / kLpp, j = tid % kLpp;
 
+    // First channel of the four that a lane loads for channels ch .. ch + 3: its own -- what lies behind a float32 row's
+    // end is read and never written, and the range check at the end of the buffer zeroes single dwords.  A dword holds
+    // two 16-bit elements, so there the last lane of a row whose length is no multiple of 4 reads the row's last four
+    // and moves its sums to their places when the rounds are done.
+    auto first_channel = [&](int ch) { return sizeof(T) == 2 && VEC == 4 ? piece_start<4>(ch, hd) : ch; };
+
     for (int cb = 0; cb < hd; cb += CH) {
         float acc[kAccPx][CHL];
 #pragma unroll
@@ -331,7 +337,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         uint32_t lane_off[NB];
 #pragma unroll
         for (int k = 0; k < NB; ++k)
-            lane_off[k] = ghead_off + (uint32_t)(my_ch + 32 * k < hd ? my_ch + 32 * k : 0) * (uint32_t)sizeof(T);
+            lane_off[k] = ghead_off + (uint32_t)(my_ch + 32 * k < hd ? first_channel(my_ch + 32 * k) : 0) * (uint32_t)sizeof(T);
         const int nch = (hd - cb) < CH ? (hd - cb) : CH;
 
         // input state of this wavefront (uniform): next group of runs, records of the current
@@ -619,6 +625,22 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 #pragma unroll
             for (int c = 0; c < CHL; ++c) acc[0][c] += cin[c];
         }
+        if constexpr (sizeof(T) == 2 && VEC == 4) {
+            if ((hd & 3) != 0) {  // (uniform)
+#pragma unroll
+                for (int kb = 0; kb < NB; ++kb) {
+                    const int ch = my_ch + 32 * kb;
+                    const int sh = ch < hd ? ch - first_channel(ch) : 0;
+#pragma unroll
+                    for (int i = 0; i < PPG; ++i) {
+                        const float v1 = acc[i][4 * kb + 1], v2 = acc[i][4 * kb + 2], v3 = acc[i][4 * kb + 3];
+                        if (sh == 1) acc[i][4 * kb] = v1, acc[i][4 * kb + 1] = v2, acc[i][4 * kb + 2] = v3;
+                        if (sh == 2) acc[i][4 * kb] = v2, acc[i][4 * kb + 1] = v3;
+                        if (sh == 3) acc[i][4 * kb] = v3;
+                    }
+                }
+            }
+        }
         // ---- write the CH channels of this tile -------------------------------------------
         // (address arithmetic derived from these opaque copies stays inside this section instead of
         // occupying registers during the rounds)
@@ -733,24 +755,18 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 template <typename T>
 static hipError_t launch_t(const KArgs& a, const TileArgs& t, hipStream_t stream)
 {
-    // an octet of lanes reads a 32-channel block of a grad_out row, 4 channels per lane: one load per lane, for float32 rows
-    // whatever their length and alignment (16-byte loads need 4-byte addresses only, and the range check at the end of the
-    // buffer zeroes single dwords), for 16-bit rows when head_dim and the pointer alignment allow it; the wider forms
-    // (tiles of 256 and 128 pixels) are built for aligned rows only
+    // an octet of lanes reads a 32-channel block of a grad_out row, 4 channels per lane: one load per lane, whatever the row's
+    // length and alignment (but for 16-bit rows of fewer than 4 channels)
     const dim3 grid(t.grid), block(t.block);
-    if (a.tile_px_log2 == 8 && t.vec >= 4)
+    if (sizeof(T) == 2 && a.hd < 4) {
+        if (a.tile_px_log2 != kTilePxLog2Max) return hipErrorInvalidConfiguration;
+        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, sizeof(T) == 2 ? 1 : 4>), grid, block, 0, stream, a, t);
+    } else if (a.tile_px_log2 == 8) {
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 8, 4>), grid, block, 0, stream, a, t);
-    else if (a.tile_px_log2 == 7 && t.vec >= 4)
+    } else if (a.tile_px_log2 == 7) {
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 16, 4>), grid, block, 0, stream, a, t);
-    else if (a.tile_px_log2 != kTilePxLog2Max)
-        return hipErrorInvalidConfiguration;
-    else if (t.vec >= 4 || sizeof(T) == 4)
+    } else {
         hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 4>), grid, block, 0, stream, a, t);
-    else if constexpr (sizeof(T) == 2) {
-        if (t.vec == 2)
-            hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 2>), grid, block, 0, stream, a, t);
-        else
-            hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 1>), grid, block, 0, stream, a, t);
     }
     return hipGetLastError();
 }

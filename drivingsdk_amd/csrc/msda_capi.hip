@@ -244,11 +244,17 @@ size_t backward_lds_bytes(int units_per_wave, int waves, bool tiles, int64_t tbl
 // two_pass_rows: rows of 17 to 32 lanes of 16 bytes are read by 16 lanes in two passes instead (four units per
 // wavefront rather than two: the first backward kernel then fills its geometry lanes and sums its dots over 16 lanes
 // with DPP alone; backward at 8 heads x 128 channels in float32 587 -> 572 us, 545 with the slab collected in LDS).
-void row_geometry(int es, int64_t hd, int align_bytes, int* vec_out, int* lpr_out, int* npass_out, bool two_pass_rows = false)
+// whole_pieces: only pieces that divide the row and that `align_bytes` allows; otherwise a row that is no multiple of the
+// piece is read in pieces of which the last one overlaps the one before it (piece_start, msda_device.h), wherever it
+// starts: pieces that divide the 37 channels of a head are single elements, 37 of 64 lanes at work and a unit per
+// wavefront (6 x 9680 queries of 4 heads x 37 channels, five levels with 3 points, float32: forward 226 -> 144 us, the backward's
+// first kernel 582 -> 212, its tile pass, which then reads the records once for up to 64 channels, 331 -> 219).
+void row_geometry(int es, int64_t hd, int lane_bytes, int* vec_out, int* lpr_out, int* npass_out, bool two_pass_rows = false,
+                  bool whole_pieces = false)
 {
-    if (align_bytes < es) align_bytes = es;
-    int vec = 16 / es;
-    while (vec > 1 && (hd % vec != 0 || align_bytes < vec * es)) vec >>= 1;
+    if (lane_bytes < es) lane_bytes = es;
+    int vec = lane_bytes / es < 16 / es ? lane_bytes / es : 16 / es;
+    while (vec > 1 && (whole_pieces ? hd % vec != 0 : hd < vec)) vec >>= 1;
     const int lanes_needed = (int)((hd + vec - 1) / vec);
     int lpr = 4;
     while (lpr < lanes_needed && lpr < mxd::kWave) lpr <<= 1;
@@ -322,12 +328,9 @@ struct BwdLayout {
 };
 
 // Pixels per tile of the grad_value pass, as a power of two: every thread of its workgroups keeps 32 sums, so 512 pixels
-// of up to 32 channels, 256 of up to 64, 128 of more (msda_plan.h).  The smaller tiles are built for rows that are read
-// four elements per lane (`wide_rows`: head_dim a multiple of 4 and pointers aligned for it); other rows keep 512-pixel
-// tiles and take one pass over the records per 32 channels.
-int preferred_tile_px_log2(const Dims& d, bool wide_rows)
+// of up to 32 channels, 256 of up to 64, 128 of more (msda_plan.h).
+int preferred_tile_px_log2(const Dims& d)
 {
-    if (!wide_rows || d.hd % 4 != 0) return mxd::kTilePxLog2Max;
     const int v = tuning().tile_px_log2;
     if (v >= 7 && v <= mxd::kTilePxLog2Max) return v;
     if (d.hd <= 32) return mxd::kTilePxLog2Max;
@@ -376,9 +379,9 @@ BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2)
 
 // The layout a launch uses: the tile size preferred for the rows, or 512-pixel tiles where the finer run table would
 // not fit the first kernel's bookkeeping.
-BwdLayout bwd_layout(int dtype, const Dims& d, bool wide_rows)
+BwdLayout bwd_layout(int dtype, const Dims& d)
 {
-    const int pref = preferred_tile_px_log2(d, wide_rows);
+    const int pref = preferred_tile_px_log2(d);
     BwdLayout L = bwd_layout_for(dtype, d, pref);
     if (!L.tiles && pref != mxd::kTilePxLog2Max) L = bwd_layout_for(dtype, d, mxd::kTilePxLog2Max);
     return L;
@@ -400,13 +403,6 @@ uint32_t run_step(int64_t nwg)
     uint32_t step = (uint32_t)(0.6180339887 * (double)nwg);
     while (step > 1 && gcd((uint32_t)nwg, step) != 1) --step;
     return step;
-}
-
-// Workspace a caller must bring: what the launch may need whichever way its pointers are aligned.
-size_t bwd_workspace_bytes(int dtype, const Dims& d)
-{
-    const size_t a = bwd_layout(dtype, d, true).total, b = bwd_layout(dtype, d, false).total;
-    return a > b ? a : b;
 }
 
 // LDS for the slab of a workgroup of the first backward kernel that makes several passes (msda_bwd_kernel.h): 12 bytes per
@@ -434,7 +430,7 @@ int plan_record_buffer(mxd_msda_plan* p, const BwdLayout& L, const Dims& d, int 
 }
 
 // Geometry of the tile-ownership grad_value kernel (msda_bwd_tiles.hip).
-int make_tile_args(const Dims& d, const BwdLayout& L, int vec, int accumulate, mxd::TileArgs* t, bool plain_operator = false)
+int make_tile_args(const Dims& d, const BwdLayout& L, int accumulate, mxd::TileArgs* t, bool plain_operator = false)
 {
     memset(t, 0, sizeof(*t));
     // pair records (counted before merging) per work item when a hot tile is split: enough items to fill the 512
@@ -475,7 +471,6 @@ int make_tile_args(const Dims& d, const BwdLayout& L, int vec, int accumulate, m
     const int64_t items = d.nl * ((2 * d.nq * d.np + t->target - 1) / t->target + 1) + L.tbl_stride;
     if (items >= (int64_t(1) << 24)) return fail(MXD_E_SHAPE, "backward needs %lld work items per (batch, head)", (long long)items);
     t->items_per_bh = (int32_t)items;  // (the callers add TileArgs::extra)
-    t->vec = vec;
     t->accumulate = accumulate;
     t->batch_major = tuning().tile_order > 0 ? 1 : 0;
     t->map.tile_q = 1;
@@ -669,17 +664,22 @@ int forward_cu_flip(int dtype)
 
 // level_cache: in/out, bytes of LDS for the forward's level cache (asked for -> granted)
 // cu_form: in/out, whether the forward may take / takes the one-workgroup-per-CU form
+// align_bytes: alignment of the rows' buffers; whole_pieces: see row_geometry (launches read rows in overlapping pieces where
+// no whole ones fit; the plan that mxd_msda_make_plan reports describes whole pieces)
 int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_plan* p, int* level_cache = nullptr,
-              int* cu_form = nullptr)
+              int* cu_form = nullptr, bool whole_pieces = false)
 {
     const int rc = check_dims(dtype, d);
     if (rc != MXD_OK) return rc;
     const int es = elem_size(dtype);
     int vec, lpr, npass;
-    if (backward && align_bytes > backward_lane_bytes(dtype, d)) align_bytes = backward_lane_bytes(dtype, d);
+    // (rows in LDS -- the one-workgroup-per-CU form, the level cache -- are copied and read in aligned pieces of 16 bytes)
+    const bool rows_of_16 = align_bytes >= 16 && d.hd * es % 16 == 0;
+    int lane_bytes = whole_pieces ? align_bytes : 16;
+    if (backward && lane_bytes > backward_lane_bytes(dtype, d)) lane_bytes = backward_lane_bytes(dtype, d);
     // (the forward keeps 32 lanes in one pass: at 8 heads x 128 channels in float32 two passes take 248 against 237 us)
-    row_geometry(es, d.hd, align_bytes, &vec, &lpr, &npass, backward && tuning().bwd_two_pass != 0);
-    if (!backward && cu_form && *cu_form && level_cache) {
+    row_geometry(es, d.hd, lane_bytes, &vec, &lpr, &npass, backward && tuning().bwd_two_pass != 0, whole_pieces);
+    if (!backward && rows_of_16 && cu_form && *cu_form && level_cache) {
         if (plan_forward_cu(dtype, d, vec, lpr, npass, p, level_cache)) return MXD_OK;
     }
     if (cu_form) *cu_form = 0;
@@ -691,7 +691,7 @@ int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_
     p->waves_per_block = 4;
     int iters = tuning().fwd_iters;
     if (iters < 1) iters = 1;
-    const BwdLayout L = bwd_layout(dtype, d, vec >= 4);
+    const BwdLayout L = bwd_layout(dtype, d);
     // the tile pass wants L.tile_q queries per workgroup of the first backward kernel
     int split = 1;  // units of the backward's first kernel that share a query
     if (backward) {
@@ -701,7 +701,7 @@ int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_
             split = (int)(p->units_per_wave * p->waves_per_block / L.tile_q);
         }
     }
-    int cache = (level_cache && *level_cache && !backward) ? forward_cache_bytes(vec, es, d, p->units_per_wave) : 0;
+    int cache = (level_cache && *level_cache && !backward && rows_of_16) ? forward_cache_bytes(vec, es, d, p->units_per_wave) : 0;
     if (cache > 0) {
         // 8 wavefronts share one copy of the cached rows and work through 128 queries (MXD_MSDA_FWD_WGQ; 256 and
         // 64 measure within 2 % of it); two such workgroups
@@ -821,7 +821,7 @@ int mxd_msda_make_plan(int backward, int dtype, int64_t bs, int64_t nk, int64_t 
     if (!plan) return fail(MXD_E_NULL, "plan is NULL");
     const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np};
     int cache = 1, cu = 1;
-    return make_plan(backward != 0, dtype, d, align_bytes, plan, &cache, &cu);
+    return make_plan(backward != 0, dtype, d, align_bytes, plan, &cache, &cu, true);
 }
 
 int mxd_msda_init(void)
@@ -984,7 +984,7 @@ size_t mxd_msda_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk, int6
     take_meta_flag(&dtype);
     const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np};
     if (check_dims(dtype, d) != MXD_OK) return 0;
-    return bwd_workspace_bytes(dtype, d);
+    return bwd_layout(dtype, d).total;
 }
 
 // What the fused form adds to a backward call.
@@ -1028,7 +1028,7 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
     memset(&a, 0, sizeof(a));
     rc = make_plan(1, dtype, d, align, &a.plan);
     if (rc != MXD_OK) return rc;
-    const BwdLayout L = bwd_layout(dtype, d, a.plan.vec >= 4);  // (as make_plan laid the first kernel's LDS out)
+    const BwdLayout L = bwd_layout(dtype, d);  // (as make_plan laid the first kernel's LDS out)
     const size_t part_bytes = (fused && fused->grad_ref) ? fused_part_bytes(d, fused->ref_dim) : 0;
     const size_t need = L.total + part_bytes;
     if (need > 0 && (!workspace || workspace_bytes < need))
@@ -1089,7 +1089,7 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
     const bool atomic_mode = !L.tiles || (flags & MXD_BWD_ANY_LAYOUT) != 0;
     mxd::TileArgs t;
     if (!atomic_mode) {
-        rc = make_tile_args(d, L, a.plan.vec, (flags & MXD_BWD_ACCUMULATE) ? 1 : 0, &t, !fused && !gka && !grid);
+        rc = make_tile_args(d, L, (flags & MXD_BWD_ACCUMULATE) ? 1 : 0, &t, !fused && !gka && !grid);
         if (rc != MXD_OK) return rc;
         plan_image(&a, &t, half, (flags & MXD_BWD_ACCUMULATE) != 0, image, grad_value, hd);
     }
@@ -1127,7 +1127,7 @@ size_t mxd_msda_fused_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk
     take_meta_flag(&dtype);
     const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
     if (check_dims(dtype, d) != MXD_OK || (ref_dim != 2 && ref_dim != 4)) return 0;
-    return bwd_workspace_bytes(dtype, d) + (want_grad_ref ? fused_part_bytes(d, ref_dim) : 0);
+    return bwd_layout(dtype, d).total + (want_grad_ref ? fused_part_bytes(d, ref_dim) : 0);
 }
 
 int mxd_msda_fused_backward(const void* value, const int32_t* spatial_shapes, const int32_t* level_start_index,
@@ -1255,7 +1255,7 @@ size_t mxd_dagg_backward_workspace_bytes(int dtype, int64_t bs, int64_t num_feat
     Dims d;
     if (dagg_dims(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &d) != MXD_OK)
         return 0;
-    return bwd_workspace_bytes(dtype, d) + dagg_part_bytes(d, num_cams);
+    return bwd_layout(dtype, d).total + dagg_part_bytes(d, num_cams);
 }
 
 int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, const int32_t* scale_start_index,
@@ -1278,7 +1278,7 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
     memset(&a, 0, sizeof(a));
     rc = make_plan(1, dtype, d, align, &a.plan);
     if (rc != MXD_OK) return rc;
-    const BwdLayout L = bwd_layout(dtype, d, a.plan.vec >= 4);  // (as make_plan laid the first kernel's LDS out)
+    const BwdLayout L = bwd_layout(dtype, d);  // (as make_plan laid the first kernel's LDS out)
     const size_t part_bytes = dagg_part_bytes(d, num_cams);
     const size_t need = L.total + part_bytes;
     if (!workspace || workspace_bytes < need)
@@ -1318,7 +1318,7 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
     const bool atomic_mode = !L.tiles;
     mxd::TileArgs t;
     if (!atomic_mode) {
-        rc = make_tile_args(d, L, a.plan.vec, 0, &t);
+        rc = make_tile_args(d, L, 0, &t);
         if (rc != MXD_OK) return rc;
         plan_image(&a, &t, half, false, image, grad_mc_ms_feat, d.hd);
     }

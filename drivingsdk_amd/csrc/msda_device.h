@@ -238,7 +238,6 @@ struct TileArgs {
     int32_t items_per_bh;  // upper bound of work items per (batch, head), including `extra`
     int32_t extra;         // workgroups per (batch, head) behind the work items that add the samples of levels whose tiles
                            // found no room in the run table (plain operator only; they leave at once otherwise)
-    int32_t vec;           // elements per load of a grad_out row
     int32_t accumulate;    // add into the existing contents of the image
     int32_t store_vec;     // 4: rows of the image are 16-byte aligned, else 1
     int32_t batch_major;   // 1: the work items of a batch element are numbered together (an XCD's L2 then holds one
@@ -326,6 +325,14 @@ __device__ inline void fused_location(const KArgs& a, const T* rp, const i32x4 l
     }
 }
 
+// First channel of the piece of VEC channels that covers channel `ch` (a multiple of VEC) of a row: the last piece of a row
+// that is no multiple of VEC long ends where the row ends and shares channels with the one before it (VEC <= hd).
+template <int VEC>
+__device__ inline int piece_start(int ch, int hd)
+{
+    return ch + VEC <= hd ? ch : hd - VEC;
+}
+
 // ---- row access: VEC elements of T at a byte offset of a bound buffer -> fp32 -------------
 template <typename T, int VEC>
 struct RowIO;
@@ -367,7 +374,10 @@ struct RawBits<T, VEC, 2> {
 
 template <typename T, int VEC>
 struct RowIO {
+    // (pieces are aligned to their elements only: a row whose length is no multiple of the piece starts anywhere.  gfx950
+    //  takes such addresses in one access, through buffer descriptors as well.)
     typedef T vec_t __attribute__((ext_vector_type(VEC)));
+    typedef vec_t mem_t __attribute__((aligned(sizeof(T))));
     typedef typename RawBits<T, VEC>::type raw_t;
 
     static __device__ inline raw_t load_raw(__amdgpu_buffer_rsrc_t r, uint32_t off)
@@ -384,13 +394,12 @@ struct RowIO {
             for (int i = 0; i < VEC; ++i) v[i] = to_f32<T>(t[i]);
         }
     }
-    // p must be aligned to VEC*sizeof(T)
     static __device__ inline void load_global(const T* p, float (&v)[VEC])
     {
         if constexpr (VEC == 1) {
             v[0] = to_f32(*p);
         } else {
-            const vec_t t = *reinterpret_cast<const vec_t*>(p);
+            const vec_t t = *reinterpret_cast<const mem_t*>(p);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) v[i] = to_f32<T>(t[i]);
         }
@@ -404,7 +413,7 @@ struct RowIO {
             vec_t t;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) t[i] = from_f32<T>(v[i]);
-            __builtin_nontemporal_store(t, reinterpret_cast<vec_t*>(p));
+            __builtin_nontemporal_store(t, reinterpret_cast<mem_t*>(p));
         }
     }
 };

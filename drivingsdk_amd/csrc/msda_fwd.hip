@@ -121,7 +121,7 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
     for (int p = 0; p < NPASS; ++p) {
         const int ch = (c + p * a.plan.lanes_per_row) * VEC;
         chan_ok[p] = ch < a.hd;
-        choff[p] = head_off + (chan_ok[p] ? ch * (uint32_t)sizeof(T) : 0u);
+        choff[p] = head_off + (chan_ok[p] ? piece_start<VEC>(ch, a.hd) * (uint32_t)sizeof(T) : 0u);
     }
     // same lane offsets inside a cached row
     uint32_t lds_choff[NPASS];
@@ -287,7 +287,8 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
             T* orow = out + (((int64_t)wk.b * a.nq + q) * a.nh + wk.h) * a.hd;
 #pragma unroll
             for (int p = 0; p < NPASS; ++p) {
-                if (chan_ok[p]) RowIO<T, VEC>::store_global(orow + (c + p * a.plan.lanes_per_row) * VEC, acc[p]);
+                // (channels that two pieces share are stored twice, with the same value)
+                if (chan_ok[p]) RowIO<T, VEC>::store_global(orow + lds_choff[p] / (uint32_t)sizeof(T), acc[p]);
             }
         }
     }
@@ -351,10 +352,7 @@ static hipError_t launch_dtype(const KArgs& a, hipStream_t stream)
 {
     const int vec = a.plan.vec, np = a.plan.npass;
     if (vec == 1 && np == 1) return launch_one<T, 1, 1>(a, stream);
-    if (vec == 1 && np == 2) return launch_one<T, 1, 2>(a, stream);
-    if (vec == 1 && np == 4) return launch_one<T, 1, 4>(a, stream);
     if (vec == 2 && np == 1) return launch_one<T, 2, 1>(a, stream);
-    if (vec == 2 && np == 2) return launch_one<T, 2, 2>(a, stream);
     if (vec == 4 && np == 1) return launch_one<T, 4, 1>(a, stream);
     if constexpr (sizeof(T) == 2) {
         if (vec == 8 && np == 1) return launch_one<T, 8, 1>(a, stream);
