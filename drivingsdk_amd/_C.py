@@ -3,6 +3,9 @@
 with the checks, output allocation and dtype policy of
 mx_driving/csrc/MultiScaleDeformableAttn.cpp:28-118, over the C ABI of libmxd_msda.so.
 
+Inputs that the kernels read as they are go straight to the extension module (csrc/torch_ops.cpp); it returns None for all
+others, which are checked here, brought into that form and handed to it again.
+
 Differences from the reference binding, all widening:
   * bfloat16 is accepted next to float16/float32;
   * float16/bfloat16 are read natively by the kernels (fp32 accumulation, one rounding at
@@ -13,6 +16,7 @@ Work is enqueued on torch's current stream of the tensors' device; nothing synch
 import torch
 
 from . import _lib
+from ._lib import native as _native
 
 _FLOAT_CODES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torch.bfloat16: _lib.DTYPE_BF16}
 
@@ -22,10 +26,11 @@ def _check(cond, msg):
         raise RuntimeError(msg)
 
 
-def _meta_flag(shapes):
-    """The reference's Python layer casts the level metadata to int32 on every call; int64 tensors are handed to the
-    library as they are instead (it reads the low words), which saves the two cast kernels."""
-    return _lib.META_I64 if shapes.dtype == torch.int64 else 0
+def _run(fn, *args):
+    """A call of the extension module with inputs that have been checked and brought into its form."""
+    out = fn(*args)
+    _check(out is not None, f"{fn.__name__}: the tensors' memory cannot be read by a kernel")
+    return out
 
 
 def _check_common(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights):
@@ -68,56 +73,33 @@ def _check_common(value, value_spatial_shapes, value_level_start_index, sampling
 def multi_scale_deformable_attn(value, value_spatial_shapes, value_level_start_index, sampling_locations,
                                 attention_weights):
     """Forward.  Returns output ``[bs, num_queries, num_heads*embed_dims]`` in value's dtype."""
-    dims = _check_common(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights)
-    bs, nk, nh, hd, nl, nl_attn, nq, npts = dims
-    lib = _lib.load()
+    output = _native.msda_forward(value, value_spatial_shapes, value_level_start_index, sampling_locations,
+                                  attention_weights)
+    if output is not None:
+        return output
+    _check_common(value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights)
     dt = value.dtype
-    value = value.contiguous()
-    shapes = value_spatial_shapes.contiguous()
-    lsi = value_level_start_index.contiguous()
-    loc = sampling_locations.to(dt).contiguous()
-    attn = attention_weights.to(dt).contiguous()
-    output = torch.empty((bs, nq, nh * hd), dtype=dt, device=value.device)
-    with torch.cuda.device(value.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.mxd_msda_forward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), loc.data_ptr(),
-                                  attn.data_ptr(), output.data_ptr(), _FLOAT_CODES[dt] | _meta_flag(shapes), bs, nk, nh,
-                                  hd, nl, nl_attn, nq, npts, stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return output
+    return _run(_native.msda_forward, value.contiguous(), value_spatial_shapes.contiguous(),
+                value_level_start_index.contiguous(), sampling_locations.to(dt).contiguous(),
+                attention_weights.to(dt).contiguous())
 
 
 def multi_scale_deformable_attn_backward(value, shape, level_start_index, location_trans, attn_weight_trans,
                                          grad_output):
     """Backward.  Returns (grad_value, grad_sampling_loc, grad_attn_weight) in value's dtype."""
+    grads = _native.msda_backward(value, shape, level_start_index, location_trans, attn_weight_trans, grad_output)
+    if grads is not None:
+        return grads
     _check(grad_output.dtype in _FLOAT_CODES,
            f"grad_output: float16, bfloat16 or float32 tensor expected but got a tensor with dtype: {grad_output.dtype}")
     dims = _check_common(value, shape, level_start_index, location_trans, attn_weight_trans)
     bs, nk, nh, hd, nl, nl_attn, nq, npts = dims
     _check(grad_output.is_cuda and grad_output.device == value.device, "grad_output: must be on value's device")
     _check(grad_output.numel() == bs * nq * nh * hd, "grad_output: expected [bs, num_queries, num_heads*embed_dims]")
-    lib = _lib.load()
     dt = value.dtype
-    value = value.contiguous()
-    shapes = shape.contiguous()
-    lsi = level_start_index.contiguous()
-    loc = location_trans.to(dt).contiguous()
-    attn = attn_weight_trans.to(dt).contiguous()
-    gout = grad_output.to(dt).contiguous()
-    grad_value = torch.empty_like(value)
-    grad_loc = torch.empty_like(loc)
-    grad_attn = torch.empty_like(attn)
-    code = _FLOAT_CODES[dt] | _meta_flag(shapes)
-    ws_bytes = lib.mxd_msda_backward_workspace_bytes(code, bs, nk, nh, hd, nl, nl_attn, nq, npts)
-    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=value.device)
-    with torch.cuda.device(value.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.mxd_msda_backward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), loc.data_ptr(), attn.data_ptr(),
-                                   gout.data_ptr(), grad_value.data_ptr(), grad_loc.data_ptr(), grad_attn.data_ptr(),
-                                   workspace.data_ptr(), ws_bytes, code, bs, nk,
-                                   nh, hd, nl, nl_attn, nq, npts, 0, stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return grad_value, grad_loc, grad_attn
+    return _run(_native.msda_backward, value.contiguous(), shape.contiguous(), level_start_index.contiguous(),
+                location_trans.to(dt).contiguous(), attn_weight_trans.to(dt).contiguous(),
+                grad_output.to(dt).contiguous())
 
 
 def msda_fused_forward(value, value_spatial_shapes, value_level_start_index, reference_points, sampling_offsets,
@@ -125,6 +107,10 @@ def msda_fused_forward(value, value_spatial_shapes, value_level_start_index, ref
     """Forward of the operator with the callers' softmax and sampling-location arithmetic folded into the
     kernel (``mxd_msda_fused_forward``): reference_points ``[bs, nq, nl, 2|4]``, sampling_offsets
     ``[bs, nq, nh, nl, np, 2]``, attention_logits ``[bs, nq, nh, nl*np]``.  Returns ``[bs, nq, nh*hd]``."""
+    output = _native.fused_forward(value, value_spatial_shapes, value_level_start_index, reference_points,
+                                   sampling_offsets, attention_logits)
+    if output is not None:
+        return output
     _check(value.dtype in _FLOAT_CODES,
            f"value: float16, bfloat16 or float32 tensor expected but got a tensor with dtype: {value.dtype}")
     _check(value_spatial_shapes.dtype in (torch.int32, torch.int64) and
@@ -152,22 +138,10 @@ def msda_fused_forward(value, value_spatial_shapes, value_level_start_index, ref
     _check(all(t.is_cuda for t in tensors),
            "msda_fused_forward: all tensors must live on a GPU (this build has no CPU implementation)")
     _check(all(t.device == value.device for t in tensors), "msda_fused_forward: tensors are on different devices")
-    lib = _lib.load()
     dt = value.dtype
-    value = value.contiguous()
-    shapes, lsi = value_spatial_shapes.contiguous(), value_level_start_index.contiguous()
-    ref = reference_points.to(dt).contiguous()
-    off = sampling_offsets.to(dt).contiguous()
-    logits = attention_logits.to(dt).contiguous()
-    output = torch.empty((bs, nq, nh * hd), dtype=dt, device=value.device)
-    with torch.cuda.device(value.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.mxd_msda_fused_forward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), ref.data_ptr(),
-                                        reference_points.size(3), off.data_ptr(), logits.data_ptr(),
-                                        output.data_ptr(), _FLOAT_CODES[dt] | _meta_flag(shapes), bs, nk, nh, hd, nl,
-                                        nq, npts, stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return output
+    return _run(_native.fused_forward, value.contiguous(), value_spatial_shapes.contiguous(),
+                value_level_start_index.contiguous(), reference_points.to(dt).contiguous(),
+                sampling_offsets.to(dt).contiguous(), attention_logits.to(dt).contiguous())
 
 
 def msda_fused_backward(value, value_spatial_shapes, value_level_start_index, reference_points, sampling_offsets,
@@ -176,6 +150,11 @@ def msda_fused_backward(value, value_spatial_shapes, value_level_start_index, re
     sampling-location arithmetic runs inside the operator's first backward kernel.  ``output`` is the forward
     result.  Returns ``(grad_value, grad_reference_points or None, grad_sampling_offsets, grad_attention_logits)``,
     each with the shape and dtype of its input."""
+    outs = (None, None if need_grad_reference_points else False, None, None)
+    grads = _native.fused_backward(value, value_spatial_shapes, value_level_start_index, reference_points,
+                                   sampling_offsets, attention_logits, output, grad_output, *outs)
+    if grads is not None:
+        return grads
     _check(value.dtype in _FLOAT_CODES,
            f"value: float16, bfloat16 or float32 tensor expected but got a tensor with dtype: {value.dtype}")
     _check(value.dim() == 4 and sampling_offsets.dim() == 6 and sampling_offsets.size(5) == 2,
@@ -202,32 +181,11 @@ def msda_fused_backward(value, value_spatial_shapes, value_level_start_index, re
     _check(all(t.is_cuda for t in tensors),
            "msda_fused_backward: all tensors must live on a GPU (this build has no CPU implementation)")
     _check(all(t.device == value.device for t in tensors), "msda_fused_backward: tensors are on different devices")
-    lib = _lib.load()
     dt = value.dtype
-    value = value.contiguous()
-    shapes, lsi = value_spatial_shapes.contiguous(), value_level_start_index.contiguous()
-    code = _FLOAT_CODES[dt] | _meta_flag(shapes)
-    ref = reference_points.to(dt).contiguous()
-    off = sampling_offsets.to(dt).contiguous()
-    logits = attention_logits.to(dt).contiguous()
-    out = output.to(dt).contiguous()
-    gout = grad_output.to(dt).contiguous()
-    grad_value = torch.empty_like(value)
-    grad_off = torch.empty_like(off)
-    grad_logits = torch.empty_like(logits)
-    grad_ref = torch.empty_like(ref) if need_grad_reference_points else None
-    want = 1 if need_grad_reference_points else 0
-    ws_bytes = lib.mxd_msda_fused_backward_workspace_bytes(code, bs, nk, nh, hd, nl, nq, npts, ref_dim, want)
-    workspace = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=value.device)
-    with torch.cuda.device(value.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        rc = lib.mxd_msda_fused_backward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), ref.data_ptr(), ref_dim,
-                                         off.data_ptr(), logits.data_ptr(), out.data_ptr(), gout.data_ptr(),
-                                         grad_value.data_ptr(), grad_ref.data_ptr() if want else None,
-                                         grad_off.data_ptr(), grad_logits.data_ptr(), workspace.data_ptr(), ws_bytes,
-                                         code, bs, nk, nh, hd, nl, nq, npts, 0, stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return grad_value, grad_ref, grad_off, grad_logits
+    return _run(_native.fused_backward, value.contiguous(), value_spatial_shapes.contiguous(),
+                value_level_start_index.contiguous(), reference_points.to(dt).contiguous(),
+                sampling_offsets.to(dt).contiguous(), attention_logits.to(dt).contiguous(),
+                output.to(dt).contiguous(), grad_output.to(dt).contiguous(), *outs)
 
 
 # ---- deformable aggregation (mx_driving/csrc/DeformableAggregation.cpp:20-82 of the reference) --------------
@@ -259,19 +217,13 @@ def _dagg_check(mc_ms_feat, spatial_shape, scale_start_index, sampling_location,
 
 def deformable_aggregation(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights):
     """Forward.  Returns ``[bs, num_anchors, num_embeds]`` in mc_ms_feat's dtype."""
-    dims = _dagg_check(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights,
-                       "deformable_aggregation")
-    lib = _lib.load()
+    out = _native.dagg_forward(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights)
+    if out is not None:
+        return out
+    _dagg_check(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights, "deformable_aggregation")
     dt = mc_ms_feat.dtype
-    feat = mc_ms_feat.contiguous()
-    ss, si = spatial_shape.contiguous(), scale_start_index.contiguous()
-    loc, w = sampling_location.to(dt).contiguous(), weights.to(dt).contiguous()
-    out = torch.empty((dims[0], dims[5], dims[2]), dtype=dt, device=feat.device)
-    with torch.cuda.device(feat.device):
-        rc = lib.mxd_dagg_forward(feat.data_ptr(), ss.data_ptr(), si.data_ptr(), loc.data_ptr(), w.data_ptr(),
-                                  out.data_ptr(), _FLOAT_CODES[dt], *dims, torch.cuda.current_stream().cuda_stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return out
+    return _run(_native.dagg_forward, mc_ms_feat.contiguous(), spatial_shape.contiguous(), scale_start_index.contiguous(),
+                sampling_location.to(dt).contiguous(), weights.to(dt).contiguous())
 
 
 def deformable_aggregation_backward(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights,
@@ -283,27 +235,16 @@ def deformable_aggregation_backward(mc_ms_feat, spatial_shape, scale_start_index
                        "deformable_aggregation_backward")
     _check(grad_output.is_cuda and grad_output.device == mc_ms_feat.device, "grad_output must be on the inputs' GPU")
     _check(tuple(grad_output.shape) == (dims[0], dims[5], dims[2]), "grad_output: expected [bs, num_anchors, num_embeds]")
-    lib = _lib.load()
     dt = mc_ms_feat.dtype
-    feat = mc_ms_feat.contiguous()
-    ss, si = spatial_shape.contiguous(), scale_start_index.contiguous()
-    loc, w = sampling_location.to(dt).contiguous(), weights.to(dt).contiguous()
-    go = grad_output.to(dt).contiguous()
+    feat, loc, w = mc_ms_feat.contiguous(), sampling_location.to(dt).contiguous(), weights.to(dt).contiguous()
 
-    def out_like(given, like):
+    def usable(given, like):
         ok = given is not None and given.is_contiguous() and given.dtype == dt and given.shape == like.shape \
             and given.device == like.device
-        return given if ok else torch.empty_like(like)
-    gf, gl, gw = out_like(grad_mc_ms_feat, feat), out_like(grad_sampling_location, loc), out_like(grad_weights, w)
-    code = _FLOAT_CODES[dt]
-    nbytes = lib.mxd_dagg_backward_workspace_bytes(code, *dims)
-    workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=feat.device)
-    with torch.cuda.device(feat.device):
-        rc = lib.mxd_dagg_backward(feat.data_ptr(), ss.data_ptr(), si.data_ptr(), loc.data_ptr(), w.data_ptr(),
-                                   go.data_ptr(), gf.data_ptr(), gl.data_ptr(), gw.data_ptr(), workspace.data_ptr(),
-                                   nbytes, code, *dims, torch.cuda.current_stream().cuda_stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return gf, gl, gw
+        return given if ok else None
+    return _run(_native.dagg_backward, feat, spatial_shape.contiguous(), scale_start_index.contiguous(), loc, w,
+                grad_output.to(dt).contiguous(), usable(grad_mc_ms_feat, feat), usable(grad_sampling_location, loc),
+                usable(grad_weights, w))
 
 
 # ---- geometric kernel attention (mx_driving/csrc/GeometricKernelAttentionFunc.cpp:33-118 of the reference) ------
@@ -342,45 +283,34 @@ def _gka_check(value, spatial_shapes, level_start_index, sampling_locations, att
 def geometric_kernel_attention_forward(value_map, spatial_shapes, level_start_index, sampling_locations,
                                        attention_weights, output):
     """Fills ``output`` ``[bs, num_queries, num_heads*dim]`` (the reference's binding has the same out-parameter)."""
+    if output.dim() == 3 and _native.gka_forward(value_map, spatial_shapes, level_start_index, sampling_locations,
+                                                 attention_weights, output) is not None:
+        return
     dims = _gka_check(value_map, spatial_shapes, level_start_index, sampling_locations, attention_weights)
-    lib = _lib.load()
     dt = value_map.dtype
     _check(output.is_cuda and output.is_contiguous() and output.dtype == dt and
            tuple(output.shape) == (dims[0], dims[5], dims[2] * dims[3]),
            "output: expected a contiguous [bs, num_queries, num_heads*dim] tensor of value's dtype")
-    value = value_map.contiguous()
-    shapes, lsi = spatial_shapes.int().contiguous(), level_start_index.int().contiguous()
     # (pixel indices travel as float32 whatever value's dtype is: exact below 2^24, where a 16-bit float is not)
-    loc, attn = sampling_locations.to(torch.float32).contiguous(), attention_weights.to(dt).contiguous()
-    with torch.cuda.device(value.device):
-        rc = lib.mxd_gka_forward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), loc.data_ptr(), attn.data_ptr(),
-                                 output.data_ptr(), _FLOAT_CODES[dt], *dims, torch.cuda.current_stream().cuda_stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
+    _run(_native.gka_forward, value_map.contiguous(), spatial_shapes.int().contiguous(),
+         level_start_index.int().contiguous(), sampling_locations.to(torch.float32).contiguous(),
+         attention_weights.to(dt).contiguous(), output)
 
 
 def geometric_kernel_attention_backward(value, spatial_shapes, level_start_index, sampling_locations, attn_weights,
                                         grad_output):
     """Returns (grad_value, grad_attn_weights)."""
+    grads = _native.gka_backward(value, spatial_shapes, level_start_index, sampling_locations, attn_weights, grad_output)
+    if grads is not None:
+        return grads
     dims = _gka_check(value, spatial_shapes, level_start_index, sampling_locations, attn_weights)
     _check(grad_output.is_cuda and grad_output.dtype in _FLOAT_CODES, "grad_output: float tensor on the GPU expected")
-    lib = _lib.load()
-    dt = value.dtype
-    value = value.contiguous()
     _check(grad_output.device == value.device and grad_output.numel() == dims[0] * dims[5] * dims[2] * dims[3],
            "grad_output: expected [bs, num_queries, num_heads*dim] on value's device")
-    shapes, lsi = spatial_shapes.int().contiguous(), level_start_index.int().contiguous()
-    loc, attn = sampling_locations.to(torch.float32).contiguous(), attn_weights.to(dt).contiguous()
-    go = grad_output.to(dt).contiguous()
-    gv, ga = torch.empty_like(value), torch.empty_like(attn)
-    code = _FLOAT_CODES[dt]
-    nbytes = lib.mxd_gka_backward_workspace_bytes(code, *dims)
-    workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=value.device)
-    with torch.cuda.device(value.device):
-        rc = lib.mxd_gka_backward(value.data_ptr(), shapes.data_ptr(), lsi.data_ptr(), loc.data_ptr(), attn.data_ptr(),
-                                  go.data_ptr(), gv.data_ptr(), ga.data_ptr(), workspace.data_ptr(), nbytes, code, *dims,
-                                  torch.cuda.current_stream().cuda_stream)
-    _check(rc == 0, _lib.last_error() if rc != 0 else "")
-    return gv, ga
+    dt = value.dtype
+    return _run(_native.gka_backward, value.contiguous(), spatial_shapes.int().contiguous(),
+                level_start_index.int().contiguous(), sampling_locations.to(torch.float32).contiguous(),
+                attn_weights.to(dt).contiguous(), grad_output.to(dt).contiguous())
 
 
 # ---- 2-D grid sampler (mx_driving/csrc/GridSampler2dV2.cpp:33-99 of the reference) ------------------------------

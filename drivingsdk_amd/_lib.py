@@ -1,8 +1,9 @@
-"""Loader for libmxd_msda.so, the C-ABI library declared in include/mxd_msda.h.
+"""Loader for libmxd_msda.so, the C-ABI library declared in include/mxd_msda.h, and for ``native``, the extension
+module that calls it with PyTorch tensors (csrc/torch_ops.cpp).
 
-The library is built in-tree (``drivingsdk_amd/lib/libmxd_msda.so``) by
+Both are built in-tree (``drivingsdk_amd/lib/libmxd_msda.so``, ``drivingsdk_amd/_native.*.so``) by
 ``drivingsdk_amd.build.build()`` / ``make -C drivingsdk_amd/csrc``.  There is no other
-implementation behind this package: if the library is missing, loading fails loudly.
+implementation behind this package: if they are missing, using them fails loudly.
 """
 import ctypes
 import os
@@ -54,6 +55,27 @@ class Plan(ctypes.Structure):
 
 
 _lib = None
+
+
+class _Missing:
+    """Stands for the extension module where it has not been built (the package is imported to build it)."""
+
+    def __init__(self, error):
+        self._error = error
+
+    def __getattr__(self, name):
+        raise ImportError(
+            "drivingsdk_amd._native is missing: the HIP library and its binding have not been built "
+            "(run `python -c 'import __graft_entry__ as g; g.build()'` or `make -C drivingsdk_amd/csrc`). "
+            "This package has no CPU or eager fallback.") from self._error
+
+
+try:
+    import torch  # noqa: F401  (the extension is linked against its libraries)
+
+    from . import _native as native
+except ImportError as e:
+    native = _Missing(e)
 
 
 def load():

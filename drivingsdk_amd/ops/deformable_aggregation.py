@@ -10,9 +10,16 @@ import torch
 from torch.autograd import Function
 
 from .. import _C
+from .._lib import native as _native
 
 
 class AdsDeformableAggregation(Function):
+    @classmethod
+    def apply(cls, *args):
+        # calls that need nothing of Python's autograd machinery are served by the extension module
+        output = _native.dagg(*args) if cls is AdsDeformableAggregation else None
+        return output if output is not None else super().apply(*args)
+
     @staticmethod
     def forward(ctx, mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights):
         if torch.numel(mc_ms_feat) == 0 or torch.numel(weights) == 0:

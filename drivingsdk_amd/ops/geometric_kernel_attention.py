@@ -9,9 +9,16 @@ Sampling locations are pixel indices (x, y), clamped to the level; there is no i
 from torch.autograd import Function
 
 from .. import _C
+from .._lib import native as _native
 
 
 class GeometricKernelAttentionFunc(Function):
+    @classmethod
+    def apply(cls, *args):
+        # calls that need nothing of Python's autograd machinery are served by the extension module
+        output = _native.gka(*args) if cls is GeometricKernelAttentionFunc else None
+        return output if output is not None else super().apply(*args)
+
     @staticmethod
     def forward(ctx, value, spatial_shapes, level_start_index, sampling_locations, attention_weights):
         ctx.save_for_backward(value, spatial_shapes, level_start_index, sampling_locations, attention_weights)

@@ -20,6 +20,7 @@ from torch.amp import custom_bwd, custom_fwd
 from torch.autograd.function import Function, once_differentiable
 
 from .. import _C
+from .._lib import native as _native
 
 
 def sampling_inputs(spatial_shapes, reference_points, sampling_offsets, attention_logits):
@@ -39,6 +40,12 @@ def sampling_inputs(spatial_shapes, reference_points, sampling_offsets, attentio
 
 
 class MultiScaleDeformableAttnFusedFunction(Function):
+    @classmethod
+    def apply(cls, *args):
+        # calls that need nothing of Python's autograd machinery are served by the extension module
+        output = _native.fused(*args) if cls is MultiScaleDeformableAttnFusedFunction else None
+        return output if output is not None else super().apply(*args)
+
     @staticmethod
     @custom_fwd(device_type="cuda", cast_inputs=torch.float32)
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, reference_points, sampling_offsets,

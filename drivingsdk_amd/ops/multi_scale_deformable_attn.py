@@ -13,9 +13,16 @@ from torch.amp import custom_bwd, custom_fwd
 from torch.autograd.function import Function, once_differentiable
 
 from .. import _C
+from .._lib import native as _native
 
 
 class MultiScaleDeformableAttnFunction(Function):
+    @classmethod
+    def apply(cls, *args):
+        # calls that need nothing of Python's autograd machinery are served by the extension module
+        output = _native.msda(*args) if cls is MultiScaleDeformableAttnFunction else None
+        return output if output is not None else super().apply(*args)
+
     @staticmethod
     @custom_fwd(device_type="cuda", cast_inputs=torch.float32)
     def forward(ctx, value, value_spatial_shapes, value_level_start_index, sampling_locations, attention_weights,
