@@ -1,0 +1,709 @@
+// Deformable aggregation for gfx950 (MI355X), wave64: forward and backward.
+//
+//   out[b,a,c] = sum over (point p, camera, scale) of w[b,a,p,camera,scale,group(c)] * bilinear(feat of (camera, scale), loc[b,a,p,camera])
+//
+// (reference: mx_driving/ops/npu_deformable_aggregation.py:10-88, kernels/deformable_aggregation/.)  A location counts only
+// strictly inside (0, 1) x (0, 1), and an anchor projects into one or two of the cameras: most samples of the sum do not exist.
+//
+// What bounds it: the feature maps of a training step (552 MB for 6 x 6 cameras of 256 x 704 pixels, 256 channels) fit no
+// cache, every row that is touched has to come from HBM once and should not come twice, and an anchor's few hundred samples
+// are one long chain when a unit of lanes works through them alone (one unit per anchor and group: forward 395 us at that
+// size, 140 us for one frame in float16, which leaves half of the CUs without a workgroup).  Here
+//
+//   * a WAVEFRONT owns an (anchor, group): its lanes look at 64 locations at a time, keep those inside the image (ballot),
+//     compute one sample per lane and then gather, 64 / lanes-per-row samples side by side, so that the chain is an eighth as
+//     long, absent samples cost a lane of one test, and 256 CUs are filled from 900 anchors on;
+//   * groups are pinned to XCDs (msda_plan.h) and the locations are taken camera by camera: the wavefronts of an XCD, which
+//     run side by side through the anchors of one batch element, then share the (camera, group) slice of the maps they are
+//     in -- 1.9 MB, of 4 MB of L2;
+//   * the gradient of the maps is gathered, not scattered: a sort by pixel of the samples' upper and lower corner pairs (LDS
+//     counters, one workgroup per (batch, level)), then every pixel row is formed once, by lanes that own its channels, from
+//     the grad_out rows of its records -- those of a batch element stay in L2 -- and stored once, whole.
+//
+// Measured (6 x 900 anchors x 13 points, 6 cameras x 4 scales, 256 channels in 8 groups, float32; float16 with one batch
+// element), before -> after: see the launchers below.
+#include "dagg.h"
+
+namespace mxd {
+
+namespace {
+
+__device__ inline i32x4 dagg_level(const DaggArgs& a, int l)
+{
+    const int sh = a.meta_i64;
+    return i32x4{a.shapes[(2 * l) << sh], a.shapes[(2 * l + 1) << sh], a.lsi[l << sh], 0};
+}
+
+__device__ inline bool inside(float x, float y) { return x > 0.0f && x < 1.0f && y > 0.0f && y < 1.0f; }  // (false for NaN)
+
+template <typename T>
+__device__ inline f32x2 load_xy(const void* loc, int64_t i)
+{
+    const T* p = static_cast<const T*>(loc) + 2 * i;
+    return f32x2{to_f32(p[0]), to_f32(p[1])};
+}
+
+// A location inside the image: {x, y, position in camera-major order << 16 | position in memory order, camera}.
+typedef u32x4 Found;
+
+// Per-wavefront LDS of the sampling kernels, in this order: found locations, the staged samples' row offsets, and then the
+// forward's corner weights and group weights or the backward's dots and location gradients.
+constexpr int kFoundBytes = kDaggList * 16, kOffBytes = kWave * 16;
+
+// Keeps the locations of anchor (b, q) from number `first` on, in camera-major order, that lie inside the image; returns
+// how many (at most kDaggList looked at).
+template <typename T>
+__device__ inline int find_locations(const DaggArgs& a, int64_t anchor, int first, Found* found, int lane)
+{
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kDaggList / kWave; ++k) {
+        const int j = first + k * kWave + lane;
+        bool ok = j < a.nloc;
+        uint32_t cam = 0;
+        int li = 0;
+        f32x2 xy = {0.f, 0.f};
+        if (ok) {
+            cam = ((uint32_t)j * a.p_magic) >> 20;
+            li = (j - (int)cam * a.P) * a.cams + (int)cam;
+            xy = load_xy<T>(a.loc, anchor * a.nloc + li);
+            ok = inside(xy.x, xy.y);
+        }
+        const uint64_t mask = __ballot(ok);
+        if (ok) {
+            const int pos = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+            const float fx = xy.x, fy = xy.y;
+            found[pos] = Found{__builtin_bit_cast(uint32_t, fx), __builtin_bit_cast(uint32_t, fy), ((uint32_t)j << 16) | (uint32_t)li, cam};
+        }
+        n += __builtin_popcountll(mask);
+    }
+    return n;
+}
+
+// ---- forward -------------------------------------------------------------------------------------------------------------
+// ONE: a row piece is the channels of one group (its weight is multiplied into the corner weights once); otherwise 128
+// bytes of several groups' channels, whose weights wait in LDS.
+template <typename T, int VEC, bool ONE>
+__global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const DaggArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ i32x4 lvl[kMaxLevels];
+    Work wk;
+    if (!decode_block(a.map, blockIdx.x, a.bs, a.pieces, a.A, &wk)) return;
+    if ((int)threadIdx.x < a.nl) lvl[threadIdx.x] = dagg_level(a, threadIdx.x);
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const int q = wk.q_begin + wave;
+    if (q >= wk.q_end) return;
+    const int64_t anchor = (int64_t)wk.b * a.A + q;
+
+    const int per_wave = kFoundBytes + kOffBytes + kWave * 16 + (ONE ? 0 : kWave * a.piece_heads * 4);
+    unsigned char* mine = smem + wave * per_wave;
+    Found* found = reinterpret_cast<Found*>(mine);
+    u32x4* off = reinterpret_cast<u32x4*>(mine + kFoundBytes);
+    f32x4* wts = reinterpret_cast<f32x4*>(mine + kFoundBytes + kOffBytes);
+    float* gws = reinterpret_cast<float*>(mine + kFoundBytes + kOffBytes + kWave * 16);
+
+    const int U = kWave >> a.lpr_log2, u = lane >> a.lpr_log2, c = lane & ((1 << a.lpr_log2) - 1);
+    const int ch0 = wk.h * a.piece_ch, nch = a.C - ch0 < a.piece_ch ? a.C - ch0 : a.piece_ch;
+    const bool chan_ok = c * VEC < nch;
+    const int ch = ch0 + (chan_ok ? piece_start<VEC>(c * VEC, nch) : 0);
+    const uint32_t choff = (uint32_t)ch * (uint32_t)sizeof(T);
+    const int h0 = ch0 / a.hd, heads = ONE ? 1 : (ch0 + nch - 1) / a.hd - h0 + 1, my_head = ONE ? 0 : ch / a.hd - h0;
+    const T* w = static_cast<const T*>(a.w) + anchor * a.nloc * a.scales * a.G + h0;
+    const __amdgpu_buffer_rsrc_t vres =
+        make_rsrc(static_cast<const char*>(a.feat) + (size_t)wk.b * a.batch_bytes, a.batch_bytes);
+
+    // lane t of a group of samples: scale t % scales of its location t / scales
+    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
+    const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);  // locations per group of samples
+    const bool tl_ok = tl < step;
+
+    float acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
+    for (int first = 0; first < a.nloc; first += kDaggList) {
+        const int n = find_locations<T>(a, anchor, first, found, lane);
+        wave_lds_sync();
+        for (int v0 = 0; v0 < n; v0 += step) {
+            const int vi = v0 + tl;
+            const bool act = tl_ok && vi < n;
+            const Found f = found[act ? vi : 0];
+            const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
+            const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
+                                              a.nf, act);
+            u32x4 o;
+            f32x4 cw;
+            const T* gw = w + (int64_t)((int)(fj & 0xFFFFu) * a.scales + ts) * a.G;
+            float aw = 1.0f;
+            if constexpr (ONE) aw = act ? to_f32(*gw) : 0.0f;
+            else
+                for (int k = 0; k < heads; ++k) gws[lane * a.piece_heads + k] = act ? to_f32(gw[k]) : 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                o[k] = sm.cvalid[k] ? (uint32_t)sm.pix[k] * a.pitch_bytes : kInvalidCorner;
+                cw[k] = sm.valid ? sm.w[k] * aw : 0.0f;
+            }
+            off[lane] = o;
+            wts[lane] = cw;
+            wave_lds_sync();
+            const int locs = n - v0 < step ? n - v0 : step;
+            const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);  // (uniform; samples that do not exist read zeros)
+#pragma unroll 2
+            for (int t = 0; t < trips; ++t) {
+                const int s = t * U + u;
+                const u32x4 ro = off[s];
+                const f32x4 rw = wts[s];
+                typename RowIO<T, VEC>::raw_t raw[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) raw[k] = RowIO<T, VEC>::load_raw(vres, ro[k] + choff);
+                const float g = ONE ? 1.0f : gws[s * a.piece_heads + my_head];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float v[VEC];
+                    RowIO<T, VEC>::unpack(raw[k], v);
+                    const float wk4 = ONE ? rw[k] : rw[k] * g;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) acc[e] = __builtin_fmaf(wk4, v[e], acc[e]);
+                }
+            }
+            wave_lds_sync();
+        }
+    }
+    // the samples were dealt to U groups of lanes: add them up, the first group stores
+    for (int d = 1 << a.lpr_log2; d < kWave; d <<= 1)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] += __shfl_xor(acc[e], d, kWave);
+    if (u == 0 && chan_ok) RowIO<T, VEC>::store_global(static_cast<T*>(a.out) + anchor * a.C + ch, acc);
+}
+
+// ---- backward, first kernel: gradients of the weights and locations, per group ---------------------------------------------
+template <typename T, int VEC>
+__global__ __launch_bounds__(kDaggWaves * kWave) void dagg_dots_kernel(const DaggArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ i32x4 lvl[kMaxLevels];
+    Work wk;
+    if (!decode_block(a.map, blockIdx.x, a.bs, a.pieces, a.A, &wk)) return;
+    if ((int)threadIdx.x < a.nl) lvl[threadIdx.x] = dagg_level(a, threadIdx.x);
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const int q = wk.q_begin + wave;
+    if (q >= wk.q_end) return;
+    const int64_t anchor = (int64_t)wk.b * a.A + q;
+
+    constexpr int kPerWave = kFoundBytes + kOffBytes + kWave * 16 + kWave * 8;
+    unsigned char* mine = smem + wave * kPerWave;
+    Found* found = reinterpret_cast<Found*>(mine);
+    u32x4* off = reinterpret_cast<u32x4*>(mine + kFoundBytes);
+    f32x4* dots = reinterpret_cast<f32x4*>(mine + kFoundBytes + kOffBytes);
+    f32x2* gxy = reinterpret_cast<f32x2*>(mine + kFoundBytes + kOffBytes + kWave * 16);
+
+    const int U = kWave >> a.lpr_log2, u = lane >> a.lpr_log2, c = lane & ((1 << a.lpr_log2) - 1);
+    const bool chan_ok = c * VEC < a.hd;
+    const int start = chan_ok ? piece_start<VEC>(c * VEC, a.hd) : 0;
+    const uint32_t choff = (uint32_t)(wk.h * a.hd + start) * (uint32_t)sizeof(T);
+    const __amdgpu_buffer_rsrc_t vres =
+        make_rsrc(static_cast<const char*>(a.feat) + (size_t)wk.b * a.batch_bytes, a.batch_bytes);
+    const T* w = static_cast<const T*>(a.w) + anchor * a.nloc * a.scales * a.G + wk.h;
+    const int64_t part = (int64_t)wk.h * a.bs * a.A + anchor;
+    float* gw = a.gw_part + part * a.nloc * a.scales;
+    f32x2* gl = reinterpret_cast<f32x2*>(a.gl_part) + part * a.nloc;
+
+    // the anchor's grad_out row, in every group of lanes (16-bit rows as pairs for v_dot2)
+    constexpr bool kDot2 = sizeof(T) == 2 && VEC % 2 == 0;
+    constexpr int kPairs = kDot2 ? VEC / 2 : 1;
+    float gv[VEC];
+    uint32_t gpk[kPairs];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) gv[e] = 0.0f;
+    if (chan_ok) {
+        RowIO<T, VEC>::load_global(static_cast<const T*>(a.grad_out) + anchor * a.C + wk.h * a.hd + start, gv);
+#pragma unroll
+        for (int e = 0; e < VEC - 1; ++e)
+            if (start + e < c * VEC) gv[e] = 0.0f;  // (counted by the piece before it)
+    }
+    if constexpr (kDot2) {
+        typedef T t2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int e = 0; e < kPairs; ++e) gpk[e] = __builtin_bit_cast(uint32_t, t2{from_f32<T>(gv[2 * e]), from_f32<T>(gv[2 * e + 1])});
+    }
+
+    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
+    const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);
+    const bool tl_ok = tl < step;
+    for (int first = 0; first < a.nloc; first += kDaggList) {
+        const int n = find_locations<T>(a, anchor, first, found, lane);
+        wave_lds_sync();
+        for (int v0 = 0; v0 < n; v0 += step) {
+            const int vi = v0 + tl;
+            const bool act = tl_ok && vi < n;
+            const Found f = found[act ? vi : 0];
+            const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
+            const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
+                                              a.nf, act);
+            const float aw = act ? to_f32(w[(int64_t)((int)(fj & 0xFFFFu) * a.scales + ts) * a.G]) : 0.0f;
+            u32x4 o;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = sm.cvalid[k] ? (uint32_t)sm.pix[k] * a.pitch_bytes : kInvalidCorner;
+            off[lane] = o;
+            wave_lds_sync();
+            const int locs = n - v0 < step ? n - v0 : step;
+            const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);
+            auto gather = [&](auto lg) {
+                constexpr int LG = decltype(lg)::value;
+#pragma unroll 2
+                for (int t = 0; t < trips; ++t) {
+                    const int s = t * (kWave >> LG) + u;
+                    const u32x4 ro = off[s];
+                    typename RowIO<T, VEC>::raw_t raw[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) raw[k] = RowIO<T, VEC>::load_raw(vres, ro[k] + choff);
+                    f32x4 d;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        float dk = 0.0f;
+                        if constexpr (kDot2) {
+                            uint32_t words[kPairs];
+                            __builtin_memcpy(words, &raw[k], sizeof(words));
+#pragma unroll
+                            for (int e = 0; e < kPairs; ++e) dk = dot2_acc<T>(words[e], gpk[e], dk);
+                        } else {
+                            float v[VEC];
+                            RowIO<T, VEC>::unpack(raw[k], v);
+#pragma unroll
+                            for (int e = 0; e < VEC; ++e) dk = __builtin_fmaf(v[e], gv[e], dk);
+                        }
+                        d[k] = group_sum<LG>(dk);
+                    }
+                    if (c == 0) dots[s] = d;
+                }
+            };
+            switch (a.lpr_log2) {
+                case 0: gather(std::integral_constant<int, 0>{}); break;
+                case 1: gather(std::integral_constant<int, 1>{}); break;
+                case 2: gather(std::integral_constant<int, 2>{}); break;
+                case 3: gather(std::integral_constant<int, 3>{}); break;
+                case 4: gather(std::integral_constant<int, 4>{}); break;
+                case 5: gather(std::integral_constant<int, 5>{}); break;
+                default: gather(std::integral_constant<int, 6>{}); break;
+            }
+            wave_lds_sync();
+            f32x2 g = {0.f, 0.f};
+            if (act) {
+                float ga = 0.f;
+                if (sm.valid) {
+                    const f32x4 dd = dots[lane];
+                    const float hw = 1.0f - sm.lw, hh = 1.0f - sm.lh;
+                    ga = sm.w[0] * dd[0] + sm.w[1] * dd[1] + sm.w[2] * dd[2] + sm.w[3] * dd[3];
+                    g.x = sm.Wf * aw * (hh * (dd[1] - dd[0]) + sm.lh * (dd[3] - dd[2]));
+                    g.y = sm.Hf * aw * (hw * (dd[2] - dd[0]) + sm.lw * (dd[3] - dd[1]));
+                }
+                gw[(int)(fj >> 16) * a.scales + ts] = ga;
+            }
+            gxy[lane] = g;
+            wave_lds_sync();
+            if (act && ts == 0) {
+                // the scales of a location share it
+                for (int k = 1; k < a.scales; ++k) g += gxy[lane + k];
+                gl[fj >> 16] = g;
+            }
+            wave_lds_sync();
+        }
+    }
+}
+
+// ---- the levels as the kernels behind it see them ---------------------------------------------------------------------------
+struct DaggLevels {
+    int32_t H[kMaxLevels], W[kMaxLevels], base[kMaxLevels];
+    int32_t px[kMaxLevels];      // pixels inside the feature tensor; 0: the level has no rows (or found no room, see csr)
+    int32_t csr[kMaxLevels];     // its first entry of DaggArgs::csr
+    int32_t chunks[kMaxLevels];  // parts its strips' records are split into
+    int32_t first[kMaxLevels + 1];  // work items of the levels before it
+    int32_t tiled;               // the levels tile the keys in order: a pixel row belongs to one level
+
+    // by the first wavefronts of the workgroup; a barrier is needed behind it
+    __device__ void fill(const DaggArgs& a)
+    {
+        for (int l = threadIdx.x; l < a.nl; l += blockDim.x) {
+            const i32x4 L = dagg_level(a, l);
+            int32_t P;
+            level_tile_count(L.x, L.y, L.z, a.nf, 0, &P);
+            H[l] = L.x;
+            W[l] = L.y;
+            base[l] = L.z;
+            px[l] = P;
+            // records of a strip if every location were inside and spread evenly
+            const float expect = P > 0 ? 2.0f * (float)a.A * (float)a.P * (float)(kDaggStrip + 1) / (float)P : 0.0f;
+            int32_t n = (int32_t)__builtin_ceilf(expect / (float)kDaggStripRecords);
+            chunks[l] = n < 1 ? 1 : n > 64 ? 64 : n;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            // (levels that overlap so far that their pixels are more than the tensor has do not fit the table of record
+            //  starts: they are left out of grad_feat)
+            int64_t next = 0, room = 0;
+            int32_t items = 0, ok = 1;
+            for (int l = 0; l < a.nl; ++l) {
+                ok = ok && H[l] > 0 && W[l] > 0 && (int64_t)base[l] == next && (int64_t)H[l] * W[l] == px[l];
+                next += px[l];
+                if (room + px[l] + 1 > (int64_t)a.nf + a.nl) px[l] = 0;
+                csr[l] = (int32_t)room;
+                if (px[l] > 0) room += px[l] + 1;
+                first[l] = items;
+                items += (px[l] + kDaggStrip - 1) / kDaggStrip * chunks[l];
+            }
+            first[a.nl] = items;
+            tiled = ok && next == a.nf;
+        }
+        __syncthreads();
+    }
+    __device__ bool direct(int l) const { return tiled && chunks[l] == 1; }
+};
+
+// ---- sort of the corner pairs by pixel -------------------------------------------------------------------------------------
+// One workgroup per (batch, level, range of kDaggSortPx pixels): counts the records of every pixel in LDS, turns the counts
+// into starts, and drops every record at its place.  10 us of a training step of 1.9 M samples.
+template <typename T>
+__global__ __launch_bounds__(1024) void dagg_sort_kernel(const DaggArgs a)
+{
+    __shared__ DaggLevels lv;
+    __shared__ uint32_t cnt[kDaggSortPx];
+    __shared__ uint32_t wsum[16];
+    __shared__ uint32_t before_s;
+    lv.fill(a);
+    const int range = blockIdx.x % a.sort_ranges, l = blockIdx.x / a.sort_ranges % a.nl, b = blockIdx.x / a.sort_ranges / a.nl;
+    const int tid = threadIdx.x;
+    const int r0 = range * kDaggSortPx, P = lv.px[l], r1 = P - r0 < kDaggSortPx ? P : r0 + kDaggSortPx;
+    if (!lv.tiled) {
+        // rows that several levels share or none has: the whole image gets zeros, and every row is added to
+        const uint64_t n = (uint64_t)a.bs * a.nf * a.C, per = (n + gridDim.x - 1) / gridDim.x;
+        const uint64_t lo = blockIdx.x * per, hi = lo + per < n ? lo + per : n;
+        for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
+    } else if (lv.chunks[l] > 1 && r0 < P) {
+        const uint64_t lo = ((uint64_t)b * a.nf + lv.base[l] + r0) * a.C, hi = lo + (uint64_t)(r1 - r0) * a.C;
+        for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
+    }
+    if (r0 >= P) return;  // (uniform)
+    for (int i = tid; i < kDaggSortPx; i += 1024) cnt[i] = 0;
+    if (tid == 0) before_s = 0;
+    __syncthreads();
+
+    const int cam = l / a.scales, sc = l - cam * a.scales;
+    const i32x4 level = {lv.H[l], lv.W[l], lv.base[l], 0};
+    const uint32_t points = (uint32_t)a.A * (uint32_t)a.P;
+    // the records of a point on this level: (key, weights) of up to two
+    auto each_record = [&](uint32_t i, auto take) {
+        const f32x2 xy = load_xy<T>(a.loc, ((int64_t)b * points + i) * a.cams + cam);
+        if (!inside(xy.x, xy.y)) return;
+        const Sample sm = sample_geometry(xy.x, xy.y, level, a.nf, true);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const bool vl = sm.cvalid[2 * r], vr = sm.cvalid[2 * r + 1];
+            if (vl || vr)
+                take((vl ? sm.pix[2 * r] : sm.pix[2 * r + 1]) - level.z, vl ? sm.w[2 * r] : sm.w[2 * r + 1], vl && vr ? sm.w[2 * r + 1] : 0.0f);
+        }
+    };
+    uint32_t before = 0;  // records of the ranges before this one
+    for (uint32_t i = tid; i < points; i += 1024)
+        each_record(i, [&](int key, float, float) {
+            if (key < r0) ++before;
+            else if (key < r1) atomicAdd(&cnt[key - r0], 1u);
+        });
+    if (r0 > 0 && before != 0) atomicAdd(&before_s, before);
+    __syncthreads();
+
+    // exclusive prefix: 12 neighbouring counters per thread, then over the threads
+    constexpr int kPer = kDaggSortPx / 1024;
+    uint32_t mine[kPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        mine[k] = sum;
+        sum += cnt[tid * kPer + k];
+    }
+    uint32_t inc = sum;
+    const int lane = tid & (kWave - 1), wave = tid >> 6;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t o = __shfl_up(inc, d, kWave);
+        if (lane >= d) inc += o;
+    }
+    if (lane == kWave - 1) wsum[wave] = inc;
+    __syncthreads();
+    uint32_t at = before_s + inc - sum;
+    for (int k = 0; k < wave; ++k) at += wsum[k];
+    uint32_t* csr = a.csr + (size_t)b * ((size_t)a.nf + a.nl) + lv.csr[l];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int p = tid * kPer + k;
+        cnt[p] = at + mine[k];
+        if (r0 + p < P) csr[r0 + p] = at + mine[k];
+        if (r0 + p == P - 1) csr[P] = at + (k + 1 < kPer ? mine[k + 1 < kPer ? k + 1 : k] : sum);
+    }
+    __syncthreads();
+
+    u32x4* rec = a.rec + ((size_t)b * a.nl + l) * 2 * points;
+    for (uint32_t i = tid; i < points; i += 1024)
+        each_record(i, [&](int key, float wa, float wb) {
+            if (key < r0 || key >= r1) return;
+            const uint32_t pos = atomicAdd(&cnt[key - r0], 1u);
+            rec[pos] = u32x4{(i / (uint32_t)a.P) << 3 | ((uint32_t)key & 7u), (i * (uint32_t)a.cams + (uint32_t)cam) * (uint32_t)a.scales + (uint32_t)sc,
+                             __builtin_bit_cast(uint32_t, wa), __builtin_bit_cast(uint32_t, wb)};
+        });
+}
+
+// ---- gradient of the feature maps --------------------------------------------------------------------------------------------
+// A unit of 2^row_lpr_log2 lanes forms the rows of a strip of 8 neighbouring pixels, or of one block of their channels, from
+// the strip's records in pixel order: one row of sums for the pixel at hand and one for the pixel to its right; the records
+// of the pixel before the strip are met for their right halves.  Every row is stored once, whole (strips split by record
+// number -- levels with few pixels -- add theirs with atomics to rows that the sort has zeroed).
+// MIXED: a lane's channels may belong to several groups.
+template <typename T, int VEC, bool MIXED>
+__global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
+{
+    __shared__ DaggLevels lv;
+    lv.fill(a);
+    const int lpr = 1 << a.row_lpr_log2, units = 256 >> a.row_lpr_log2;
+    const int c = threadIdx.x & (lpr - 1);
+    const uint32_t per_b = (uint32_t)lv.first[a.nl] * (uint32_t)a.row_blocks;
+    const uint64_t total = (uint64_t)per_b * a.bs;
+    const T* gout = static_cast<const T*>(a.grad_out);
+    const uint32_t points = (uint32_t)a.A * (uint32_t)a.P;
+    const uint32_t per_anchor = (uint32_t)a.nloc * (uint32_t)a.scales;
+    for (uint64_t item = (uint64_t)blockIdx.x * units + (threadIdx.x >> a.row_lpr_log2); item < total; item += (uint64_t)gridDim.x * units) {
+        const int b = (int)(item / per_b);
+        const uint32_t r = (uint32_t)(item - (uint64_t)b * per_b);
+        const int blk = (int)(r % (uint32_t)a.row_blocks);
+        // (the coarse levels, whose strips have the most records, are numbered last and start first)
+        const int it = lv.first[a.nl] - 1 - (int)(r / (uint32_t)a.row_blocks);
+        int l = 0;
+        for (int s = 32; s > 0; s >>= 1)
+            if (l + s < a.nl && lv.first[l + s] <= it) l += s;
+        const int k = it - lv.first[l], chunks = lv.chunks[l], strip = k / chunks, chunk = k - strip * chunks;
+        const int p0 = strip * kDaggStrip, p1 = p0 + kDaggStrip < lv.px[l] ? p0 + kDaggStrip : lv.px[l];
+        const bool direct = lv.direct(l);
+        const uint32_t* csr = a.csr + (size_t)b * ((size_t)a.nf + a.nl) + lv.csr[l];
+        const uint32_t s1 = csr[p0];
+        uint32_t lo = p0 > 0 ? csr[p0 - 1] : s1, hi = csr[p1];
+        if (chunks > 1) {
+            const uint32_t s0 = lo, n = hi - lo;
+            lo = s0 + (uint32_t)((uint64_t)n * chunk / chunks);
+            hi = s0 + (uint32_t)((uint64_t)n * (chunk + 1) / chunks);
+        }
+        const int chn = (blk * lpr + c) * VEC;
+        const bool chan_ok = chn < a.C;
+        const int ch = chan_ok ? piece_start<VEC>(chn, a.C) : 0;
+        const T* grow = gout + (size_t)b * a.A * a.C + ch;
+        const T* w = static_cast<const T*>(a.w) + (size_t)b * a.A * per_anchor * a.G + ch / a.hd;
+        const u32x4* rec = a.rec + ((size_t)b * a.nl + l) * 2 * points;
+
+        float acc[VEC], nxt[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] = nxt[e] = 0.0f;
+        int cur = 0;         // pixel of the strip whose sums are in acc
+        auto flush = [&]() { // its row is complete
+            const size_t row = ((size_t)b * a.nf + lv.base[l] + p0 + cur) * a.C + ch;
+            if (chan_ok) {
+                if (direct) {
+                    RowIO<T, VEC>::store_global(static_cast<T*>(a.grad_feat) + row, acc);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        if (ch + e >= chn && acc[e] != 0.0f) unsafeAtomicAdd(a.image + row + e, acc[e]);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[e] = nxt[e], nxt[e] = 0.0f;
+            ++cur;
+        };
+        constexpr int kAhead = 4;  // records whose rows are in flight together
+        for (uint32_t e0 = lo; e0 < hi; e0 += kAhead) {
+            u32x4 rc[kAhead];
+            typename RowIO<T, VEC>::held_t row[kAhead];
+            float aw[kAhead][MIXED ? VEC : 1];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) rc[j] = rec[e0 + j < hi ? e0 + j : hi - 1];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                row[j] = RowIO<T, VEC>::load_held(grow + (size_t)(rc[j].x >> 3) * a.C);
+                const T* wj = w + (size_t)rc[j].y * a.G;
+                if constexpr (MIXED) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) aw[j][e] = to_f32(wj[(ch + e) / a.hd - ch / a.hd]);
+                } else {
+                    aw[j][0] = to_f32(*wj);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                if (e0 + j >= hi) break;
+                const uint32_t za = rc[j].z, zb = rc[j].w;
+                float wa = __builtin_bit_cast(float, za), wb = __builtin_bit_cast(float, zb);
+                if (e0 + j < s1) {  // a pair that starts on the pixel before the strip
+                    wa = wb;
+                    wb = 0.0f;
+                } else {
+                    const int px = (int)(rc[j].x & 7u);
+                    while (cur < px) flush();
+                }
+                float g[VEC];
+                RowIO<T, VEC>::unpack_held(row[j], g);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    const float gw = g[e] * aw[j][MIXED ? e : 0];
+                    acc[e] = __builtin_fmaf(wa, gw, acc[e]);
+                    nxt[e] = __builtin_fmaf(wb, gw, nxt[e]);
+                }
+            }
+        }
+        while (cur < p1 - p0) flush();
+    }
+}
+
+// ---- the rest: weights' and locations' gradients in the caller's layout, rounding ---------------------------------------------
+// A workgroup per anchor turns the per-group images into the caller's tensors (zeros for locations outside the image); for
+// 16-bit dtypes further ones round the rows of grad_feat that were added to in the float32 image.
+template <typename T>
+__global__ __launch_bounds__(256) void dagg_finish_kernel(const DaggArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int anchors = a.bs * a.A;
+    if ((int)blockIdx.x >= anchors) {
+        __shared__ DaggLevels lv;
+        lv.fill(a);
+        const uint64_t part = blockIdx.x - anchors, parts = gridDim.x - anchors;
+        auto round = [&](uint64_t lo, uint64_t n) {
+            for (uint64_t i = part * 256 + threadIdx.x; i < n; i += parts * 256) static_cast<T*>(a.grad_feat)[lo + i] = from_f32<T>(a.image[lo + i]);
+        };
+        if (!lv.tiled) {
+            round(0, (uint64_t)a.bs * a.nf * a.C);
+        } else {
+            for (int b = 0; b < a.bs; ++b)
+                for (int l = 0; l < a.nl; ++l)
+                    if (lv.chunks[l] > 1) round(((uint64_t)b * a.nf + lv.base[l]) * a.C, (uint64_t)lv.px[l] * a.C);
+        }
+        return;
+    }
+    // position of a location in the images, or 0xFFFF outside the image
+    uint16_t* pos = reinterpret_cast<uint16_t*>(smem);
+    const int64_t anchor = blockIdx.x;
+    const int64_t stride = (int64_t)anchors * a.nloc;  // locations per group
+    const f32x2* gl = reinterpret_cast<const f32x2*>(a.gl_part) + anchor * a.nloc;
+    T* out_l = static_cast<T*>(a.grad_loc) + anchor * a.nloc * 2;
+    for (int li = threadIdx.x; li < a.nloc; li += 256) {
+        const int p = li / a.cams, j = (li - p * a.cams) * a.P + p;
+        const f32x2 xy = load_xy<T>(a.loc, anchor * a.nloc + li);
+        const bool in = inside(xy.x, xy.y);
+        pos[li] = in ? (uint16_t)j : (uint16_t)0xFFFFu;
+        f32x2 s = {0.f, 0.f};
+        if (in)
+            for (int g = 0; g < a.G; ++g) s += gl[g * stride + j];
+        out_l[2 * li] = from_f32<T>(s.x);
+        out_l[2 * li + 1] = from_f32<T>(s.y);
+    }
+    __syncthreads();
+    const int gs = a.G < 256 ? a.G : 256, rows = 256 / gs;  // groups and (location, scale) pairs side by side
+    const int g0 = threadIdx.x % gs, r0 = threadIdx.x / gs, n = a.nloc * a.scales;
+    const float* gw = a.gw_part + anchor * n;
+    T* out_w = static_cast<T*>(a.grad_w) + anchor * n * a.G;
+    if (r0 < rows)
+        for (int r = r0; r < n; r += rows) {
+            const int li = (int)(((uint32_t)r * a.sc_magic) >> 20), sc = r - li * a.scales;
+            const uint32_t j = pos[li];
+            for (int g = g0; g < a.G; g += gs)
+                out_w[(int64_t)r * a.G + g] =
+                    from_f32<T>(j != 0xFFFFu ? gw[(int64_t)g * stride * a.scales + (int)j * a.scales + sc] : 0.0f);
+        }
+}
+
+template <typename F>
+hipError_t by_vec(int es, int vec, F f)
+{
+    switch (vec) {
+        case 8: if (es == 2) return f(std::integral_constant<int, 8>{}); break;
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 2: return f(std::integral_constant<int, 2>{});
+        case 1: return f(std::integral_constant<int, 1>{});
+    }
+    return hipErrorInvalidConfiguration;
+}
+
+template <typename T>
+hipError_t forward_t(const DaggArgs& a, hipStream_t stream)
+{
+    const dim3 grid(a.map.grid), block(kDaggWaves * kWave);
+    return by_vec(sizeof(T), dagg_vec(sizeof(T), a.piece_heads == 1 ? a.piece_ch : a.hd), [&](auto v) {
+        constexpr int VEC = decltype(v)::value;
+        if constexpr (VEC * sizeof(T) <= 16) {
+            const size_t lds = kDaggWaves * (kFoundBytes + kOffBytes + kWave * 16 + (a.piece_heads == 1 ? 0 : kWave * a.piece_heads * 4));
+            if (a.piece_heads == 1) hipLaunchKernelGGL((dagg_fwd_kernel<T, VEC, true>), grid, block, lds, stream, a);
+            else hipLaunchKernelGGL((dagg_fwd_kernel<T, VEC, false>), grid, block, lds, stream, a);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidConfiguration;
+        }
+    });
+}
+
+template <typename T>
+hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
+{
+    hipError_t e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
+        constexpr int VEC = decltype(v)::value;
+        if constexpr (VEC * sizeof(T) <= 16) {
+            const size_t lds = kDaggWaves * (kFoundBytes + kOffBytes + kWave * 16 + kWave * 8);
+            hipLaunchKernelGGL((dagg_dots_kernel<T, VEC>), dim3(a.map.grid), dim3(kDaggWaves * kWave), lds, stream, a);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidConfiguration;
+        }
+    });
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(dagg_sort_kernel<T>, dim3((unsigned)(a.bs * a.nl * a.sort_ranges)), dim3(1024), 0, stream, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.C), [&](auto v) {
+        constexpr int VEC = decltype(v)::value;
+        if constexpr (VEC * sizeof(T) <= 16) {
+            // enough workgroups to fill the chip eight times over, or a strip per unit
+            const int units = 256 >> a.row_lpr_log2;
+            int64_t blocks = ((int64_t)a.bs * ((a.nf + kDaggStrip - 1) / kDaggStrip + a.nl) * a.row_blocks + units - 1) / units;
+            if (blocks > 256 * 32) blocks = 256 * 32;
+            if (a.hd % VEC == 0)
+                hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+            else
+                hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidConfiguration;
+        }
+    });
+    if (e != hipSuccess) return e;
+    const unsigned rounding = sizeof(T) == 2 ? 512u : 0u;
+    hipLaunchKernelGGL(dagg_finish_kernel<T>, dim3((unsigned)(a.bs * a.A) + rounding), dim3(256), (size_t)((a.nloc + 1) & ~1) * 2, stream, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_dagg_forward(int dtype, const DaggArgs& a, hipStream_t stream)
+{
+    switch (dtype) {
+        case MXD_DTYPE_F32: return forward_t<float>(a, stream);
+        case MXD_DTYPE_F16: return forward_t<f16_t>(a, stream);
+        case MXD_DTYPE_BF16: return forward_t<bf16_t>(a, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_dagg_backward(int dtype, const DaggArgs& a, hipStream_t stream)
+{
+    switch (dtype) {
+        case MXD_DTYPE_F32: return backward_t<float>(a, stream);
+        case MXD_DTYPE_F16: return backward_t<f16_t>(a, stream);
+        case MXD_DTYPE_BF16: return backward_t<bf16_t>(a, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace mxd

@@ -80,9 +80,9 @@ hipError_t launch_round_rows(int dtype, const KArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-// deformable aggregation: grad_location[i] = sum over heads of the per-head partial images
+// fused form: gradient of the reference points[i] = sum over heads of the per-head partial images
 template <typename T>
-__global__ __launch_bounds__(256) void dagg_sum_heads_kernel(const float* part, T* dst, size_t n, int nh)
+__global__ __launch_bounds__(256) void sum_heads_kernel(const float* part, T* dst, size_t n, int nh)
 {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -99,11 +99,11 @@ hipError_t launch_sum_heads(int dtype, const float* part, void* dst, size_t n, i
     if (blocks > 256 * 16) blocks = 256 * 16;
     const dim3 grid((unsigned)blocks), block(256);
     if (dtype == MXD_DTYPE_F32)
-        hipLaunchKernelGGL(dagg_sum_heads_kernel<float>, grid, block, 0, stream, part, static_cast<float*>(dst), n, nh);
+        hipLaunchKernelGGL(sum_heads_kernel<float>, grid, block, 0, stream, part, static_cast<float*>(dst), n, nh);
     else if (dtype == MXD_DTYPE_F16)
-        hipLaunchKernelGGL(dagg_sum_heads_kernel<f16_t>, grid, block, 0, stream, part, static_cast<f16_t*>(dst), n, nh);
+        hipLaunchKernelGGL(sum_heads_kernel<f16_t>, grid, block, 0, stream, part, static_cast<f16_t*>(dst), n, nh);
     else if (dtype == MXD_DTYPE_BF16)
-        hipLaunchKernelGGL(dagg_sum_heads_kernel<bf16_t>, grid, block, 0, stream, part, static_cast<bf16_t*>(dst), n, nh);
+        hipLaunchKernelGGL(sum_heads_kernel<bf16_t>, grid, block, 0, stream, part, static_cast<bf16_t*>(dst), n, nh);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -222,9 +222,9 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     // their dots are reduced: for the first kKeep of them (all, with up to 8 units per wavefront)
     // fractions, weight, first pixel and validity bits stay in registers until then instead of being
     // derived from the location a second time.
-    // (Only for the plain operator and deformable aggregation: the other sample sources run with fewer registers
-    // and more wavefronts per SIMD without it, which is worth more to them.)
-    constexpr int kLaneSamples = 4, kKeep = (SRC == kSrcPlain || SRC == kSrcDagg) ? 2 : 0, kKeepRegs = kKeep > 0 ? kKeep : 1;
+    // (Only for the plain operator: the other sample sources run with fewer registers and more wavefronts per SIMD
+    // without it, which is worth more to them.)
+    constexpr int kLaneSamples = 4, kKeep = SRC == kSrcPlain ? 2 : 0, kKeepRegs = kKeep > 0 ? kKeep : 1;
     constexpr int kUnroll = kKeep > 0 ? kLaneSamples : 1;  // (registers are indexed by ks: unrolled)
     float keep_lw[kKeepRegs], keep_lh[kKeepRegs], keep_aw[kKeepRegs];
     int32_t keep_pix[kKeepRegs];
@@ -265,8 +265,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             const bool active = rd.active;
             const float x = rd.x, y = rd.y, aw = rd.aw;
             const int l = rd.l;
-            const bool inside = SRC != kSrcDagg || (x > 0.0f && x < 1.0f && y > 0.0f && y < 1.0f);
-            const Sample sm = source_geometry<SRC>(x, y, lvl[l], a.nk, active && inside, a.grid);
+            const Sample sm = source_geometry<SRC>(x, y, lvl[l], a.nk, active, a.grid);
             Entry en;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -365,8 +364,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 if constexpr (FUSED)
                     fused_location(a, static_cast<const T*>(a.ref) + (((int64_t)wk.b * a.nq + wk.q_begin + qr) * a.nl + l) * a.ref_dim,
                                    lvl[l], cx, cy);
-                const bool inside = SRC != kSrcDagg || (cx > 0.0f && cx < 1.0f && cy > 0.0f && cy < 1.0f);
-                sm = source_geometry<SRC>(cx, cy, lvl[l], a.nk, inside, a.grid);
+                sm = source_geometry<SRC>(cx, cy, lvl[l], a.nk, true, a.grid);
             }
             bool have[2], keep[2];
             int32_t key[2];
@@ -638,8 +636,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                             fused_location(a, ref + (((int64_t)wk.b * a.nq + q) * a.nl + l) * a.ref_dim, lvl[l], x, y);
                             aw = expf(aw - unit_stats(u)[0]) / unit_stats(u)[1];
                         }
-                        const bool inside = SRC != kSrcDagg || (x > 0.0f && x < 1.0f && y > 0.0f && y < 1.0f);
-                        sm = source_geometry<SRC>(x, y, lvl[l], a.nk, inside, a.grid);
+                        sm = source_geometry<SRC>(x, y, lvl[l], a.nk, true, a.grid);
                     }
                     const T* rp = nullptr;
                     if constexpr (FUSED) rp = ref + (((int64_t)wk.b * a.nq + q) * a.nl + l) * a.ref_dim;
@@ -695,25 +692,6 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                         }
                     } else if constexpr (SRC != kSrcGrid) __builtin_nontemporal_store(from_f32<T>(ga), gattn + sr.w_e);
                     if constexpr (FUSED) {
-                    } else if constexpr (SRC == kSrcDagg) {
-                        // one location serves the scales of its camera and every head: sum over the
-                        // scales here (neighbouring lanes), per head into a float32 partial image that a
-                        // small kernel adds up over the heads afterwards
-                        float* part = reinterpret_cast<float*>(a.grad_loc) +
-                                      2 * ((int64_t)wk.h * ((int64_t)a.bs * a.nq * a.np * a.cams) + sr.loc_e);
-                        if (a.sc_pow2) {
-                            for (int d = 1; d < a.scales; d <<= 1) {
-                                gx += __shfl_xor(gx, d, kWave);
-                                gy += __shfl_xor(gy, d, kWave);
-                            }
-                            if ((l & (a.scales - 1)) == 0) {
-                                part[0] = gx;
-                                part[1] = gy;
-                            }
-                        } else {
-                            unsafeAtomicAdd(part, gx);
-                            unsafeAtomicAdd(part + 1, gy);
-                        }
                     } else if constexpr (SRC != kSrcGka) {  // (pixel-index locations have no gradient)
                         // (streamed out like the records: results should not push value rows out of L2)
                         __builtin_nontemporal_store(from_f32<T>(gx), gloc + 2 * sr.loc_e);
@@ -809,11 +787,6 @@ inline hipError_t launch_one(const KArgs& a, bool scatter, hipStream_t stream)
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, true, kSrcGka>), grid, block, a.plan.lds_bytes, stream, a);
         else
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcGka>), grid, block, a.plan.lds_bytes, stream, a);
-    } else if (a.cams > 0) {
-        if (scatter)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, true, kSrcDagg>), grid, block, a.plan.lds_bytes, stream, a);
-        else
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcDagg>), grid, block, a.plan.lds_bytes, stream, a);
     } else if (a.ref != nullptr) {
         if (scatter)
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, true, kSrcFused>), grid, block, a.plan.lds_bytes, stream, a);

@@ -1,7 +1,7 @@
 // C ABI entry points (include/mxd_msda.h): argument checks, launch geometry, enqueue.
 // Host code only; the kernels live in msda_fwd.hip, msda_fwd_cu.hip, msda_bwd_kernel.h (with msda_bwd*.hip) and msda_bwd_tiles.hip.  Multi-scale
-// deformable attention, its fused form, deformable aggregation and geometric kernel attention are the same
-// three kernels with different sample sources (msda_device.h: sample_ref, source_geometry).
+// deformable attention, its fused form, geometric kernel attention and the grid sampler are the same three kernels with
+// different sample sources (msda_device.h: sample_ref, source_geometry); deformable aggregation has its own (dagg.hip).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdarg.h>
@@ -12,6 +12,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "dagg.h"
 #include "msda_device.h"
 
 namespace mxd {
@@ -289,7 +290,7 @@ int backward_lane_bytes(int dtype, const Dims& d)
 // wavefront, 4 wavefronts), 32 otherwise.  MXD_MSDA_BWD_TILE_Q overrides (32/64/128/256).
 static int64_t bwd_tile_q(int dtype, const Dims& d)
 {
-    // (units with very many samples -- deformable aggregation's 312 -- measured 1 to 2 % better with 64)
+    // (units with very many samples measured 1 to 2 % better with 64)
     int vec, lpr, npass;
     row_geometry(elem_size(dtype), d.hd, backward_lane_bytes(dtype, d), &vec, &lpr, &npass, tuning().bwd_two_pass != 0);
     const int64_t least = (mxd::kWave / lpr > 8 || d.nl * d.np >= 256) ? 64 : 32;
@@ -773,38 +774,89 @@ void fill_args(mxd::KArgs* a, int dtype, const Dims& d)
     a->gbatch_bytes = (uint32_t)(d.nk * d.nh * d.hd * 4);
 }
 
-// Deformable aggregation in the terms of the kernels: channel group = head, (camera, scale) = level,
-// anchor = query, points per anchor = points.
-int dagg_dims(int dtype, int64_t bs, int64_t nf, int64_t C, int64_t cams, int64_t scales, int64_t A, int64_t P,
-              int64_t G, Dims* d)
+size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
+
+int log2_lanes(int64_t lanes)
+{
+    int s = 0;
+    while ((int64_t(1) << s) < lanes && s < 6) ++s;
+    return s;
+}
+
+// Checks the sizes of a deformable aggregation and fills in what follows from them.
+int dagg_args(int dtype, int64_t bs, int64_t nf, int64_t C, int64_t cams, int64_t scales, int64_t A, int64_t P, int64_t G,
+              mxd::DaggArgs* a)
 {
     if (G <= 0 || cams <= 0 || scales <= 0 || C <= 0)
         return fail(MXD_E_SHAPE, "Input Tensor can not be a empty Tensor (C=%lld cams=%lld scales=%lld groups=%lld)",
                     (long long)C, (long long)cams, (long long)scales, (long long)G);
     if (C % G != 0) return fail(MXD_E_SHAPE, "num_embeds (%lld) must be a multiple of num_groups (%lld)", (long long)C, (long long)G);
-    *d = Dims{bs, nf, G, C / G, cams * scales, cams * scales, A, P};
-    const int rc = check_dims(dtype, *d);
+    const Dims d{bs, nf, G, C / G, cams * scales, cams * scales, A, P};  // (a group is a head, a (camera, scale) pair a level)
+    const int rc = check_dims(dtype, d);
     if (rc != MXD_OK) return rc;
-    // sample index -> (point, level) by a multiply-shift that is exact while samples * levels < 2^20
-    if (d->nl * d->np * d->nl >= (1 << 20))
-        return fail(MXD_E_SHAPE, "num_pts*(num_cams*num_scale)^2 = %lld is beyond what this build indexes",
-                    (long long)(d->nl * d->np * d->nl));
+    if (A >= (int64_t(1) << 29) || A * P * d.nl >= (int64_t(1) << 31) || bs * A >= (int64_t(1) << 30))
+        return fail(MXD_E_SHAPE, "num_anchors*num_pts*num_cams*num_scale = %lld is beyond what this build indexes", (long long)(A * P * d.nl));
+    memset(a, 0, sizeof(*a));
+    const int es = elem_size(dtype);
+    a->bs = (int32_t)bs;
+    a->nf = (int32_t)nf;
+    a->C = (int32_t)C;
+    a->G = (int32_t)G;
+    a->hd = (int32_t)d.hd;
+    a->cams = (int32_t)cams;
+    a->scales = (int32_t)scales;
+    a->nl = (int32_t)d.nl;
+    a->A = (int32_t)A;
+    a->P = (int32_t)P;
+    a->nloc = (int32_t)(P * cams);
+    a->p_magic = (uint32_t)(((1u << 20) + P - 1) / P);
+    a->sc_magic = (uint32_t)(((1u << 20) + scales - 1) / scales);
+    a->pitch_bytes = (uint32_t)(C * es);
+    a->batch_bytes = (uint32_t)(nf * C * es);
+    const int vec = mxd::dagg_vec(es, C);
+    a->row_lpr_log2 = log2_lanes((C + vec - 1) / vec);
+    a->row_blocks = (int32_t)(((C + vec - 1) / vec + mxd::kWave - 1) / mxd::kWave);
+    a->sort_ranges = (int32_t)((nf + mxd::kDaggSortPx - 1) / mxd::kDaggSortPx);
     return MXD_OK;
 }
 
-void fill_dagg(mxd::KArgs* a, int64_t cams, int64_t scales)
+// Launch geometry of the forward (or of the backward's first kernel): an anchor per wavefront and row piece.
+int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
 {
-    a->cams = (int32_t)cams;
-    a->scales = (int32_t)scales;
-    a->np_magic = (uint32_t)(((1u << 20) + a->nl - 1) / a->nl);  // sample / levels
-    a->sc_magic = (uint32_t)(((1u << 20) + scales - 1) / scales);
-    a->sc_pow2 = (scales & (scales - 1)) == 0 && scales <= 16;
+    // A piece is a group's channels.  In the forward several groups share one where a group's row is short of the 128
+    // bytes of a cache line (float16, groups of 32 channels: a line that two XCDs fetch for half of it each), if the lanes'
+    // channels do not straddle groups; the backward's dot products belong to one group each.
+    int vec = mxd::dagg_vec(es, a->hd);
+    a->piece_ch = a->hd;
+    a->piece_heads = 1;
+    if (!backward && a->hd % vec == 0 && a->hd * es < 128 && a->G > 1) {
+        a->piece_ch = 128 / es < a->C ? 128 / es : a->C;
+        a->piece_heads = a->piece_ch % a->hd == 0 ? a->piece_ch / a->hd : (a->piece_ch - 1) / a->hd + 2;
+    }
+    a->pieces = (a->C + a->piece_ch - 1) / a->piece_ch;
+    a->lpr_log2 = log2_lanes((a->piece_ch + vec - 1) / vec);
+    a->map.tile_q = mxd::kDaggWaves;
+    const int64_t grid = fill_xcd_map(&a->map, a->bs, a->pieces, (a->A + mxd::kDaggWaves - 1) / mxd::kDaggWaves);
+    if (grid >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs %lld workgroups, beyond the launch limit", (long long)grid);
+    if ((int64_t)a->bs * a->nl * a->sort_ranges >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs too many workgroups");
+    a->map.grid = (uint32_t)grid;
+    return MXD_OK;
 }
 
-size_t dagg_part_bytes(const Dims& d, int64_t cams)
-{
-    return (size_t)d.nh * d.bs * d.nq * d.np * cams * 2 * sizeof(float);
-}
+// Workspace of the backward: {weights' gradients per group, location gradients per group, record starts, records, float32
+// image of grad_mc_ms_feat for 16-bit dtypes}.
+struct DaggSpace {
+    size_t gl, csr, rec, image, total;
+    DaggSpace(const mxd::DaggArgs& a, int es)
+    {
+        const size_t locs = (size_t)a.bs * a.A * a.nloc;
+        gl = round_up((size_t)a.G * locs * a.scales * 4, 256);
+        csr = gl + round_up((size_t)a.G * locs * 8, 256);
+        rec = csr + round_up((size_t)a.bs * ((size_t)a.nf + a.nl) * 4, 256);
+        image = rec + (size_t)a.bs * a.nl * 2 * a.A * a.P * 16;
+        total = image + (es == 2 ? (size_t)a.bs * a.nf * a.C * 4 : 0);
+    }
+};
 
 }  // namespace
 
@@ -1223,27 +1275,20 @@ int mxd_dagg_forward(const void* mc_ms_feat, const int32_t* spatial_shape, const
                      int64_t num_pts, int64_t num_groups, void* hip_stream)
 {
     const int meta64 = take_meta_flag(&dtype);
-    Dims d;
-    int rc = dagg_dims(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &d);
+    mxd::DaggArgs a;
+    int rc = dagg_args(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &a);
+    if (rc == MXD_OK && (!mc_ms_feat || !spatial_shape || !scale_start_index || !sampling_location || !weights || !output))
+        rc = fail(MXD_E_NULL, "mxd_dagg_forward: NULL data pointer");
+    if (rc == MXD_OK) rc = dagg_plan(&a, elem_size(dtype), false);
     if (rc != MXD_OK) return rc;
-    if (!mc_ms_feat || !spatial_shape || !scale_start_index || !sampling_location || !weights || !output)
-        return fail(MXD_E_NULL, "mxd_dagg_forward: NULL data pointer");
-    int align = ptr_align(mc_ms_feat);
-    if (ptr_align(output) < align) align = ptr_align(output);
-    mxd::KArgs a;
-    memset(&a, 0, sizeof(a));
-    rc = make_plan(0, dtype, d, align, &a.plan);
-    if (rc != MXD_OK) return rc;
-    fill_args(&a, dtype, d);
     a.meta_i64 = meta64;
-    fill_dagg(&a, num_cams, num_scale);
-    a.value = mc_ms_feat;
+    a.feat = mc_ms_feat;
     a.shapes = spatial_shape;
     a.lsi = scale_start_index;
     a.loc = sampling_location;
-    a.attn = weights;
+    a.w = weights;
     a.out = output;
-    const hipError_t e = mxd::launch_forward(dtype, a, static_cast<hipStream_t>(hip_stream));
+    const hipError_t e = mxd::launch_dagg_forward(dtype, a, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_forward: launch failed: %s", hipGetErrorString(e));
     return MXD_OK;
 }
@@ -1252,10 +1297,9 @@ size_t mxd_dagg_backward_workspace_bytes(int dtype, int64_t bs, int64_t num_feat
                                          int64_t num_scale, int64_t num_anchors, int64_t num_pts, int64_t num_groups)
 {
     take_meta_flag(&dtype);
-    Dims d;
-    if (dagg_dims(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &d) != MXD_OK)
-        return 0;
-    return bwd_layout(dtype, d).total + dagg_part_bytes(d, num_cams);
+    mxd::DaggArgs a;
+    if (dagg_args(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &a) != MXD_OK) return 0;
+    return DaggSpace(a, elem_size(dtype)).total;
 }
 
 int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, const int32_t* scale_start_index,
@@ -1266,82 +1310,40 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
                       void* hip_stream)
 {
     const int meta64 = take_meta_flag(&dtype);
-    Dims d;
-    int rc = dagg_dims(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &d);
+    mxd::DaggArgs a;
+    int rc = dagg_args(dtype, bs, num_feat, num_embeds, num_cams, num_scale, num_anchors, num_pts, num_groups, &a);
     if (rc != MXD_OK) return rc;
     if (!mc_ms_feat || !spatial_shape || !scale_start_index || !sampling_location || !weights || !grad_output ||
         !grad_mc_ms_feat || !grad_sampling_location || !grad_weights)
         return fail(MXD_E_NULL, "mxd_dagg_backward: NULL data pointer");
-    int align = ptr_align(mc_ms_feat);
-    if (ptr_align(grad_output) < align) align = ptr_align(grad_output);
-    mxd::KArgs a;
-    memset(&a, 0, sizeof(a));
-    rc = make_plan(1, dtype, d, align, &a.plan);
+    const int es = elem_size(dtype);
+    rc = dagg_plan(&a, es, true);
     if (rc != MXD_OK) return rc;
-    const BwdLayout L = bwd_layout(dtype, d);  // (as make_plan laid the first kernel's LDS out)
-    const size_t part_bytes = dagg_part_bytes(d, num_cams);
-    const size_t need = L.total + part_bytes;
-    if (!workspace || workspace_bytes < need)
-        return fail(MXD_E_WORKSPACE, "mxd_dagg_backward: workspace of %zu bytes required, %zu given", need,
+    const DaggSpace space(a, es);
+    if (!workspace || workspace_bytes < space.total)
+        return fail(MXD_E_WORKSPACE, "mxd_dagg_backward: workspace of %zu bytes required, %zu given", space.total,
                     workspace ? workspace_bytes : (size_t)0);
     if (reinterpret_cast<uintptr_t>(workspace) & 15u)
         return fail(MXD_E_WORKSPACE, "mxd_dagg_backward: workspace must be 16-byte aligned");
-    const bool half = elem_size(dtype) == 2;
     char* ws = static_cast<char*>(workspace);
-    float* image = half ? reinterpret_cast<float*>(ws + L.tbl_bytes + L.rec_bytes) : static_cast<float*>(grad_mc_ms_feat);
-    float* part = reinterpret_cast<float*>(ws + L.total);
-    if (reinterpret_cast<uintptr_t>(image) & 3u) return fail(MXD_E_SHAPE, "mxd_dagg_backward: grad_mc_ms_feat is not 4-byte aligned");
-    fill_args(&a, dtype, d);
-    a.tile_px_log2 = L.tile_px_log2;
-    a.unit_split_log2 = unit_split_log2(a.plan);
-    a.rec_lds_bytes = plan_record_buffer(&a.plan, L, d, dtype, false, a.unit_split_log2);
     a.meta_i64 = meta64;
-    fill_dagg(&a, num_cams, num_scale);
-    a.value = mc_ms_feat;
+    a.feat = mc_ms_feat;
     a.shapes = spatial_shape;
     a.lsi = scale_start_index;
     a.loc = sampling_location;
-    a.attn = weights;
+    a.w = weights;
     a.grad_out = grad_output;
-    a.grad_value = image;
-    a.tbl = reinterpret_cast<uint32_t*>(ws);
-    a.rec = reinterpret_cast<uint32_t*>(ws + L.tbl_bytes);
-    a.nwg = (int32_t)L.nwg;
-    a.run_step = run_step(L.nwg);
-    a.rec_cap = (int32_t)L.rec_cap;
-    a.tbl_stride = (int32_t)L.tbl_stride;
-    a.grad_loc = part;  // per-head partial images, summed below
-    a.grad_attn = grad_weights;
-    hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-    const size_t n = (size_t)bs * num_feat * num_embeds;
-    // every step that can fail for the sizes given comes before the first launch
-    const bool atomic_mode = !L.tiles;
-    mxd::TileArgs t;
-    if (!atomic_mode) {
-        rc = make_tile_args(d, L, 0, &t);
-        if (rc != MXD_OK) return rc;
-        plan_image(&a, &t, half, false, image, grad_mc_ms_feat, d.hd);
-    }
-    hipError_t e = hipSuccess;
-    if (L.tiles && n % 4 == 0 && (reinterpret_cast<uintptr_t>(image) & 15u) == 0 && tuning().bwd_fill_kernel == 0)
-        a.fill_n4 = n / 4;  // zero-filled by the first kernel's workgroups
-    else
-        e = mxd::launch_fill_zero(image, n, stream);
-    if (e == hipSuccess && !a.sc_pow2) e = mxd::launch_fill_zero(part, part_bytes / sizeof(float), stream);
-    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: zero-fill launch failed: %s", hipGetErrorString(e));
-    e = mxd::launch_backward(dtype, a, atomic_mode, stream);
+    a.grad_feat = grad_mc_ms_feat;
+    a.grad_loc = grad_sampling_location;
+    a.grad_w = grad_weights;
+    a.image = es == 2 ? reinterpret_cast<float*>(ws + space.image) : static_cast<float*>(grad_mc_ms_feat);
+    if (reinterpret_cast<uintptr_t>(a.image) & 3u) return fail(MXD_E_SHAPE, "mxd_dagg_backward: grad_mc_ms_feat is not 4-byte aligned");
+    a.gw_part = reinterpret_cast<float*>(ws);
+    a.gl_part = reinterpret_cast<float*>(ws + space.gl);
+    a.csr = reinterpret_cast<uint32_t*>(ws + space.csr);
+    a.rec = reinterpret_cast<mxd::u32x4*>(ws + space.rec);
+    const hipError_t e = mxd::launch_dagg_backward(dtype, a, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: launch failed: %s", hipGetErrorString(e));
-    if (!atomic_mode) {
-        e = mxd::launch_gradv_tiles(dtype, a, t, stream);
-        if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: tile kernel launch failed: %s", hipGetErrorString(e));
-    }
-    if (half) {
-        e = a.sparse ? mxd::launch_round_rows(dtype, a, stream) : mxd::launch_round(dtype, image, grad_mc_ms_feat, n, stream);
-        if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: rounding launch failed: %s", hipGetErrorString(e));
-    }
-    e = mxd::launch_sum_heads(dtype, part, grad_sampling_location, (size_t)bs * num_anchors * num_pts * num_cams * 2,
-                              (int)num_groups, stream);
-    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: head sum launch failed: %s", hipGetErrorString(e));
     return MXD_OK;
 }
 

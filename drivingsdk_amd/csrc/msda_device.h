@@ -31,20 +31,12 @@ struct KArgs {
     // the kernel), and the sampling location is reference point + offset / normaliser
     const void* ref;       // [bs, nq, nl, ref_dim] reference points
     int32_t ref_dim;       // 2: (x, y); 4: (x, y, w, h) boxes
-    // deformable aggregation only (source = kSrcDagg): a level is a (camera, scale) pair, nl = cams*scales,
-    // np = points per anchor, sample s = point*nl + level; `loc` is [bs, nq, np, cams, 2] (shared by the
-    // scales of a camera and by all heads = channel groups), `attn` is [bs, nq, np, cams, scales, nh]
-    int32_t cams;
-    int32_t scales;
-    uint32_t sc_magic;     // ceil(2^20/scales): level / scales
     int32_t lds_cache_bytes;  // forward: LDS set aside for the rows of the last (coarsest) levels, 0 = none
     int32_t fwd_ahead;        // forward: request an iteration's samples before the gather of the one before it
     int32_t fwd_cu_flip;      // forward, one workgroup per CU: half of the wavefronts take their LDS groups first
     int32_t grid_h, grid_w;  // grid sampler: the one level's shape comes with the call, not from device memory
     int32_t grid;          // grid sampler: 1 + padding mode (0 zeros, 1 border) + 2*align_corners; 0 = not a grid sampler
     int32_t gka;           // geometric kernel attention: locations are pixel indices, one pixel per sample
-    int32_t sc_pow2;       // scales is a power of two that divides 16: location gradients are summed over the
-                           // scales across lanes and stored once; otherwise they are added with atomics
     const void* grad_out;  // backward only from here
     float* grad_value;     // fp32 accumulation image of grad_value
     uint64_t fill_n4;      // first backward kernel, tile mode: 16-byte pieces of the image its workgroups zero-fill
@@ -206,7 +198,7 @@ __device__ inline bool atomic_rows_of_part(const KArgs& a, int32_t tile, int32_t
 }
 
 // Where a kernel takes the location and the weight of sample s of unit (b, q, h) from.
-enum : int { kSrcPlain = 0, kSrcFused = 1, kSrcDagg = 2, kSrcGka = 3, kSrcGrid = 4 };
+enum : int { kSrcPlain = 0, kSrcFused = 1, kSrcGka = 2, kSrcGrid = 3 };
 struct SampleRef {
     int64_t loc_e;  // index of the (x, y) pair
     int64_t w_e;    // index of the weight
@@ -216,16 +208,8 @@ template <int SRC>
 __device__ inline SampleRef sample_ref(const KArgs& a, int b, int q, int h, int s)
 {
     SampleRef r;
-    if constexpr (SRC == kSrcDagg) {
-        const int p = (int)(((uint32_t)s * a.np_magic) >> 20);  // s / nl (np_magic is built for the divisor nl here)
-        r.l = s - p * a.nl;
-        const int cam = (int)(((uint32_t)r.l * a.sc_magic) >> 20);
-        r.loc_e = (((int64_t)b * a.nq + q) * a.np + p) * a.cams + cam;
-        r.w_e = (((int64_t)b * a.nq + q) * a.S + s) * a.nh + h;
-    } else {
-        r.loc_e = r.w_e = (((int64_t)b * a.nq + q) * a.nh + h) * a.S_full + s;
-        r.l = (int)(((uint32_t)s * a.np_magic) >> 20);
-    }
+    r.loc_e = r.w_e = (((int64_t)b * a.nq + q) * a.nh + h) * a.S_full + s;
+    r.l = (int)(((uint32_t)s * a.np_magic) >> 20);
     return r;
 }
 
@@ -400,6 +384,22 @@ struct RowIO {
             v[0] = to_f32(*p);
         } else {
             const vec_t t = *reinterpret_cast<const mem_t*>(p);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) v[i] = to_f32<T>(t[i]);
+        }
+    }
+    // a piece as it was loaded (unpacked where it is used)
+    typedef typename std::conditional<VEC == 1, T, vec_t>::type held_t;
+    static __device__ inline held_t load_held(const T* p)
+    {
+        if constexpr (VEC == 1) return *p;
+        else return *reinterpret_cast<const mem_t*>(p);
+    }
+    static __device__ inline void unpack_held(held_t t, float (&v)[VEC])
+    {
+        if constexpr (VEC == 1) {
+            v[0] = to_f32(t);
+        } else {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) v[i] = to_f32<T>(t[i]);
         }

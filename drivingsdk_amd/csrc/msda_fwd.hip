@@ -27,10 +27,6 @@
 // offset / (W, H)  [2-d reference points]  or  + offset / np * (w, h) * 0.5  [boxes].
 // The normalised locations and weights then never exist in memory.
 //
-// SRC = kSrcDagg is deformable aggregation (reference: mx_driving/ops/npu_deformable_aggregation.py,
-// kernels/deformable_aggregation/): the same sum with a channel group as head, a (camera, scale) pair as
-// level, one location per (anchor, point, camera) shared by scales and groups, weights laid out
-// [.., point, camera, scale, group], and samples counted only strictly inside (0, 1) x (0, 1).
 // SRC = kSrcGka: geometric kernel attention (the location is a clamped pixel index, one row per sample).
 // SRC = kSrcGrid: bilinear 2-D grid sampler (one level, one head, one point, weight 1, grid coordinates).
 #include "msda_device.h"
@@ -159,9 +155,7 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
     };
     auto place = [&](const RawSample& r, int i) {
         const int sl = i & (kChunk - 1);
-        // deformable aggregation samples only strictly inside the image (0 < x, y < 1)
-        const bool inside = SRC != kSrcDagg || (r.x > 0.0f && r.x < 1.0f && r.y > 0.0f && r.y < 1.0f);
-        const Sample sm = source_geometry<SRC>(r.x, r.y, lvl[r.l], a.nk, r.active && inside, a.grid);
+        const Sample sm = source_geometry<SRC>(r.x, r.y, lvl[r.l], a.nk, r.active, a.grid);
         Entry en;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -302,8 +296,6 @@ static hipError_t launch_one(const KArgs& a, hipStream_t stream)
         hipLaunchKernelGGL((msda_fwd_kernel<T, VEC, NPASS, kSrcGrid, false>), grid, block, a.plan.lds_bytes, stream, a);
     else if (a.gka)
         hipLaunchKernelGGL((msda_fwd_kernel<T, VEC, NPASS, kSrcGka, false>), grid, block, a.plan.lds_bytes, stream, a);
-    else if (a.cams > 0)
-        hipLaunchKernelGGL((msda_fwd_kernel<T, VEC, NPASS, kSrcDagg, false>), grid, block, a.plan.lds_bytes, stream, a);
     else if (a.ref != nullptr)
         hipLaunchKernelGGL((msda_fwd_kernel<T, VEC, NPASS, kSrcFused, false>), grid, block, a.plan.lds_bytes, stream, a);
     else {

@@ -1,0 +1,53 @@
+"""Deformable aggregation at the sizes where its kernels change course, against the oracle: groups narrower and wider than a cache
+line and than a lane's piece, more locations than a wavefront looks through at once, scale counts that do not divide 64, levels
+with so few pixels that their records are split, levels larger than one sort workgroup counts, and level starts that do not
+tile the features (rows shared by two levels, rows of none)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dagg_oracle as dagg
+from test_dagg_gpu import check, make_inputs, run_gpu
+from util import BWD_FP32, FWD_FP32, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("C,G", [(16, 4), (40, 8), (32, 8), (64, 16), (80, 4), (256, 8), (36, 2), (37, 1), (6, 3), (512, 8), (520, 4), (128, 128)])
+def test_group_widths(gpu_device, C, G):
+    print(check(make_inputs(2, C, G, 21, 5, [[(9, 13), (5, 7)]] * 2, seed=C, pad=True), gpu_device))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("C,G", [(256, 8), (32, 8), (40, 8), (36, 2), (12, 2)])
+def test_group_widths_16_bit(gpu_device, C, G, dtype):
+    inp = [np.asarray(torch.from_numpy(t).to(dtype).float()) if t.dtype == np.float32 else t
+           for t in make_inputs(2, C, G, 21, 5, [[(9, 13), (2, 3)]] * 2, seed=C, pad=True)]
+    want = (dagg.direct_forward(*inp[:5]),) + dagg.direct_backward(*inp)
+    tol = {torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
+    for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
+        assert rel_err(g, r) <= tol, k
+
+
+@pytest.mark.parametrize("P,cams,scales", [(1, 1, 1), (65, 1, 1), (43, 3, 3), (130, 2, 1), (7, 5, 7), (2, 1, 40)])
+def test_location_and_scale_counts(gpu_device, P, cams, scales):
+    print(check(make_inputs(1, 32, 4, 9, P, [[(6 + s % 3, 7) for s in range(scales)]] * cams, seed=P, pad=True), gpu_device))
+
+
+def test_few_pixels_many_records(gpu_device):
+    print(check(make_inputs(2, 64, 8, 700, 13, [[(11, 12), (2, 3), (1, 1)]], seed=8, pad=True), gpu_device))
+
+
+def test_a_level_of_several_sort_ranges(gpu_device):
+    print(check(make_inputs(1, 16, 2, 150, 9, [[(130, 197), (33, 50)]], seed=9), gpu_device))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_levels_that_do_not_tile_the_features(gpu_device, dtype):
+    feat, ss, ssi, loc, w, go = make_inputs(2, 32, 4, 33, 5, [[(9, 13), (5, 7)]], seed=10, pad=True)
+    feat = np.concatenate([feat, feat[:, :20]], 1)          # rows that no level covers
+    ssi = np.array([[3, 3 + 60]], dtype=np.int32)           # the second level starts inside the first
+    inp = (feat, ss, ssi, loc, w, go)
+    want = (dagg.direct_forward(*inp[:5]),) + dagg.direct_backward(*inp)
+    for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
+        assert rel_err(g, r) <= ((FWD_FP32 if k == 0 else BWD_FP32) if dtype == torch.float32 else 4e-3), k
