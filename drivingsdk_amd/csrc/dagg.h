@@ -6,7 +6,7 @@ namespace mxd {
 
 constexpr int kDaggWaves = 4;        // wavefronts per workgroup of the forward and of the backward's first kernel: an anchor each
 constexpr int kDaggList = 128;       // locations of an anchor that a wavefront looks through before it samples
-constexpr int kDaggSortPx = 12288;   // pixels of a level that a workgroup of the sort counts in LDS
+constexpr int kDaggSortPx = 4096;    // pixels of a level that a workgroup of the sort counts in LDS
 constexpr int kDaggStrip = 8;        // neighbouring pixels whose gradient rows are formed together
 constexpr int kDaggStripRecords = 1024;  // records per strip aimed at where the strips of a level are split
 

@@ -178,13 +178,14 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
 }
 
 // ---- backward, first kernel: gradients of the weights and locations, per group ---------------------------------------------
+// LDS per wavefront: found locations, row offsets, dots, location gradients
+constexpr int kDotsLds = kFoundBytes + kOffBytes + kWave * 16 + kWave * 8;
+
 template <typename T, int VEC>
-__global__ __launch_bounds__(kDaggWaves * kWave) void dagg_dots_kernel(const DaggArgs a)
+__device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned char* smem, i32x4* lvl)
 {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ i32x4 lvl[kMaxLevels];
     Work wk;
-    if (!decode_block(a.map, blockIdx.x, a.bs, a.pieces, a.A, &wk)) return;
+    if (!decode_block(a.map, block, a.bs, a.pieces, a.A, &wk)) return;
     if ((int)threadIdx.x < a.nl) lvl[threadIdx.x] = dagg_level(a, threadIdx.x);
     __syncthreads();
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
@@ -192,8 +193,7 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_dots_kernel(const Dag
     if (q >= wk.q_end) return;
     const int64_t anchor = (int64_t)wk.b * a.A + q;
 
-    constexpr int kPerWave = kFoundBytes + kOffBytes + kWave * 16 + kWave * 8;
-    unsigned char* mine = smem + wave * kPerWave;
+    unsigned char* mine = smem + wave * kDotsLds;
     Found* found = reinterpret_cast<Found*>(mine);
     u32x4* off = reinterpret_cast<u32x4*>(mine + kFoundBytes);
     f32x4* dots = reinterpret_cast<f32x4*>(mine + kFoundBytes + kOffBytes);
@@ -363,38 +363,43 @@ struct DaggLevels {
 
 // ---- sort of the corner pairs by pixel -------------------------------------------------------------------------------------
 // One workgroup per (batch, level, range of kDaggSortPx pixels): counts the records of every pixel in LDS, turns the counts
-// into starts, and drops every record at its place.  10 us of a training step of 1.9 M samples.
+// into starts, and drops every record at its place.
+struct DaggSort {
+    DaggLevels lv;
+    uint32_t wsum[kDaggWaves];
+    uint32_t before_s;
+    uint32_t cnt[kDaggSortPx];
+};
 template <typename T>
-__global__ __launch_bounds__(1024) void dagg_sort_kernel(const DaggArgs a)
+__device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, uint32_t blocks, unsigned char* smem)
 {
-    __shared__ DaggLevels lv;
-    __shared__ uint32_t cnt[kDaggSortPx];
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t before_s;
+    constexpr int kThreads = kDaggWaves * kWave;
+    DaggSort& sh = *reinterpret_cast<DaggSort*>(smem);
+    DaggLevels& lv = sh.lv;
+    uint32_t *cnt = sh.cnt, *wsum = sh.wsum, &before_s = sh.before_s;
     lv.fill(a);
-    const int range = blockIdx.x % a.sort_ranges, l = blockIdx.x / a.sort_ranges % a.nl, b = blockIdx.x / a.sort_ranges / a.nl;
+    const int range = block % a.sort_ranges, l = block / a.sort_ranges % a.nl, b = block / a.sort_ranges / a.nl;
     const int tid = threadIdx.x;
     const int r0 = range * kDaggSortPx, P = lv.px[l], r1 = P - r0 < kDaggSortPx ? P : r0 + kDaggSortPx;
     if (!lv.tiled) {
         // rows that several levels share or none has: the whole image gets zeros, and every row is added to
-        const uint64_t n = (uint64_t)a.bs * a.nf * a.C, per = (n + gridDim.x - 1) / gridDim.x;
-        const uint64_t lo = blockIdx.x * per, hi = lo + per < n ? lo + per : n;
+        const uint64_t n = (uint64_t)a.bs * a.nf * a.C, per = (n + blocks - 1) / blocks;
+        const uint64_t lo = block * per, hi = lo + per < n ? lo + per : n;
         for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
-    } else if (lv.chunks[l] > 1 && r0 < P) {
+    } else if (b < a.bs && lv.chunks[l] > 1 && r0 < P) {
         const uint64_t lo = ((uint64_t)b * a.nf + lv.base[l] + r0) * a.C, hi = lo + (uint64_t)(r1 - r0) * a.C;
         for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
     }
-    if (r0 >= P) return;  // (uniform)
-    for (int i = tid; i < kDaggSortPx; i += 1024) cnt[i] = 0;
+    if (b >= a.bs || r0 >= P) return;  // (uniform; the launch has a multiple of 8 sort workgroups)
+    for (int i = tid; i < kDaggSortPx; i += kThreads) cnt[i] = 0;
     if (tid == 0) before_s = 0;
     __syncthreads();
 
     const int cam = l / a.scales, sc = l - cam * a.scales;
     const i32x4 level = {lv.H[l], lv.W[l], lv.base[l], 0};
     const uint32_t points = (uint32_t)a.A * (uint32_t)a.P;
-    // the records of a point on this level: (key, weights) of up to two
-    auto each_record = [&](uint32_t i, auto take) {
-        const f32x2 xy = load_xy<T>(a.loc, ((int64_t)b * points + i) * a.cams + cam);
+    // the records of a location on this level: (key, weights) of up to two
+    auto each_record = [&](const f32x2 xy, auto take) {
         if (!inside(xy.x, xy.y)) return;
         const Sample sm = sample_geometry(xy.x, xy.y, level, a.nf, true);
 #pragma unroll
@@ -404,23 +409,35 @@ __global__ __launch_bounds__(1024) void dagg_sort_kernel(const DaggArgs a)
                 take((vl ? sm.pix[2 * r] : sm.pix[2 * r + 1]) - level.z, vl ? sm.w[2 * r] : sm.w[2 * r + 1], vl && vr ? sm.w[2 * r + 1] : 0.0f);
         }
     };
+    // eight points' locations are requested together: one at a time, the two passes are a chain of trips to memory
+    constexpr int kTogether = 8;
+    auto each_point = [&](auto take) {
+        for (uint32_t i0 = tid; i0 < points; i0 += kTogether * kThreads) {
+            f32x2 xy[kTogether];
+#pragma unroll
+            for (int k = 0; k < kTogether; ++k) {
+                const uint32_t i = i0 + k * kThreads;
+                xy[k] = i < points ? load_xy<T>(a.loc, ((int64_t)b * points + i) * a.cams + cam) : f32x2{0.f, 0.f};
+            }
+            for (int k = 0; k < kTogether; ++k) {
+                each_record(xy[0], [&](int key, float wa, float wb) { take(i0 + k * kThreads, key, wa, wb); });
+#pragma unroll
+                for (int m = 0; m + 1 < kTogether; ++m) xy[m] = xy[m + 1];
+            }
+        }
+    };
     uint32_t before = 0;  // records of the ranges before this one
-    for (uint32_t i = tid; i < points; i += 1024)
-        each_record(i, [&](int key, float, float) {
-            if (key < r0) ++before;
-            else if (key < r1) atomicAdd(&cnt[key - r0], 1u);
-        });
+    each_point([&](uint32_t, int key, float, float) {
+        if (key < r0) ++before;
+        else if (key < r1) atomicAdd(&cnt[key - r0], 1u);
+    });
     if (r0 > 0 && before != 0) atomicAdd(&before_s, before);
     __syncthreads();
 
-    // exclusive prefix: 12 neighbouring counters per thread, then over the threads
-    constexpr int kPer = kDaggSortPx / 1024;
-    uint32_t mine[kPer], sum = 0;
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        mine[k] = sum;
-        sum += cnt[tid * kPer + k];
-    }
+    // exclusive prefix: neighbouring counters per thread, then over the threads
+    constexpr int kPer = kDaggSortPx / kThreads;
+    uint32_t sum = 0;
+    for (int k = 0; k < kPer; ++k) sum += cnt[tid * kPer + k];
     uint32_t inc = sum;
     const int lane = tid & (kWave - 1), wave = tid >> 6;
 #pragma unroll
@@ -433,23 +450,34 @@ __global__ __launch_bounds__(1024) void dagg_sort_kernel(const DaggArgs a)
     uint32_t at = before_s + inc - sum;
     for (int k = 0; k < wave; ++k) at += wsum[k];
     uint32_t* csr = a.csr + (size_t)b * ((size_t)a.nf + a.nl) + lv.csr[l];
-#pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const int p = tid * kPer + k;
-        cnt[p] = at + mine[k];
-        if (r0 + p < P) csr[r0 + p] = at + mine[k];
-        if (r0 + p == P - 1) csr[P] = at + (k + 1 < kPer ? mine[k + 1 < kPer ? k + 1 : k] : sum);
+        const uint32_t v = cnt[p];
+        cnt[p] = at;
+        if (r0 + p < P) csr[r0 + p] = at;
+        at += v;
+        if (r0 + p == P - 1) csr[P] = at;
     }
     __syncthreads();
 
     u32x4* rec = a.rec + ((size_t)b * a.nl + l) * 2 * points;
-    for (uint32_t i = tid; i < points; i += 1024)
-        each_record(i, [&](int key, float wa, float wb) {
-            if (key < r0 || key >= r1) return;
-            const uint32_t pos = atomicAdd(&cnt[key - r0], 1u);
-            rec[pos] = u32x4{(i / (uint32_t)a.P) << 3 | ((uint32_t)key & 7u), (i * (uint32_t)a.cams + (uint32_t)cam) * (uint32_t)a.scales + (uint32_t)sc,
-                             __builtin_bit_cast(uint32_t, wa), __builtin_bit_cast(uint32_t, wb)};
-        });
+    each_point([&](uint32_t i, int key, float wa, float wb) {
+        if (key < r0 || key >= r1) return;
+        const uint32_t pos = atomicAdd(&cnt[key - r0], 1u);
+        rec[pos] = u32x4{(i / (uint32_t)a.P) << 3 | ((uint32_t)key & 7u), (i * (uint32_t)a.cams + (uint32_t)cam) * (uint32_t)a.scales + (uint32_t)sc,
+                         __builtin_bit_cast(uint32_t, wa), __builtin_bit_cast(uint32_t, wb)};
+    });
+}
+
+// The two kernels side by side in one launch: the sort has work for a few workgroups, whose time the others' gathers cover
+// (131 us as a launch of its own).
+template <typename T, int VEC>
+__global__ __launch_bounds__(kDaggWaves * kWave) void dagg_dots_and_sort_kernel(const DaggArgs a, uint32_t sorts)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ i32x4 lvl[kMaxLevels];
+    if (blockIdx.x < sorts) dagg_sort<T>(a, blockIdx.x, sorts, smem);
+    else dagg_dots<T, VEC>(a, blockIdx.x - sorts, smem, lvl);
 }
 
 // ---- gradient of the feature maps --------------------------------------------------------------------------------------------
@@ -458,11 +486,17 @@ __global__ __launch_bounds__(1024) void dagg_sort_kernel(const DaggArgs a)
 // of the pixel before the strip are met for their right halves.  Every row is stored once, whole (strips split by record
 // number -- levels with few pixels -- add theirs with atomics to rows that the sort has zeroed).
 // MIXED: a lane's channels may belong to several groups.
-template <typename T, int VEC, bool MIXED>
+// WAVE: a unit is a wavefront -- what it reads of records and starts is the same for all lanes and comes through the scalar
+// cache.
+template <typename T, int VEC, bool MIXED, bool WAVE>
 __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
 {
+    // (memory that this kernel does not write, as far as the compiler is concerned: uniform loads become scalar ones)
+    typedef const __attribute__((address_space(4))) u32x4* rec_ptr;
+    typedef const __attribute__((address_space(4))) uint32_t* csr_ptr;
     __shared__ DaggLevels lv;
     lv.fill(a);
+    auto scalar = [](int v) { return WAVE ? __builtin_amdgcn_readfirstlane(v) : v; };
     const int lpr = 1 << a.row_lpr_log2, units = 256 >> a.row_lpr_log2;
     const int c = threadIdx.x & (lpr - 1);
     const uint32_t per_b = (uint32_t)lv.first[a.nl] * (uint32_t)a.row_blocks;
@@ -470,7 +504,8 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
     const T* gout = static_cast<const T*>(a.grad_out);
     const uint32_t points = (uint32_t)a.A * (uint32_t)a.P;
     const uint32_t per_anchor = (uint32_t)a.nloc * (uint32_t)a.scales;
-    for (uint64_t item = (uint64_t)blockIdx.x * units + (threadIdx.x >> a.row_lpr_log2); item < total; item += (uint64_t)gridDim.x * units) {
+    const uint32_t unit = threadIdx.x >> a.row_lpr_log2;
+    for (uint64_t item = (uint64_t)blockIdx.x * units + (WAVE ? (uint32_t)__builtin_amdgcn_readfirstlane((int)unit) : unit); item < total; item += (uint64_t)gridDim.x * units) {
         const int b = (int)(item / per_b);
         const uint32_t r = (uint32_t)(item - (uint64_t)b * per_b);
         const int blk = (int)(r % (uint32_t)a.row_blocks);
@@ -479,10 +514,11 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
         int l = 0;
         for (int s = 32; s > 0; s >>= 1)
             if (l + s < a.nl && lv.first[l + s] <= it) l += s;
-        const int k = it - lv.first[l], chunks = lv.chunks[l], strip = k / chunks, chunk = k - strip * chunks;
-        const int p0 = strip * kDaggStrip, p1 = p0 + kDaggStrip < lv.px[l] ? p0 + kDaggStrip : lv.px[l];
+        l = scalar(l);
+        const int k = scalar(it - lv.first[l]), chunks = scalar(lv.chunks[l]), strip = k / chunks, chunk = k - strip * chunks;
+        const int p0 = strip * kDaggStrip, px_l = scalar(lv.px[l]), p1 = p0 + kDaggStrip < px_l ? p0 + kDaggStrip : px_l;
         const bool direct = lv.direct(l);
-        const uint32_t* csr = a.csr + (size_t)b * ((size_t)a.nf + a.nl) + lv.csr[l];
+        const csr_ptr csr = (csr_ptr)(a.csr + (size_t)b * ((size_t)a.nf + a.nl) + scalar(lv.csr[l]));
         const uint32_t s1 = csr[p0];
         uint32_t lo = p0 > 0 ? csr[p0 - 1] : s1, hi = csr[p1];
         if (chunks > 1) {
@@ -495,7 +531,7 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
         const int ch = chan_ok ? piece_start<VEC>(chn, a.C) : 0;
         const T* grow = gout + (size_t)b * a.A * a.C + ch;
         const T* w = static_cast<const T*>(a.w) + (size_t)b * a.A * per_anchor * a.G + ch / a.hd;
-        const u32x4* rec = a.rec + ((size_t)b * a.nl + l) * 2 * points;
+        const rec_ptr rec = (rec_ptr)(a.rec + ((size_t)b * a.nl + l) * 2 * points);
 
         float acc[VEC], nxt[VEC];
 #pragma unroll
@@ -651,16 +687,16 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
     hipError_t e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
         constexpr int VEC = decltype(v)::value;
         if constexpr (VEC * sizeof(T) <= 16) {
-            const size_t lds = kDaggWaves * (kFoundBytes + kOffBytes + kWave * 16 + kWave * 8);
-            hipLaunchKernelGGL((dagg_dots_kernel<T, VEC>), dim3(a.map.grid), dim3(kDaggWaves * kWave), lds, stream, a);
+            size_t lds = kDaggWaves * kDotsLds;
+            if (lds < sizeof(DaggSort)) lds = sizeof(DaggSort);
+            // (a multiple of 8 sort workgroups: the others keep their places in the XCD mapping)
+            const uint32_t sorts = ((uint32_t)(a.bs * a.nl * a.sort_ranges) + kNumXcd - 1) / kNumXcd * kNumXcd;
+            hipLaunchKernelGGL((dagg_dots_and_sort_kernel<T, VEC>), dim3(sorts + a.map.grid), dim3(kDaggWaves * kWave), lds, stream, a, sorts);
             return hipGetLastError();
         } else {
             return hipErrorInvalidConfiguration;
         }
     });
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(dagg_sort_kernel<T>, dim3((unsigned)(a.bs * a.nl * a.sort_ranges)), dim3(1024), 0, stream, a);
-    e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.C), [&](auto v) {
         constexpr int VEC = decltype(v)::value;
@@ -669,10 +705,10 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
             const int units = 256 >> a.row_lpr_log2;
             int64_t blocks = ((int64_t)a.bs * ((a.nf + kDaggStrip - 1) / kDaggStrip + a.nl) * a.row_blocks + units - 1) / units;
             if (blocks > 256 * 32) blocks = 256 * 32;
-            if (a.hd % VEC == 0)
-                hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-            else
-                hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+            const dim3 grid((unsigned)blocks), block(256);
+            if (a.hd % VEC != 0) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true, false>), grid, block, 0, stream, a);
+            else if (a.row_lpr_log2 == 6) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, true>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, false>), grid, block, 0, stream, a);
             return hipGetLastError();
         } else {
             return hipErrorInvalidConfiguration;
