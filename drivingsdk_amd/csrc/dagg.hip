@@ -552,13 +552,21 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
             for (int e = 0; e < VEC; ++e) acc[e] = nxt[e], nxt[e] = 0.0f;
             ++cur;
         };
-        constexpr int kAhead = 4;  // records whose rows are in flight together
+        // (records whose rows are in flight together; the records after them are requested with those rows, or else every
+        //  batch would be two trips to memory one after the other)
+        constexpr int kAhead = WAVE ? 6 : 4;  // (4, 6, 8, 12 with a wavefront per row: 250, 236, 237, 279 us)
+        u32x4 next[kAhead];
+        auto request = [&](uint32_t e0) {
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) next[j] = rec[e0 + j < hi ? e0 + j : hi - 1];
+        };
+        if (lo < hi) request(lo);
         for (uint32_t e0 = lo; e0 < hi; e0 += kAhead) {
             u32x4 rc[kAhead];
             typename RowIO<T, VEC>::held_t row[kAhead];
             float aw[kAhead][MIXED ? VEC : 1];
 #pragma unroll
-            for (int j = 0; j < kAhead; ++j) rc[j] = rec[e0 + j < hi ? e0 + j : hi - 1];
+            for (int j = 0; j < kAhead; ++j) rc[j] = next[j];
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 row[j] = RowIO<T, VEC>::load_held(grow + (size_t)(rc[j].x >> 3) * a.C);
@@ -570,6 +578,7 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
                     aw[j][0] = to_f32(*wj);
                 }
             }
+            if (e0 + kAhead < hi) request(e0 + kAhead);
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 if (e0 + j >= hi) break;
