@@ -316,8 +316,9 @@ def geometric_kernel_attention_backward(value, spatial_shapes, level_start_index
 # ---- 2-D grid sampler (mx_driving/csrc/GridSampler2dV2.cpp:33-99 of the reference) ------------------------------
 
 def grid_sampler2d_v2(input, grid, interpolation_mode, padding_mode, align_corners):
-    """input [N, C, H, W], grid [N, H_out, W_out, 2] -> output [N, C, H_out, W_out] (bilinear).  As in the reference's
-    binding the kernel works on channel-last data: input is permuted to NHWC before and the output back after.
+    """input [N, C, H, W], grid [N, H_out, W_out, 2] -> output [N, C, H_out, W_out] (bilinear).  A contiguous input of
+    planes that fit the LDS of a compute unit is sampled as it is; otherwise, as in the reference's binding, the kernel works
+    on channel-last data: input is permuted to NHWC before and the output back after.
     An input in torch's channels_last memory format needs no copy and gets its output in that format too (torch's
     convention for memory formats); any other input gets a contiguous NCHW output as in the reference."""
     _check(input.layout == torch.strided and grid.layout == torch.strided,
@@ -335,6 +336,10 @@ def grid_sampler2d_v2(input, grid, interpolation_mode, padding_mode, align_corne
            f"grid_sampler2d_v2(): grid must have size 2 in last dimension, but got grid with sizes {tuple(grid.shape)}")
     _check(input.is_cuda and grid.is_cuda and input.device == grid.device,
            "grid_sampler2d_v2(): input and grid must live on one GPU (this build has no CPU implementation)")
+    if input.is_contiguous():  # planes as they are, where they fit the kernels for planes
+        out = _native.grid_forward(input, grid.contiguous(), int(interpolation_mode), int(padding_mode), int(bool(align_corners)))
+        if out is not None:
+            return out
     n, c, h_in, w_in = input.shape
     _, h_out, w_out, _ = grid.shape
     lib = _lib.load()

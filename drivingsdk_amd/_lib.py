@@ -39,6 +39,10 @@ EXPORTS = (
     "mxd_grid_sampler2d_forward",
     "mxd_grid_sampler2d_backward_workspace_bytes",
     "mxd_grid_sampler2d_backward",
+    "mxd_grid_sampler2d_planes_fit",
+    "mxd_grid_sampler2d_planes_forward",
+    "mxd_grid_sampler2d_planes_backward_workspace_bytes",
+    "mxd_grid_sampler2d_planes_backward",
 )
 
 

@@ -1,0 +1,36 @@
+// Grid sampler on planes (NCHW): arguments of its kernels (grid_planes.hip), filled by the entry points in msda_capi.hip.
+#pragma once
+#include "msda_device.h"
+
+namespace mxd {
+
+constexpr int kGridThreads = 512;           // per workgroup; 1024 where its LDS leaves no room for a second workgroup on the CU
+constexpr int kGridStageBytes = 48 * 1024;  // LDS that several planes of a workgroup share: three workgroups fit a CU
+constexpr int kGridMaxPx = 9;               // output pixels whose sums a thread of the grid's gradient keeps in registers
+
+struct GridArgs {
+    const void* x;         // [n, c, h, w]
+    const void* grid;      // [n, outs, 2]
+    void* out;             // [n, c, outs]
+    const void* grad_out;
+    void* grad_x;          // nullptr: not wanted
+    void* grad_grid;       // nullptr: not wanted
+    float* part;           // [gg_chunks][n, outs, 2]: the gradient of the grid before its sum over the channel chunks
+    int32_t n, c, h, w, outs;
+    int32_t mode;          // 1 + padding mode (0 zeros, 1 border) + 2 * align_corners
+    // forward: planes per workgroup, chunks of them per image, splits of the output pixels
+    int32_t planes, chunks, splits, split_px;
+    // gradient of the maps: planes per workgroup, chunks per image, bands of a large plane and their pixels, workgroups
+    int32_t gx_planes, gx_chunks, gx_bands, gx_band_px, gx_wgs;
+    // gradient of the grid: channels per workgroup, of which so many planes are staged at a time, chunks per image, ranges of
+    // output pixels, output pixels per thread, workgroups
+    int32_t gg_channels, gg_planes, gg_chunks, gg_ranges, gg_px, gg_wgs;
+    int32_t block;
+    uint32_t lds;
+};
+
+hipError_t raise_grid_lds();
+hipError_t launch_grid_planes_forward(int dtype, const GridArgs& a, hipStream_t stream);
+hipError_t launch_grid_planes_backward(int dtype, const GridArgs& a, hipStream_t stream);
+
+}  // namespace mxd

@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "dagg.h"
+#include "grid_planes.h"
 #include "msda_device.h"
 
 namespace mxd {
@@ -161,6 +162,7 @@ int ensure_device_ready()
     if (g_device_ready[dev].load(std::memory_order_relaxed)) return MXD_OK;
     e = mxd::raise_forward_lds();
     if (e == hipSuccess) e = mxd::raise_forward_cu_lds();
+    if (e == hipSuccess) e = mxd::raise_grid_lds();
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "raising the dynamic LDS limit failed: %s", hipGetErrorString(e));
     void* ptr = nullptr;
     e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));  // (this device's copy of the array: the device is current)
@@ -858,6 +860,110 @@ struct DaggSpace {
     }
 };
 
+// Grid sampler on planes: whether a plane fits the LDS of a CU (as float32, whatever the dtype) and every index its type.
+bool grid_planes_fit(int64_t n, int64_t c, int64_t h, int64_t w, int64_t h_out, int64_t w_out)
+{
+    const int64_t lim = int64_t(1) << 28;
+    if (n <= 0 || c <= 0 || h <= 0 || w <= 0 || h_out <= 0 || w_out <= 0 || c > 256 || n >= (1 << 20)) return false;
+    if (h >= lim || w >= lim || h_out >= lim || w_out >= lim || h_out * w_out >= lim) return false;
+    return h * w * 4 <= mxd::kCuLdsBytes;
+}
+
+// Sizes, and the work split: how many planes a workgroup takes and, where there are few, how the output pixels are shared out.
+// Small planes share a workgroup (one geometry for all of them) as long as two workgroups per CU are left; large ones (one
+// workgroup per CU) get more threads.
+int grid_planes_args(int dtype, int64_t n, int64_t c, int64_t h, int64_t w, int64_t h_out, int64_t w_out, int mode, mxd::GridArgs* a)
+{
+    const int es = elem_size(dtype);
+    if (es == 0) return fail(MXD_E_DTYPE, "dtype code %d is not float32(0)/float16(1)/bfloat16(2)", dtype);
+    if (!grid_planes_fit(n, c, h, w, h_out, w_out))
+        return fail(MXD_E_SHAPE, "grid_sampler2d: [%lld, %lld, %lld, %lld] is beyond what the kernels for planes take", (long long)n,
+                    (long long)c, (long long)h, (long long)w);
+    memset(a, 0, sizeof(*a));
+    a->n = (int32_t)n;
+    a->c = (int32_t)c;
+    a->h = (int32_t)h;
+    a->w = (int32_t)w;
+    a->outs = (int32_t)(h_out * w_out);
+    a->mode = mode;
+    return MXD_OK;
+}
+
+constexpr int64_t kGridFill = 512;  // workgroups aimed at: two per CU
+
+int64_t ceil_div(int64_t x, int64_t y) { return (x + y - 1) / y; }
+
+// Planes of `bytes` that a workgroup takes when `items` of them have to be shared out.
+int64_t grid_planes_together(int64_t bytes, int64_t c, int64_t n)
+{
+    int64_t k = mxd::kGridStageBytes / bytes;
+    if (k > ceil_div(n * c, kGridFill)) k = ceil_div(n * c, kGridFill);
+    if (k > c) k = c;
+    return k < 1 ? 1 : k;
+}
+
+int grid_block(int64_t lds) { return 2 * lds > mxd::kCuLdsBytes ? 2 * mxd::kGridThreads : mxd::kGridThreads; }
+
+int grid_planes_forward_plan(int es, mxd::GridArgs* a)
+{
+    const int64_t bytes = (int64_t)a->h * a->w * es;
+    a->planes = (int32_t)grid_planes_together(bytes, a->c, a->n);
+    a->chunks = (int32_t)ceil_div(a->c, a->planes);
+    a->lds = (uint32_t)((a->planes * bytes + 15) & ~15);
+    a->block = grid_block(a->lds);
+    // few planes: each is read by several workgroups, of at least one pass of their threads
+    int64_t splits = ceil_div(kGridFill, (int64_t)a->n * a->chunks);
+    if (splits > ceil_div(a->outs, a->block)) splits = ceil_div(a->outs, a->block);
+    a->split_px = (int32_t)ceil_div(a->outs, splits);
+    a->splits = (int32_t)ceil_div(a->outs, a->split_px);
+    if ((int64_t)a->n * a->chunks * a->splits >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs too many workgroups");
+    return MXD_OK;
+}
+
+int grid_planes_backward_plan(int es, bool maps, bool points, mxd::GridArgs* a)
+{
+    const int64_t px = (int64_t)a->h * a->w, images = a->n;
+    int64_t lds = 0, wgs = 0;
+    a->gx_planes = (int32_t)grid_planes_together(px * 8, a->c, images);
+    a->gx_chunks = (int32_t)ceil_div(a->c, a->gx_planes);
+    a->gx_bands = (int32_t)ceil_div(px * 8, mxd::kCuLdsBytes);  // (a plane whole where it fits: two bands of 45 KB took 85 us, one plane 77)
+    a->gx_band_px = (int32_t)ceil_div(px, a->gx_bands);
+    a->gx_bands = (int32_t)ceil_div(px, a->gx_band_px);
+    if (maps) {
+        wgs = images * a->gx_chunks * a->gx_bands;
+        lds = (int64_t)a->gx_planes * a->gx_band_px * 8;
+    }
+    a->gx_wgs = (int32_t)wgs;
+    a->block = grid_block((int64_t)a->gx_planes * a->gx_band_px * 8);
+    a->gg_ranges = (int32_t)ceil_div(a->outs, (int64_t)a->block * mxd::kGridMaxPx);
+    a->gg_px = (int32_t)ceil_div(a->outs, (int64_t)a->block * a->gg_ranges);
+    a->gg_ranges = (int32_t)ceil_div(a->outs, (int64_t)a->block * a->gg_px);
+    // as many channels per workgroup as leave the chip full: every chunk more is one more image of sums to write and to read
+    int64_t channels = images * a->gg_ranges * a->c / kGridFill;
+    if (channels > a->c) channels = a->c;
+    if (channels < 1) channels = 1;
+    a->gg_chunks = (int32_t)ceil_div(a->c, channels);
+    a->gg_channels = (int32_t)ceil_div(a->c, a->gg_chunks);
+    a->gg_chunks = (int32_t)ceil_div(a->c, a->gg_channels);
+    int64_t staged = (lds > mxd::kGridStageBytes ? lds : mxd::kGridStageBytes) / (px * es);
+    if (staged > a->gg_channels) staged = a->gg_channels;
+    a->gg_planes = (int32_t)(staged < 1 ? 1 : staged);
+    if (points) {
+        const int64_t gg = images * a->gg_chunks * a->gg_ranges;
+        if (a->gg_planes * px * es > lds) lds = a->gg_planes * px * es;
+        wgs += gg;
+        a->gg_wgs = (int32_t)gg;
+    }
+    if (wgs >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs too many workgroups");
+    a->lds = (uint32_t)((lds + 15) & ~15);
+    return MXD_OK;
+}
+
+size_t grid_part_bytes(const mxd::GridArgs& a)
+{
+    return a.gg_chunks > 1 ? (size_t)a.gg_chunks * a.n * a.outs * 2 * sizeof(float) : 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1344,6 +1450,71 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
     a.rec = reinterpret_cast<mxd::u32x4*>(ws + space.rec);
     const hipError_t e = mxd::launch_dagg_backward(dtype, a, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_dagg_backward: launch failed: %s", hipGetErrorString(e));
+    return MXD_OK;
+}
+
+int mxd_grid_sampler2d_planes_fit(int64_t n, int64_t c, int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out)
+{
+    return grid_planes_fit(n, c, h_in, w_in, h_out, w_out) ? 1 : 0;
+}
+
+int mxd_grid_sampler2d_planes_forward(const void* input, const void* grid, void* output, int dtype, int64_t n, int64_t c,
+                                      int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out, int interpolation_mode,
+                                      int padding_mode, int align_corners, void* hip_stream)
+{
+    const int mode = grid_mode(interpolation_mode, padding_mode, align_corners);
+    if (mode < 0) return mode;
+    mxd::GridArgs a;
+    int rc = grid_planes_args(dtype, n, c, h_in, w_in, h_out, w_out, mode, &a);
+    if (rc == MXD_OK && (!input || !grid || !output)) rc = fail(MXD_E_NULL, "mxd_grid_sampler2d_planes_forward: NULL data pointer");
+    if (rc == MXD_OK) rc = grid_planes_forward_plan(elem_size(dtype), &a);
+    if (rc == MXD_OK) rc = ensure_device_ready();
+    if (rc != MXD_OK) return rc;
+    a.x = input;
+    a.grid = grid;
+    a.out = output;
+    const hipError_t e = mxd::launch_grid_planes_forward(dtype, a, static_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_grid_sampler2d_planes_forward: launch failed: %s", hipGetErrorString(e));
+    return MXD_OK;
+}
+
+size_t mxd_grid_sampler2d_planes_backward_workspace_bytes(int dtype, int64_t n, int64_t c, int64_t h_in, int64_t w_in,
+                                                          int64_t h_out, int64_t w_out)
+{
+    mxd::GridArgs a;
+    if (grid_planes_args(dtype, n, c, h_in, w_in, h_out, w_out, 1, &a) != MXD_OK) return 0;
+    if (grid_planes_backward_plan(elem_size(dtype), true, true, &a) != MXD_OK) return 0;
+    return grid_part_bytes(a);
+}
+
+int mxd_grid_sampler2d_planes_backward(const void* grad_output, const void* input, const void* grid, void* grad_input,
+                                       void* grad_grid, void* workspace, size_t workspace_bytes, int dtype, int64_t n,
+                                       int64_t c, int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out,
+                                       int interpolation_mode, int padding_mode, int align_corners, void* hip_stream)
+{
+    const int mode = grid_mode(interpolation_mode, padding_mode, align_corners);
+    if (mode < 0) return mode;
+    mxd::GridArgs a;
+    int rc = grid_planes_args(dtype, n, c, h_in, w_in, h_out, w_out, mode, &a);
+    if (rc == MXD_OK && (!grad_output || !input || !grid || (!grad_input && !grad_grid)))
+        rc = fail(MXD_E_NULL, "mxd_grid_sampler2d_planes_backward: NULL data pointer");
+    if (rc == MXD_OK) rc = grid_planes_backward_plan(elem_size(dtype), grad_input != nullptr, grad_grid != nullptr, &a);
+    if (rc == MXD_OK) rc = ensure_device_ready();
+    if (rc != MXD_OK) return rc;
+    const size_t need = grad_grid ? grid_part_bytes(a) : 0;
+    if (need > 0 && (!workspace || workspace_bytes < need))
+        return fail(MXD_E_WORKSPACE, "mxd_grid_sampler2d_planes_backward: workspace of %zu bytes required, %zu given", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    if (need > 0 && (reinterpret_cast<uintptr_t>(workspace) & 15u))
+        return fail(MXD_E_WORKSPACE, "mxd_grid_sampler2d_planes_backward: workspace must be 16-byte aligned");
+    a.x = input;
+    a.grid = grid;
+    a.grad_out = grad_output;
+    a.grad_x = grad_input;
+    a.grad_grid = grad_grid;
+    a.part = static_cast<float*>(workspace);
+    const hipError_t e = mxd::launch_grid_planes_backward(dtype, a, static_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_grid_sampler2d_planes_backward: launch failed: %s", hipGetErrorString(e));
     return MXD_OK;
 }
 

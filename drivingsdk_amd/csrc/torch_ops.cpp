@@ -257,6 +257,42 @@ struct Gka {
     }
 };
 
+struct Grid {
+    static constexpr const char* kNode = "GridSampler2dV2FunctionBackward";
+    static constexpr int kTensors = 2, kInts = 3;  // interpolation and padding mode, align_corners: see mxd_grid_sampler2d_forward
+    static constexpr std::array<int, 2> kGradOf{0, 1};
+    static constexpr bool kKeepsOutput = false, kOnce = true, kFloat32InAutocast = false;
+    static bool takes(const Args& a)
+    {
+        const Tensor &x = a.t[0], &grid = a.t[1];
+        if (dtype_code(x) < 0 || !plain(x, x) || !plain(grid, x, x.scalar_type()) || x.dim() != 4 || grid.dim() != 4) return false;
+        return a.i[0] == 0 && (a.i[1] == 0 || a.i[1] == 1) && (a.i[2] == 0 || a.i[2] == 1) && grid.size(0) == x.size(0) && grid.size(3) == 2 &&
+               mxd_grid_sampler2d_planes_fit(x.size(0), x.size(1), x.size(2), x.size(3), grid.size(1), grid.size(2));
+    }
+    static Tensor new_output(const Args& a) { return new_tensor({a.t[0].size(0), a.t[0].size(1), a.t[1].size(1), a.t[1].size(2)}, a.t[0]); }
+    static void forward(const Args& a, Tensor& out)
+    {
+        const Tensor &x = a.t[0], &grid = a.t[1];
+        Launch l(x);
+        check(mxd_grid_sampler2d_planes_forward(x.data_ptr(), grid.data_ptr(), out.data_ptr(), dtype_code(x), x.size(0), x.size(1), x.size(2),
+                                                x.size(3), grid.size(1), grid.size(2), (int)a.i[0], (int)a.i[1], (int)a.i[2], l.stream()));
+    }
+    static void backward(const Args& a, const Tensor& grad, std::array<Tensor, 2>& g, unsigned need)
+    {
+        const Tensor &x = a.t[0], &grid = a.t[1];
+        const int code = dtype_code(x);
+        if ((need & 3) == 0) return;
+        Launch l(x);
+        const size_t bytes = (need & 2) ? mxd_grid_sampler2d_planes_backward_workspace_bytes(code, x.size(0), x.size(1), x.size(2), x.size(3),
+                                                                                              grid.size(1), grid.size(2))
+                                        : 0;
+        check(mxd_grid_sampler2d_planes_backward(grad.data_ptr(), x.data_ptr(), grid.data_ptr(), (need & 1) ? g[0].data_ptr() : nullptr,
+                                                 (need & 2) ? g[1].data_ptr() : nullptr, l.scratch(bytes), bytes, code, x.size(0), x.size(1),
+                                                 x.size(2), x.size(3), grid.size(1), grid.size(2), (int)a.i[0], (int)a.i[1], (int)a.i[2],
+                                                 l.stream()));
+    }
+};
+
 // ---- autograd ----------------------------------------------------------------------------------------------------------
 
 bool usable_grad(const Tensor& grad, const Tensor& like, int64_t numel)
@@ -275,6 +311,8 @@ template <>
 int64_t output_numel<Fused>(const Args& a) { return a.t[4].size(0) * a.t[4].size(1) * a.t[0].size(2) * a.t[0].size(3); }
 template <>
 int64_t output_numel<Dagg>(const Args& a) { return a.t[0].size(0) * a.t[4].size(1) * a.t[0].size(2); }
+template <>
+int64_t output_numel<Grid>(const Args& a) { return a.t[0].size(0) * a.t[0].size(1) * a.t[1].size(1) * a.t[1].size(2); }
 template <>
 int64_t output_numel<Gka>(const Args& a) { return output_numel<Msda>(a); }
 
@@ -484,7 +522,7 @@ PyObject* py_backward(PyObject*, PyObject* const* args, Py_ssize_t n)
     {name "_forward", (PyCFunction)(void (*)(void)) & py_forward<op>, METH_FASTCALL, nullptr},       \
     {name "_backward", (PyCFunction)(void (*)(void)) & py_backward<op>, METH_FASTCALL, nullptr}
 
-PyMethodDef methods[] = {MXD_OP("msda", Msda), MXD_OP("fused", Fused), MXD_OP("dagg", Dagg), MXD_OP("gka", Gka),
+PyMethodDef methods[] = {MXD_OP("msda", Msda), MXD_OP("fused", Fused), MXD_OP("dagg", Dagg), MXD_OP("gka", Gka), MXD_OP("grid", Grid),
                          {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "The operators on PyTorch tensors (csrc/torch_ops.cpp).", -1, methods,

@@ -12,11 +12,19 @@ from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
 from .. import _C
+from .._lib import native as _native
 
 MAX_CHANNELS = 256
 
 
 class GridSampler2dV2Function(Function):
+    @classmethod
+    def apply(cls, input_tensor, grid_tensor, mode="bilinear", padding_mode="zeros", align_corners=False):
+        # calls that need nothing of Python's autograd machinery are served by the extension module
+        padding = {"zeros": 0, "border": 1}.get(padding_mode) if mode == "bilinear" and cls is GridSampler2dV2Function else None
+        output = None if padding is None else _native.grid(input_tensor, grid_tensor, 0, padding, 1 if align_corners else 0)
+        return output if output is not None else super().apply(input_tensor, grid_tensor, mode, padding_mode, align_corners)
+
     @staticmethod
     def forward(ctx, input_tensor, grid_tensor, mode="bilinear", padding_mode="zeros", align_corners=False):
         if torch.numel(input_tensor) == 0 or torch.numel(grid_tensor) == 0:
@@ -47,10 +55,15 @@ class GridSampler2dV2Function(Function):
     @once_differentiable
     def backward(ctx, grad_output):
         input_x, input_grid = ctx.saved_tensors
-        nhwc_input_x = input_x.permute(0, 2, 3, 1).contiguous()
-        nhwc_grad_output = grad_output.permute(0, 2, 3, 1).contiguous()
         interpolation = {"bilinear": 0, "nearest": 1}.get(ctx.interpolation, 0)
         padding = {"zeros": 0, "border": 1, "reflection": 2}.get(ctx.padding_mode, 0)
+        if input_x.is_contiguous():  # planes as they are, where they fit the kernels for planes
+            grads = _native.grid_backward(input_x, input_grid.contiguous(), interpolation, padding, int(bool(ctx.align_corners)),
+                                          grad_output.contiguous())
+            if grads is not None:
+                return grads[0], grads[1], None, None, None
+        nhwc_input_x = input_x.permute(0, 2, 3, 1).contiguous()
+        nhwc_grad_output = grad_output.permute(0, 2, 3, 1).contiguous()
         grad_x, grad_grid = _C.grid_sampler2d_v2_backward(nhwc_grad_output, nhwc_input_x, input_grid, interpolation,
                                                           padding, ctx.align_corners)
         return grad_x, grad_grid, None, None, None

@@ -290,6 +290,20 @@ int mxd_grid_sampler2d_backward(const void* grad_output_nhwc, const void* input_
                                 int64_t w_out, int interpolation_mode, int padding_mode, int align_corners,
                                 void* hip_stream);
 
+/* The same on planes: input [n, c, h_in, w_in], output [n, c, h_out, w_out], no transposition.  For planes that fit the
+ * LDS of a compute unit as float32 (h_in * w_in <= 40960): planes_fit() says whether a problem can be given to these.
+ * The backward leaves out the gradient whose pointer is NULL. */
+int mxd_grid_sampler2d_planes_fit(int64_t n, int64_t c, int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out);
+int mxd_grid_sampler2d_planes_forward(const void* input, const void* grid, void* output, int dtype, int64_t n, int64_t c,
+                                      int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out, int interpolation_mode,
+                                      int padding_mode, int align_corners, void* hip_stream);
+size_t mxd_grid_sampler2d_planes_backward_workspace_bytes(int dtype, int64_t n, int64_t c, int64_t h_in, int64_t w_in,
+                                                          int64_t h_out, int64_t w_out);
+int mxd_grid_sampler2d_planes_backward(const void* grad_output, const void* input, const void* grid, void* grad_input,
+                                       void* grad_grid, void* workspace, size_t workspace_bytes, int dtype, int64_t n,
+                                       int64_t c, int64_t h_in, int64_t w_in, int64_t h_out, int64_t w_out,
+                                       int interpolation_mode, int padding_mode, int align_corners, void* hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

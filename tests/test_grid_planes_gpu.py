@@ -1,0 +1,64 @@
+"""Grid sampler on planes at the sizes where its kernels change course, against torch on the CPU in float64: planes of odd size
+(no 16-byte boundaries), one and many planes per workgroup, one and several output pixels per thread, ranges and splits of
+the output pixels, chunks of the channels, planes that take a CU's LDS whole, and planes too large for it (channel-last form)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import mx_driving
+from drivingsdk_amd.ops.grid_sampler2d_v2 import GridSampler2dV2Function
+from test_grid_sampler_gpu import check, make_inputs
+from util import BF16, BWD_FP32, FWD_FP32, HALF, rel_err
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [([1, 1, 1, 1], [1, 1, 1, 2]), ([2, 3, 5, 7], [2, 3, 5, 2]), ([3, 5, 37, 41], [3, 23, 29, 2]), ([1, 19, 20, 31], [1, 70, 90, 2]),
+          ([2, 33, 16, 20], [2, 13, 200, 2]), ([24, 40, 17, 21], [24, 9, 11, 2]), ([1, 2, 101, 181], [1, 100, 181, 2]),
+          ([1, 4, 160, 256], [1, 40, 50, 2]), ([1, 3, 161, 256], [1, 10, 10, 2]), ([2, 256, 9, 33], [2, 31, 17, 2])]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("input_shape,grid_shape", SHAPES)
+def test_planes(gpu_device, input_shape, grid_shape, dtype):
+    x, grid, go = make_inputs(input_shape, grid_shape, seed=input_shape[1], span=1.2)
+    if dtype == torch.float32:
+        # (a float32 pixel coordinate of up to 180 is off by up to 1e-5)
+        print(check(x, grid, go, "zeros", False, gpu_device, fwd_tol=2 * FWD_FP32, bwd_tol=BWD_FP32))
+        return
+    x, grid, go = x.to(dtype), grid.to(dtype), go.to(dtype)
+    xr, gr = x.double().requires_grad_(), grid.double().requires_grad_()
+    want = F.grid_sample(xr, gr, "bilinear", "border", True)
+    want.backward(go.double())
+    xd, gd = x.to(gpu_device).requires_grad_(), grid.to(gpu_device).requires_grad_()
+    out = mx_driving.grid_sampler2d_v2(xd, gd, "bilinear", "border", True)
+    out.backward(go.to(gpu_device))
+    tol = HALF if dtype == torch.float16 else BF16
+    for got, ref in ((out.detach(), want.detach()), (xd.grad, xr.grad)):
+        assert got.dtype == dtype and rel_err(got.double().cpu().numpy(), ref.numpy()) <= tol
+
+
+def test_single_gradients_and_the_python_function(gpu_device):
+    x, grid, go = [t.to(gpu_device) for t in make_inputs([2, 20, 30, 40], [2, 25, 35, 2], seed=2)]
+
+    class PythonPath(GridSampler2dV2Function):
+        pass
+
+    x.requires_grad_()
+    grid.requires_grad_()
+    a, b = (f(x, grid, "bilinear", "zeros", False) for f in (mx_driving.grid_sampler2d_v2, PythonPath.apply))
+    assert torch.equal(a, b) and a.grad_fn.name() == b.grad_fn.name().replace("PythonPath", "GridSampler2dV2Function")
+    both = torch.autograd.grad(a, [x, grid], go, retain_graph=True)
+    for k, t in enumerate((x, grid)):
+        for o in (a, b):
+            assert torch.allclose(torch.autograd.grad(o, t, go, retain_graph=True)[0], both[k], rtol=1e-5, atol=1e-5)
+
+
+def test_infinite_pixels_outside_the_samples(gpu_device):
+    """A pixel that no sample reaches must not enter a result, whatever it holds (corners outside the image read some pixel)."""
+    x, grid, go = make_inputs([1, 4, 8, 8], [1, 6, 6, 2], seed=6)
+    grid = grid * 0.05 + torch.tensor([1.0, 1.0])   # around the lower right corner, part of it outside
+    x[:, :, 0, 0] = float("inf")
+    xd, gd = x.to(gpu_device).requires_grad_(), grid.to(gpu_device).requires_grad_()
+    out = mx_driving.grid_sampler2d_v2(xd, gd, "bilinear", "zeros", False)
+    out.backward(go.to(gpu_device))
+    assert all(torch.isfinite(t).all() for t in (out, xd.grad, gd.grad))
