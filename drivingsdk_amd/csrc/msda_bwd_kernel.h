@@ -63,10 +63,19 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
 
     extern __shared__ __align__(16) unsigned char smem[];
     i32x4* lvl = reinterpret_cast<i32x4*>(smem);
+    int32_t* tile_first = reinterpret_cast<int32_t*>(
+        smem + kMaxLevels * sizeof(i32x4) +
+        (size_t)a.plan.waves_per_block * a.plan.units_per_wave * (kChunkStride * sizeof(Entry) + kChunk * sizeof(f32x4)));
     if constexpr (!SCATTER) {
         // this workgroup's share of the zero-fill of the image (every workgroup of the launch takes one, also those
         // without work): the stores ride along with this kernel instead of taking a launch of their own
-        if (a.fill_n4 != 0 && a.sparse != 0 && levels_tile_the_keys(a)) {
+        const LevelLanes lv(a, (int)threadIdx.x & (kWave - 1));
+        // the levels and their first tiles (-1: a level that does not fit the run table is left out of grad_value)
+        if ((int)threadIdx.x < a.nl) {
+            lvl[threadIdx.x] = lv.geo;
+            tile_first[threadIdx.x] = lv.first;
+        }
+        if (a.fill_n4 != 0 && a.sparse != 0 && lv.canonical) {
             // only the rows that receive atomic additions in the tile pass (tiles split by query range, small tiles,
             // and the first pixel of every other tile); a row of the image is nh*hd floats, a multiple of 16 bytes here
             const int32_t tiles = a.tbl_stride - 1;  // (bound: pieces of tiles that do not exist are skipped)
@@ -76,7 +85,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             for (int64_t w = blockIdx.x; w < pieces; w += gridDim.x) {
                 const int32_t b = (int32_t)(w / (tiles * kRowParts)), r = (int32_t)(w % (tiles * kRowParts));
                 int32_t r0, r1;
-                if (!atomic_rows_of_part(a, r / kRowParts, r % kRowParts, &r0, &r1)) continue;
+                if (!lv.atomic_rows_of_part(a, r / kRowParts, r % kRowParts, &r0, &r1)) continue;
                 f32x4* img = reinterpret_cast<f32x4*>(a.grad_value) + ((size_t)b * a.nk + r0) * row4;
                 const uint32_t n4 = (uint32_t)(r1 - r0) * row4;
                 for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x) __builtin_nontemporal_store(z, img + i);
@@ -97,10 +106,10 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     Work wk;
     if (!decode_block(a.plan, blockIdx.x, a.bs, a.nh, a.nq, &wk)) return;
 
-    for (int i = threadIdx.x; i < a.nl; i += blockDim.x) {
-        lvl[i] = load_level(a, i);
+    if constexpr (SCATTER) {
+        for (int i = threadIdx.x; i < a.nl; i += blockDim.x) lvl[i] = load_level(a, i);
+        __syncthreads();
     }
-    __syncthreads();
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
@@ -141,9 +150,6 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     const uint32_t ghead_off = (uint32_t)wk.h * a.hd * 4u;
 
     // ---- records per tile of this workgroup: count, prefix, publish -----------------------
-    int32_t* tile_first = reinterpret_cast<int32_t*>(
-        smem + kMaxLevels * sizeof(i32x4) +
-        (size_t)a.plan.waves_per_block * a.plan.units_per_wave * (kChunkStride * sizeof(Entry) + kChunk * sizeof(f32x4)));
     int32_t* cursor = tile_first + kMaxLevels;  // [tbl_stride] counts, then next free position per tile
     uint32_t* slab = nullptr;
     const int entries = U * kChunk;
@@ -320,18 +326,6 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     if constexpr (!SCATTER) {
         const int64_t wg_row = ((int64_t)wk.b * a.nh + wk.h) * a.nwg + wk.q_begin / a.plan.tile_q;
         slab = a.rec + wg_row * a.rec_cap * kRecDwords;
-        if (threadIdx.x == 0) {
-            // the run table has room for tbl_stride - 1 tiles, which is every tile when the levels do not
-            // overlap; a level that does not fit (malformed shapes) is left out of grad_value: -1
-            int32_t first = 0;
-            for (int l = 0; l < a.nl; ++l) {
-                int32_t px;
-                const int32_t nt = level_tile_count(lvl[l].x, lvl[l].y, lvl[l].z, a.nk, a.tile_px_log2, &px);
-                const bool fits = first + nt <= a.tbl_stride - 1;
-                tile_first[l] = fits ? first : -1;
-                if (fits) first += nt;
-            }
-        }
         for (int i = threadIdx.x; i < a.tbl_stride; i += blockDim.x) cursor[i] = 0;
         __syncthreads();
         // queries whose first `span` samples are counted here:
@@ -773,7 +767,10 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
 template <typename T, int VEC, int NPASS>
 inline hipError_t launch_one(const KArgs& a, bool scatter, hipStream_t stream)
 {
-    const dim3 grid(a.plan.grid), block(a.plan.block);
+    // (few queries: the zero-fill of the image gets workgroups that do nothing else -- it was 27 us of a backward of 2 x 100
+    //  queries that 64 workgroups shared)
+    const uint32_t fill_wgs = a.fill_n4 != 0 ? 1024u : 0u;
+    const dim3 grid(a.plan.grid > fill_wgs ? a.plan.grid : fill_wgs), block(a.plan.block);
     // (the 16-lane fixed geometry is built for lanes of 16 bytes and one row pass: rows of 256 bytes; with two passes --
     //  heads of 128 float32 channels -- it changes nothing, 544 us)
     constexpr bool kWide = sizeof(T) * VEC == 16 && NPASS == 1;

@@ -43,10 +43,8 @@
 
 namespace mxd {
 
-
-// Work item table, evaluated identically by every workgroup.
+// A work item: a tile, or the share of a hot one that a range of the slabs holds.
 struct TileItem {
-    int32_t level, H, W, base;   // level geometry
     int32_t p0, p1;              // pixel range of the tile, relative to the batch element
     int32_t c0, cstep;           // the item takes slabs c0, c0 + cstep, c0 + 2 cstep, ... in the order of KArgs::run_step
     int32_t tile;                // index of the tile within the (batch, head): column of the run table
@@ -54,85 +52,27 @@ struct TileItem {
                                  // levels tile the keys, so that no tile of another level holds the same rows)
 };
 
-// What a workgroup needs of every level, derived by one lane per level (LevelInfo::fill) so that the thread that looks up
-// the work item afterwards goes through LDS values only: the level loads and the divisions behind the chunk count
-// would otherwise be made one level after the other by that one thread, in front of everything the workgroup does.
-struct LevelInfo {
-    int32_t H[kMaxLevels], W[kMaxLevels], base[kMaxLevels];
-    int32_t px[kMaxLevels];      // pixels of the level inside the value tensor
-    int32_t nt[kMaxLevels];      // its tiles (before the run table's room is considered)
-    int32_t chunks[kMaxLevels];  // query chunks per tile
-    __device__ void fill(const KArgs& a, int l)
-    {
-        const i32x4 L = load_level(a, l);
-        int32_t P;
-        const int32_t n = level_tile_count(L.x, L.y, L.z, a.nk, a.tile_px_log2, &P);
-        H[l] = L.x;
-        W[l] = L.y;
-        base[l] = L.z;
-        px[l] = P;
-        nt[l] = n;
-        chunks[l] = n > 0 ? level_tile_chunks(a, n) : 0;
-    }
-    // levels_tile_the_keys() on the values held here
-    __device__ bool tile_the_keys(const KArgs& a) const
-    {
-        int64_t next = 0;
-        int32_t tiles = 0;
-        for (int l = 0; l < a.nl; ++l) {
-            if (H[l] <= 0 || W[l] <= 0 || (int64_t)base[l] != next) return false;
-            const int64_t p = (int64_t)H[l] * W[l];
-            next += p;
-            if (next > a.nk) return false;
-            tiles += (int32_t)((p + ((int64_t)1 << a.tile_px_log2) - 1) >> a.tile_px_log2);
-        }
-        return next == a.nk && tiles <= a.tbl_stride - 1;
-    }
-};
-
-// lv_first / lv_nt: scratch of kMaxLevels entries each (first tile and tile count per level).
-__device__ inline bool decode_tile_item(const KArgs& a, const TileArgs& t, const LevelInfo& lv, int32_t item, TileItem* out,
-                                        int32_t* lv_first, int32_t* lv_nt)
+// Work item number `item` of a (batch, head).  Items are numbered from the last level to the first: the coarse levels, whose
+// tiles are split into many long-running items, start first and the short items of the fine levels fill the end of the launch.
+// (by whole wavefronts)
+__device__ inline bool decode_tile_item(const KArgs& a, int32_t item, int lane, TileItem* out)
 {
-    // Tiles are numbered level by level as in the first kernel; a level that does not fit the run table
-    // (only possible when the levels overlap) has no tiles.
-    int32_t total = 0;
-    for (int l = 0; l < a.nl; ++l) {
-        const int32_t nt = lv.nt[l];
-        const bool fits = total + nt <= a.tbl_stride - 1;
-        lv_first[l] = total;
-        lv_nt[l] = fits ? nt : 0;
-        if (fits) total += nt;
-    }
-    const bool canonical = lv.tile_the_keys(a);
-    // Items are numbered from the last level to the first: the coarse levels, whose tiles are
-    // split into many long-running items, start first and the short items of the fine levels
-    // fill the end of the launch.
-    int32_t first = 0;
-    for (int l = a.nl - 1; l >= 0; --l) {
-        const int32_t nt = lv_nt[l];
-        if (nt == 0) continue;
-        const int32_t base = lv.base[l], P = lv.px[l];
-        const int32_t chunks = lv.chunks[l];
-        const int32_t n = nt * chunks;
-        if (item < first + n) {
-            const int32_t ti = (item - first) / chunks, ci = (item - first) % chunks;
-            out->level = l;
-            out->H = lv.H[l];
-            out->W = lv.W[l];
-            out->base = base;
-            const int32_t tile_px = 1 << a.tile_px_log2;
-            out->p0 = base + ti * tile_px;
-            out->p1 = (out->p0 + tile_px) < (base + P) ? (out->p0 + tile_px) : (base + P);
-            out->c0 = ci;
-            out->cstep = chunks;
-            out->tile = lv_first[l] + ti;
-            out->exclusive = chunks == 1 && canonical;
-            return true;
-        }
-        first += n;
-    }
-    return false;
+    const LevelLanes lv(a, lane);
+    const int32_t n = lv.nt * lv.chunks, inc = LevelLanes::prefix(a, n, lane);
+    const int32_t start = __builtin_amdgcn_readlane(inc, a.nl - 1) - inc;
+    const uint64_t owner = __ballot(item >= start && item < start + n);
+    if (owner == 0) return false;
+    const int l = __builtin_ctzll(owner);
+    const int32_t chunks = __builtin_amdgcn_readlane(lv.chunks, l), at = item - __builtin_amdgcn_readlane(start, l);
+    const int32_t ti = (int32_t)((uint32_t)at / (uint32_t)chunks), tile_px = 1 << a.tile_px_log2;
+    const int32_t end = lv.base(l) + __builtin_amdgcn_readlane(lv.px, l);
+    out->p0 = lv.base(l) + ti * tile_px;
+    out->p1 = (out->p0 + tile_px) < end ? (out->p0 + tile_px) : end;
+    out->c0 = at - ti * chunks;
+    out->cstep = chunks;
+    out->tile = __builtin_amdgcn_readlane(lv.first, l) + ti;
+    out->exclusive = chunks == 1 && lv.canonical;
+    return true;
 }
 
 // The samples of levels whose tiles found no room in the run table, added to grad_value one sample per thread with
@@ -217,9 +157,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     // up to 64 runs of records per wavefront at a time: first record, records before the run
     __shared__ uint32_t run_src_all[NW * kWave];
     __shared__ uint32_t run_pre_all[NW * kWave];
-    __shared__ TileItem item_s;
-    __shared__ int32_t lv_first[kMaxLevels], lv_nt[kMaxLevels];
-    __shared__ int item_ok;
+    __shared__ int32_t lv_unfit[kMaxLevels];
     __shared__ int done_count;
     // Pixels that collect far more entries than the others (inputs that pile samples on a few pixels) get extra
     // lists in the slots of the workgroup that no pixel of the tile uses -- when there are such slots.  The first
@@ -239,28 +177,21 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         wk.q_begin = (int32_t)(r / a.bs);
     }
     if (wk.q_begin >= t.items_per_bh - t.extra) {  // (uniform: one of the workgroups behind the work items)
-        add_levels_without_tiles<T>(a, wk.b, wk.h, wk.q_begin - (t.items_per_bh - t.extra), t.extra, lv_first);
+        add_levels_without_tiles<T>(a, wk.b, wk.h, wk.q_begin - (t.items_per_bh - t.extra), t.extra, lv_unfit);
         return;
     }
-    // (the per-level values live in the entry storage, which is not written before the work item is known: the kernel's
-    //  static LDS is 450 bytes short of the 80 KiB that let two workgroups share a CU)
-    static_assert(sizeof(LevelInfo) <= sizeof(u32x4) * kTileEntCap, "the level values must fit one wavefront's entry storage");
-    LevelInfo& lv_info = *reinterpret_cast<LevelInfo*>(&ent[0]);
-    if ((int)threadIdx.x < a.nl) lv_info.fill(a, (int)threadIdx.x);
     if (threadIdx.x < kTileThreads / 2) slot_info[threadIdx.x] = 0;
     // an empty list points at the dummy entry of the wavefront that owns the pixel slot (slot s belongs to lane group
     // s / PPG, i.e. to wavefront s / (8 PPG); slots past the tile size are never used)
     heads[threadIdx.x] = ((threadIdx.x / (kLpp * PPG)) % NW * kTileEntCap + kDummyOfWave) * 16u;
-    __syncthreads();
     if (threadIdx.x == 0) {
-        item_ok = decode_tile_item(a, t, lv_info, wk.q_begin, &item_s, lv_first, lv_nt) ? 1 : 0;
         done_count = 0;
         spare_next = 0;
         round1_total = 0;
     }
+    TileItem it;
+    if (!decode_tile_item(a, wk.q_begin, (int)threadIdx.x & (kWave - 1), &it)) return;  // uniform
     __syncthreads();
-    if (!item_ok) return;  // uniform
-    const TileItem it = item_s;
 
     const int hd = a.hd;
     const int tid = threadIdx.x;
@@ -735,7 +666,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                         else if (t.accumulate)
                             *dst += v;
                         else
-                            *dst = v;
+                            __builtin_nontemporal_store(v, dst);
                     }
                 }
             }

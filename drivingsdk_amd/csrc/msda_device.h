@@ -135,67 +135,84 @@ __device__ inline bool tile_stored_directly(int32_t chunks, int32_t npx, int32_t
     return chunks == 1 && (1 << tile_px_log2) - ((npx + g - 1) / g * g) < g;
 }
 
-// Whether the levels tile the keys exactly and in order -- the first level starts at key 0, every other one where the
-// one before it ends, the last one ends at key nk -- and all their tiles fit the run table.  Only then is every row of
-// grad_value covered by exactly one tile, which is what lets the owner of a tile store its rows (instead of adding to
-// them) and lets the rows that nobody adds to go without zeros.  level_start_index is the caller's: for any other
-// layout (keys that no level covers, levels out of order or overlapping) every row is zero-filled and every tile adds
-// its sums with atomics.
-// (level(l): {H, W, first key} of level l, from wherever the caller holds it)
-template <typename GetLevel>
-__device__ inline bool levels_tile_the_keys_of(const KArgs& a, GetLevel level)
-{
-    int64_t next = 0;
-    int32_t tiles = 0;
-    for (int l = 0; l < a.nl; ++l) {
-        const i32x4 L = level(l);
-        if (L.x <= 0 || L.y <= 0 || (int64_t)L.z != next) return false;
-        const int64_t px = (int64_t)L.x * L.y;
-        next += px;
-        if (next > a.nk) return false;
-        tiles += (int32_t)((px + ((int64_t)1 << a.tile_px_log2) - 1) >> a.tile_px_log2);
-    }
-    return next == a.nk && tiles <= a.tbl_stride - 1;
-}
-__device__ inline bool levels_tile_the_keys(const KArgs& a)
-{
-    return levels_tile_the_keys_of(a, [&](int l) { return load_level(a, l); });
-}
+// What the kernels of the backward need to know of the levels, one level per lane of a wavefront.  Every workgroup goes through this
+// before it starts: walked through one level after the other it is a chain of memory and LDS latencies that short work items wait
+// for longer than they work (backward of 900 queries, two images, float32: first kernel 18.4 -> 15.5 us).
+struct LevelLanes {
+    i32x4 geo;       // this lane's level {H, W, first key, 0}; zeros past the last level
+    int32_t px, nt;  // its pixels inside the value tensor, its tiles in the run table
+    int32_t first;   // number of its first tile (tiles are numbered level by level); -1: the table has no room for its tiles
+    int32_t chunks;  // query chunks per tile
+    // Whether the levels tile the keys exactly and in order -- the first level starts at key 0, every other one where the
+    // one before it ends, the last one ends at key nk -- and all their tiles fit the run table.  Only then is every row of
+    // grad_value covered by exactly one tile, which is what lets the owner of a tile store its rows (instead of adding to
+    // them) and lets the rows that nobody adds to go without zeros.  level_start_index is the caller's: for any other
+    // layout (keys that no level covers, levels out of order or overlapping) every row is zero-filled and every tile adds
+    // its sums with atomics.
+    bool canonical;
 
-// Rows (pixels of a batch element) [*r0, *r1) of piece `part` (< kRowParts) of tile `tile` of a batch element that
-// receive atomic additions in the tile pass; false when there is no such tile.  Tiles are numbered level by level as
-// in the first kernel and the tile pass.
-template <typename GetLevel>
-__device__ inline bool atomic_rows_of_part_of(const KArgs& a, GetLevel level, int32_t tile, int32_t part, int32_t* r0, int32_t* r1)
-{
-    int32_t first = 0;
-    for (int l = 0; l < a.nl; ++l) {
-        const i32x4 L = level(l);
-        int32_t P;
-        const int32_t nt = level_tile_count(L.x, L.y, L.z, a.nk, a.tile_px_log2, &P);
-        if (first + nt > a.tbl_stride - 1) continue;  // (a level that does not fit the run table has no tiles)
-        if (tile < first + nt) {
-            const int32_t ti = tile - first, tile_px = 1 << a.tile_px_log2;
-            const int32_t p0 = L.z + ti * tile_px;
-            const int32_t npx = (P - ti * tile_px) < tile_px ? (P - ti * tile_px) : tile_px;
-            if (tile_stored_directly(level_tile_chunks(a, nt), npx, a.tile_px_log2)) {
-                *r0 = p0;
-                *r1 = part == 0 ? p0 + 1 : p0;
-            } else {
-                const int per = tile_px / kRowParts;
-                *r0 = p0 + (part * per < npx ? part * per : npx);
-                *r1 = p0 + ((part + 1) * per < npx ? (part + 1) * per : npx);
+    // (by whole wavefronts: the lanes exchange values)
+    __device__ LevelLanes(const KArgs& a, int lane)
+    {
+        geo = lane < a.nl ? load_level(a, lane) : i32x4{0, 0, 0, 0};
+        const int32_t tiles = level_tile_count(geo.x, geo.y, geo.z, a.nk, a.tile_px_log2, &px), room = a.tbl_stride - 1;
+        const int32_t inc = prefix(a, tiles, lane), total = __builtin_amdgcn_readlane(inc, a.nl - 1);
+        nt = tiles;
+        first = inc - tiles;
+        if (total > room) {
+            // levels that overlap: one whose tiles find no room is left out, a later one may still fit
+            nt = 0;
+            first = -1;
+            int32_t at = 0;
+            for (int l = 0; l < a.nl; ++l) {
+                const int32_t n = __builtin_amdgcn_readlane(tiles, l);
+                if (at + n > room) continue;
+                if (lane == l) nt = n, first = at;
+                at += n;
             }
-            return true;
         }
-        first += nt;
+        const int64_t p = (int64_t)geo.x * geo.y;
+        const bool inside = geo.x > 0 && geo.y > 0 && geo.z >= 0 && p <= (int64_t)a.nk - geo.z;
+        const int32_t end = inside ? geo.z + (int32_t)p : -1, before = __shfl_up(end, 1, kWave);
+        const bool follows = inside && geo.z == (lane == 0 ? 0 : before);
+        canonical = __ballot(lane < a.nl && !follows) == 0 && __builtin_amdgcn_readlane(end, a.nl - 1) == a.nk && total <= room;
+        chunks = nt > 0 ? level_tile_chunks(a, nt) : 0;
     }
-    return false;
-}
-__device__ inline bool atomic_rows_of_part(const KArgs& a, int32_t tile, int32_t part, int32_t* r0, int32_t* r1)
-{
-    return atomic_rows_of_part_of(a, [&](int l) { return load_level(a, l); }, tile, part, r0, r1);
-}
+    // inclusive sum over the levels
+    static __device__ int32_t prefix(const KArgs& a, int32_t v, int lane)
+    {
+        for (int d = 1; d < a.nl; d <<= 1) {
+            const int32_t o = __shfl_up(v, d, kWave);
+            if (lane >= d) v += o;
+        }
+        return v;
+    }
+    // {H, W, first key, 0} of level l (the same in all lanes)
+    __device__ int32_t H(int l) const { return __builtin_amdgcn_readlane(geo.x, l); }
+    __device__ int32_t W(int l) const { return __builtin_amdgcn_readlane(geo.y, l); }
+    __device__ int32_t base(int l) const { return __builtin_amdgcn_readlane(geo.z, l); }
+
+    // Rows (pixels of a batch element) [*r0, *r1) of piece `part` (< kRowParts) of tile `tile` of a batch element that
+    // receive atomic additions in the tile pass; false when there is no such tile.
+    __device__ bool atomic_rows_of_part(const KArgs& a, int32_t tile, int32_t part, int32_t* r0, int32_t* r1) const
+    {
+        const uint64_t owner = __ballot(first >= 0 && tile >= first && tile < first + nt);
+        if (owner == 0) return false;
+        const int l = __builtin_ctzll(owner);
+        const int32_t ti = tile - __builtin_amdgcn_readlane(first, l), tile_px = 1 << a.tile_px_log2, P = __builtin_amdgcn_readlane(px, l);
+        const int32_t p0 = base(l) + ti * tile_px;
+        const int32_t npx = (P - ti * tile_px) < tile_px ? (P - ti * tile_px) : tile_px;
+        if (tile_stored_directly(__builtin_amdgcn_readlane(chunks, l), npx, a.tile_px_log2)) {
+            *r0 = p0;
+            *r1 = part == 0 ? p0 + 1 : p0;
+        } else {
+            const int per = tile_px / kRowParts;
+            *r0 = p0 + (part * per < npx ? part * per : npx);
+            *r1 = p0 + ((part + 1) * per < npx ? (part + 1) * per : npx);
+        }
+        return true;
+    }
+};
 
 // Where a kernel takes the location and the weight of sample s of unit (b, q, h) from.
 enum : int { kSrcPlain = 0, kSrcFused = 1, kSrcGka = 2, kSrcGrid = 3 };
