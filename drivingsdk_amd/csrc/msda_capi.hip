@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "dagg.h"
+#include "gka.h"
 #include "grid_planes.h"
 #include "msda_device.h"
 
@@ -163,6 +164,7 @@ int ensure_device_ready()
     e = mxd::raise_forward_lds();
     if (e == hipSuccess) e = mxd::raise_forward_cu_lds();
     if (e == hipSuccess) e = mxd::raise_grid_lds();
+    if (e == hipSuccess) e = mxd::raise_gka_lds();
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "raising the dynamic LDS limit failed: %s", hipGetErrorString(e));
     void* ptr = nullptr;
     e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));  // (this device's copy of the array: the device is current)
@@ -860,6 +862,78 @@ struct DaggSpace {
     }
 };
 
+int64_t ceil_div(int64_t x, int64_t y) { return (x + y - 1) / y; }
+
+// Workgroups per (batch, head) such that `slots` of them run side by side: as many rounds of whole launches as cost least, each
+// paying `fixed` (in units of one query's work) before its queries.
+int64_t gka_splits(int64_t slabs, int64_t nq, int64_t slots, double fixed, int64_t least)
+{
+    int64_t best = 1;
+    double best_cost = -1.0;
+    for (int64_t s = 1; s <= 64 && (s == 1 || nq / s >= least); ++s) {
+        const double cost = (double)ceil_div(slabs * s, slots) * ((double)ceil_div(nq, s) + fixed);
+        if (best_cost < 0.0 || cost < best_cost) {
+            best_cost = cost;
+            best = s;
+        }
+    }
+    return best;
+}
+
+// Geometric kernel attention with the (batch, head)'s slab of value in LDS (gka.hip): whether a problem's slab, in the dtype for the
+// gather and as float32 sums in registers for grad_value, fits, and the launch geometry.
+bool gka_plan(int dtype, const Dims& d, mxd::GkaArgs* a)
+{
+    memset(a, 0, sizeof(*a));
+    const int es = elem_size(dtype);
+    const int64_t row = d.hd * es, lanes = row / 16, sc_lanes = d.hd / 4, S = d.nl * d.np;
+    if (tuning().bwd_atomic || row % 16 != 0 || (lanes & (lanes - 1)) != 0 || lanes < 2 || lanes > 32) return false;
+    if (sc_lanes > 64 || d.nk >= 32768 || S > 256 || d.nl != d.nl_attn || d.bs * d.nh > 65536) return false;
+    a->bs = (int32_t)d.bs;
+    a->nk = (int32_t)d.nk;
+    a->nh = (int32_t)d.nh;
+    a->hd = (int32_t)d.hd;
+    a->nl = (int32_t)d.nl;
+    a->np = (int32_t)d.np;
+    a->nq = (int32_t)d.nq;
+    a->S = (int32_t)S;
+    a->np_magic = (uint32_t)(((1u << 20) + d.np - 1) / d.np);
+    a->s_magic = (uint32_t)(((1u << 20) + S - 1) / S);
+    a->lpr_log2 = log2_lanes((int)lanes);
+    // gather: two workgroups of 8 wavefronts per CU, or one of 16
+    const int64_t slab = (d.nk + 1) * row, strip = (64 / lanes) * mxd::kChunkStride * 8, lim = mxd::kCuLdsBytes - 256;
+    const int64_t lds2 = mxd::kGkaLevelBytes + slab + 8 * strip, lds1 = mxd::kGkaLevelBytes + slab + 16 * strip;
+    const bool two = 2 * lds2 <= lim || lds1 > lim;
+    a->block = two ? 512 : 1024;
+    a->lds = (uint32_t)(two ? lds2 : lds1);
+    if (a->lds > lim) return false;
+    const int64_t slabs = d.bs * d.nh;
+    int64_t s = gka_splits(slabs, d.nq, 2 * (int64_t)a->lds <= lim ? 512 : 256, (double)d.nk / 2, 64 / lanes * (a->block / 64));
+    a->split_q = (int32_t)ceil_div(d.nq, s);
+    a->splits = (int32_t)ceil_div(d.nq, a->split_q);
+    // grad_value: tiles of queries that let two workgroups share a CU's LDS
+    a->sc_lanes_log2 = log2_lanes((int)sc_lanes);
+    a->sc_block = ceil_div(d.nk, 512 / sc_lanes) <= mxd::kGkaPixels ? 512 : 1024;
+    a->sc_px = (int32_t)ceil_div(d.nk, a->sc_block / sc_lanes);
+    if (a->sc_px > mxd::kGkaPixels) return false;
+    const int64_t room = (a->sc_block == 512 ? lim / 2 : lim) - mxd::kGkaLevelBytes - (2 * d.nk + 1) * 4 - 32;
+    int64_t tile = room / (row + S * 8);
+    if (tile > mxd::kGkaSamples * a->sc_block / S) tile = mxd::kGkaSamples * a->sc_block / S;
+    if (tile * S * S >= (1 << 20)) tile = (1 << 20) / (S * S) - 1;
+    if (tile > 4088) tile = 4088;  // (32-bit products of the division by S)
+    if (tile > d.nq) tile = d.nq;
+    if (tile >= 8) tile &= ~(int64_t)7;
+    if (tile < 8 && tile < d.nq) return false;
+    a->sc_tile_q = (int32_t)tile;
+    s = gka_splits(slabs, d.nq, a->sc_block == 512 ? 512 : 256, (double)tile, tile);
+    a->sc_split_q = (int32_t)ceil_div(d.nq, s);
+    a->sc_splits = (int32_t)ceil_div(d.nq, a->sc_split_q);
+    a->sc_lds = (uint32_t)(mxd::kGkaLevelBytes + ((tile * S * 8 + 15) & ~15) + tile * row + (2 * d.nk + 1) * 4);
+    return true;
+}
+
+size_t gka_part_bytes(const mxd::GkaArgs& a) { return (size_t)a.sc_splits * a.bs * a.nk * a.nh * a.hd * sizeof(float); }
+
 // Grid sampler on planes: whether a plane fits the LDS of a CU (as float32, whatever the dtype) and every index its type.
 bool grid_planes_fit(int64_t n, int64_t c, int64_t h, int64_t w, int64_t h_out, int64_t w_out)
 {
@@ -890,8 +964,6 @@ int grid_planes_args(int dtype, int64_t n, int64_t c, int64_t h, int64_t w, int6
 }
 
 constexpr int64_t kGridFill = 512;  // workgroups aimed at: two per CU
-
-int64_t ceil_div(int64_t x, int64_t y) { return (x + y - 1) / y; }
 
 // Planes of `bytes` that a workgroup takes when `items` of them have to be shared out.
 int64_t grid_planes_together(int64_t bytes, int64_t c, int64_t n)
@@ -1061,8 +1133,27 @@ int mxd_gka_forward(const void* value, const int32_t* spatial_shapes, const int3
                     const void* sampling_locations, const void* attn_weights, void* output, int dtype, int64_t bs,
                     int64_t nk, int64_t nh, int64_t hd, int64_t nl, int64_t nq, int64_t np, void* hip_stream)
 {
-    return forward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, output, dtype,
-                          bs, nk, nh, hd, nl, nl, nq, np, hip_stream);
+    int code = dtype;
+    const int meta64 = take_meta_flag(&code);
+    const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
+    mxd::GkaArgs a;
+    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, &a))
+        return forward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, output, dtype,
+                              bs, nk, nh, hd, nl, nl, nq, np, hip_stream);
+    if (!value || !spatial_shapes || !level_start_index || !sampling_locations || !attn_weights || !output)
+        return fail(MXD_E_NULL, "mxd_gka_forward: NULL data pointer");
+    const int rc = ensure_device_ready();
+    if (rc != MXD_OK) return rc;
+    a.meta_i64 = meta64;
+    a.value = value;
+    a.shapes = spatial_shapes;
+    a.lsi = level_start_index;
+    a.loc = static_cast<const float*>(sampling_locations);
+    a.attn = attn_weights;
+    a.out = output;
+    const hipError_t e = mxd::launch_gka_forward(code, a, static_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_gka_forward: launch failed: %s", hipGetErrorString(e));
+    return MXD_OK;
 }
 
 static int grid_mode(int interpolation_mode, int padding_mode, int align_corners)
@@ -1339,6 +1430,11 @@ int mxd_msda_backward_static(const void* value, const int32_t* spatial_shapes, c
 size_t mxd_gka_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk, int64_t nh, int64_t hd, int64_t nl,
                                         int64_t nq, int64_t np)
 {
+    int code = dtype;
+    take_meta_flag(&code);
+    const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
+    mxd::GkaArgs a;
+    if (check_dims(code, d) == MXD_OK && gka_plan(code, d, &a)) return gka_part_bytes(a);
     return mxd_msda_backward_workspace_bytes(dtype, bs, nk, nh, hd, nl, nl, nq, np);
 }
 
@@ -1348,9 +1444,37 @@ int mxd_gka_backward(const void* value, const int32_t* spatial_shapes, const int
                      int64_t bs, int64_t nk, int64_t nh, int64_t hd, int64_t nl, int64_t nq, int64_t np,
                      void* hip_stream)
 {
-    return backward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, grad_output,
-                           grad_value, nullptr, grad_attn_weights, workspace, workspace_bytes, dtype, bs, nk, nh, hd, nl,
-                           nl, nq, np, 0, hip_stream);
+    int code = dtype;
+    const int meta64 = take_meta_flag(&code);
+    const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
+    mxd::GkaArgs a;
+    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, &a))
+        return backward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, grad_output,
+                               grad_value, nullptr, grad_attn_weights, workspace, workspace_bytes, dtype, bs, nk, nh, hd, nl,
+                               nl, nq, np, 0, hip_stream);
+    if (!value || !spatial_shapes || !level_start_index || !sampling_locations || !attn_weights || !grad_output || !grad_value ||
+        !grad_attn_weights)
+        return fail(MXD_E_NULL, "mxd_gka_backward: NULL data pointer");
+    const size_t need = gka_part_bytes(a);
+    if (!workspace || workspace_bytes < need)
+        return fail(MXD_E_WORKSPACE, "mxd_gka_backward: workspace of %zu bytes required, %zu given", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    if (reinterpret_cast<uintptr_t>(workspace) & 15u) return fail(MXD_E_WORKSPACE, "mxd_gka_backward: workspace must be 16-byte aligned");
+    const int rc = ensure_device_ready();
+    if (rc != MXD_OK) return rc;
+    a.meta_i64 = meta64;
+    a.value = value;
+    a.shapes = spatial_shapes;
+    a.lsi = level_start_index;
+    a.loc = static_cast<const float*>(sampling_locations);
+    a.attn = attn_weights;
+    a.grad_out = grad_output;
+    a.grad_value = grad_value;
+    a.grad_attn = grad_attn_weights;
+    a.part = static_cast<float*>(workspace);
+    const hipError_t e = mxd::launch_gka_backward(code, a, static_cast<hipStream_t>(hip_stream));
+    if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_gka_backward: launch failed: %s", hipGetErrorString(e));
+    return MXD_OK;
 }
 
 size_t mxd_grid_sampler2d_backward_workspace_bytes(int dtype, int64_t n, int64_t c, int64_t h_in, int64_t w_in,
