@@ -4,11 +4,12 @@
 
 namespace mxd {
 
-constexpr int kDaggWaves = 4;        // wavefronts per workgroup of the forward and of the backward's first kernel: an anchor each
+constexpr int kDaggWaves = 4;        // wavefronts per workgroup of the forward: an anchor each
+constexpr int kDaggBackWaves = 8;    // the same for the backward's first kernel, whose sort is the shorter for it (442 anchors: 52 -> 44 us with 8, 43 with
+                                     // 16; 6 x 900 anchors lose 5 % with 16)
 constexpr int kDaggList = 128;       // locations of an anchor that a wavefront looks through before it samples
 constexpr int kDaggSortPx = 4096;    // pixels of a level that a workgroup of the sort counts in LDS
 constexpr int kDaggStrip = 8;        // neighbouring pixels whose gradient rows are formed together
-constexpr int kDaggStripRecords = 1024;  // records per strip aimed at where the strips of a level are split
 
 struct DaggArgs {
     const void* feat;      // [bs, nf, C]
@@ -40,6 +41,7 @@ struct DaggArgs {
     int32_t lpr_log2;      // lanes that share it
     // grad_feat: lanes that share a pixel row, channel blocks per row
     int32_t row_lpr_log2, row_blocks, sort_ranges;
+    int32_t strip_records; // records per strip aimed at where the strips of a level are split
     mxd_msda_plan map;     // XCD mapping: piece = head, anchor = query
 };
 

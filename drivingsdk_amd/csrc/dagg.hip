@@ -322,39 +322,57 @@ struct DaggLevels {
     int32_t first[kMaxLevels + 1];  // work items of the levels before it
     int32_t tiled;               // the levels tile the keys in order: a pixel row belongs to one level
 
-    // by the first wavefronts of the workgroup; a barrier is needed behind it
+    // (a level per lane of the first wavefront: one after the other, 24 levels were 5 us in front of every workgroup)
     __device__ void fill(const DaggArgs& a)
     {
-        for (int l = threadIdx.x; l < a.nl; l += blockDim.x) {
-            const i32x4 L = dagg_level(a, l);
+        static_assert(kMaxLevels <= kWave, "a lane per level");
+        if (threadIdx.x < kWave) {
+            const int lane = (int)threadIdx.x;
+            const i32x4 L = lane < a.nl ? dagg_level(a, lane) : i32x4{0, 0, 0, 0};
             int32_t P;
             level_tile_count(L.x, L.y, L.z, a.nf, 0, &P);
-            H[l] = L.x;
-            W[l] = L.y;
-            base[l] = L.z;
-            px[l] = P;
-            // records of a strip if every location were inside and spread evenly
-            const float expect = P > 0 ? 2.0f * (float)a.A * (float)a.P * (float)(kDaggStrip + 1) / (float)P : 0.0f;
-            int32_t n = (int32_t)__builtin_ceilf(expect / (float)kDaggStripRecords);
-            chunks[l] = n < 1 ? 1 : n > 64 ? 64 : n;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
+            auto prefix = [&](int64_t v) {
+                for (int d = 1; d < a.nl; d <<= 1) {
+                    const int64_t o = __shfl_up(v, d, kWave);
+                    if (lane >= d) v += o;
+                }
+                return v;
+            };
+            const int64_t p = (int64_t)L.x * L.y;
+            const bool whole = L.x > 0 && L.y > 0 && p == P;
+            const int32_t end = L.z + P, before = __shfl_up(end, 1, kWave);
+            const bool follows = whole && L.z == (lane == 0 ? 0 : before);
+            tiled = __ballot(lane < a.nl && !follows) == 0 && __builtin_amdgcn_readlane(end, a.nl - 1) == a.nf;
             // (levels that overlap so far that their pixels are more than the tensor has do not fit the table of record
             //  starts: they are left out of grad_feat)
-            int64_t next = 0, room = 0;
-            int32_t items = 0, ok = 1;
-            for (int l = 0; l < a.nl; ++l) {
-                ok = ok && H[l] > 0 && W[l] > 0 && (int64_t)base[l] == next && (int64_t)H[l] * W[l] == px[l];
-                next += px[l];
-                if (room + px[l] + 1 > (int64_t)a.nf + a.nl) px[l] = 0;
-                csr[l] = (int32_t)room;
-                if (px[l] > 0) room += px[l] + 1;
-                first[l] = items;
-                items += (px[l] + kDaggStrip - 1) / kDaggStrip * chunks[l];
+            int64_t used = P > 0 ? P + 1 : 0, at = prefix(used) - used;
+            if (__ballot(at + used > (int64_t)a.nf + a.nl) != 0) {
+                int64_t room = 0;
+                for (int l = 0; l < a.nl; ++l) {
+                    const int32_t u = __builtin_amdgcn_readlane((int32_t)used, l);
+                    const bool fits = room + u <= (int64_t)a.nf + a.nl;
+                    if (lane == l) {
+                        at = room;
+                        if (!fits) P = 0;
+                    }
+                    if (fits) room += u;
+                }
             }
-            first[a.nl] = items;
-            tiled = ok && next == a.nf;
+            // records of a strip if every location were inside and spread evenly
+            const float expect = P > 0 ? 2.0f * (float)a.A * (float)a.P * (float)(kDaggStrip + 1) / (float)P : 0.0f;
+            int32_t n = (int32_t)__builtin_ceilf(expect / (float)a.strip_records);
+            n = n < 1 ? 1 : n > 64 ? 64 : n;
+            const int32_t items = (P + kDaggStrip - 1) / kDaggStrip * n, upto = (int32_t)prefix(items);
+            if (lane < a.nl) {
+                H[lane] = L.x;
+                W[lane] = L.y;
+                base[lane] = L.z;
+                px[lane] = P;
+                csr[lane] = (int32_t)at;
+                chunks[lane] = n;
+                first[lane] = upto - items;
+                if (lane == a.nl - 1) first[a.nl] = upto;
+            }
         }
         __syncthreads();
     }
@@ -366,14 +384,14 @@ struct DaggLevels {
 // into starts, and drops every record at its place.
 struct DaggSort {
     DaggLevels lv;
-    uint32_t wsum[kDaggWaves];
+    uint32_t wsum[kDaggBackWaves];
     uint32_t before_s;
     uint32_t cnt[kDaggSortPx];
 };
 template <typename T>
-__device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, uint32_t blocks, unsigned char* smem)
+__device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned char* smem)
 {
-    constexpr int kThreads = kDaggWaves * kWave;
+    constexpr int kThreads = kDaggBackWaves * kWave;
     DaggSort& sh = *reinterpret_cast<DaggSort*>(smem);
     DaggLevels& lv = sh.lv;
     uint32_t *cnt = sh.cnt, *wsum = sh.wsum, &before_s = sh.before_s;
@@ -381,15 +399,6 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, uint32_t blo
     const int range = block % a.sort_ranges, l = block / a.sort_ranges % a.nl, b = block / a.sort_ranges / a.nl;
     const int tid = threadIdx.x;
     const int r0 = range * kDaggSortPx, P = lv.px[l], r1 = P - r0 < kDaggSortPx ? P : r0 + kDaggSortPx;
-    if (!lv.tiled) {
-        // rows that several levels share or none has: the whole image gets zeros, and every row is added to
-        const uint64_t n = (uint64_t)a.bs * a.nf * a.C, per = (n + blocks - 1) / blocks;
-        const uint64_t lo = block * per, hi = lo + per < n ? lo + per : n;
-        for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
-    } else if (b < a.bs && lv.chunks[l] > 1 && r0 < P) {
-        const uint64_t lo = ((uint64_t)b * a.nf + lv.base[l] + r0) * a.C, hi = lo + (uint64_t)(r1 - r0) * a.C;
-        for (uint64_t i = lo + tid; i < hi; i += blockDim.x) a.image[i] = 0.0f;
-    }
     if (b >= a.bs || r0 >= P) return;  // (uniform; the launch has a multiple of 8 sort workgroups)
     for (int i = tid; i < kDaggSortPx; i += kThreads) cnt[i] = 0;
     if (tid == 0) before_s = 0;
@@ -469,15 +478,43 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, uint32_t blo
     });
 }
 
-// The two kernels side by side in one launch: the sort has work for a few workgroups, whose time the others' gathers cover
+// Zeros for the rows of grad_feat's float32 image that the kernel behind it adds to: those of levels whose strips are split, or,
+// where the levels do not tile the features (rows that several levels share or none has), all.  (By workgroups of their own: a level's
+// rows zeroed by the workgroup that sorts it kept the launch 100 us longer with 512 channels.)
+constexpr uint32_t kDaggZeroWgs = 128;
+__device__ inline void dagg_zero(const DaggArgs& a, uint32_t block, unsigned char* smem)
+{
+    DaggLevels& lv = reinterpret_cast<DaggSort*>(smem)->lv;
+    lv.fill(a);
+    const uint32_t step = kDaggZeroWgs * blockDim.x;
+    auto zero = [&](uint64_t lo, uint64_t hi) {
+        if (((lo | hi) & 3) == 0 && (reinterpret_cast<uintptr_t>(a.image) & 15) == 0)
+            for (uint64_t i = lo / 4 + block * blockDim.x + threadIdx.x; i < hi / 4; i += step) reinterpret_cast<f32x4*>(a.image)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        else
+            for (uint64_t i = lo + block * blockDim.x + threadIdx.x; i < hi; i += step) a.image[i] = 0.0f;
+    };
+    if (!lv.tiled) {
+        zero(0, (uint64_t)a.bs * a.nf * a.C);
+        return;
+    }
+    for (int l = 0; l < a.nl; ++l)
+        if (lv.chunks[l] > 1)
+            for (int b = 0; b < a.bs; ++b) {
+                const uint64_t lo = ((uint64_t)b * a.nf + lv.base[l]) * a.C;
+                zero(lo, lo + (uint64_t)lv.px[l] * a.C);
+            }
+}
+
+// The kernels side by side in one launch: the sort has work for a few workgroups, whose time the others' gathers cover
 // (131 us as a launch of its own).
 template <typename T, int VEC>
-__global__ __launch_bounds__(kDaggWaves * kWave) void dagg_dots_and_sort_kernel(const DaggArgs a, uint32_t sorts)
+__global__ __launch_bounds__(kDaggBackWaves * kWave) void dagg_dots_and_sort_kernel(const DaggArgs a, uint32_t sorts)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ i32x4 lvl[kMaxLevels];
-    if (blockIdx.x < sorts) dagg_sort<T>(a, blockIdx.x, sorts, smem);
-    else dagg_dots<T, VEC>(a, blockIdx.x - sorts, smem, lvl);
+    if (blockIdx.x < sorts) dagg_sort<T>(a, blockIdx.x, smem);
+    else if (blockIdx.x < sorts + kDaggZeroWgs) dagg_zero(a, blockIdx.x - sorts, smem);
+    else dagg_dots<T, VEC>(a, blockIdx.x - sorts - kDaggZeroWgs, smem, lvl);
 }
 
 // ---- gradient of the feature maps --------------------------------------------------------------------------------------------
@@ -495,7 +532,9 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
     typedef const __attribute__((address_space(4))) u32x4* rec_ptr;
     typedef const __attribute__((address_space(4))) uint32_t* csr_ptr;
     __shared__ DaggLevels lv;
+    __shared__ float turn_all[WAVE ? 256 * VEC : 1];
     lv.fill(a);
+    [[maybe_unused]] float* turn = turn_all + (WAVE ? (threadIdx.x & ~63u) * VEC : 0u);
     auto scalar = [](int v) { return WAVE ? __builtin_amdgcn_readfirstlane(v) : v; };
     const int lpr = 1 << a.row_lpr_log2, units = 256 >> a.row_lpr_log2;
     const int c = threadIdx.x & (lpr - 1);
@@ -539,14 +578,29 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
         int cur = 0;         // pixel of the strip whose sums are in acc
         auto flush = [&]() { // its row is complete
             const size_t row = ((size_t)b * a.nf + lv.base[l] + p0 + cur) * a.C + ch;
-            if (chan_ok) {
-                if (direct) {
-                    RowIO<T, VEC>::store_global(static_cast<T*>(a.grad_feat) + row, acc);
-                } else {
+            if (direct) {
+                if (chan_ok) RowIO<T, VEC>::store_global(static_cast<T*>(a.grad_feat) + row, acc);
+            } else if constexpr (WAVE) {
+                // through LDS, so that neighbouring lanes add to neighbouring channels: an addition is carried out per 64 bytes that
+                // an instruction touches, and a lane's own channels are 4 VEC bytes from the next lane's (6 x 900 anchors,
+                // 256 channels in float32: backward 628 -> 585 us; shorter rows, whose units diverge, lose by it)
+                if (chan_ok) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e)
-                        if (ch + e >= chn && acc[e] != 0.0f) unsafeAtomicAdd(a.image + row + e, acc[e]);
+                        if (ch + e >= chn) turn[ch + e - blk * kWave * VEC] = acc[e];
                 }
+                wave_lds_sync();
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    const int i = blk * kWave * VEC + e * kWave + c;
+                    const float v = i < a.C ? turn[e * kWave + c] : 0.0f;
+                    if (v != 0.0f) unsafeAtomicAdd(a.image + row - ch + i, v);
+                }
+                wave_lds_sync();
+            } else if (chan_ok) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e)
+                    if (ch + e >= chn && acc[e] != 0.0f) unsafeAtomicAdd(a.image + row + e, acc[e]);
             }
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] = nxt[e], nxt[e] = 0.0f;
@@ -696,11 +750,11 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
     hipError_t e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
         constexpr int VEC = decltype(v)::value;
         if constexpr (VEC * sizeof(T) <= 16) {
-            size_t lds = kDaggWaves * kDotsLds;
+            size_t lds = kDaggBackWaves * kDotsLds;
             if (lds < sizeof(DaggSort)) lds = sizeof(DaggSort);
             // (a multiple of 8 sort workgroups: the others keep their places in the XCD mapping)
             const uint32_t sorts = ((uint32_t)(a.bs * a.nl * a.sort_ranges) + kNumXcd - 1) / kNumXcd * kNumXcd;
-            hipLaunchKernelGGL((dagg_dots_and_sort_kernel<T, VEC>), dim3(sorts + a.map.grid), dim3(kDaggWaves * kWave), lds, stream, a, sorts);
+            hipLaunchKernelGGL((dagg_dots_and_sort_kernel<T, VEC>), dim3(sorts + kDaggZeroWgs + a.map.grid), dim3(kDaggBackWaves * kWave), lds, stream, a, sorts);
             return hipGetLastError();
         } else {
             return hipErrorInvalidConfiguration;
@@ -712,7 +766,10 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
         if constexpr (VEC * sizeof(T) <= 16) {
             // enough workgroups to fill the chip eight times over, or a strip per unit
             const int units = 256 >> a.row_lpr_log2;
-            int64_t blocks = ((int64_t)a.bs * ((a.nf + kDaggStrip - 1) / kDaggStrip + a.nl) * a.row_blocks + units - 1) / units;
+            // (strips, and the parts of those that are split: at most one per strip_records records)
+            int64_t items = (a.nf + kDaggStrip - 1) / kDaggStrip + 2 * (int64_t)a.nl;
+            items += 2 * (int64_t)a.nl * a.A * a.P * (kDaggStrip + 1) / kDaggStrip / a.strip_records;
+            int64_t blocks = (a.bs * items * a.row_blocks + units - 1) / units;
             if (blocks > 256 * 32) blocks = 256 * 32;
             const dim3 grid((unsigned)blocks), block(256);
             if (a.hd % VEC != 0) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true, false>), grid, block, 0, stream, a);

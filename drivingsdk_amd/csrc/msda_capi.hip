@@ -821,6 +821,12 @@ int dagg_args(int dtype, int64_t bs, int64_t nf, int64_t C, int64_t cams, int64_
     a->row_lpr_log2 = log2_lanes((C + vec - 1) / vec);
     a->row_blocks = (int32_t)(((C + vec - 1) / vec + mxd::kWave - 1) / mxd::kWave);
     a->sort_ranges = (int32_t)((nf + mxd::kDaggSortPx - 1) / mxd::kDaggSortPx);
+    // A unit of lanes goes through a strip's records one batch after the other, a trip to memory each.  Where the strips alone leave
+    // the chip short of units they are split down to 96 records (829 anchors x 9 points, 4 levels from 58 x 28, 64 channels: 90 us
+    // with parts of 1024 records, 27 with 96, 31 with 64); a split costs zeros and atomic additions, so that strips enough for two
+    // thirds of 16 wavefronts per CU are split only where samples pile up.
+    const int64_t strips = bs * (nf / mxd::kDaggStrip + d.nl) * a->row_blocks, units = 16 * 256 * (mxd::kWave >> a->row_lpr_log2);
+    a->strip_records = 3 * strips >= 2 * units ? 1024 : 96;
     return MXD_OK;
 }
 
@@ -839,8 +845,9 @@ int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
     }
     a->pieces = (a->C + a->piece_ch - 1) / a->piece_ch;
     a->lpr_log2 = log2_lanes((a->piece_ch + vec - 1) / vec);
-    a->map.tile_q = mxd::kDaggWaves;
-    const int64_t grid = fill_xcd_map(&a->map, a->bs, a->pieces, (a->A + mxd::kDaggWaves - 1) / mxd::kDaggWaves);
+    const int waves = backward ? mxd::kDaggBackWaves : mxd::kDaggWaves;
+    a->map.tile_q = waves;
+    const int64_t grid = fill_xcd_map(&a->map, a->bs, a->pieces, (a->A + waves - 1) / waves);
     if (grid >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs %lld workgroups, beyond the launch limit", (long long)grid);
     if ((int64_t)a->bs * a->nl * a->sort_ranges >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs too many workgroups");
     a->map.grid = (uint32_t)grid;
