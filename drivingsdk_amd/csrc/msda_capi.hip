@@ -339,12 +339,6 @@ int preferred_tile_px_log2(const Dims& d)
     const int v = tuning().tile_px_log2;
     if (v >= 7 && v <= mxd::kTilePxLog2Max) return v;
     if (d.hd <= 32) return mxd::kTilePxLog2Max;
-    // Maps so small that a level is a tile of 512 pixels or less keep that tile and take two or four passes: the slots
-    // of the workgroup that the tile leaves free are what a pixel that collects far more entries than the others gets
-    // its extra lists from, and a tile cut in two has none (geometric kernel attention at 15 x 25 pixels and 64 channels,
-    // where clamping piles half of the samples on the border: 0.80 ms per step with one tile of 375 pixels and two
-    // passes, 0.90 ms with tiles of 256 + 119 pixels and one).
-    if (d.nk <= (int64_t)d.nl << mxd::kTilePxLog2Max) return mxd::kTilePxLog2Max;
     // (measured at 8 heads x 128 channels, encoder levels: float16 backward 588 us with tiles of 512 pixels, 431 with 256,
     //  383 with 128; float32 722, 590, 586)
     return d.hd <= 64 ? 8 : 7;
@@ -467,7 +461,10 @@ int make_tile_args(const Dims& d, const BwdLayout& L, int accumulate, mxd::TileA
                 best_c = c;
             }
         }
-        target = (per_tile + best_c - 1) / best_c;
+        // (few records: a tile split in two pays zeros, atomic additions and, in 16 bits, a rounding pass for its rows, which weighs
+        //  more than an item that lasts longer -- 28 x 57 pixels, 1596 queries x 2, 128 channels, bfloat16: 57 -> 37 us)
+        const int64_t equal = (per_tile + best_c - 1) / best_c;
+        if (target >= 8192 || equal > target) target = equal;
     }
     t->target = tuning().tile_target > 0 ? tuning().tile_target : (int)target;
     if (t->target < 128) t->target = 128;
