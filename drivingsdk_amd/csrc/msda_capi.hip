@@ -769,6 +769,9 @@ void fill_args(mxd::KArgs* a, int dtype, const Dims& d)
     a->nq = (int32_t)d.nq;
     a->S = (int32_t)(d.nl * d.np);
     a->S_full = (int32_t)(d.nl_attn * d.np);
+    const int64_t S = d.nl * d.np, n0 = S < mxd::kChunk ? S : mxd::kChunk, n1 = S % mxd::kChunk ? S % mxd::kChunk : mxd::kChunk;
+    a->chunk_magic = (uint32_t)(((1 << 16) + n0 - 1) / n0);
+    a->tail_magic = (uint32_t)(((1 << 16) + n1 - 1) / n1);
     a->np_magic = (uint32_t)(((1u << 20) + d.np - 1) / d.np);
     a->pitch_bytes = (uint32_t)(d.nh * d.hd * es);
     a->batch_bytes = (uint32_t)(d.nk * d.nh * d.hd * es);

@@ -80,6 +80,8 @@ struct KArgs {
     int32_t bs, nk, nh, hd, nl, np, nq;
     int32_t S;             // nl*np: samples per unit that are evaluated
     int32_t S_full;        // nl_attn*np: samples per unit that are stored
+    uint32_t chunk_magic;  // ceil(2^16/n) for the samples n of a unit's first pass (at most kChunk) ...
+    uint32_t tail_magic;   // ... and of its last one
     uint32_t np_magic;     // ceil(2^20/np): s/np == (s*np_magic)>>20 while s*np < 2^20
     uint32_t pitch_bytes;  // nh*hd*sizeof(T): distance between neighbouring pixels of value
     uint32_t batch_bytes;  // nk*pitch_bytes

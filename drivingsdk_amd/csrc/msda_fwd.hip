@@ -129,15 +129,19 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
     // A sample as it is read from memory, and its way into the staging strip.
     struct RawSample {
         float x, y, aw;
-        int l, u;
+        int l, u, sl;
         bool active;
     };
+    // Samples of a pass: `ns` (at most kChunk) of each unit, packed, so that units of few samples do not leave lanes without one
+    // (2 levels x 4 points, bfloat16, 6 x 1199 queries: 16.9 -> 14.9 us).
+    int ns = a.S < kChunk ? a.S : kChunk;
+    uint32_t ns_magic = a.chunk_magic;  // ceil(2^16 / ns)
     auto fetch = [&](int q0, int c0, int i) -> RawSample {
         RawSample r;
-        r.u = i >> 4;
-        const int sl = i & (kChunk - 1);
-        const int s = c0 + sl, q = q0 + r.u;
-        r.active = (i < entries) && (q < wk.q_end) && (s < a.S);
+        r.u = (int)(((uint32_t)i * ns_magic) >> 16);
+        r.sl = i - r.u * ns;
+        const int s = c0 + r.sl, q = q0 + r.u;
+        r.active = (i < U * ns) && (q < wk.q_end);
         r.x = 0.f, r.y = 0.f, r.aw = 0.f, r.l = 0;
         if (r.active) {
             const SampleRef sr = sample_ref<SRC>(a, wk.b, q, wk.h, s);
@@ -153,8 +157,7 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
         }
         return r;
     };
-    auto place = [&](const RawSample& r, int i) {
-        const int sl = i & (kChunk - 1);
+    auto place = [&](const RawSample& r) {
         const Sample sm = source_geometry<SRC>(r.x, r.y, lvl[r.l], a.nk, r.active, a.grid);
         Entry en;
 #pragma unroll
@@ -167,7 +170,7 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
                 if (r.l >= c_first) en.off[k] = (uint32_t)(sm.cvalid[k] ? sm.pix[k] - c_base : c_rows) * row_bytes;
             }
         }
-        stage[r.u * kChunkStride + sl] = en;
+        stage[r.u * kChunkStride + r.sl] = en;
     };
     // AHEAD (one chunk of samples per unit, at most two samples per lane; chosen by the launcher): the samples of an
     // iteration are requested before the gather of the iteration before it, so their way from memory is covered by
@@ -210,12 +213,16 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
         }
 
         for (int c0 = 0; c0 < a.S; c0 += kChunk) {
+            if (!ahead) {
+                ns = a.S - c0 < kChunk ? a.S - c0 : kChunk;
+                ns_magic = ns == kChunk ? 65536u / kChunk : a.tail_magic;
+            }
             // ---- geometry: one sample per lane --------------------------------------------
             if (ahead) {
-                if (lane < entries) place(nxt[0], lane);
-                if (lane + kWave < entries) place(nxt[1], lane + kWave);
+                if (lane < U * ns) place(nxt[0]);
+                if (lane + kWave < U * ns) place(nxt[1]);
             } else {
-                for (int i = lane; i < entries; i += kWave) place(fetch(q0, c0, i), i);
+                for (int i = lane; i < U * ns; i += kWave) place(fetch(q0, c0, i));
             }
             wave_lds_sync();
             if (ahead) {
@@ -226,7 +233,6 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
             }
 
             // ---- gather + weighted sum ----------------------------------------------------
-            const int ns = (a.S - c0) < kChunk ? (a.S - c0) : kChunk;
             const Entry* mine = stage + g * kChunkStride;
             // samples are level-major: those of the cached levels are the tail of the unit's list
             int n_mem = ns;
