@@ -152,7 +152,10 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     // ---- records per tile of this workgroup: count, prefix, publish -----------------------
     int32_t* cursor = tile_first + kMaxLevels;  // [tbl_stride] counts, then next free position per tile
     uint32_t* slab = nullptr;
-    const int entries = U * kChunk;
+    // Lanes of a pass per unit: 16, or 8 or 4 for queries of so few samples, whose geometry and gradients then take half or a quarter
+    // of the passes (aligned groups of 4 lanes belong to one query either way: the merging of records relies on it).
+    const int pk = a.S <= 4 ? 2 : a.S <= 8 ? 3 : 4, pk_mask = (1 << pk) - 1;
+    const int entries = U << pk;
     // ---- per unit: the grad_out row in the value-load layout and, for the fused form, the softmax terms ----
     float gv[NPASS][VEC];
     // 16-bit rows: the same row as packed pairs, for dot products that multiply two pairs of 16-bit elements exactly
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             for (int d = 1; d < LPR; d <<= 1) dsum += __shfl_xor(dsum, d, kWave);
             if (c == 0 && g < U) unit_stats(g)[2] = dsum;
             // softmax statistics: lanes 16u..16u+15 share unit u, each takes every 16th logit
-            for (int i = lane; i < entries; i += kWave) {
+            for (int i = lane; i < U * kChunk; i += kWave) {
                 const int u = i >> 4, sl = i & (kChunk - 1), q = q0 + (u >> sp);
                 const T* lg = attn + (((int64_t)wk.b * a.nq + (q < wk.q_end ? q : wk.q_begin)) * a.nh + wk.h) * a.S_full;
                 float m = -__builtin_inff();
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
         };
         auto read_sample = [&](int i) -> Read {
             Read r{0.f, 0.f, 0.f, 0, false};
-            const int u = i >> 4, sl = i & (kChunk - 1);
+            const int u = i >> pk, sl = i & pk_mask;
             const int s = c0 + ((u & sp_mask) << 4) + sl, q = q0 + (u >> sp);
             r.active = (i < entries) && (q < wk.q_end) && (s < a.S);
             if (r.active) {
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
         };
         auto stage_sample = [&](auto ks_c, int i, const Read& rd) {
             constexpr int ks = decltype(ks_c)::value;  // (which registers keep the sample; i = lane + ks * 64 then)
-            const int u = i >> 4, sl = i & (kChunk - 1);
+            const int u = i >> pk, sl = i & pk_mask;
             const bool active = rd.active;
             const float x = rd.x, y = rd.y, aw = rd.aw;
             const int l = rd.l;
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             for (int ks = 0; ks < kLaneSamples; ++ks) {
                 const int i = lane + ks * kWave;
                 if (i >= entries) break;
-                const int u = i >> 4, sl = i & (kChunk - 1);
+                const int u = i >> pk, sl = i & pk_mask;
                 const int s = c0 + ((u & sp_mask) << 4) + sl, q = q0 + (u >> sp);
                 // the sample's pair records (upper and lower corners), written after the gradients
                 bool rec_have[2] = {false, false};
