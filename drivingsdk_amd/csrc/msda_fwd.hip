@@ -240,7 +240,8 @@ __global__ __launch_bounds__(LDSC ? 512 : 256) void msda_fwd_kernel(const KArgs 
                 n_mem = c_first * a.np - c0;
                 n_mem = n_mem < 0 ? 0 : (n_mem > ns ? ns : n_mem);
             }
-#pragma unroll 4
+            // (two samples' rows in flight per wavefront: four take 100 registers, and the wavefronts that they cost fetch more)
+#pragma unroll 2
             for (int sl = 0; sl < n_mem; ++sl) {
                 const u32x4 off = *reinterpret_cast<const u32x4*>(mine[sl].off);
                 const f32x4 w = *reinterpret_cast<const f32x4*>(mine[sl].w);
