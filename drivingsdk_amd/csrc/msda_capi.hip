@@ -280,7 +280,10 @@ int backward_lane_bytes(int dtype, const Dims& d)
     // staging strips of a workgroup take 51 KiB of LDS, which leaves 3 wavefronts per SIMD, and a lane stages four
     // samples of which it keeps two in registers (measured, encoder shape in float16 / bfloat16: backward 322 -> 300 us;
     // BEVFormer shape in float16 1114 -> 1075 us; with rows of 256 bytes halving the lane width costs 10 %).
+    // Rows of up to 32 bytes: 8 lanes of 4, from 5 samples per query on (16 channels in float16, 2 x 13253 queries of 18 samples:
+    // backward 289 -> 251 us; 3 samples 53 -> 55).
     const int64_t row = d.hd * elem_size(dtype);
+    if (row > 16 && row <= 32) return d.nl * d.np > 4 ? 4 : 16;
     return (row > 32 && row <= 64) ? 8 : 16;
 }
 
@@ -685,6 +688,9 @@ int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_
         if (plan_forward_cu(dtype, d, vec, lpr, npass, p, level_cache)) return MXD_OK;
     }
     if (cu_form) *cu_form = 0;
+    // (a row is shared by four lanes at least: 8 bytes each for rows of 32 -- 16 channels in float16, 2 x 13253 queries of 18
+    //  samples: forward 75 -> 63 us)
+    if (!backward && d.hd * es <= 32 && lane_bytes > 8) row_geometry(es, d.hd, 8, &vec, &lpr, &npass, false, whole_pieces);
     memset(p, 0, sizeof(*p));
     p->vec = vec;
     p->lanes_per_row = lpr;
