@@ -23,7 +23,10 @@ struct GkaArgs {
     int32_t bs, nk, nh, hd, nl, np, nq, S;
     uint32_t np_magic;     // ceil(2^20 / np)
     uint32_t s_magic;      // ceil(2^20 / S)
-    int32_t lpr_log2;      // lanes of 16 bytes that share a row
+    // maps too large for LDS with whole rows: the channels of a head in parts, each with workgroups of its own
+    int32_t parts, part_ch;
+    float* dots;           // [parts][bs, nq, nh, S]: the parts' dots, where there are several
+    int32_t lpr_log2;      // lanes of 16 bytes that share a part's row
     // forward and dots: workgroups per (batch, head), queries each
     int32_t splits, split_q, block;
     uint32_t lds;

@@ -71,6 +71,8 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
     uint32_t wg = xcd_order(blockIdx.x, gridDim.x);
     const int h = (int)(wg % (uint32_t)a.nh);
     wg /= (uint32_t)a.nh;
+    const int part = (int)(wg % (uint32_t)a.parts), ch = h * a.hd + part * a.part_ch;  // first channel of the rows
+    wg /= (uint32_t)a.parts;
     const int b = (int)(wg / (uint32_t)a.splits), q_begin = (int)(wg % (uint32_t)a.splits) * a.split_q;
     const int q_end = q_begin + a.split_q < a.nq ? q_begin + a.split_q : a.nq;
     const int g = lane >> LPR_LOG2, c = lane & (LPR - 1);
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
 
     load_levels(a, lvl);
     {
-        const T* src = static_cast<const T*>(a.value) + ((int64_t)b * a.nk * a.nh + h) * a.hd;
+        const T* src = static_cast<const T*>(a.value) + (int64_t)b * a.nk * a.nh * a.hd + ch;
         const int64_t pitch = (int64_t)a.nh * a.hd;
         const int total = a.nk << LPR_LOG2, step = (int)blockDim.x;
         for (int i0 = (int)threadIdx.x; i0 < total; i0 += 4 * step) {
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
     };
     auto fetch_row = [&](int q0) {
         const int q = q0 + g < q_end ? q0 + g : q_begin;
-        return Row::load_held(gout + (((int64_t)b * a.nq + q) * a.nh + h) * a.hd + c * VEC);
+        return Row::load_held(gout + ((int64_t)b * a.nq + q) * a.nh * a.hd + ch + c * VEC);
     };
     // (the samples, and grad_out rows, of the next pass are on their way while this one's are gathered)
     int q0 = q_begin + wave * U;
@@ -193,16 +195,21 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
                     }
                 }
                 T* dst = static_cast<T*>(a.grad_attn);
+                float* dots = a.dots + (int64_t)part * a.bs * a.nq * a.nh * a.S;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const int s = c + k * LPR;
-                    if (s < ns && q0 + g < q_end) dst[index(q0 + g, c0 + s)] = from_f32<T>(mine[s].row == zero_row ? 0.0f : dot[k]);
+                    if (s < ns && q0 + g < q_end) {
+                        const float d = mine[s].row == zero_row ? 0.0f : dot[k];
+                        if (a.parts == 1) dst[index(q0 + g, c0 + s)] = from_f32<T>(d);
+                        else dots[index(q0 + g, c0 + s)] = d;
+                    }
                 }
             }
             wave_lds_sync();
         }
         if constexpr (!DOTS) {
-            if (q0 + g < q_end) Row::store_global(static_cast<T*>(a.out) + (((int64_t)b * a.nq + q0 + g) * a.nh + h) * a.hd + c * VEC, acc);
+            if (q0 + g < q_end) Row::store_global(static_cast<T*>(a.out) + ((int64_t)b * a.nq + q0 + g) * a.nh * a.hd + ch + c * VEC, acc);
         }
     }
 }
@@ -215,7 +222,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ uint32_t wave_sum[16];
     const int tid = (int)threadIdx.x, block = (int)blockDim.x, lane = tid & (kWave - 1);
-    const int row_bytes = a.hd * (int)sizeof(T);
+    const int row_bytes = a.part_ch * (int)sizeof(T);
     i32x4* lvl = reinterpret_cast<i32x4*>(smem);
     u32x2* ent = reinterpret_cast<u32x2*>(smem + kGkaLevelBytes);                    // sorted samples: {row in `rows`, weight}
     unsigned char* rows = reinterpret_cast<unsigned char*>(ent) + (((size_t)a.sc_tile_q * a.S * 8 + 15) & ~(size_t)15);
@@ -224,10 +231,12 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
     uint32_t wg = xcd_order(blockIdx.x, gridDim.x);
     const int h = (int)(wg % (uint32_t)a.nh);
     wg /= (uint32_t)a.nh;
+    const int ch = h * a.hd + (int)(wg % (uint32_t)a.parts) * a.part_ch;  // first channel of the rows
+    wg /= (uint32_t)a.parts;
     const int split = (int)(wg % (uint32_t)a.sc_splits), b = (int)(wg / (uint32_t)a.sc_splits);
     const int q_begin = split * a.sc_split_q, q_end = q_begin + a.sc_split_q < a.nq ? q_begin + a.sc_split_q : a.nq;
     const T* attn = static_cast<const T*>(a.attn);
-    const T* gout = static_cast<const T*>(a.grad_out) + ((int64_t)b * a.nq * a.nh + h) * a.hd;
+    const T* gout = static_cast<const T*>(a.grad_out) + (int64_t)b * a.nq * a.nh * a.hd + ch;
     const int64_t pitch = (int64_t)a.nh * a.hd;
     load_levels(a, lvl);
     for (int i = tid; i < a.nk; i += block) count[i] = 0;
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
         }
         __syncthreads();
     }
-    float* part = a.part + (((int64_t)split * a.bs + b) * a.nk * a.nh + h) * a.hd + j * 4;
+    float* part = a.part + ((int64_t)split * a.bs + b) * a.nk * a.nh * a.hd + ch + j * 4;
     int g0 = grp;
 #pragma unroll
     for (int i = 0; i < PX; ++i) {
@@ -359,10 +368,18 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
     }
 }
 
-// Adds up the parts of grad_value.
+// Adds up the query ranges' images of grad_value and, behind those workgroups, the channel parts' dots.
 template <typename T>
-__global__ __launch_bounds__(256) void gka_sum_kernel(const GkaArgs a)
+__global__ __launch_bounds__(256) void gka_sum_kernel(const GkaArgs a, uint32_t image_wgs)
 {
+    if (blockIdx.x >= image_wgs) {
+        const int64_t n = (int64_t)a.bs * a.nq * a.nh * a.S, i = (int64_t)(blockIdx.x - image_wgs) * 256 + threadIdx.x;
+        if (i >= n) return;
+        float sum = a.dots[i];
+        for (int p = 1; p < a.parts; ++p) sum += a.dots[p * n + i];
+        static_cast<T*>(a.grad_attn)[i] = from_f32<T>(sum);
+        return;
+    }
     const int64_t n4 = (int64_t)a.bs * a.nk * a.nh * a.hd / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
     const f32x4* part = reinterpret_cast<const f32x4*>(a.part) + i;
@@ -416,7 +433,7 @@ template <typename T, bool DOTS>
 hipError_t slab_t(const GkaArgs& a, hipStream_t stream)
 {
     return by_lanes<T, DOTS>(a.lpr_log2, [&](auto* kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.splits)), dim3(a.block), a.lds, stream, a);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.splits)), dim3(a.block), a.lds, stream, a);
         return hipGetLastError();
     });
 }
@@ -427,12 +444,14 @@ hipError_t backward_t(const GkaArgs& a, hipStream_t stream)
     hipError_t e = slab_t<T, true>(a, stream);
     if (e != hipSuccess) return e;
     e = by_pixels<T>(a.sc_px, [&](auto* kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.sc_splits)), dim3(a.sc_block), a.sc_lds, stream, a);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.sc_splits)), dim3(a.sc_block), a.sc_lds, stream, a);
         return hipGetLastError();
     });
     if (e != hipSuccess) return e;
     const int64_t n4 = (int64_t)a.bs * a.nk * a.nh * a.hd / 4;
-    hipLaunchKernelGGL(gka_sum_kernel<T>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, a);
+    const uint32_t image_wgs = (uint32_t)((n4 + 255) / 256);
+    const int64_t dot_wgs = a.parts > 1 ? ((int64_t)a.bs * a.nq * a.nh * a.S + 255) / 256 : 0;
+    hipLaunchKernelGGL(gka_sum_kernel<T>, dim3(image_wgs + (uint32_t)dot_wgs), dim3(256), 0, stream, a, image_wgs);
     return hipGetLastError();
 }
 

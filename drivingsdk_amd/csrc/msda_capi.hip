@@ -95,6 +95,7 @@ struct Tuning {
     int bwd_lane_bytes;  // MXD_MSDA_BWD_LANE_BYTES: most bytes of a row one lane of the first backward kernel loads
                          // (16, 8, 4), 0 = chosen here
     int tile_px_log2;    // MXD_MSDA_TILE_PX_LOG2: log2 of the pixels per tile of the grad_value pass (9, 8, 7), 0 = chosen here
+    int gka_slab;        // MXD_MSDA_GKA_SLAB: geometric kernel attention with value in LDS: 0 = never, 1 = wherever it fits, -1 = chosen here
     int bwd_fixed;       // MXD_MSDA_BWD_FIXED: 0 = the first backward kernel never takes the instantiation with the common launch
                          // geometry as constants (default 1: where the launch has that geometry)
     int bwd_two_pass;    // MXD_MSDA_BWD_TWO_PASS: 1 = the first backward kernel reads rows of 17 to 32 lanes of 16 bytes with 16
@@ -127,6 +128,7 @@ void read_tuning()
     t.bwd_unit_split = env_int("MXD_MSDA_BWD_UNIT_SPLIT", 1);
     t.tile_px_log2 = env_int("MXD_MSDA_TILE_PX_LOG2", 0);
     t.bwd_rec_lds = env_int("MXD_MSDA_BWD_REC_LDS", -1);
+    t.gka_slab = env_int("MXD_MSDA_GKA_SLAB", -1);
     t.bwd_fixed = env_int("MXD_MSDA_BWD_FIXED", 1);
     t.bwd_two_pass = env_int("MXD_MSDA_BWD_TWO_PASS", 1);
     g_tuning = t;
@@ -897,15 +899,14 @@ int64_t gka_splits(int64_t slabs, int64_t nq, int64_t slots, double fixed, int64
     return best;
 }
 
-// Geometric kernel attention with the (batch, head)'s slab of value in LDS (gka.hip): whether a problem's slab, in the dtype for the
-// gather and as float32 sums in registers for grad_value, fits, and the launch geometry.
-bool gka_plan(int dtype, const Dims& d, mxd::GkaArgs* a)
+// Geometric kernel attention with the (batch, head)'s slab of value in LDS (gka.hip), `parts` of its channels at a time: whether the
+// part's slab, in the dtype for the gather and as float32 sums in registers for grad_value, fits, and the launch geometry.
+bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
 {
     memset(a, 0, sizeof(*a));
     const int es = elem_size(dtype);
-    const int64_t row = d.hd * es, lanes = row / 16, sc_lanes = d.hd / 4, S = d.nl * d.np;
-    if (tuning().bwd_atomic || row % 16 != 0 || (lanes & (lanes - 1)) != 0 || lanes < 2 || lanes > 32) return false;
-    if (sc_lanes > 64 || d.nk >= 32768 || S > 256 || d.nl != d.nl_attn || d.bs * d.nh > 65536) return false;
+    const int64_t ch = d.hd / parts, row = ch * es, lanes = row / 16, sc_lanes = ch / 4, S = d.nl * d.np;
+    if (d.hd % parts != 0 || row % 16 != 0 || (lanes & (lanes - 1)) != 0 || lanes < 2 || lanes > 32 || sc_lanes > 64) return false;
     a->bs = (int32_t)d.bs;
     a->nk = (int32_t)d.nk;
     a->nh = (int32_t)d.nh;
@@ -916,6 +917,8 @@ bool gka_plan(int dtype, const Dims& d, mxd::GkaArgs* a)
     a->S = (int32_t)S;
     a->np_magic = (uint32_t)(((1u << 20) + d.np - 1) / d.np);
     a->s_magic = (uint32_t)(((1u << 20) + S - 1) / S);
+    a->parts = (int32_t)parts;
+    a->part_ch = (int32_t)ch;
     a->lpr_log2 = log2_lanes((int)lanes);
     // gather: two workgroups of 8 wavefronts per CU, or one of 16
     const int64_t slab = (d.nk + 1) * row, strip = (64 / lanes) * mxd::kChunkStride * 8, lim = mxd::kCuLdsBytes - 256;
@@ -923,8 +926,8 @@ bool gka_plan(int dtype, const Dims& d, mxd::GkaArgs* a)
     const bool two = 2 * lds2 <= lim || lds1 > lim;
     a->block = two ? 512 : 1024;
     a->lds = (uint32_t)(two ? lds2 : lds1);
-    if (a->lds > lim) return false;
-    const int64_t slabs = d.bs * d.nh;
+    if ((two ? lds2 : lds1) > lim) return false;
+    const int64_t slabs = d.bs * d.nh * parts;
     int64_t s = gka_splits(slabs, d.nq, 2 * (int64_t)a->lds <= lim ? 512 : 256, (double)d.nk / 2, 64 / lanes * (a->block / 64));
     a->split_q = (int32_t)ceil_div(d.nq, s);
     a->splits = (int32_t)ceil_div(d.nq, a->split_q);
@@ -949,7 +952,24 @@ bool gka_plan(int dtype, const Dims& d, mxd::GkaArgs* a)
     return true;
 }
 
-size_t gka_part_bytes(const mxd::GkaArgs& a) { return (size_t)a.sc_splits * a.bs * a.nk * a.nh * a.hd * sizeof(float); }
+// Whether these kernels take a problem.  Forward: whole rows only (with the channels in two parts, which read the locations twice, it
+// takes 36 us where the general kernel takes 29), and from half a million samples on (446 000 samples 6.7 -> 8.7 us, 685 000
+// 11.6 -> 9.5, 2.4 million 23 -> 16).  Backward: wherever the slab fits, whole or in two parts (48 x 24 pixels, 64 channels, float32,
+// two parts: 180 -> 112 us; in four parts 64 x 46 pixels of 32 channels went from 80 to 107 us).
+bool gka_plan(int dtype, const Dims& d, bool backward, mxd::GkaArgs* a)
+{
+    const int mode = tuning().gka_slab;
+    if (mode == 0 || tuning().bwd_atomic || d.nk >= 32768 || d.nl * d.np > 256 || d.nl != d.nl_attn || d.bs * d.nh > 65536) return false;
+    if (!backward) return (mode > 0 || d.bs * d.nh * d.nq * d.nl * d.np >= (int64_t(1) << 19)) && gka_plan_parts(dtype, d, 1, a);
+    return gka_plan_parts(dtype, d, 1, a) || gka_plan_parts(dtype, d, 2, a);
+}
+
+// Workspace of its backward: images of grad_value, dots of the channel parts.
+size_t gka_image_bytes(const mxd::GkaArgs& a) { return round_up((size_t)a.sc_splits * a.bs * a.nk * a.nh * a.hd * sizeof(float), 256); }
+size_t gka_part_bytes(const mxd::GkaArgs& a)
+{
+    return gka_image_bytes(a) + (a.parts > 1 ? (size_t)a.parts * a.bs * a.nq * a.nh * a.S * sizeof(float) : 0);
+}
 
 // Grid sampler on planes: whether a plane fits the LDS of a CU (as float32, whatever the dtype) and every index its type.
 bool grid_planes_fit(int64_t n, int64_t c, int64_t h, int64_t w, int64_t h_out, int64_t w_out)
@@ -1154,7 +1174,7 @@ int mxd_gka_forward(const void* value, const int32_t* spatial_shapes, const int3
     const int meta64 = take_meta_flag(&code);
     const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
     mxd::GkaArgs a;
-    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, &a))
+    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, false, &a))
         return forward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, output, dtype,
                               bs, nk, nh, hd, nl, nl, nq, np, hip_stream);
     if (!value || !spatial_shapes || !level_start_index || !sampling_locations || !attn_weights || !output)
@@ -1451,7 +1471,7 @@ size_t mxd_gka_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk, int64
     take_meta_flag(&code);
     const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
     mxd::GkaArgs a;
-    if (check_dims(code, d) == MXD_OK && gka_plan(code, d, &a)) return gka_part_bytes(a);
+    if (check_dims(code, d) == MXD_OK && gka_plan(code, d, true, &a)) return gka_part_bytes(a);
     return mxd_msda_backward_workspace_bytes(dtype, bs, nk, nh, hd, nl, nl, nq, np);
 }
 
@@ -1465,7 +1485,7 @@ int mxd_gka_backward(const void* value, const int32_t* spatial_shapes, const int
     const int meta64 = take_meta_flag(&code);
     const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
     mxd::GkaArgs a;
-    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, &a))
+    if (check_dims(code, d) != MXD_OK || !gka_plan(code, d, true, &a))
         return backward_common(1, value, spatial_shapes, level_start_index, sampling_locations, attn_weights, grad_output,
                                grad_value, nullptr, grad_attn_weights, workspace, workspace_bytes, dtype, bs, nk, nh, hd, nl,
                                nl, nq, np, 0, hip_stream);
@@ -1489,6 +1509,7 @@ int mxd_gka_backward(const void* value, const int32_t* spatial_shapes, const int
     a.grad_value = grad_value;
     a.grad_attn = grad_attn_weights;
     a.part = static_cast<float*>(workspace);
+    a.dots = reinterpret_cast<float*>(static_cast<char*>(workspace) + gka_image_bytes(a));
     const hipError_t e = mxd::launch_gka_backward(code, a, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_gka_backward: launch failed: %s", hipGetErrorString(e));
     return MXD_OK;

@@ -1,14 +1,19 @@
 """Geometric kernel attention with value in LDS at the sizes where its kernels change course, against the CPU oracle: rows of two
 to 32 lanes, one to 16 pixels per lane group, more samples than one pass stages, one query and many tiles of them, all samples
-on one pixel, rows of no query, maps just inside and outside of what fits, levels that overlap."""
+on one pixel, channels in two parts, maps just inside and outside of what fits, levels that overlap."""
 import pytest
 import torch
 
 from oracle import gka_oracle as gka
 from test_gka_gpu import make_inputs, run_gpu
-from util import BWD_FP32, FWD_FP32, HALF, rel_err
+from util import BWD_FP32, FWD_FP32, HALF, rel_err, set_tuning
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _wherever_it_fits(monkeypatch):
+    set_tuning(monkeypatch, MXD_MSDA_GKA_SLAB=1)
 
 
 def compare(inp, device, dtype=torch.float32):
@@ -26,7 +31,8 @@ def compare(inp, device, dtype=torch.float32):
     # bs, nq, hd, nh, nl, np; map
     ([2, 700, 8, 2, 1, 7], (9, 13)), ([1, 1, 16, 2, 1, 4], (8, 12)), ([2, 333, 16, 3, 1, 20], (40, 60)), ([1, 911, 32, 2, 2, 9], (17, 19)),
     ([3, 257, 64, 4, 1, 16], (24, 25)), ([1, 130, 128, 2, 1, 5], (10, 20)), ([1, 5000, 32, 1, 1, 1], (3, 5)), ([2, 90, 64, 1, 3, 17], (7, 11)),
-    ([1, 300, 16, 2, 1, 17], (60, 68)), ([1, 300, 64, 2, 1, 6], (25, 26)), ([1, 300, 64, 2, 1, 6], (31, 33))])
+    ([1, 300, 16, 2, 1, 17], (60, 68)), ([1, 300, 64, 2, 1, 6], (25, 26)), ([1, 300, 64, 2, 1, 6], (31, 33)), ([2, 257, 64, 2, 1, 18], (24, 48)),
+    ([1, 40, 16, 2, 1, 6], (64, 74))])
 def test_sizes(gpu_device, shape, hw, dtype):
     compare(make_inputs(shape, hw, seed=shape[1]), gpu_device, dtype)
 
