@@ -282,10 +282,10 @@ int backward_lane_bytes(int dtype, const Dims& d)
     // staging strips of a workgroup take 51 KiB of LDS, which leaves 3 wavefronts per SIMD, and a lane stages four
     // samples of which it keeps two in registers (measured, encoder shape in float16 / bfloat16: backward 322 -> 300 us;
     // BEVFormer shape in float16 1114 -> 1075 us; with rows of 256 bytes halving the lane width costs 10 %).
-    // Rows of up to 32 bytes: 8 lanes of 4, from 5 samples per query on (16 channels in float16, 2 x 13253 queries of 18 samples:
-    // backward 289 -> 251 us; 3 samples 53 -> 55).
+    // Rows of up to 32 bytes: 8 lanes of 4 for units that fill a chunk of 16 samples (16 channels in float16, 2 x 13253 queries of 18
+    // samples: backward 289 -> 251 us; 3 samples 53 -> 55), with half as many queries per workgroup.
     const int64_t row = d.hd * elem_size(dtype);
-    if (row > 16 && row <= 32) return d.nl * d.np > 4 ? 4 : 16;
+    if (row > 16 && row <= 32) return d.nl * d.np > 12 ? 4 : 16;
     return (row > 32 && row <= 64) ? 8 : 16;
 }
 
@@ -584,7 +584,15 @@ bool plan_forward_cu(int dtype, const Dims& d, int vec, int lpr, int npass, mxd_
             ++levels_cached;
         }
         if (levels_cached == 0 || d.bs * d.nh * d.nq * d.nl * d.np < (int64_t(1) << 20)) return false;
-        const int64_t slice = d.nk * d.hd * es;
+        // Its units work through whole chunks of 16 samples, the general kernel's through as many as there are: up to 8 samples
+        // (3 x 15247 queries, 4 heads, levels from 58 x 197: float32 48 against 35 us, float16 39 against 30), and 17 to 20 with rows
+        // of 16 lanes (2 x 5355 queries of 18 samples, 256-byte rows: 57 against 54 / 76 against 55), go there; so do rows of 16
+        // lanes in bfloat16, whose conversions the four wavefronts per SIMD of this form do not hide, where an XCD's L2 holds the
+        // slice (3 x 6321 queries, 128 channels, 1.6 MB: 100 against 86; 3.8 MB 80 against 70; the encoder's levels, 5.1 MB, 103
+        // against 106).
+        const int64_t samples = d.nl * d.np, slice = d.nk * d.hd * es;
+        if (samples <= mxd::kChunk / 2 || (lpr == 16 && ((samples > mxd::kChunk && samples <= mxd::kChunk + 4) || (dtype == MXD_DTYPE_BF16 && slice <= (int64_t(4) << 20)))))
+            return false;
         // (rows of 256 bytes, 16 samples per unit, one level of four cached: 0.88 to 0.93 of the general kernel's time at
         //  the encoder's levels -- head_dim 64 and 48 in float32, 128 and 96 in float16, slices of 5 MB -- but 1.18 to
         //  1.33 at slices of 8 MB and more, and 0.93 to 1.25 with 8 samples per unit)
