@@ -26,7 +26,7 @@ struct DaggArgs {
     float* image;          // float32 image of grad_feat: grad_feat itself, or in the workspace for 16-bit dtypes
     float* gw_part;        // [G][bs, A][cams, P, scales]: gradients of the weights of one group, locations inside the image only
     float* gl_part;        // [G][bs, A][cams, P][2]: one group's part of the location gradients, summed over the scales
-    uint32_t* csr;         // [bs][nf + nl]: per level, first record of every pixel, then their number
+    uint32_t* csr;         // [bs][starts]: per level, first record of every pixel, then their number
     u32x4* rec;            // [bs][nl][2 A P] records sorted by pixel: {anchor << 3 | pixel & 7, index of the weight of group 0 / G,
                            //   bilinear weight of the pixel, of the pixel to its right}
     int32_t bs, nf, C, G, hd, cams, scales, nl, A, P;
@@ -41,12 +41,18 @@ struct DaggArgs {
     int32_t lpr_log2;      // lanes that share it
     // grad_feat: lanes that share a pixel row, channel blocks per row
     int32_t row_lpr_log2, row_blocks, sort_ranges;
+    int64_t starts;        // entries of a batch element's table of record starts (dagg_starts)
     int32_t strip_records; // records per strip aimed at where the strips of a level are split
     mxd_msda_plan map;     // XCD mapping: piece = head, anchor = query
 };
 
 hipError_t launch_dagg_forward(int dtype, const DaggArgs& a, hipStream_t stream);
 hipError_t launch_dagg_backward(int dtype, const DaggArgs& a, hipStream_t stream);
+
+// Entries of a batch element's table of record starts.  A level takes one per pixel and one more; levels that do not overlap have at
+// most the tensor's pixels between them, and 512 entries more per level are room for levels that share rows (cameras that name the
+// same map).  What does not fit all the same is added sample by sample (dagg_levels_without_room).
+inline int64_t dagg_starts(int64_t nf, int64_t nl) { return nf + nl * (512 + 1); }
 
 // Elements per lane of a row piece of `ch` channels (what the kernels are instantiated for).
 inline int dagg_vec(int elem_size, int64_t ch)

@@ -316,11 +316,12 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
 // ---- the levels as the kernels behind it see them ---------------------------------------------------------------------------
 struct DaggLevels {
     int32_t H[kMaxLevels], W[kMaxLevels], base[kMaxLevels];
-    int32_t px[kMaxLevels];      // pixels inside the feature tensor; 0: the level has no rows (or found no room, see csr)
+    int32_t px[kMaxLevels];      // pixels inside the feature tensor; 0: the level has no rows (or is one of `lost`)
     int32_t csr[kMaxLevels];     // its first entry of DaggArgs::csr
     int32_t chunks[kMaxLevels];  // parts its strips' records are split into
     int32_t first[kMaxLevels + 1];  // work items of the levels before it
     int32_t tiled;               // the levels tile the keys in order: a pixel row belongs to one level
+    uint64_t lost;               // levels, by bit, that found no room in csr: dagg_levels_without_room
 
     // (a level per lane of the first wavefront: one after the other, 24 levels were 5 us in front of every workgroup)
     __device__ void fill(const DaggArgs& a)
@@ -343,21 +344,23 @@ struct DaggLevels {
             const int32_t end = L.z + P, before = __shfl_up(end, 1, kWave);
             const bool follows = whole && L.z == (lane == 0 ? 0 : before);
             tiled = __ballot(lane < a.nl && !follows) == 0 && __builtin_amdgcn_readlane(end, a.nl - 1) == a.nf;
-            // (levels that overlap so far that their pixels are more than the tensor has do not fit the table of record
-            //  starts: they are left out of grad_feat)
+            // (levels that overlap far: the ones that find no room in the table of record starts have no records)
             int64_t used = P > 0 ? P + 1 : 0, at = prefix(used) - used;
-            if (__ballot(at + used > (int64_t)a.nf + a.nl) != 0) {
+            bool fits = true;
+            if (__ballot(at + used > a.starts) != 0) {
                 int64_t room = 0;
                 for (int l = 0; l < a.nl; ++l) {
                     const int32_t u = __builtin_amdgcn_readlane((int32_t)used, l);
-                    const bool fits = room + u <= (int64_t)a.nf + a.nl;
+                    const bool room_left = room + u <= a.starts;
                     if (lane == l) {
                         at = room;
-                        if (!fits) P = 0;
+                        fits = room_left;
                     }
-                    if (fits) room += u;
+                    if (room_left) room += u;
                 }
+                if (!fits) P = 0;
             }
+            lost = __ballot(!fits);
             // records of a strip if every location were inside and spread evenly
             const float expect = P > 0 ? 2.0f * (float)a.A * (float)a.P * (float)(kDaggStrip + 1) / (float)P : 0.0f;
             int32_t n = (int32_t)__builtin_ceilf(expect / (float)a.strip_records);
@@ -458,7 +461,7 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
     __syncthreads();
     uint32_t at = before_s + inc - sum;
     for (int k = 0; k < wave; ++k) at += wsum[k];
-    uint32_t* csr = a.csr + (size_t)b * ((size_t)a.nf + a.nl) + lv.csr[l];
+    uint32_t* csr = a.csr + (size_t)b * (size_t)a.starts + lv.csr[l];
     for (int k = 0; k < kPer; ++k) {
         const int p = tid * kPer + k;
         const uint32_t v = cnt[p];
@@ -518,6 +521,34 @@ __global__ __launch_bounds__(kDaggBackWaves * kWave) void dagg_dots_and_sort_ker
 }
 
 // ---- gradient of the feature maps --------------------------------------------------------------------------------------------
+// The samples of levels that found no room in the table of record starts, added to grad_feat's float32 image by atomics: a sample per
+// wavefront, a channel per lane.  Only levels that overlap come here, and then every row has been zeroed and every other level
+// adds with atomics as well.  Slow, and there so that scale_start_index is honoured however it comes.
+template <typename T>
+__device__ inline void dagg_levels_without_room(const DaggArgs& a, const DaggLevels& lv)
+{
+    const T* gout = static_cast<const T*>(a.grad_out);
+    const uint32_t lane = threadIdx.x & (kWave - 1), waves = gridDim.x * (blockDim.x / kWave);
+    const uint64_t points = (uint64_t)a.A * (uint64_t)a.P, total = points * a.bs;
+    for (uint64_t i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < total; i += waves) {
+        const uint64_t b = i / points, anchor = i / (uint64_t)a.P;  // (anchor of all batch elements)
+        for (uint64_t m = lv.lost; m != 0; m &= m - 1) {
+            const int l = __builtin_ctzll(m), cam = l / a.scales;
+            const uint64_t li = i * a.cams + cam;
+            const f32x2 xy = load_xy<T>(a.loc, (int64_t)li);
+            if (!inside(xy.x, xy.y)) continue;
+            const Sample sm = sample_geometry(xy.x, xy.y, i32x4{lv.H[l], lv.W[l], lv.base[l], 0}, a.nf, true);
+            const T* w = static_cast<const T*>(a.w) + (li * a.scales + (l - cam * a.scales)) * a.G;
+            float* image = a.image + b * a.nf * a.C;
+            for (int ch = (int)lane; ch < a.C; ch += kWave) {
+                const float g = to_f32(gout[anchor * a.C + ch]) * to_f32(w[ch / a.hd]);
+                for (int k = 0; k < 4; ++k)
+                    if (sm.cvalid[k]) unsafeAtomicAdd(image + (size_t)sm.pix[k] * a.C + ch, sm.w[k] * g);
+            }
+        }
+    }
+}
+
 // A unit of 2^row_lpr_log2 lanes forms the rows of a strip of 8 neighbouring pixels, or of one block of their channels, from
 // the strip's records in pixel order: one row of sums for the pixel at hand and one for the pixel to its right; the records
 // of the pixel before the strip are met for their right halves.  Every row is stored once, whole (strips split by record
@@ -557,7 +588,7 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
         const int k = scalar(it - lv.first[l]), chunks = scalar(lv.chunks[l]), strip = k / chunks, chunk = k - strip * chunks;
         const int p0 = strip * kDaggStrip, px_l = scalar(lv.px[l]), p1 = p0 + kDaggStrip < px_l ? p0 + kDaggStrip : px_l;
         const bool direct = lv.direct(l);
-        const csr_ptr csr = (csr_ptr)(a.csr + (size_t)b * ((size_t)a.nf + a.nl) + scalar(lv.csr[l]));
+        const csr_ptr csr = (csr_ptr)(a.csr + (size_t)b * (size_t)a.starts + scalar(lv.csr[l]));
         const uint32_t s1 = csr[p0];
         uint32_t lo = p0 > 0 ? csr[p0 - 1] : s1, hi = csr[p1];
         if (chunks > 1) {
@@ -657,6 +688,7 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
         }
         while (cur < p1 - p0) flush();
     }
+    if (lv.lost != 0) dagg_levels_without_room<T>(a, lv);
 }
 
 // ---- the rest: weights' and locations' gradients in the caller's layout, rounding ---------------------------------------------

@@ -841,6 +841,7 @@ int dagg_args(int dtype, int64_t bs, int64_t nf, int64_t C, int64_t cams, int64_
     a->row_lpr_log2 = log2_lanes((C + vec - 1) / vec);
     a->row_blocks = (int32_t)(((C + vec - 1) / vec + mxd::kWave - 1) / mxd::kWave);
     a->sort_ranges = (int32_t)((nf + mxd::kDaggSortPx - 1) / mxd::kDaggSortPx);
+    a->starts = mxd::dagg_starts(nf, d.nl);
     // A unit of lanes goes through a strip's records one batch after the other, a trip to memory each.  Where the strips alone leave
     // the chip short of units they are split down to 96 records (829 anchors x 9 points, 4 levels from 58 x 28, 64 channels: 90 us
     // with parts of 1024 records, 27 with 96, 31 with 64); a split costs zeros and atomic additions, so that strips enough for two
@@ -883,7 +884,7 @@ struct DaggSpace {
         const size_t locs = (size_t)a.bs * a.A * a.nloc;
         gl = round_up((size_t)a.G * locs * a.scales * 4, 256);
         csr = gl + round_up((size_t)a.G * locs * 8, 256);
-        rec = csr + round_up((size_t)a.bs * ((size_t)a.nf + a.nl) * 4, 256);
+        rec = csr + round_up((size_t)a.bs * (size_t)a.starts * 4, 256);
         image = rec + (size_t)a.bs * a.nl * 2 * a.A * a.P * 16;
         total = image + (es == 2 ? (size_t)a.bs * a.nf * a.C * 4 : 0);
     }

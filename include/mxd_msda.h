@@ -229,16 +229,16 @@ int mxd_msda_backward_static(const void* value, const int32_t* spatial_shapes, c
  *   sampling_location [bs, num_anchors, num_pts, num_cams, 2] = (x, y)
  *   weights [bs, num_anchors, num_pts, num_cams, num_scale, num_groups]     output [bs, num_anchors, num_embeds]
  * output[b,a,c] = sum over (pt, cam, scale) of weights[..., group(c)] * bilinear(feat of (cam, scale), location);
- * a location counts only when 0 < x < 1 and 0 < y < 1; zero padding outside the map.  The same kernels as
- * multi-scale deformable attention run it (group = head, (camera, scale) = level, anchor = query). */
+ * a location counts only when 0 < x < 1 and 0 < y < 1; zero padding outside the map.  Levels may share rows of the
+ * features in any way (cameras that name the same map): all of them count in every gradient. */
 int mxd_dagg_forward(const void* mc_ms_feat, const int32_t* spatial_shape, const int32_t* scale_start_index,
                      const void* sampling_location, const void* weights, void* output, int dtype, int64_t bs,
                      int64_t num_feat, int64_t num_embeds, int64_t num_cams, int64_t num_scale, int64_t num_anchors,
                      int64_t num_pts, int64_t num_groups, void* hip_stream);
 
 /* Bytes of scratch mxd_dagg_backward needs (0 if the sizes are invalid): the hand-over between the two
- * backward kernels, the fp32 image of grad_mc_ms_feat for 16-bit dtypes, and one float32 partial image of
- * grad_sampling_location per group. */
+ * backward kernels (records sorted by pixel and where each pixel's begin), the fp32 image of grad_mc_ms_feat for
+ * 16-bit dtypes, and one float32 partial image of grad_sampling_location and of grad_weights per group. */
 size_t mxd_dagg_backward_workspace_bytes(int dtype, int64_t bs, int64_t num_feat, int64_t num_embeds, int64_t num_cams,
                                          int64_t num_scale, int64_t num_anchors, int64_t num_pts, int64_t num_groups);
 

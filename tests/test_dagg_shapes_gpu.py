@@ -51,3 +51,30 @@ def test_levels_that_do_not_tile_the_features(gpu_device, dtype):
     want = (dagg.direct_forward(*inp[:5]),) + dagg.direct_backward(*inp)
     for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
         assert rel_err(g, r) <= ((FWD_FP32 if k == 0 else BWD_FP32) if dtype == torch.float32 else 4e-3), k
+
+
+def _shared_map(cams, maps, starts, nf, C, G, A, P, dtype, seed):
+    """Inputs (float32 arrays that `dtype` holds exactly) for `cams` cameras whose levels start at `starts` in nf rows."""
+    inp = list(make_inputs(2, C, G, A, P, [maps] * cams, seed=seed, pad=True))
+    inp[0] = np.random.default_rng(seed).random((2, nf, C), dtype=np.float32)
+    inp[2] = np.array(starts, dtype=np.int32).reshape(cams, len(maps))
+    return [np.asarray(torch.from_numpy(t).to(dtype).float()) if t.dtype == np.float32 else t for t in inp]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cams,maps,starts,nf,C,G,A,P", [
+    # two cameras that name one map: more pixels between them than the tensor has rows
+    (2, [(9, 13)], [0, 0], 117, 32, 4, 33, 5),
+    (2, [(9, 13)], [0, 0], 117, 256, 8, 33, 5),
+    # eight levels of 36 x 41 pixels in 2000 rows: the table of record starts (2000 + 8 * 513 entries) holds four of them
+    (8, [(36, 41)], [0, 10, 100, 37, 500, 524, 3, 0], 2000, 64, 8, 41, 3),
+    (8, [(36, 41)], [0, 10, 100, 37, 500, 524, 3, 0], 2000, 256, 8, 9, 3),
+    # groups that lanes straddle; two scales, the first of which finds room in the first six cameras only, the second everywhere
+    (8, [(36, 41), (2, 3)], [0, 1994] * 6 + [524, 5, 3, 1990], 2000, 40, 8, 23, 4)])
+def test_levels_that_share_rows(gpu_device, cams, maps, starts, nf, C, G, A, P, dtype):
+    """Every level counts in the gradient of the maps, however far the levels overlap."""
+    inp = _shared_map(cams, maps, starts, nf, C, G, A, P, dtype, cams + C)
+    want = (dagg.direct_forward(*inp[:5]),) + dagg.direct_backward(*inp)
+    tol = {torch.float32: BWD_FP32, torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
+    for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
+        assert rel_err(g, r) <= tol, k
