@@ -106,12 +106,13 @@ struct Args {
 };
 
 // ---- the operators ---------------------------------------------------------------------------------------------------
-// kGradOf: which tensors have gradients.  kKeepsOutput: the backward reads the result.  kOnce: gradients of gradients raise an
-// error.  kFloat32InAutocast: autocast has the inputs cast to float32 (left to Python).  takes(): whether a call is in the form the kernels read, grad_output aside.
+// kGradOf: which tensors have gradients.  kFloat32: the tensor that is float32 whatever the others are (-1: none).  kKeepsOutput:
+// the backward reads the result.  kOnce: gradients of gradients raise an error.  kFloat32InAutocast: autocast has the inputs cast to
+// float32 (left to Python).  takes(): whether a call is in the form the kernels read, grad_output aside.
 
 struct Msda {
     static constexpr const char* kNode = "MultiScaleDeformableAttnFunctionBackward";
-    static constexpr int kTensors = 5, kInts = 0;
+    static constexpr int kTensors = 5, kInts = 0, kFloat32 = -1;
     static constexpr std::array<int, 3> kGradOf{0, 3, 4};
     static constexpr bool kKeepsOutput = false, kOnce = true, kFloat32InAutocast = true;
     static bool takes(const Args& a)
@@ -149,7 +150,7 @@ struct Msda {
 
 struct Fused {
     static constexpr const char* kNode = "MultiScaleDeformableAttnFusedFunctionBackward";
-    static constexpr int kTensors = 6, kInts = 0;
+    static constexpr int kTensors = 6, kInts = 0, kFloat32 = -1;
     static constexpr std::array<int, 4> kGradOf{0, 3, 4, 5};
     static constexpr bool kKeepsOutput = true, kOnce = true, kFloat32InAutocast = true;
     static bool takes(const Args& a)
@@ -187,7 +188,7 @@ struct Fused {
 
 struct Dagg {
     static constexpr const char* kNode = "AdsDeformableAggregationBackward";
-    static constexpr int kTensors = 5, kInts = 0;
+    static constexpr int kTensors = 5, kInts = 0, kFloat32 = -1;
     static constexpr std::array<int, 3> kGradOf{0, 3, 4};
     static constexpr bool kKeepsOutput = false, kOnce = false, kFloat32InAutocast = false;
     static bool takes(const Args& a)
@@ -224,7 +225,7 @@ struct Dagg {
 
 struct Gka {
     static constexpr const char* kNode = "GeometricKernelAttentionFuncBackward";
-    static constexpr int kTensors = 5, kInts = 0;
+    static constexpr int kTensors = 5, kInts = 0, kFloat32 = 3;
     static constexpr std::array<int, 2> kGradOf{0, 4};
     static constexpr bool kKeepsOutput = false, kOnce = false, kFloat32InAutocast = false;
     static bool takes(const Args& a)
@@ -259,7 +260,7 @@ struct Gka {
 
 struct Grid {
     static constexpr const char* kNode = "GridSampler2dV2FunctionBackward";
-    static constexpr int kTensors = 2, kInts = 3;  // interpolation and padding mode, align_corners: see mxd_grid_sampler2d_forward
+    static constexpr int kTensors = 2, kInts = 3, kFloat32 = -1;  // interpolation and padding mode, align_corners: see mxd_grid_sampler2d_forward
     static constexpr std::array<int, 2> kGradOf{0, 1};
     static constexpr bool kKeepsOutput = false, kOnce = true, kFloat32InAutocast = false;
     static bool takes(const Args& a)
@@ -297,7 +298,7 @@ struct Grid {
 
 bool usable_grad(const Tensor& grad, const Tensor& like, int64_t numel)
 {
-    return plain(grad, like, like.scalar_type()) && grad.numel() == numel;
+    return like.defined() && plain(grad, like, like.scalar_type()) && grad.numel() == numel;
 }
 
 template <class Op>
@@ -315,6 +316,32 @@ template <>
 int64_t output_numel<Grid>(const Args& a) { return a.t[0].size(0) * a.t[0].size(1) * a.t[1].size(1) * a.t[1].size(2); }
 template <>
 int64_t output_numel<Gka>(const Args& a) { return output_numel<Msda>(a); }
+
+template <class Op>
+bool kept_as_taken(const Args& a)
+{
+    for (int k = 0; k < Op::kTensors; ++k)
+        if (!a.t[k].defined()) return false;
+    return Op::takes(a) && (!Op::kKeepsOutput || usable_grad(a.out, a.t[0], output_numel<Op>(a)));
+}
+
+// What is unpacked in the backward need not be what the forward checked: hooks for saved tensors (torch.autograd.graph) hand
+// back whatever they like -- a view with other strides, another dtype, a tensor of another device.  Strides and dtypes are brought
+// into the form that the kernels read, value's dtype deciding as in the forward; everything else is an error.
+template <class Op>
+void bring_into_form(Args& a)
+{
+    auto bring = [&](Tensor& t, at::ScalarType type) {
+        TORCH_CHECK(t.defined() && t.is_cuda() && t.device() == a.t[0].device(), Op::kNode,
+                    ": a tensor saved for the backward was handed back on another device (this build has no CPU implementation)");
+        t = (t.is_floating_point() ? t.to(type) : t).contiguous();
+    };
+    TORCH_CHECK(a.t[0].defined(), Op::kNode, ": a tensor saved for the backward was not handed back");
+    const at::ScalarType type = a.t[0].scalar_type();
+    for (int k = 0; k < Op::kTensors; ++k) bring(a.t[k], k == Op::kFloat32 ? at::kFloat : type);
+    if (Op::kKeepsOutput) bring(a.out, type);
+    TORCH_CHECK(kept_as_taken<Op>(a), Op::kNode, ": the tensors saved for the backward were handed back in a form that the kernels do not take");
+}
 
 template <class Op>
 struct Backward : torch::autograd::Node {
@@ -342,6 +369,7 @@ struct Backward : torch::autograd::Node {
         const bool again = at::GradMode::is_enabled();  // (a graph of the backward is wanted)
         {
             at::AutoDispatchBelowAutograd below;
+            if (!kept_as_taken<Op>(a)) bring_into_form<Op>(a);
             Tensor grad = grads[0];
             if (!grad.defined()) {
                 grad = Op::new_output(a);
@@ -349,6 +377,7 @@ struct Backward : torch::autograd::Node {
             } else if (!usable_grad(grad, a.t[0], output_numel<Op>(a))) {
                 grad = grad.to(a.t[0].options()).contiguous();
                 TORCH_CHECK(grad.numel() == output_numel<Op>(a), Op::kNode, ": grad_output has another size than the output");
+                TORCH_CHECK(usable_grad(grad, a.t[0], output_numel<Op>(a)), Op::kNode, ": grad_output is no tensor that the kernels can read");
             }
             unsigned need = 0;
             for (size_t k = 0; k < kGrads<Op>; ++k) {
