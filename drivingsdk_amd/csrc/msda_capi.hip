@@ -862,6 +862,10 @@ int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
     a->piece_heads = 1;
     if (!backward && a->hd % vec == 0 && a->hd * es < 128 && a->G > 1) {
         a->piece_ch = 128 / es < a->C ? 128 / es : a->C;
+        // (at most 32 of them: a wavefront keeps the weights of 64 samples per group in LDS, and those of 64 groups would take the
+        //  workgroup to 80 KiB, beyond what a kernel is promised without opting in; 128 groups of one channel, 900 anchors x 13 points in six
+        //  cameras, float16: 64 / 32 groups a piece 114 / 85 us)
+        if (a->piece_ch > 32 * a->hd) a->piece_ch = 32 * a->hd;
         a->piece_heads = a->piece_ch % a->hd == 0 ? a->piece_ch / a->hd : (a->piece_ch - 1) / a->hd + 2;
     }
     a->pieces = (a->C + a->piece_ch - 1) / a->piece_ch;

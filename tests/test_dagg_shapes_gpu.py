@@ -29,6 +29,18 @@ def test_group_widths_16_bit(gpu_device, C, G, dtype):
         assert rel_err(g, r) <= tol, k
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("C,G", [(128, 128), (64, 64), (70, 70), (130, 65), (48, 48)])
+def test_many_narrow_groups_in_16_bits(gpu_device, C, G, dtype):
+    """128 bytes of a row hold 64 groups of one channel: the weights of a wavefront's samples have to fit its share of LDS."""
+    inp = [np.asarray(torch.from_numpy(t).to(dtype).float()) if t.dtype == np.float32 else t
+           for t in make_inputs(1, C, G, 9, 5, [[(9, 13), (5, 7)]] * 2, seed=C, pad=True)]
+    want = (dagg.direct_forward(*inp[:5]),) + dagg.direct_backward(*inp)
+    tol = {torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
+    for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
+        assert rel_err(g, r) <= tol, k
+
+
 @pytest.mark.parametrize("P,cams,scales", [(1, 1, 1), (65, 1, 1), (43, 3, 3), (130, 2, 1), (7, 5, 7), (2, 1, 40)])
 def test_location_and_scale_counts(gpu_device, P, cams, scales):
     print(check(make_inputs(1, 32, 4, 9, P, [[(6 + s % 3, 7) for s in range(scales)]] * cams, seed=P, pad=True), gpu_device))
