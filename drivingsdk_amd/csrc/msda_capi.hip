@@ -339,8 +339,10 @@ struct BwdLayout {
 
 // Pixels per tile of the grad_value pass, as a power of two: every thread of its workgroups keeps 32 sums, so 512 pixels
 // of up to 32 channels, 256 of up to 64, 128 of more (msda_plan.h).
-int preferred_tile_px_log2(const Dims& d)
+int preferred_tile_px_log2(int dtype, const Dims& d)
 {
+    // (16-bit rows of fewer than 4 channels, which no lane can read four of, have the tile pass for 512 pixels alone)
+    if (elem_size(dtype) == 2 && d.hd < 4) return mxd::kTilePxLog2Max;
     const int v = tuning().tile_px_log2;
     if (v >= 7 && v <= mxd::kTilePxLog2Max) return v;
     if (d.hd <= 32) return mxd::kTilePxLog2Max;
@@ -385,7 +387,7 @@ BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2)
 // not fit the first kernel's bookkeeping.
 BwdLayout bwd_layout(int dtype, const Dims& d)
 {
-    const int pref = preferred_tile_px_log2(d);
+    const int pref = preferred_tile_px_log2(dtype, d);
     BwdLayout L = bwd_layout_for(dtype, d, pref);
     if (!L.tiles && pref != mxd::kTilePxLog2Max) L = bwd_layout_for(dtype, d, mxd::kTilePxLog2Max);
     return L;

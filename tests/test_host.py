@@ -363,3 +363,16 @@ def test_forward_cu_form_is_refused_beyond_its_index_arithmetic(monkeypatch, for
     if forced:
         plan = _lib.make_plan(0, 0, 1, 60, 32768, 64, 1, 1, 1 << 16, 16)
         assert plan.block != 1024, plan.as_dict()
+
+
+@pytest.mark.parametrize("code,hd,honoured", [(1, 3, False), (2, 1, False), (1, 4, True), (0, 3, True)])
+def test_tile_sizes_that_no_kernel_is_built_for_are_not_taken(monkeypatch, code, hd, honoured):
+    """16-bit rows of fewer than 4 channels have the grad_value pass for tiles of 512 pixels alone: there MXD_MSDA_TILE_PX_LOG2
+    changes nothing (the size of the workspace tells which tiles a backward call lays its run table out for)."""
+    lib = _lib.load()
+    dims = (2, 20000, 8, hd, 1, 1, 3000, 4)
+    default = lib.mxd_msda_backward_workspace_bytes(code, *dims)
+    for v in (7, 8):
+        monkeypatch.setenv("MXD_MSDA_TILE_PX_LOG2", str(v))
+        _lib.reload_tuning()
+        assert (lib.mxd_msda_backward_workspace_bytes(code, *dims) != default) == honoured

@@ -5,7 +5,7 @@ import torch
 
 from drivingsdk_amd import workloads
 from test_msda_gpu import _check_all
-from util import BWD_FP32, FWD_FP32, half_tol
+from util import BWD_FP32, FWD_FP32, half_tol, set_tuning
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,10 @@ def test_sample_counts_around_a_pass(gpu_device, nl, npts, dtype):
 def test_short_rows(gpu_device, nl, npts, dtype, hd):
     fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
     _check_all(_inputs(_MAPS[:nl], npts, 131, 4, hd, dtype, hd + npts), gpu_device, fwd, bwd)
+
+
+@pytest.mark.parametrize("hd", [1, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_narrow_16_bit_rows_with_a_forced_tile_size(gpu_device, monkeypatch, dtype, hd):
+    set_tuning(monkeypatch, MXD_MSDA_TILE_PX_LOG2=7)
+    _check_all(_inputs(_MAPS, 4, 131, 4, hd, dtype, hd), gpu_device, half_tol(dtype), half_tol(dtype))
