@@ -187,6 +187,7 @@ void* device_scratch()
 
 struct Dims {
     int64_t bs, nk, nh, hd, nl, nl_attn, nq, np;
+    int gka = 0;  // geometric kernel attention (on the shared kernels)
 };
 
 int check_dims(int dtype, const Dims& d)
@@ -346,6 +347,16 @@ int preferred_tile_px_log2(int dtype, const Dims& d)
     const int v = tuning().tile_px_log2;
     if (v >= 7 && v <= mxd::kTilePxLog2Max) return v;
     if (d.hd <= 32) return mxd::kTilePxLog2Max;
+    // Geometric kernel attention clamps its samples to the map, which piles many of them on the border's pixels.  Those get extra
+    // lists in the slots of a workgroup that its tile leaves free; a map cut in tiles of 256 or 128 pixels has none to speak of.
+    // With enough samples that is worth two to four passes over the records.  15 x 25 pixels, 24 x 7156 queries x 15, backward,
+    // tiles by head size -> one tile of 512: float32 48 channels 692 -> 584 us, 96 channels 1076 -> 918, 160 channels
+    // 2417 -> 1791; float16 646 -> 576, 812 -> 758, 1546 -> 1232.  From 3.6 million samples on 18 of 24 sizes of 280 to 360
+    // pixels gain 10 to 30 %, the others are within 5 % of even (but for one at +15 %: 96 channels in float16, 280 pixels, 20.6
+    // million).  Not with fewer samples (half a million 1.3 to 1.7 times as long), not on maps that one smaller tile holds (6 x 10:
+    // 1.04 to 1.5), not where the free slots are fewer than the pixels that want them (420 pixels, 48 channels: 1.13 to
+    // 1.3) and not for several levels (15 x 25 and 8 x 13, 48 channels, 11 million: 1.13 and 1.21).
+    if (d.gka && d.nl == 1 && d.nk > 256 && d.nk <= 384 && d.bs * d.nh * d.nq * d.np >= (int64_t(3) << 20)) return mxd::kTilePxLog2Max;
     // (measured at 8 heads x 128 channels, encoder levels: float16 backward 588 us with tiles of 512 pixels, 431 with 256,
     //  383 with 128; float32 722, 590, 586)
     return d.hd <= 64 ? 8 : 7;
@@ -1309,8 +1320,8 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
                            const FusedBackward* fused = nullptr)
 {
     const int meta64 = take_meta_flag(&dtype);
-    const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np};
     const int gka = kind == 1, grid = kind >= 2 ? kind - 1 : 0;
+    const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np, gka};
     const char* who = fused  ? "mxd_msda_fused_backward"
                       : grid ? "mxd_grid_sampler2d_backward"
                       : gka  ? "mxd_gka_backward"
@@ -1482,12 +1493,11 @@ int mxd_msda_backward_static(const void* value, const int32_t* spatial_shapes, c
 size_t mxd_gka_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk, int64_t nh, int64_t hd, int64_t nl,
                                         int64_t nq, int64_t np)
 {
-    int code = dtype;
-    take_meta_flag(&code);
-    const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
+    take_meta_flag(&dtype);
+    const Dims d{bs, nk, nh, hd, nl, nl, nq, np, 1};
+    if (check_dims(dtype, d) != MXD_OK) return 0;
     mxd::GkaArgs a;
-    if (check_dims(code, d) == MXD_OK && gka_plan(code, d, true, &a)) return gka_part_bytes(a);
-    return mxd_msda_backward_workspace_bytes(dtype, bs, nk, nh, hd, nl, nl, nq, np);
+    return gka_plan(dtype, d, true, &a) ? gka_part_bytes(a) : bwd_layout(dtype, d).total;
 }
 
 int mxd_gka_backward(const void* value, const int32_t* spatial_shapes, const int32_t* level_start_index,

@@ -119,6 +119,19 @@ def test_largest_reference_shape_at_full_batch(gpu_device):
         assert rel_err(g_, w_) <= tol, (name, rel_err(g_, w_))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("hd,hw,nq", [(48, (15, 25), 4681), (96, (257, 1), 4682), (160, (24, 16), 4682), (37, (16, 16), 4682)])
+def test_small_maps_and_many_samples_on_the_shared_kernels(gpu_device, hd, hw, nq, dtype):
+    """Head sizes that the kernels with value in LDS do not take, on both sides of the rule that keeps a small map in one tile."""
+    inp = make_inputs([16, nq, hd, 2, 1, 21], hw, seed=hd)
+    value, sh, lsi, loc, attn, go = inp
+    v, a, g = (t.to(dtype).double() for t in (value, attn, go))
+    want = (gka.forward(v, sh, lsi, loc, a),) + gka.backward(v, sh, lsi, loc, a, g)
+    got = run_gpu(*inp, gpu_device, dtype=dtype, loc_dtype=torch.float32)
+    for k, (g_, w_) in enumerate(zip(got, want)):
+        assert rel_err(g_, w_) <= (HALF if dtype == torch.float16 else FWD_FP32 if k == 0 else BWD_FP32)
+
+
 def test_levels_that_overlap_beyond_the_run_table_take_the_atomic_form(gpu_device, monkeypatch):
     """level_start_index is the caller's.  Three levels of 513 pixels that overlap inside 600 keys have six tiles of 512
     pixels between them where the run table of the tile-mode backward has room for four (num_keys / 512 + num_levels).

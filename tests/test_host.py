@@ -365,6 +365,28 @@ def test_forward_cu_form_is_refused_beyond_its_index_arithmetic(monkeypatch, for
         assert plan.block != 1024, plan.as_dict()
 
 
+@pytest.mark.parametrize("code", [0, 1, 2])
+@pytest.mark.parametrize("nk,nq,nl,one_tile", [(257, 2185, 1, True), (375, 7156, 1, True), (384, 2185, 1, True), (256, 2185, 1, False),
+                                               (385, 2185, 1, False), (375, 2184, 1, False), (375, 2185, 2, False)])
+def test_geometric_kernel_attention_keeps_a_small_map_in_one_tile(monkeypatch, code, nk, nq, nl, one_tile):
+    """From 3 * 2^20 samples on maps of 257 to 384 pixels go through the grad_value pass as one tile (the size of the workspace
+    tells the tile size), for geometric kernel attention alone."""
+    lib = _lib.load()
+    for hd in (48, 96, 160):
+        dims, rest = (24, nk, 4, hd), (nq, 15)
+
+        def sizes():
+            return (lib.mxd_gka_backward_workspace_bytes(code, *dims, nl, *rest),
+                    lib.mxd_msda_backward_workspace_bytes(code, *dims, nl, nl, *rest))
+        by_rule = sizes()
+        monkeypatch.setenv("MXD_MSDA_TILE_PX_LOG2", "9")
+        _lib.reload_tuning()
+        forced = sizes()
+        assert (by_rule[0] == forced[0]) == one_tile and by_rule[1] != forced[1]
+        monkeypatch.delenv("MXD_MSDA_TILE_PX_LOG2")
+        _lib.reload_tuning()
+
+
 @pytest.mark.parametrize("code,hd,honoured", [(1, 3, False), (2, 1, False), (1, 4, True), (0, 3, True)])
 def test_tile_sizes_that_no_kernel_is_built_for_are_not_taken(monkeypatch, code, hd, honoured):
     """16-bit rows of fewer than 4 channels have the grad_value pass for tiles of 512 pixels alone: there MXD_MSDA_TILE_PX_LOG2
