@@ -190,6 +190,8 @@ struct Dims {
     int gka = 0;  // geometric kernel attention (on the shared kernels)
 };
 
+size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
+
 int check_dims(int dtype, const Dims& d)
 {
     if (elem_size(dtype) == 0) return fail(MXD_E_DTYPE, "dtype code %d is not float32(0)/float16(1)/bfloat16(2)", dtype);
@@ -557,10 +559,30 @@ int64_t estimated_cached_rows(const Dims& d, int64_t cap_rows)
     return (int64_t)total;
 }
 
+// Time of the forward's one-workgroup-per-CU form over that of the general kernel, estimated.  What the form gains: a row takes fewer
+// instructions, and rows of cached levels come from LDS.  What it loses: its units work through whole chunks of 16 samples, the
+// general kernel's through as many as there are; rows from memory cost more where the slices that run side by side on an XCD
+// overflow its L2, because four wavefronts per SIMD hide less of it; every workgroup pays its launch and cache fill (`start`, in
+// rows of its share) before its share of the rows.  Conversions weigh more here (bfloat16 has no mixed multiply-add), most with 16
+// lanes per row.  The fused form's general kernel computes its softmax in a pass of its own over the samples.
+// Weights fitted to 2 827 pairs of timings: one to five levels of 20 x 20 to 130 x 200 pixels, 1 to 8 points, 4, 8 and 16 heads of 16
+// to 128 channels, 500 to 60 000 queries, from a million samples on, all three types, plain and fused, uniformly random
+// locations: the form chosen takes 2.1 % longer than the better of the two on average, always the general kernel 9.0 %.
+// 179 problems drawn from the same ranges afterwards: plain 2.2 % (3.5 % with separate lines for samples, levels and slices; six instead
+// of 16 beyond 15 %), fused 1.5 % (1.7 %).
+double cu_over_general(int dtype, bool fused, int lpr, int64_t samples, double from_memory, double over, double start)
+{
+    double row = lpr <= 8 ? 0.55 : 0.6;
+    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.65 : lpr <= 8 ? 0.7 : dtype == MXD_DTYPE_F16 ? 0.8 : 1.3;
+    if (fused) row *= 0.75;
+    const double padded = (double)round_up((size_t)samples, mxd::kChunk) / (double)samples;
+    return row * (from_memory * (1.0 + 0.85 * over) + 0.85 * (1.0 - from_memory)) * (0.25 + 0.75 * padded) + start;
+}
+
 // The forward's one-workgroup-per-CU form (msda_fwd_cu.hip): whether a problem takes it, and its launch geometry.
-// It needs 16-byte lanes, rows of at most 16 lanes and the plain operator; it pays when at least the last level fits
-// the CU's LDS and the problem is large enough to keep 256 such workgroups busy well beyond their cache fill.
-bool plan_forward_cu(int dtype, const Dims& d, int vec, int lpr, int npass, mxd_msda_plan* p, int* cache_bytes)
+// It needs 16-byte lanes, rows of at most 16 lanes and the plain operator or its fused form; it pays when at least the last level fits
+// the CU's LDS and the problem is large enough to keep 256 such workgroups busy well beyond their cache fill (cu_over_general).
+bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int npass, mxd_msda_plan* p, int* cache_bytes)
 {
     const int mode = tuning().fwd_cu;
     const int es = elem_size(dtype);
@@ -576,42 +598,19 @@ bool plan_forward_cu(int dtype, const Dims& d, int vec, int lpr, int npass, mxd_
     const int cap = mxd::kCuLdsBytes - mxd::kCuTableBytes;  // (two level tables come first)
     const int64_t cap_rows = cap / (d.hd * es) - 1;
     const int64_t cached = estimated_cached_rows(d, cap_rows);
-    // By default (measured on MI355X, uniformly random locations, this form against the general kernel, float32 /
-    // float16).  Units of up to 16 samples (one chunk): it wins where about half of the samples are gathered from LDS
-    // -- the Deformable-DETR encoder shape, 79 against 86 us / 71 against 86 us; one level of 64 x 64 with 8 points,
-    // 85 against 106 / 77 against 97 -- and is level or behind where fewer are (BEVFormer's levels with 4 points: 214
-    // against 215 / 149 against 151; five levels: 258 against 206 / 185 against 179).  Units of more samples: it wins
-    // as soon as the last level is cached -- the encoder's levels with 5, 6, 8, 12, 16 points: 0.93, 0.91, 0.79, 0.76,
-    // 0.73 of the general kernel's time / 0.82, 0.78, 0.74, 0.68, 0.70; the BEVFormer shape 395 against 433 / 237
-    // against 288 -- unless a (batch, head) slice of value is far beyond an XCD's 4 MiB of L2, where the general
-    // kernel's larger number of wavefronts hides more of the memory latency (pyramid from 256 x 256, 11 MB in
-    // float32: 1750 against 1504 us; 5.6 MB in float16: 1109 against 1147; five levels from 200 x 300, 10 MB: 441
-    // against 404 / 5 MB: 287 against 308), and not where nothing is cached (one level of 100 x 150, 32 points: 153
-    // against 147 / 174 against 138).  Small problems stay with the general kernel (8 x 900 queries: 59 against 37).
-    if (mode < 0) {
-        double last = (double)d.nk, rows = 0.0;
-        if (d.nl > 1) last = (double)d.nk * 3.0 / ((double)(int64_t(1) << (2 * (d.nl < 16 ? d.nl : 16))) - 1.0);
-        int levels_cached = 0;
-        for (double r = last; levels_cached < d.nl && rows + r <= (double)cap_rows; r *= 4.0) {
-            rows += r;
-            ++levels_cached;
-        }
-        if (levels_cached == 0 || d.bs * d.nh * d.nq * d.nl * d.np < (int64_t(1) << 20)) return false;
-        // Its units work through whole chunks of 16 samples, the general kernel's through as many as there are: up to 8 samples
-        // (3 x 15247 queries, 4 heads, levels from 58 x 197: float32 48 against 35 us, float16 39 against 30), and 17 to 20 with rows
-        // of 16 lanes (2 x 5355 queries of 18 samples, 256-byte rows: 57 against 54 / 76 against 55), go there; so do rows of 16
-        // lanes in bfloat16, whose conversions the four wavefronts per SIMD of this form do not hide, where an XCD's L2 holds the
-        // slice (3 x 6321 queries, 128 channels, 1.6 MB: 100 against 86; 3.8 MB 80 against 70; the encoder's levels, 5.1 MB, 103
-        // against 106).
-        const int64_t samples = d.nl * d.np, slice = d.nk * d.hd * es;
-        if (samples <= mxd::kChunk / 2 || (lpr == 16 && ((samples > mxd::kChunk && samples <= mxd::kChunk + 4) || (dtype == MXD_DTYPE_BF16 && slice <= (int64_t(4) << 20)))))
-            return false;
-        // (rows of 256 bytes, 16 samples per unit, one level of four cached: 0.88 to 0.93 of the general kernel's time at
-        //  the encoder's levels -- head_dim 64 and 48 in float32, 128 and 96 in float16, slices of 5 MB -- but 1.18 to
-        //  1.33 at slices of 8 MB and more, and 0.93 to 1.25 with 8 samples per unit)
-        const bool long_rows = lpr == 16 && d.nl * d.np == mxd::kChunk && slice <= (int64_t(6) << 20);
-        if (d.nl * d.np <= mxd::kChunk ? 2 * levels_cached < d.nl && !long_rows : slice > (int64_t(8) << 20)) return false;
+    // Levels whose rows come from LDS, estimated as above.
+    double last = (double)d.nk, rows = 0.0;
+    if (d.nl > 1) last = (double)d.nk * 3.0 / ((double)(int64_t(1) << (2 * (d.nl < 16 ? d.nl : 16))) - 1.0);
+    int levels_cached = 0;
+    for (double r = last; levels_cached < d.nl && rows + r <= (double)cap_rows; r *= 4.0) {
+        rows += r;
+        ++levels_cached;
     }
+    // (nothing cached is nothing gained; 8 x 900 queries, under a million samples: 59 against 37 us)
+    const double from_memory = (double)(d.nl - levels_cached) / (double)d.nl;
+    if (mode < 0 && (levels_cached == 0 || d.bs * d.nh * d.nq * d.nl * d.np < (int64_t(1) << 20) ||
+                     cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, 0.0, 0.0) >= 1.0))
+        return false;
     const int U = mxd::kWave / lpr;
     const int64_t groups = (d.nq + U - 1) / U;
     // Workgroups per (batch, head): every XCD has 32 CUs, each of which runs one workgroup at a time; the launch
@@ -619,7 +618,7 @@ bool plan_forward_cu(int dtype, const Dims& d, int vec, int lpr, int npass, mxd_
     // are not cached come from the XCD's 4 MiB L2: the workgroups that run side by side on an XCD should work on as
     // few (batch, head) slices as possible (workgroups of an XCD are numbered head, query range, batch element).
     int64_t best_p = 1;
-    double best_cost = -1.0;
+    double best_cost = -1.0, best_over = 0.0, best_rows = 1.0;
     const int64_t max_p = groups < 512 ? groups : 512;
     const double slice_bytes = (double)(d.nk - cached) * (double)(d.hd * es);
     const double launch = 3000.0, fill = (double)cached + 1000.0;   // in units of one gathered row
@@ -653,9 +652,13 @@ bool plan_forward_cu(int dtype, const Dims& d, int vec, int lpr, int npass, mxd_
         if (best_cost < 0.0 || cost < best_cost) {
             best_cost = cost;
             best_p = P;
+            best_over = over;
+            best_rows = (double)tq * (double)(d.nl * d.np) * 4.0;
         }
     }
     if (best_cost < 0.0) return false;  // (not a shape for this form)
+    if (mode < 0 && cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, best_over, (launch + 1500.0 + (double)cached) / best_rows) >= 1.0)
+        return false;
     const int64_t tq = U * (((d.nq + best_p - 1) / best_p + U - 1) / U);
     const int64_t nt = (d.nq + tq - 1) / tq;
     memset(p, 0, sizeof(*p));
@@ -691,7 +694,7 @@ int forward_cu_flip(int dtype)
 }
 
 // level_cache: in/out, bytes of LDS for the forward's level cache (asked for -> granted)
-// cu_form: in/out, whether the forward may take / takes the one-workgroup-per-CU form
+// cu_form: in/out, whether the forward may take (2: in its fused form) / takes the one-workgroup-per-CU form
 // align_bytes: alignment of the rows' buffers; whole_pieces: see row_geometry (launches read rows in overlapping pieces where
 // no whole ones fit; the plan that mxd_msda_make_plan reports describes whole pieces)
 int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_plan* p, int* level_cache = nullptr,
@@ -708,7 +711,7 @@ int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_
     // (the forward keeps 32 lanes in one pass: at 8 heads x 128 channels in float32 two passes take 248 against 237 us)
     row_geometry(es, d.hd, lane_bytes, &vec, &lpr, &npass, backward && tuning().bwd_two_pass != 0, whole_pieces);
     if (!backward && rows_of_16 && cu_form && *cu_form && level_cache) {
-        if (plan_forward_cu(dtype, d, vec, lpr, npass, p, level_cache)) return MXD_OK;
+        if (plan_forward_cu(dtype, d, *cu_form == 2, vec, lpr, npass, p, level_cache)) return MXD_OK;
     }
     if (cu_form) *cu_form = 0;
     // (a row is shared by four lanes at least: 8 bytes each for rows of 32 -- 16 channels in float16, 2 x 13253 queries of 18
@@ -810,8 +813,6 @@ void fill_args(mxd::KArgs* a, int dtype, const Dims& d)
     a->batch_bytes = (uint32_t)(d.nk * d.nh * d.hd * es);
     a->gbatch_bytes = (uint32_t)(d.nk * d.nh * d.hd * 4);
 }
-
-size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
 
 int log2_lanes(int64_t lanes)
 {
@@ -1264,6 +1265,7 @@ int mxd_msda_fused_forward(const void* value, const int32_t* spatial_shapes, con
                         ptr_align(reference_points) >= 2 * elem_size(dtype);
     if (cu) {
         cache = 1;
+        cu = 2;
         rc = make_plan(0, dtype, d, align, &a.plan, &cache, &cu);
         if (rc != MXD_OK) return rc;
     }

@@ -398,3 +398,24 @@ def test_tile_sizes_that_no_kernel_is_built_for_are_not_taken(monkeypatch, code,
         monkeypatch.setenv("MXD_MSDA_TILE_PX_LOG2", str(v))
         _lib.reload_tuning()
         assert (lib.mxd_msda_backward_workspace_bytes(code, *dims) != default) == honoured
+
+
+@pytest.mark.parametrize("code,dims,takes", [
+    # bs, nk, nh, hd, nl, nq, np: measured, this form / the general kernel in us
+    (0, (1, 6180, 8, 16, 4, 30000, 8), True),         # 52 / 97: half of the rows from LDS, chunks full
+    (1, (1, 19947, 8, 16, 4, 30000, 4), True),        # 40 / 58
+    (0, (4, 20017, 8, 16, 5, 14000, 6), True),        # 161 / 218: two chunks, the second nearly full
+    (2, (2, 6180, 8, 32, 4, 19947, 4), True),         # 53 / 69
+    (1, (1, 30825, 8, 16, 4, 30000, 4), True),        # 51 / 65
+    (1, (6, 19700, 8, 64, 3, 9675, 2), False),        # 147 / 83: chunks of 6 samples of 16
+    (1, (4, 30825, 8, 96, 4, 14000, 3), False),       # 411 / 244: rows of 16 lanes, most of them from memory
+    (0, (3, 30825, 16, 32, 4, 7001, 1), False),       # 107 / 54
+    (0, (4, 19947, 16, 32, 4, 14000, 2), False),      # 292 / 193
+    (2, (6, 20017, 8, 128, 5, 9675, 4), False),       # 529 / 396: 20 samples in two chunks, conversions
+    (0, (2, 30825, 8, 64, 4, 5355, 6), False),        # 138 / 96: slices of 8 MB
+    (0, (2, 19947, 8, 32, 4, 900, 4), False),         # too few samples
+    (0, (2, 40000, 8, 32, 1, 19947, 16), False),      # no level fits the LDS
+])
+def test_forward_takes_the_form_that_measured_faster(code, dims, takes):
+    bs, nk, nh, hd, nl, nq, npts = dims
+    assert (_lib.make_plan(0, code, bs, nk, nh, hd, nl, nl, nq, npts).block == 1024) == takes
