@@ -980,14 +980,23 @@ bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
 }
 
 // Whether these kernels take a problem.  Forward: whole rows only (with the channels in two parts, which read the locations twice, it
-// takes 36 us where the general kernel takes 29), and from half a million samples on (446 000 samples 6.7 -> 8.7 us, 685 000
-// 11.6 -> 9.5, 2.4 million 23 -> 16).  Backward: wherever the slab fits, whole or in two parts (48 x 24 pixels, 64 channels, float32,
+// takes 36 us where the general kernel takes 29), and from as many samples on as pay for the slabs' way into LDS, general kernel / this
+// one at 64 channels, 375 pixels, 15 points, 2 batch elements x 4 heads: float32 0.52 million samples 8.7 / 6.6 us, 1.0 million 14.4 /
+// 8.8, 3 million 39 / 20; float16, whose rows cost the general kernel half as many lines, 0.52 million 6.7 / 7.4, 0.7 million 7.5 /
+// 7.6, 1.0 million 11.0 / 9.3, 3 million 27.6 / 19.4 (of five maps of 160 to 2400 pixels two are even or better at 0.7 million and
+// three at 1.0 million; in float32 three of four at half a million).  16-bit units of fewer than 4 samples stay with the general
+// kernel (1 to 3 samples: 0.9 to 1.2 of its time), with fewer than 8 slabs those of fewer than 12 (four slabs: 1 sample 1.5, 4 samples 1.1
+// to 1.3, 8 samples 1.0 to 1.2, 12 samples 0.9 to 1.0).  Backward: wherever the slab fits, whole or in two parts (48 x 24 pixels, 64 channels, float32,
 // two parts: 180 -> 112 us; in four parts 64 x 46 pixels of 32 channels went from 80 to 107 us).
 bool gka_plan(int dtype, const Dims& d, bool backward, mxd::GkaArgs* a)
 {
     const int mode = tuning().gka_slab;
     if (mode == 0 || tuning().bwd_atomic || d.nk >= 32768 || d.nl * d.np > 256 || d.nl != d.nl_attn || d.bs * d.nh > 65536) return false;
-    if (!backward) return (mode > 0 || d.bs * d.nh * d.nq * d.nl * d.np >= (int64_t(1) << 19)) && gka_plan_parts(dtype, d, 1, a);
+    if (!backward) {
+        const bool half = elem_size(dtype) == 2, pays = d.bs * d.nh * d.nq * d.nl * d.np >= (half ? int64_t(7) << 17 : int64_t(1) << 19) &&
+                                                        (!half || d.nl * d.np >= (d.bs * d.nh < 8 ? 12 : 4));
+        return (mode > 0 || pays) && gka_plan_parts(dtype, d, 1, a);
+    }
     return gka_plan_parts(dtype, d, 1, a) || gka_plan_parts(dtype, d, 2, a);
 }
 
