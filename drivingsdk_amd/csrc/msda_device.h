@@ -189,9 +189,7 @@ struct LevelLanes {
         }
         return v;
     }
-    // {H, W, first key, 0} of level l (the same in all lanes)
-    __device__ int32_t H(int l) const { return __builtin_amdgcn_readlane(geo.x, l); }
-    __device__ int32_t W(int l) const { return __builtin_amdgcn_readlane(geo.y, l); }
+    // first key of level l (the same in all lanes)
     __device__ int32_t base(int l) const { return __builtin_amdgcn_readlane(geo.z, l); }
 
     // Rows (pixels of a batch element) [*r0, *r1) of piece `part` (< kRowParts) of tile `tile` of a batch element that
