@@ -20,8 +20,10 @@
 //     counters, one workgroup per (batch, level)), then every pixel row is formed once, by lanes that own its channels, from
 //     the grad_out rows of its records -- those of a batch element stay in L2 -- and stored once, whole.
 //
-// Measured (6 x 900 anchors x 13 points, 6 cameras x 4 scales, 256 channels in 8 groups, float32; float16 with one batch
-// element), before -> after: see the launchers below.
+// Measured (6 x 900 anchors x 13 points, 6 cameras x 4 scales, 256 channels in 8 groups, float32), one unit of lanes per anchor and
+// group and the tile pass -> these: forward 395 -> 270 us (float16, one batch element 140 -> 25), forward and backward 1969 ->
+// 855.  Of the 585 us of the backward the dots with the sort beside them take 318, the gradient of the maps 221, the caller's
+// layouts 40 (kernel times one at a time; rows from HBM bound all but the last).
 #include "dagg.h"
 
 namespace mxd {

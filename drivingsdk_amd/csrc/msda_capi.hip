@@ -560,23 +560,24 @@ int64_t estimated_cached_rows(const Dims& d, int64_t cap_rows)
 }
 
 // Time of the forward's one-workgroup-per-CU form over that of the general kernel, estimated.  What the form gains: a row takes fewer
-// instructions, and rows of cached levels come from LDS.  What it loses: its units work through whole chunks of 16 samples, the
-// general kernel's through as many as there are; rows from memory cost more where the slices that run side by side on an XCD
-// overflow its L2, because four wavefronts per SIMD hide less of it; every workgroup pays its launch and cache fill (`start`, in
-// rows of its share) before its share of the rows.  Conversions weigh more here (bfloat16 has no mixed multiply-add), most with 16
-// lanes per row.  The fused form's general kernel computes its softmax in a pass of its own over the samples.
-// Weights fitted to 2 827 pairs of timings: one to five levels of 20 x 20 to 130 x 200 pixels, 1 to 8 points, 4, 8 and 16 heads of 16
-// to 128 channels, 500 to 60 000 queries, from a million samples on, all three types, plain and fused, uniformly random
-// locations: the form chosen takes 2.1 % longer than the better of the two on average, always the general kernel 9.0 %.
-// 179 problems drawn from the same ranges afterwards: plain 2.2 % (3.5 % with separate lines for samples, levels and slices; six instead
-// of 16 beyond 15 %), fused 1.5 % (1.7 %).
-double cu_over_general(int dtype, bool fused, int lpr, int64_t samples, double from_memory, double over, double start)
+// instructions, and rows of cached levels come from LDS beside the others.  What it loses: its units work through whole chunks of 16
+// samples, the general kernel's through as many as there are; rows from memory cost more where the slices that run side by side on
+// an XCD overflow its L2 (`spill`: by how many L2s, beyond 1.4 of them), because four wavefronts per SIMD hide less of it; every
+// workgroup pays its launch and cache fill (`start`, in rows of its share) before its share of the rows.  Conversions weigh more
+// here, most with 16 lanes per row (bfloat16, which has no mixed multiply-add, never pays there).  The fused form's general kernel computes
+// its softmax in a pass of its own over the samples.
+// Weights fitted to 3 339 pairs of timings: one to six levels of 20 x 20 to 300 x 400 pixels, 1 to 8 points, 4, 8 and 16 heads of 16
+// to 128 channels, 500 to 60 000 queries or every pixel, from a million samples on, all three types, plain and fused, uniformly
+// random locations: the form chosen takes 1.6 % longer than the better of the two on average (110 of them more than 15 % longer),
+// always the general kernel 8.2 %.  On 275 problems drawn afterwards: plain 2.8 % (5.0 % with separate lines for samples, cached
+// levels, slices and types before it; always the general kernel 9.5 %), fused 2.1 % (2.4, 8.4).
+double cu_over_general(int dtype, bool fused, int lpr, int64_t samples, double from_memory, double spill, double start)
 {
-    double row = lpr <= 8 ? 0.55 : 0.6;
-    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.65 : lpr <= 8 ? 0.7 : dtype == MXD_DTYPE_F16 ? 0.8 : 1.3;
-    if (fused) row *= 0.75;
+    double row = 0.46;
+    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.52 : lpr <= 8 ? 0.62 : dtype == MXD_DTYPE_F16 ? 0.7 : 1.1;
+    if (fused) row *= 0.84;
     const double padded = (double)round_up((size_t)samples, mxd::kChunk) / (double)samples;
-    return row * (from_memory * (1.0 + 0.85 * over) + 0.85 * (1.0 - from_memory)) * (0.25 + 0.75 * padded) + start;
+    return row * (1.0 + from_memory * spill) * (0.2 + 0.8 * padded) + start;
 }
 
 // The forward's one-workgroup-per-CU form (msda_fwd_cu.hip): whether a problem takes it, and its launch geometry.
@@ -618,7 +619,7 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
     // are not cached come from the XCD's 4 MiB L2: the workgroups that run side by side on an XCD should work on as
     // few (batch, head) slices as possible (workgroups of an XCD are numbered head, query range, batch element).
     int64_t best_p = 1;
-    double best_cost = -1.0, best_over = 0.0, best_rows = 1.0;
+    double best_cost = -1.0, best_spill = 0.0, best_rows = 1.0;
     const int64_t max_p = groups < 512 ? groups : 512;
     const double slice_bytes = (double)(d.nk - cached) * (double)(d.hd * es);
     const double launch = 3000.0, fill = (double)cached + 1000.0;   // in units of one gathered row
@@ -646,18 +647,19 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
         if (mode < 0 && !((trial.xcd_mode == 1 && trial.heads_per_xcd <= 2) || (trial.xcd_mode == 2 && trial.xcds_per_head <= 2)))
             continue;
         double over = ceil(slices) * slice_bytes / (4.0 * 1024 * 1024) - 0.4;
+        const double spill = over < 1.0 ? 0.0 : (over > 3.0 ? 2.0 : over - 1.0);
         over = over < 0.0 ? 0.0 : (over > 1.0 ? 1.0 : over);
         const double gather = (1.0 + 0.5 * over) * (double)tq * (double)(d.nl * d.np) * 4.0;
         const double cost = rounds * (launch + fill + gather);
         if (best_cost < 0.0 || cost < best_cost) {
             best_cost = cost;
             best_p = P;
-            best_over = over;
+            best_spill = spill;
             best_rows = (double)tq * (double)(d.nl * d.np) * 4.0;
         }
     }
     if (best_cost < 0.0) return false;  // (not a shape for this form)
-    if (mode < 0 && cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, best_over, (launch + 1500.0 + (double)cached) / best_rows) >= 1.0)
+    if (mode < 0 && cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, best_spill, (launch + 2500.0 + (double)cached) / best_rows) >= 1.0)
         return false;
     const int64_t tq = U * (((d.nq + best_p - 1) / best_p + U - 1) / U);
     const int64_t nt = (d.nq + tq - 1) / tq;

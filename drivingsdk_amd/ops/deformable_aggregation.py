@@ -3,8 +3,8 @@
 Same class name, argument order, coercions, saved tensors and return structure as the reference's Python layer
 (mx_driving/ops/npu_deformable_aggregation.py:10-88): ``forward(ctx, mc_ms_feat, spatial_shape,
 scale_start_index, sampling_location, weights)`` and ``backward -> (grad_mc_ms_feat, None, None,
-grad_sampling_location, grad_weights)``.  The compute sits in ``drivingsdk_amd._C`` (the HIP kernels of
-multi-scale deformable attention, run with a channel group as head and a (camera, scale) pair as level).
+grad_sampling_location, grad_weights)``.  The compute sits in ``drivingsdk_amd._C`` (HIP kernels of its own,
+csrc/dagg.hip).
 """
 import torch
 from torch.autograd import Function
