@@ -91,7 +91,7 @@ struct Tuning {
     int bwd_sparse;      // MXD_MSDA_BWD_SPARSE: 0 = zero-fill (and, for 16-bit dtypes, round) the whole fp32 image of
                          // grad_value, 1 = only the rows that receive atomic additions
     int bwd_unit_split;  // MXD_MSDA_BWD_UNIT_SPLIT: 0 = a unit of the first backward kernel is always a whole query, 1 = queries
-                         // of 25 to 32 samples get two units, 2 = queries of 17 to 32 samples
+                         // of 25 to 32 samples get two units, those of 17 to 24 where it pays, 2 = queries of 17 to 32 samples
     int bwd_lane_bytes;  // MXD_MSDA_BWD_LANE_BYTES: most bytes of a row one lane of the first backward kernel loads
                          // (16, 8, 4), 0 = chosen here
     int tile_px_log2;    // MXD_MSDA_TILE_PX_LOG2: log2 of the pixels per tile of the grad_value pass (9, 8, 7), 0 = chosen here
@@ -187,7 +187,7 @@ void* device_scratch()
 
 struct Dims {
     int64_t bs, nk, nh, hd, nl, nl_attn, nq, np;
-    int gka = 0;  // geometric kernel attention (on the shared kernels)
+    int kind = 0;  // which operator the shared kernels run for: 0 the plain one, 1 geometric kernel attention, 2 the fused form
 };
 
 size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
@@ -300,7 +300,7 @@ int backward_lane_bytes(int dtype, const Dims& d)
 // longer runs; with few queries they leave the chip short of workgroups, so the size steps down until the
 // launch has about six workgroups per CU.  64 is the least for rows of up to 64 bytes (16 units per
 // wavefront, 4 wavefronts), 32 otherwise.  MXD_MSDA_BWD_TILE_Q overrides (32/64/128/256).
-static int64_t bwd_tile_q(int dtype, const Dims& d)
+static int64_t bwd_tile_q(int dtype, const Dims& d, bool early_split)
 {
     // (units with very many samples measured 1 to 2 % better with 64)
     int vec, lpr, npass;
@@ -321,11 +321,18 @@ static int64_t bwd_tile_q(int dtype, const Dims& d)
     // 16 of its samples, so that the workgroup -- half as many queries -- stages all its samples while it counts its
     // records (their geometry is derived once) and collects its records in LDS to write its slab in whole lines, as
     // with up to 16 samples per query.
-    // (it pays when the second unit has work for most of its lanes -- encoder levels, float32: 32 samples per query 544
-    //  against 571 us, BEVFormer 1036 against 1094; 24 samples 2370 against 2301, 20 samples 442 against 420 --: from 25
-    //  samples on; MXD_MSDA_BWD_UNIT_SPLIT=2 splits from 17 on)
+    // From 25 samples on the second unit has work for most of its lanes (encoder levels, float32, 32 samples: one unit / two 566 /
+    // 486 us, BEVFormer 1044 / 967).  With 17 to 24 samples, most of whose second units idle, it depends on what the shorter
+    // slabs cost the tile pass: it pays from 16 000 keys on (18, 22, 21 and 24 samples, three types, 40 000 to 58 000 queries: 19 000
+    // keys 0.85 to 1.01 of the time with one unit, 32 000 keys 0.79 to 0.98; 12 000 keys 0.93 to 1.06, 5 000 keys 0.96 to 1.10),
+    // for rows of more than 64 bytes in float32 (5 000 keys 0.96 to 1.03, 12 000 keys 0.93 to 1.03) and where queries are
+    // few (5 000 queries x 8 heads: 5 000 keys 0.89 to 1.04, 12 000 keys 0.83 to 0.98).  The plain operator's only, whose workgroups
+    // collect their slab in LDS by it: the fused form takes 0.96 to 1.22, geometric kernel attention 0.99 to 1.14 of the
+    // time with one unit.  MXD_MSDA_BWD_UNIT_SPLIT=2 splits from 17 on.
     const int units = mxd::kWave / lpr * 4;
-    const int64_t split_from = tuning().bwd_unit_split >= 2 ? mxd::kChunk + 1 : mxd::kChunk + mxd::kChunk / 2 + 1;
+    const bool early = tuning().bwd_unit_split >= 2 ||
+                       (early_split && d.kind == 0 && (d.nk >= 16384 || (elem_size(dtype) == 4 && d.hd > 16) || d.bs * d.nh * d.nq <= 65536));
+    const int64_t split_from = early ? mxd::kChunk + 1 : mxd::kChunk + mxd::kChunk / 2 + 1;
     if (tuning().bwd_unit_split && least == units && units >= 8 && d.nl * d.np >= split_from && d.nl * d.np <= 2 * mxd::kChunk)
         return least / 2;
     return least;
@@ -358,18 +365,18 @@ int preferred_tile_px_log2(int dtype, const Dims& d)
     // million).  Not with fewer samples (half a million 1.3 to 1.7 times as long), not on maps that one smaller tile holds (6 x 10:
     // 1.04 to 1.5), not where the free slots are fewer than the pixels that want them (420 pixels, 48 channels: 1.13 to
     // 1.3) and not for several levels (15 x 25 and 8 x 13, 48 channels, 11 million: 1.13 and 1.21).
-    if (d.gka && d.nl == 1 && d.nk > 256 && d.nk <= 384 && d.bs * d.nh * d.nq * d.np >= (int64_t(3) << 20)) return mxd::kTilePxLog2Max;
+    if (d.kind == 1 && d.nl == 1 && d.nk > 256 && d.nk <= 384 && d.bs * d.nh * d.nq * d.np >= (int64_t(3) << 20)) return mxd::kTilePxLog2Max;
     // (measured at 8 heads x 128 channels, encoder levels: float16 backward 588 us with tiles of 512 pixels, 431 with 256,
     //  383 with 128; float32 722, 590, 586)
     return d.hd <= 64 ? 8 : 7;
 }
 
-BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2)
+BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2, bool early_split)
 {
     BwdLayout L;
     memset(&L, 0, sizeof(L));
     L.tile_px_log2 = tile_px_log2;
-    L.tile_q = bwd_tile_q(dtype, d);
+    L.tile_q = bwd_tile_q(dtype, d, early_split);
     L.nwg = (d.nq + L.tile_q - 1) / L.tile_q;
     L.rec_cap = 2 * L.tile_q * d.nl * d.np;
     // tiles per (batch, head) when the levels do not overlap: sum of ceil(pixels / tile) <= nk / tile + nl
@@ -397,12 +404,17 @@ BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2)
 }
 
 // The layout a launch uses: the tile size preferred for the rows, or 512-pixel tiles where the finer run table would
-// not fit the first kernel's bookkeeping.
+// not fit the first kernel's bookkeeping.  Queries of 17 to 24 samples keep one unit where the longer run table of two would not
+// fit, or would take the workspace beyond the static array that the one of whole queries fits.
 BwdLayout bwd_layout(int dtype, const Dims& d)
 {
     const int pref = preferred_tile_px_log2(dtype, d);
-    BwdLayout L = bwd_layout_for(dtype, d, pref);
-    if (!L.tiles && pref != mxd::kTilePxLog2Max) L = bwd_layout_for(dtype, d, mxd::kTilePxLog2Max);
+    BwdLayout L = bwd_layout_for(dtype, d, pref, true);
+    if (!L.tiles || L.total > kStaticScratchBytes) {
+        const BwdLayout whole = bwd_layout_for(dtype, d, pref, false);
+        if (whole.tiles && (!L.tiles || whole.total <= kStaticScratchBytes)) L = whole;
+    }
+    if (!L.tiles && pref != mxd::kTilePxLog2Max) L = bwd_layout_for(dtype, d, mxd::kTilePxLog2Max, false);
     return L;
 }
 
@@ -1334,7 +1346,7 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
 {
     const int meta64 = take_meta_flag(&dtype);
     const int gka = kind == 1, grid = kind >= 2 ? kind - 1 : 0;
-    const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np, gka};
+    const Dims d{bs, nk, nh, hd, nl, nl_attn, nq, np, fused ? 2 : gka};
     const char* who = fused  ? "mxd_msda_fused_backward"
                       : grid ? "mxd_grid_sampler2d_backward"
                       : gka  ? "mxd_gka_backward"
@@ -1450,7 +1462,7 @@ size_t mxd_msda_fused_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk
                                                int64_t nl, int64_t nq, int64_t np, int ref_dim, int want_grad_ref)
 {
     take_meta_flag(&dtype);
-    const Dims d{bs, nk, nh, hd, nl, nl, nq, np};
+    const Dims d{bs, nk, nh, hd, nl, nl, nq, np, 2};
     if (check_dims(dtype, d) != MXD_OK || (ref_dim != 2 && ref_dim != 4)) return 0;
     return bwd_layout(dtype, d).total + (want_grad_ref ? fused_part_bytes(d, ref_dim) : 0);
 }

@@ -419,3 +419,40 @@ def test_tile_sizes_that_no_kernel_is_built_for_are_not_taken(monkeypatch, code,
 def test_forward_takes_the_form_that_measured_faster(code, dims, takes):
     bs, nk, nh, hd, nl, nq, npts = dims
     assert (_lib.make_plan(0, code, bs, nk, nh, hd, nl, nl, nq, npts).block == 1024) == takes
+
+
+@pytest.mark.parametrize("code,nk,nh,hd,nq,npts,split", [
+    (1, 19947, 8, 32, 20000, 5, True),      # from 16 384 keys on
+    (1, 12000, 8, 32, 20000, 5, False),
+    (0, 6000, 8, 32, 20000, 5, True),       # rows of 128 bytes in float32
+    (0, 6000, 8, 16, 20000, 5, False),
+    (1, 6000, 8, 32, 4096, 5, True),        # 2 x 8 x 4096 units
+    (1, 6000, 8, 32, 4097, 5, False),
+    (1, 6000, 8, 32, 20000, 7, True),       # from 25 samples on
+    (0, 19947, 8, 32, 20000, 4, False)])    # a unit of 16
+def test_queries_of_17_to_24_samples_get_two_units_where_it_pays(code, nk, nh, hd, nq, npts, split):
+    """The queries per workgroup of the first backward kernel tell: a workgroup that makes one pass holds half as many."""
+    plan = _lib.make_plan(1, code, 2, nk, nh, hd, 4, 4, nq, npts)
+    assert (plan.tile_q * 2 == plan.units_per_wave * plan.waves_per_block) == split
+    # the fused form's workspace is that of whole queries, or of queries from 25 samples on
+    lib = _lib.load()
+    fused = lib.mxd_msda_fused_backward_workspace_bytes(code, 2, nk, nh, hd, 4, nq, npts, 2, 0)
+    assert (fused == lib.mxd_msda_backward_workspace_bytes(code, 2, nk, nh, hd, 4, 4, nq, npts)) == (not split or 4 * npts >= 25)
+
+
+def test_two_units_for_17_samples_never_cost_a_problem_its_form_or_the_static_array():
+    """Sizes just below the limits of the hand-over with whole queries: they keep it (and the static array) although two units per
+    query, with twice as many workgroups, would not."""
+    lib = _lib.load()
+    limit = lib.mxd_msda_backward_static_limit()
+    fits = [nq for nq in range(4000, 7000, 16) if lib.mxd_msda_backward_workspace_bytes(0, 1, 19947, 8, 32, 4, 4, nq, 5) <= limit]
+    records = 2 * 8 * 20 * 12                                # bytes per query, 2 records of 12 bytes per sample
+    whole = lambda nq: -(-nq // 32) * 32 * records + -(-8 * -(-nq // 32) * 43 * 4 // 256) * 256   # (43 = 19947 // 512 + 4 + 1 columns)
+    assert max(fits) == max(nq for nq in range(4000, 7000, 16) if -(-whole(nq) // 256) * 256 <= limit)
+    # a run table of 256 MiB: 48 (batch, head) pairs, 129 columns
+    nk, nl = 64000, 4
+    for nq in (320_000, 338_000):
+        rows = 48 * -(-nq // 32)
+        assert rows * (nk // 512 + nl + 1) * 4 <= 1 << 28 < 2 * rows * (nk // 512 + nl + 1) * 4
+        total = lib.mxd_msda_backward_workspace_bytes(1, 6, nk, 8, 32, nl, nl, nq, 5)
+        assert total > 48 * nq * 20 * 2 * 12                 # the hand-over is there: not the form with global atomics
