@@ -10,7 +10,7 @@ float32).  Prints ONE JSON line: whole-step throughput in queries/s, the HBM roo
 dominant kernel (timed live with HIP events on the launch stream), per-kernel figures, and
 the CPU oracle timed on the host cores of the same box as a reported baseline.
 Other workloads: the named shapes of drivingsdk_amd.workloads (with --dtype), and the sibling operators
-that run on the same kernels: sparse4d_dagg (deformable aggregation), gka (geometric kernel attention),
+beside it: sparse4d_dagg (deformable aggregation), gka (geometric kernel attention),
 grid_sampler2d (grid_sampler2d_v2), each at a shape of the reference's recipes or tests; `heuristics` times the
 launcher's default choices against every forced variant on shapes around the benchmark shapes.
 """
@@ -461,7 +461,7 @@ def _bench_heuristics(args):
     lib = _lib.load()
     dev = torch.device("cuda", 0)
     enc, bev = workloads._DETR_LEVELS, workloads._BEV_LEVELS
-    f32, f16 = torch.float32, torch.float16
+    f32, f16, bf16 = torch.float32, torch.float16, torch.bfloat16
     # name, dtype, bs, queries (None = keys), levels, heads, head_dim, points
     shapes = [
         ("encoder", f32, 2, None, enc, 8, 32, 4), ("encoder fp16", f16, 2, None, enc, 8, 32, 4),
@@ -475,6 +475,12 @@ def _bench_heuristics(args):
         ("decoder 300 queries", f32, 2, 300, enc, 8, 32, 4), ("decoder 900 queries bs8", f32, 8, 900, enc, 8, 32, 4),
         ("BEVFormer", f32, 6, 9675, bev, 8, 32, 8), ("BEVFormer fp16", f16, 6, 9675, bev, 8, 32, 8),
         ("BEVFormer 4 points", f32, 6, 9675, bev, 8, 32, 4),
+        # where the forward's two forms meet: few samples per unit, units a little over a chunk of 16, rows of 16 lanes
+        ("encoder 1 point", f32, 2, None, enc, 8, 32, 1), ("encoder 3 points fp16", f16, 2, None, enc, 8, 32, 3),
+        ("encoder 5 points", f32, 2, None, enc, 8, 32, 5), ("encoder 6 points fp16", f16, 2, None, enc, 8, 32, 6),
+        ("3 levels 6 points hd64 fp16", f16, 2, 5355, enc[:3], 8, 64, 6), ("BEVFormer hd64 6 points", f32, 2, 5355, bev, 8, 64, 6),
+        ("encoder head_dim 128 bf16", bf16, 1, None, enc, 8, 128, 4), ("BEVFormer hd128 bf16", bf16, 3, 6321, bev, 8, 128, 4),
+        ("16 heads 2 points", f32, 4, 14000, enc, 16, 32, 2), ("4 heads 8 points fp16", f16, 2, 9000, enc, 4, 32, 8),
     ]
     fwd_variants = [{}, {"MXD_MSDA_FWD_CU": 0}, {"MXD_MSDA_FWD_CU": 1}, {"MXD_MSDA_FWD_CU": 0, "MXD_MSDA_FWD_LDS": 0},
                     {"MXD_MSDA_FWD_CU": 0, "MXD_MSDA_FWD_LDS": 40960}, {"MXD_MSDA_FWD_CU_FLIP": 0}, {"MXD_MSDA_FWD_CU_FLIP": 1}]

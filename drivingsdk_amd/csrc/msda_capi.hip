@@ -576,7 +576,7 @@ int64_t estimated_cached_rows(const Dims& d, int64_t cap_rows)
 // samples, the general kernel's through as many as there are; rows from memory cost more where the slices that run side by side on
 // an XCD overflow its L2 (`spill`: by how many L2s, beyond 1.4 of them), because four wavefronts per SIMD hide less of it; every
 // workgroup pays its launch and cache fill (`start`, in rows of its share) before its share of the rows.  Conversions weigh more
-// here, most with 16 lanes per row (bfloat16, which has no mixed multiply-add, never pays there).  The fused form's general kernel computes
+// here, most with 16 lanes per row (and in bfloat16, which has no mixed multiply-add).  The fused form's general kernel computes
 // its softmax in a pass of its own over the samples.
 // Weights fitted to 3 339 pairs of timings: one to six levels of 20 x 20 to 300 x 400 pixels, 1 to 8 points, 4, 8 and 16 heads of 16
 // to 128 channels, 500 to 60 000 queries or every pixel, from a million samples on, all three types, plain and fused, uniformly
@@ -586,7 +586,7 @@ int64_t estimated_cached_rows(const Dims& d, int64_t cap_rows)
 double cu_over_general(int dtype, bool fused, int lpr, int64_t samples, double from_memory, double spill, double start)
 {
     double row = 0.46;
-    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.52 : lpr <= 8 ? 0.62 : dtype == MXD_DTYPE_F16 ? 0.7 : 1.1;
+    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.52 : lpr <= 8 ? 0.62 : dtype == MXD_DTYPE_F16 ? 0.75 : 0.85;
     if (fused) row *= 0.84;
     const double padded = (double)round_up((size_t)samples, mxd::kChunk) / (double)samples;
     return row * (1.0 + from_memory * spill) * (0.2 + 0.8 * padded) + start;
