@@ -547,9 +547,12 @@ int forward_cache_bytes(int vec, int es, const Dims& d, int units_per_wave)
     if (!forced) {
         if (units_per_wave > 8) return 0;
         // Small problems lose more to the cache fill of every workgroup than the gather gains (float32, with / without:
-        // 2 x 300 queries 11.3 / 6.1 us, 8 x 900 queries 37 / 34, the encoder's queries with 2 heads 18 / 14, five
-        // levels with 4 points and 6.4 M samples 206 / 201; with 8 points and 12.8 M samples 406 / 421).
-        if (d.bs * d.nh * d.nq * d.nl * d.np < (int64_t(1) << 23)) return 0;
+        // 2 x 300 queries 11.3 / 6.1 us, 8 x 900 queries 37 / 34; five levels with 4 points and 6.4 M samples 120 / 139).  Over 300
+        // problems whose last level fits, with / without: float32 rows of up to 256 bytes at 1 to 2 M samples 0.77 to 1.31 (median 1.00), at
+        // 2 to 4 M 0.80 to 1.13 (0.95), at 4 to 8 M 0.69 to 1.17 (0.91); 16-bit rows, whose conversions take the wavefronts that
+        // hide the memory's latency, at 2 to 4 M 0.87 to 1.39 (1.04), at 4 to 8 M 0.85 to 1.11 (1.00), beyond 0.88 to 1.11 (0.95).
+        const bool words = es == 4 && d.hd * es <= 256;
+        if (d.bs * d.nh * d.nq * d.nl * d.np < (int64_t(1) << (words ? 21 : 23))) return 0;
         double last = (double)d.nk;
         if (d.nl > 1) last = (double)d.nk * 3.0 / ((double)(int64_t(1) << (2 * (d.nl < 16 ? d.nl : 16))) - 1.0);
         if (last * 1.1 * (double)(d.hd * es) > (double)v) return 0;
@@ -573,23 +576,22 @@ int64_t estimated_cached_rows(const Dims& d, int64_t cap_rows)
 
 // Time of the forward's one-workgroup-per-CU form over that of the general kernel, estimated.  What the form gains: a row takes fewer
 // instructions, and rows of cached levels come from LDS beside the others.  What it loses: its units work through whole chunks of 16
-// samples, the general kernel's through as many as there are; rows from memory cost more where the slices that run side by side on
-// an XCD overflow its L2 (`spill`: by how many L2s, beyond 1.4 of them), because four wavefronts per SIMD hide less of it; every
-// workgroup pays its launch and cache fill (`start`, in rows of its share) before its share of the rows.  Conversions weigh more
-// here, most with 16 lanes per row (and in bfloat16, which has no mixed multiply-add).  The fused form's general kernel computes
-// its softmax in a pass of its own over the samples.
+// samples, the general kernel's through as many as there are and three samples' worth of a unit's start; rows from memory cost more
+// where the slices that run side by side on an XCD overflow its L2 (`spill`: by how many L2s, beyond 1.4 of them), because four
+// wavefronts per SIMD hide less of it; every workgroup pays its launch and cache fill (`start`, in rows of its share) before its share
+// of the rows.  Conversions weigh more here, most with 16 lanes per row (and in bfloat16, which has no mixed multiply-add).  The
+// fused form's general kernel computes its softmax in a pass of its own over the samples.
 // Weights fitted to 3 339 pairs of timings: one to six levels of 20 x 20 to 300 x 400 pixels, 1 to 8 points, 4, 8 and 16 heads of 16
 // to 128 channels, 500 to 60 000 queries or every pixel, from a million samples on, all three types, plain and fused, uniformly
-// random locations: the form chosen takes 1.6 % longer than the better of the two on average (110 of them more than 15 % longer),
-// always the general kernel 8.2 %.  On 275 problems drawn afterwards: plain 2.8 % (5.0 % with separate lines for samples, cached
-// levels, slices and types before it; always the general kernel 9.5 %), fused 2.1 % (2.4, 8.4).
+// random locations: the form chosen takes 1.6 % longer than the better of the two on average (104 of them more than 15 % longer),
+// always the general kernel 7.8 %.  On 408 problems drawn afterwards: plain 1.9 % (3.9 % with separate lines for samples, cached
+// levels, slices and types before it; always the general kernel 8.3 %), fused 1.5 % (1.7, 7.5).
 double cu_over_general(int dtype, bool fused, int lpr, int64_t samples, double from_memory, double spill, double start)
 {
-    double row = 0.46;
-    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.52 : lpr <= 8 ? 0.62 : dtype == MXD_DTYPE_F16 ? 0.75 : 0.85;
-    if (fused) row *= 0.84;
-    const double padded = (double)round_up((size_t)samples, mxd::kChunk) / (double)samples;
-    return row * (1.0 + from_memory * spill) * (0.2 + 0.8 * padded) + start;
+    double row = 0.64;
+    if (dtype != MXD_DTYPE_F32) row = lpr <= 4 ? 0.64 : lpr <= 8 ? 0.72 : dtype == MXD_DTYPE_F16 ? 0.82 : 0.9;
+    if (fused) row *= 0.8;
+    return row * (1.0 + 1.5 * from_memory * spill) * (double)round_up((size_t)samples, mxd::kChunk) / (double)(samples + 3) + start;
 }
 
 // The forward's one-workgroup-per-CU form (msda_fwd_cu.hip): whether a problem takes it, and its launch geometry.
@@ -671,7 +673,7 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
         }
     }
     if (best_cost < 0.0) return false;  // (not a shape for this form)
-    if (mode < 0 && cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, best_spill, (launch + 2500.0 + (double)cached) / best_rows) >= 1.0)
+    if (mode < 0 && cu_over_general(dtype, fused, lpr, d.nl * d.np, from_memory, best_spill, (launch + 3000.0 + (double)cached) / best_rows) >= 1.0)
         return false;
     const int64_t tq = U * (((d.nq + best_p - 1) / best_p + U - 1) / U);
     const int64_t nt = (d.nq + tq - 1) / tq;
