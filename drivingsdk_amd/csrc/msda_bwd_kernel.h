@@ -34,28 +34,21 @@
 #pragma once
 #include <type_traits>
 
-#include "msda_device.h"
+#include "msda_bwd_pass.h"
 
 namespace mxd {
 
 // RECBUF: workgroups that make several passes collect their slab of records in LDS (see `recbuf` below); an
 // instantiation of its own, for the plain operator and its fused form, because the extra paths cost the others scalar
 // registers (spilled ones travel through vector lanes) that they have no use for.
-// FIXED != 0: the launch geometry of the common cases as compile-time constants -- rows read by 8 lanes (8 units per
-// wavefront), one iteration of one chunk, the plain operator's tile form, with a unit per query (1: up to 16 samples per
-// query) or two (2: up to 32): the paths for anything else and the scalar registers that steer them fall away (57
-// vector registers instead of 96 and no spilled scalar ones; encoder shape 281.7 -> 276.3 us, float16 294.0 -> 286.7).
-// FIXED == 3: rows of 256 bytes read by 16 lanes (4 units per wavefront), a unit per query, any number of iterations
-// and chunks (heads of 128 channels in the 16-bit types: backward 380.2 -> 366.1 us in float16, 382.9 -> 369.7 in bfloat16).
-template <typename T, int VEC, int NPASS, bool SCATTER, int SRC, bool RECBUF = false, int FIXED = 0>
+// WIDE: rows of 256 bytes read by 16 lanes (4 units per wavefront), a unit per query, any number of iterations and chunks, as
+// compile-time constants: the paths for anything else and the scalar registers that steer them fall away (heads of 128 channels in
+// the 16-bit types: backward 380.2 -> 366.1 us in float16, 382.9 -> 369.7 in bfloat16).  Rows read by 8 lanes whose workgroups
+// make one pass have a kernel of their own (msda_bwd_pass.h).
+template <typename T, int VEC, int NPASS, bool SCATTER, int SRC, bool RECBUF = false, bool WIDE = false>
 __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
 {
-    static_assert(!FIXED || (!SCATTER && (SRC == kSrcPlain || (SRC == kSrcFused && FIXED == 1))),
-                  "the fixed geometry is built for the tile form of the plain operator (and, one unit per query in one pass, of its fused form)");
-    // 1, 2: 8 lanes per row, one pass of one chunk, one / two units per query; 3: 16 lanes per row (4 units per wavefront), a
-    // unit per query, any number of iterations and chunks (rows of 256 bytes: heads of 128 channels in the 16-bit types)
-    constexpr bool kOnePass = FIXED == 1 || FIXED == 2;
-    static_assert(!(kOnePass && RECBUF), "a workgroup that makes one pass collects its records in its staging strips");
+    static_assert(!WIDE || (!SCATTER && SRC == kSrcPlain), "the fixed geometry is built for the tile form of the plain operator");
     static_assert(!RECBUF || (!SCATTER && (SRC == kSrcPlain || SRC == kSrcFused)), "the record buffer is built for the tile form of the operator and its fused form");
     constexpr int GSHIFT = sizeof(T) == 4 ? 0 : 1;  // value byte offset -> fp32 image byte offset
     constexpr bool FUSED = SRC == kSrcFused;
@@ -75,34 +68,12 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             lvl[threadIdx.x] = lv.geo;
             tile_first[threadIdx.x] = lv.first;
         }
-        if (a.fill_n4 != 0 && a.sparse != 0 && lv.canonical) {
-            // only the rows that receive atomic additions in the tile pass (tiles split by query range, small tiles,
-            // and the first pixel of every other tile); a row of the image is nh*hd floats, a multiple of 16 bytes here
-            const int32_t tiles = a.tbl_stride - 1;  // (bound: pieces of tiles that do not exist are skipped)
-            const int64_t pieces = (int64_t)a.bs * tiles * kRowParts;
-            const uint32_t row4 = (uint32_t)(a.nh * a.hd) / 4;
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            for (int64_t w = blockIdx.x; w < pieces; w += gridDim.x) {
-                const int32_t b = (int32_t)(w / (tiles * kRowParts)), r = (int32_t)(w % (tiles * kRowParts));
-                int32_t r0, r1;
-                if (!lv.atomic_rows_of_part(a, r / kRowParts, r % kRowParts, &r0, &r1)) continue;
-                f32x4* img = reinterpret_cast<f32x4*>(a.grad_value) + ((size_t)b * a.nk + r0) * row4;
-                const uint32_t n4 = (uint32_t)(r1 - r0) * row4;
-                for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x) __builtin_nontemporal_store(z, img + i);
-            }
-        } else if (a.fill_n4 != 0) {
-            f32x4* img = reinterpret_cast<f32x4*>(a.grad_value);
-            const uint64_t per = (a.fill_n4 + gridDim.x - 1) / gridDim.x;
-            const uint64_t lo = (uint64_t)blockIdx.x * per;
-            const uint64_t hi = lo + per < a.fill_n4 ? lo + per : a.fill_n4;
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) __builtin_nontemporal_store(z, img + i);
-        }
+        zero_fill(a, lv);
     }
     // (fixed geometry: the arithmetic phases of a wavefront -- geometry and counting, gradients and records -- run at a
     //  raised priority, the gather at the default one: BEVFormer shape 988.6 -> 964.8 us, encoder shape unchanged; the
     //  other way round the encoder shape loses 7 us)
-    if constexpr (FIXED != 0) __builtin_amdgcn_s_setprio(2);
+    if constexpr (WIDE) __builtin_amdgcn_s_setprio(2);
     Work wk;
     if (!decode_block(a.plan, blockIdx.x, a.bs, a.nh, a.nq, &wk)) return;
 
@@ -114,13 +85,13 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
 
-    const int LPR = FIXED == 3 ? 16 : FIXED ? 8 : a.plan.lanes_per_row;
-    const int lpr_log2 = FIXED == 3 ? 4 : FIXED ? 3 : __builtin_ctz(LPR);
-    const int U = FIXED == 3 ? 4 : FIXED ? 8 : a.plan.units_per_wave;
-    const int iters = kOnePass ? 1 : a.plan.iters;
+    const int LPR = WIDE ? 16 : a.plan.lanes_per_row;
+    const int lpr_log2 = WIDE ? 4 : __builtin_ctz(LPR);
+    const int U = WIDE ? 4 : a.plan.units_per_wave;
+    const int iters = a.plan.iters;
     // 2^sp neighbouring units share a query, each taking kChunk of its samples: a pass of a wavefront covers `span`
     // samples of U >> sp queries (sp = 0: a unit is a query and goes through its samples kChunk at a time)
-    const int sp = FIXED == 3 ? 0 : FIXED ? FIXED - 1 : a.unit_split_log2, sp_mask = (1 << sp) - 1, span = kChunk << sp;
+    const int sp = WIDE ? 0 : a.unit_split_log2, sp_mask = (1 << sp) - 1, span = kChunk << sp;
     const int g = lane >> lpr_log2;
     const int c = lane & (LPR - 1);
     // lanes per row in the scatter phase: the power of two covering head_dim, within [LPR, 64]
@@ -345,7 +316,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
         // the workgroup goes through every trip (the lane exchanges need their partners).
         const int S4 = (a.S + 3) & ~3;
         const int n = (wk.q_end - wk.q_begin) * S4;
-        const bool all_early = kOnePass || (early_units >= wk.q_end - wk.q_begin && a.S <= span);  // nothing left to count
+        const bool all_early = early_units >= wk.q_end - wk.q_begin && a.S <= span;  // nothing left to count
         for (int base = 0; base < n && !all_early; base += blockDim.x) {
             const int i = base + (int)threadIdx.x;
             const int qr = i / S4, s = i - qr * S4;
@@ -411,8 +382,8 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     // wavefront has gathered, the staged entries are free, and a unit's 32 records (two per sample) fit the 16 entries
     // before its pad entry (which the fused form still needs).  Record `pos` of the slab lives at record pos % 32 of
     // unit pos / 32 of the workgroup.
-    const bool rec_in_lds = kOnePass || ((SRC == kSrcPlain || SRC == kSrcFused) && !SCATTER && iters == 1 && a.S <= span);
-    const int u_log2 = FIXED == 3 ? 2 : FIXED ? 3 : __builtin_ctz(U);
+    const bool rec_in_lds = (SRC == kSrcPlain || SRC == kSrcFused) && !SCATTER && iters == 1 && a.S <= span;
+    const int u_log2 = WIDE ? 2 : __builtin_ctz(U);
     auto rec_lds = [&](int pos) {
         const int unit = pos >> 5;  // of the workgroup: wavefront unit >> u_log2, its unit & (U - 1)
         return reinterpret_cast<u32x4*>(smem + kMaxLevels * sizeof(i32x4) +
@@ -455,7 +426,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
 
         if (!(kEarly && FUSED && it == 0)) unit_prologue(q0);  // (the fused form's first iteration: done before the count)
 
-        for (int c0 = 0; c0 < (kOnePass ? 1 : a.S); c0 += span) {
+        for (int c0 = 0; c0 < a.S; c0 += span) {
             // ---- geometry (the first chunk of the first iteration was staged while records were counted) ----
             if (!(kEarly && it == 0 && c0 == 0)) geometry(q0, c0, std::false_type{});
             wave_lds_sync();
@@ -499,7 +470,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 // (where it measured faster: the fixed geometry, and geometric kernel attention -- step 0.807 -> 0.786 ms;
                 //  the fused form, 0.440 -> 0.459 ms for forward + backward, and the grid sampler, 0.192 -> 0.200 ms, lose
                 //  more to the registers than they gain)
-                constexpr bool kAhead = (FIXED != 0 || SRC == kSrcGka) && NPASS <= 2;
+                constexpr bool kAhead = (WIDE || SRC == kSrcGka) && NPASS <= 2;
                 if constexpr (kAhead) {
                     // the rows of the next sample (of the row's second half, with two passes) are requested before the
                     // rows at hand are used: a wavefront otherwise goes through the samples of its chunk one trip to
@@ -541,7 +512,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                     }
                 }
             };
-            if constexpr (FIXED != 0) __builtin_amdgcn_s_setprio(0);
+            if constexpr (WIDE) __builtin_amdgcn_s_setprio(0);
             switch (lpr_log2) {
                 case 2: gather_dots(std::integral_constant<int, 2>{}); break;
                 case 3: gather_dots(std::integral_constant<int, 3>{}); break;
@@ -549,7 +520,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 case 5: gather_dots(std::integral_constant<int, 5>{}); break;
                 default: gather_dots(std::integral_constant<int, 6>{}); break;
             }
-            if constexpr (FIXED != 0) __builtin_amdgcn_s_setprio(2);
+            if constexpr (WIDE) __builtin_amdgcn_s_setprio(2);
             wave_lds_sync();
             if (rec_in_lds) __syncthreads();  // every wavefront's staged entries have been used: the strips take records
             // ---- scatter: grad_value[row_c] += (w_c*attn) * grad_out row --------------------
@@ -639,12 +610,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                     if constexpr (FUSED) rp = ref + (((int64_t)wk.b * a.nq + q) * a.nl + l) * a.ref_dim;
                     const f32x4 dd = dots[u * kChunk + sl];
                     float ga = 0.f, gx = 0.f, gy = 0.f;
-                    if (sm.valid) {
-                        const float hw = 1.0f - sm.lw, hh = 1.0f - sm.lh;
-                        ga = sm.w[0] * dd[0] + sm.w[1] * dd[1] + sm.w[2] * dd[2] + sm.w[3] * dd[3];
-                        gx = sm.Wf * aw * (hh * (dd[1] - dd[0]) + sm.lh * (dd[3] - dd[2]));
-                        gy = sm.Hf * aw * (hw * (dd[2] - dd[0]) + sm.lw * (dd[3] - dd[1]));
-                    }
+                    if (sm.valid) sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, aw, dd, ga, gx, gy);
                     if constexpr (FUSED) {
                         // chain rule through the softmax and through location = reference + offset * scale
                         gattn[sr.w_e] = from_f32<T>(aw * (ga - unit_stats(u)[2]));
@@ -767,6 +733,19 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     }
 }
 
+template <typename T, int VEC, int SRC, int UPQ>
+inline hipError_t launch_pass(const KArgs& a, hipStream_t stream)
+{
+    // (rows that 8 lanes would read 8 bytes each, those of 33 to 64 bytes, take 4 lanes of 16)
+    constexpr bool kFour = VEC * sizeof(T) == 8;
+    constexpr int V = kFour ? 2 * VEC : VEC, LPR = kFour ? 4 : 8;
+    // (few queries: the zero-fill of the image gets workgroups that do nothing else, as below)
+    const uint32_t fill_wgs = a.fill_n4 != 0 ? 1024u : 0u;
+    const dim3 grid(a.plan.grid > fill_wgs ? a.plan.grid : fill_wgs);
+    hipLaunchKernelGGL((msda_bwd_pass_kernel<T, V, LPR, SRC, UPQ>), grid, dim3(kPassUnits * LPR), pass_lds_bytes(a.nl, a.tbl_stride, LPR, SRC == kSrcFused), stream, a);
+    return hipGetLastError();
+}
+
 template <typename T, int VEC, int NPASS>
 inline hipError_t launch_one(const KArgs& a, bool scatter, hipStream_t stream)
 {
@@ -793,22 +772,22 @@ inline hipError_t launch_one(const KArgs& a, bool scatter, hipStream_t stream)
         else if (a.rec_lds_bytes != 0)
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcFused, true>), grid, block, a.plan.lds_bytes, stream, a);
         else if (a.bwd_fixed == 1 && NPASS == 1)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, 1, false, kSrcFused, false, 1>), grid, block, a.plan.lds_bytes, stream, a);
+            return launch_pass<T, VEC, kSrcFused, 1>(a, stream);
         else
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcFused>), grid, block, a.plan.lds_bytes, stream, a);
     } else {
         if (scatter)
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, true, kSrcPlain>), grid, block, a.plan.lds_bytes, stream, a);
         else if (a.bwd_fixed == 3 && kWide && a.rec_lds_bytes != 0)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, kWide ? NPASS : 1, false, kSrcPlain, true, 3>), grid, block, a.plan.lds_bytes, stream, a);
+            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, kWide ? NPASS : 1, false, kSrcPlain, true, true>), grid, block, a.plan.lds_bytes, stream, a);
         else if (a.bwd_fixed == 3 && kWide)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, kWide ? NPASS : 1, false, kSrcPlain, false, 3>), grid, block, a.plan.lds_bytes, stream, a);
+            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, kWide ? NPASS : 1, false, kSrcPlain, false, true>), grid, block, a.plan.lds_bytes, stream, a);
         else if (a.rec_lds_bytes != 0)
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcPlain, true>), grid, block, a.plan.lds_bytes, stream, a);
         else if (a.bwd_fixed == 1 && NPASS == 1)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, 1, false, kSrcPlain, false, 1>), grid, block, a.plan.lds_bytes, stream, a);
+            return launch_pass<T, VEC, kSrcPlain, 1>(a, stream);
         else if (a.bwd_fixed == 2 && NPASS == 1)
-            hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, 1, false, kSrcPlain, false, 2>), grid, block, a.plan.lds_bytes, stream, a);
+            return launch_pass<T, VEC, kSrcPlain, 2>(a, stream);
         else
             hipLaunchKernelGGL((msda_bwd_kernel<T, VEC, NPASS, false, kSrcPlain>), grid, block, a.plan.lds_bytes, stream, a);
     }

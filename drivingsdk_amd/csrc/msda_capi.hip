@@ -1387,7 +1387,8 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
     a.rec_lds_bytes = plan_record_buffer(&a.plan, L, d, dtype, !gka && !grid, a.unit_split_log2);
     a.bwd_fixed = (tuning().bwd_fixed != 0 && (!fused || a.unit_split_log2 == 0) && !gka && !grid && L.tiles && a.plan.lanes_per_row == 8 &&
                    a.plan.units_per_wave == 8 && a.plan.npass == 1 && a.plan.iters == 1 && a.unit_split_log2 <= 1 &&
-                   d.nl * d.np <= ((int64_t)mxd::kChunk << a.unit_split_log2) && a.rec_lds_bytes == 0)
+                   d.nl * d.np <= ((int64_t)mxd::kChunk << a.unit_split_log2) && a.rec_lds_bytes == 0 &&
+                   d.nh * d.nl_attn * d.np < (int64_t(1) << 24))  // (32-bit offsets of a wavefront's samples)
                       ? 1 + a.unit_split_log2 : 0;
     if (tuning().bwd_fixed != 0 && !fused && !gka && !grid && L.tiles && a.plan.lanes_per_row == 16 && a.plan.units_per_wave == 4 &&
         a.plan.npass == 1 && a.plan.vec * (int)elem_size(dtype) == 16 && a.unit_split_log2 == 0)

@@ -66,9 +66,9 @@ struct KArgs {
     int32_t tile_px_log2;  // log2 of the pixels per tile of the grad_value pass (9, 8 or 7: see msda_plan.h)
     int32_t rec_lds_bytes; // first backward kernel: LDS behind its counters (16-byte aligned) in which a workgroup that makes
                            // several passes collects its slab before it writes it; 0 = none (records stored one by one)
-    int32_t bwd_fixed;     // first backward kernel, plain operator's tile form: 1, 2 = the launch has the common geometry (rows read
-                           // by 8 lanes, one iteration of one chunk, this many units per query), 3 = rows of 256 bytes read by 16
-                           // lanes of 16 bytes, a unit per query: it takes the instantiation built for that geometry
+    int32_t bwd_fixed;     // first backward kernel, tile form: 1, 2 = one iteration of one chunk of rows read by 8 lanes, with this many
+                           // units per query: it takes the kernel built for that (msda_bwd_pass.h); 3 = plain operator, rows of 256
+                           // bytes read by 16 lanes of 16 bytes, a unit per query: the general kernel's instantiation for them
     int32_t tile_target;   // pair records per work item of the tile pass aimed at when a hot tile is split by query range
     int32_t tile_max_chunks;  // most query chunks a tile is split into
     int32_t sparse;        // 1: only the rows of the image that receive atomic additions are zero-filled (and, for 16-bit
@@ -213,6 +213,35 @@ struct LevelLanes {
         return true;
     }
 };
+
+// A workgroup's share of the zero-fill of the float32 image of grad_value, by the first backward kernel: the stores ride along with
+// it instead of taking a launch of their own (every workgroup takes a share, also those without other work).
+__device__ inline void zero_fill(const KArgs& a, const LevelLanes& lv)
+{
+    if (a.fill_n4 != 0 && a.sparse != 0 && lv.canonical) {
+        // only the rows that receive atomic additions in the tile pass (tiles split by query range, small tiles,
+        // and the first pixel of every other tile); a row of the image is nh*hd floats, a multiple of 16 bytes here
+        const int32_t tiles = a.tbl_stride - 1;  // (bound: pieces of tiles that do not exist are skipped)
+        const int64_t pieces = (int64_t)a.bs * tiles * kRowParts;
+        const uint32_t row4 = (uint32_t)(a.nh * a.hd) / 4;
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        for (int64_t w = blockIdx.x; w < pieces; w += gridDim.x) {
+            const int32_t b = (int32_t)(w / (tiles * kRowParts)), r = (int32_t)(w % (tiles * kRowParts));
+            int32_t r0, r1;
+            if (!lv.atomic_rows_of_part(a, r / kRowParts, r % kRowParts, &r0, &r1)) continue;
+            f32x4* img = reinterpret_cast<f32x4*>(a.grad_value) + ((size_t)b * a.nk + r0) * row4;
+            const uint32_t n4 = (uint32_t)(r1 - r0) * row4;
+            for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x) __builtin_nontemporal_store(z, img + i);
+        }
+    } else if (a.fill_n4 != 0) {
+        f32x4* img = reinterpret_cast<f32x4*>(a.grad_value);
+        const uint64_t per = (a.fill_n4 + gridDim.x - 1) / gridDim.x;
+        const uint64_t lo = (uint64_t)blockIdx.x * per;
+        const uint64_t hi = lo + per < a.fill_n4 ? lo + per : a.fill_n4;
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) __builtin_nontemporal_store(z, img + i);
+    }
+}
 
 // Where a kernel takes the location and the weight of sample s of unit (b, q, h) from.
 enum : int { kSrcPlain = 0, kSrcFused = 1, kSrcGka = 2, kSrcGrid = 3 };
@@ -456,6 +485,19 @@ __device__ inline void bilinear_weights(float lw, float lh, float (&w)[4])
     w[3] = lh * lw;
 }
 
+// Gradients of a sample's weight and location from the dots of its four rows with the grad_out row.  (Every operation is named, so
+// that the kernels that form them agree to the bit, whatever the compiler would fuse.)
+__device__ inline void sample_gradients(float lw, float lh, float Wf, float Hf, float aw, const f32x4 d, float& ga, float& gx, float& gy)
+{
+#pragma clang fp contract(off)
+    float w[4];
+    bilinear_weights(lw, lh, w);
+    const float hw = 1.0f - lw, hh = 1.0f - lh;
+    ga = __builtin_fmaf(w[3], d[3], __builtin_fmaf(w[2], d[2], __builtin_fmaf(w[1], d[1], w[0] * d[0])));
+    gx = Wf * aw * __builtin_fmaf(lh, d[3] - d[2], hh * (d[1] - d[0]));
+    gy = Hf * aw * __builtin_fmaf(lw, d[3] - d[1], hw * (d[2] - d[0]));
+}
+
 // level = {H, W, level_start_index, unused}
 __device__ inline Sample sample_geometry(float x, float y, i32x4 level, int32_t nk, bool active)
 {
@@ -617,6 +659,8 @@ __device__ inline float group_sum(float v)
 // wa / wb of a surviving record carry the sums.  All four lanes of a group must make the call together; a lane
 // without a record passes have = false.  `key` is a record's pixel index (>= 0); the lanes of a group belong to
 // one query.
+// PIN: the sums are formed lane by lane (left to itself the compiler fetches all three lanes' values first: two dozen registers).
+template <bool PIN = false>
 __device__ inline void merge_pair_records_in_quad(const bool (&have)[2], const int32_t (&key)[2], float (&wa)[2],
                                                   float (&wb)[2], bool (&keep)[2])
 {
@@ -644,6 +688,7 @@ __device__ inline void merge_pair_records_in_quad(const bool (&have)[2], const i
         b1 += m11 ? ob1 : 0.0f;
         keep0 = keep0 && !(lower && m00);
         keep1 = keep1 && !m01 && !(lower && m11);  // (m01: an upper record takes it)
+        if constexpr (PIN) asm volatile("" : "+v"(a0), "+v"(b0), "+v"(a1), "+v"(b1));
     };
     look(std::integral_constant<int, 0x39>{}, 1);
     look(std::integral_constant<int, 0x4E>{}, 2);
