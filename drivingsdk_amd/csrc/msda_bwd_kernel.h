@@ -645,12 +645,8 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                                     }
                                 }
                             } else {
-                                unsafeAtomicAdd(part, gx);
-                                unsafeAtomicAdd(part + 1, gy);
-                                if (a.ref_dim == 4) {
-                                    unsafeAtomicAdd(part + 2, r2);
-                                    unsafeAtomicAdd(part + 3, r3);
-                                }
+                                // (any other number of points: summed below, from the place of the dots)
+                                dots[u * kChunk + sl] = f32x4{gx, gy, r2, r3};
                             }
                         }
                     } else if constexpr (SRC != kSrcGrid) __builtin_nontemporal_store(from_f32<T>(ga), gattn + sr.w_e);
@@ -699,6 +695,26 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 }
             }
             wave_lds_sync();
+            if constexpr (FUSED) {
+                if (a.grad_ref != nullptr && !a.np_pow2) {
+                    const int end = a.S < c0 + span ? a.S : c0 + span;
+                    for (int i = lane; i < (U >> sp) * a.nl; i += kWave) {
+                        const int u = i / a.nl, l = i - u * a.nl, q = q0 + u, l0 = l * a.np, l1 = l0 + a.np;
+                        const int s0 = l0 > c0 ? l0 : c0, s1 = l1 < end ? l1 : end;
+                        if (q >= wk.q_end || s0 >= s1) continue;
+                        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                        for (int s = s0; s < s1; ++s) sum += dots[((u << sp) + ((s - c0) >> 4)) * kChunk + ((s - c0) & (kChunk - 1))];
+                        float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + q) * (a.nl * a.ref_dim) + l * a.ref_dim;
+                        const bool whole = s0 == l0 && s1 == l1;  // (a level that lies in two chunks is added up in memory)
+                        for (int k = 0; k < a.ref_dim; ++k) {
+                            const float v = k == 0 ? sum[0] : k == 1 ? sum[1] : k == 2 ? sum[2] : sum[3];
+                            if (whole) part[k] = v;
+                            else unsafeAtomicAdd(part + k, v);
+                        }
+                    }
+                    wave_lds_sync();
+                }
+            }
             if (rec_in_lds) {  // every wavefront's records are in the strips: the slab is written in whole lines
                 __syncthreads();
                 copy_records_out();

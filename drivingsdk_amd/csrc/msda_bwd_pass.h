@@ -417,12 +417,8 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
                         }
                     }
                 } else {
-                    unsafeAtomicAdd(part, gx);
-                    unsafeAtomicAdd(part + 1, gy);
-                    if (a.ref_dim == 4) {
-                        unsafeAtomicAdd(part + 2, r2);
-                        unsafeAtomicAdd(part + 3, r3);
-                    }
+                    // (any other number of points: summed below, from the place of the dots)
+                    strip[p.u * kChunkStride + p.sn] = __builtin_bit_cast(u32x4, f32x4{gx, gy, r2, r3});
                 }
             }
         } else {
@@ -430,6 +426,25 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
             __builtin_nontemporal_store(from_f32<T>(ga), la + p.e);
             __builtin_nontemporal_store(from_f32<T>(gx), ll + 2 * p.e);
             __builtin_nontemporal_store(from_f32<T>(gy), ll + 2 * p.e + 1);
+        }
+    }
+
+    if constexpr (FUSED) {
+        if (a.grad_ref != nullptr && !a.np_pow2) {
+            wave_lds_sync();
+            for (int i = lane; i < U * a.nl; i += kWave) {
+                const int u = i / a.nl, l = i - u * a.nl, q = q0 + u;
+                if (q >= wk.q_end) continue;
+                f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < a.np; ++t) sum += __builtin_bit_cast(f32x4, strip[u * kChunkStride + l * a.np + t]);
+                float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + q) * (a.nl * a.ref_dim) + l * a.ref_dim;
+                part[0] = sum[0];
+                part[1] = sum[1];
+                if (a.ref_dim == 4) {
+                    part[2] = sum[2];
+                    part[3] = sum[3];
+                }
+            }
         }
     }
 

@@ -1442,7 +1442,8 @@ static int backward_common(int kind, const void* value, const int32_t* spatial_s
         if (fill_inside) a.fill_n4 = n / 4;
         else e = mxd::launch_fill_zero(image, n, stream);
     }
-    if (e == hipSuccess && part && !a.np_pow2) e = mxd::launch_fill_zero(part, part_bytes / sizeof(float), stream);
+    // (a level whose points lie in two chunks is added up in memory: not where a query is one chunk)
+    if (e == hipSuccess && part && !a.np_pow2 && nl * np > mxd::kChunk) e = mxd::launch_fill_zero(part, part_bytes / sizeof(float), stream);
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "%s: zero-fill launch failed: %s", who, hipGetErrorString(e));
     e = mxd::launch_backward(dtype, a, atomic_mode, stream);
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));

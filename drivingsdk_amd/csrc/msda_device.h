@@ -47,8 +47,8 @@ struct KArgs {
     // dot product of its row with the grad_out row); grad_loc / grad_attn receive the gradients of the offsets
     // and of the logits; the reference points' gradient is summed over points here and over heads afterwards
     float* grad_ref;       // [nh][bs, nq, nl, ref_dim] float32 per-head partial sums, or nullptr: not wanted
-    int32_t np_pow2;       // np is a power of two that divides 16: the point sum is taken across lanes and
-                           // stored once; otherwise added with atomics into the zero-filled partial sums
+    int32_t np_pow2;       // np is a power of two that divides 16: the point sum is taken across lanes and stored once; otherwise
+                           // from LDS, and for levels that lie in two chunks added with atomics into zero-filled sums
     // Hand-over from the first backward kernel to the grad_value pass.  Every workgroup of the
     // first kernel (tile_q queries of one (batch, head)) owns a slab of rec_cap pair records,
     // which it fills sorted by tile; row [w] of the table holds the start of every tile's run
