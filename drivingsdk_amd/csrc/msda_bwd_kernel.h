@@ -749,17 +749,28 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     }
 }
 
-template <typename T, int VEC, int SRC, int UPQ>
-inline hipError_t launch_pass(const KArgs& a, hipStream_t stream)
+template <typename T, int VEC, int LPR, int SRC, int UPQ>
+inline hipError_t launch_pass_lanes(const KArgs& a, hipStream_t stream)
 {
-    // (rows that 8 lanes would read 8 bytes each, those of 33 to 64 bytes, take 4 lanes of 16)
-    constexpr bool kFour = VEC * sizeof(T) == 8;
-    constexpr int V = kFour ? 2 * VEC : VEC, LPR = kFour ? 4 : 8;
     // (few queries: the zero-fill of the image gets workgroups that do nothing else, as below)
     const uint32_t fill_wgs = a.fill_n4 != 0 ? 1024u : 0u;
     const dim3 grid(a.plan.grid > fill_wgs ? a.plan.grid : fill_wgs);
-    hipLaunchKernelGGL((msda_bwd_pass_kernel<T, V, LPR, SRC, UPQ>), grid, dim3(kPassUnits * LPR), pass_lds_bytes(a.nl, a.tbl_stride, LPR, SRC == kSrcFused), stream, a);
+    hipLaunchKernelGGL((msda_bwd_pass_kernel<T, VEC, LPR, SRC, UPQ>), grid, dim3(kPassUnits * LPR),
+                       pass_lds_bytes(a.nl, a.tbl_stride, LPR, SRC == kSrcFused), stream, a);
     return hipGetLastError();
+}
+
+template <typename T, int VEC, int SRC, int UPQ>
+inline hipError_t launch_pass(const KArgs& a, hipStream_t stream)
+{
+    // Rows of 33 to 64 bytes: 4 lanes of 16 bytes where there are more workgroups than 8 lanes of 8 have side by side (7 per CU).  Below,
+    // what counts is how long one takes, and four samples per lane take longer than two (backward, 8 heads, 32 channels, 4937 keys
+    // of three levels x 4 points, float16, 4 lanes / 8: 300 queries 36.0 / 32.9 us, 3000 43.7 / 41.9, 6000 (1504 workgroups) 67.2 /
+    // 65.1, 8000 (2000) 74.6 / 77.7; fused 42.5 / 37.3, 51.2 / 47.1, 77.9 / 72.8, 84.9 / 86.4; float32 with 16 channels alike).
+    if constexpr (VEC * sizeof(T) == 8) {
+        if (a.plan.grid > 7u * 256u) return launch_pass_lanes<T, 2 * VEC, 4, SRC, UPQ>(a, stream);
+    }
+    return launch_pass_lanes<T, VEC, 8, SRC, UPQ>(a, stream);
 }
 
 template <typename T, int VEC, int NPASS>

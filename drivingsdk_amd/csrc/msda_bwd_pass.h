@@ -9,7 +9,7 @@
 //     to memory;
 //   * run starts are a scan that every wavefront makes for itself (up to 64 tiles): three barriers per slab;
 //   * the dots replace the row offsets that they were gathered by, in place;
-//   * rows of 33 to 64 bytes are read by 4 lanes of 16 bytes: a row of 64 bytes costs the L1 a line of 128 however it is read, but half
+//   * rows of 33 to 64 bytes are read by 4 lanes of 16 bytes (where there are enough of them: launch_pass): a row of 64 bytes costs the L1 a line of 128 however it is read, but half
 //     of the instructions of 8 lanes of 8 bytes (181 -> 117 million at the second shape below).
 // Measured, this kernel against the instantiations of the general one that it replaces (two batch elements of the encoder in float32 /
 // the same in bfloat16, fused / 6 x 9675 queries of 32 samples over 30 825 keys in float16): 142 -> 132, 185 -> 132, 399 -> 379 us.
