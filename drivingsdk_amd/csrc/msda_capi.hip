@@ -216,10 +216,30 @@ int check_dims(int dtype, const Dims& d)
 }
 
 // Fills the XCD mapping fields of a plan for `ntiles` work items per (batch, head); returns the grid.
-int64_t fill_xcd_map(mxd_msda_plan* p, int64_t bs, int64_t nh, int64_t ntiles)
+//
+// row_bytes: length of the rows that are gathered (0: of no matter).  Rows of up to 64 bytes of neighbouring heads share the lines of
+// 128 bytes that move between memory, L2 and L1: pinned to an XCD each, such heads fetch every line twice and fill twice the L2 for the
+// same rows.  Heads that share a line then share an XCD, and where that leaves XCDs without a head of their own, several XCDs share
+// the heads' (batch element, tile) pairs, each taking a contiguous part of them (mode 3).  A head per XCD / this: 6 x 9675 queries of 32
+// samples over 30 825 keys in float16, forward 231 / 203 us, first backward kernel 379 / 356; two batch elements of the encoder in
+// bfloat16, fused forward 79.6 / 74.6 (one round of workgroups: the slices of two heads side by side fill no more of an L2 than one
+// did); 43 problems of 16 to 32 channels, one to five levels, 300 to 20 000 queries: forward 0.71 to 1.03 of the time, 0.90 on average,
+// backward 0.94 to 1.03, 0.98.  The tile pass gains nothing by it (408 / 409 us at the first of these) and keeps a head per XCD.
+int64_t fill_xcd_map(mxd_msda_plan* p, int64_t bs, int64_t nh, int64_t ntiles, int64_t row_bytes = 0)
 {
     p->ntiles = (int32_t)ntiles;
     const int mode_override = tuning().xcd_mode;
+    int64_t share = 1;  // heads that share a line
+    while (row_bytes > 0 && 2 * share * row_bytes <= 128 && nh % (2 * share) == 0) share *= 2;
+    const int64_t groups = nh / share;
+    if (mode_override != 0 && share > 1 && groups < mxd::kNumXcd && mxd::kNumXcd % groups == 0) {
+        p->xcd_mode = 3;
+        p->heads_per_xcd = (int32_t)share;
+        p->xcds_per_head = (int32_t)(mxd::kNumXcd / groups);
+        const int64_t each = (bs * ntiles * share + p->xcds_per_head - 1) / p->xcds_per_head;
+        p->tiles_per_part = (int32_t)each;  // (the callers refuse grids beyond 2^31)
+        return (int64_t)mxd::kNumXcd * each;
+    }
     if (mode_override != 0 && nh % mxd::kNumXcd == 0) {
         p->xcd_mode = 1;
         p->heads_per_xcd = (int32_t)(nh / mxd::kNumXcd);
@@ -643,10 +663,11 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
         const int64_t nt = (d.nq + tq - 1) / tq;
         mxd_msda_plan trial;
         memset(&trial, 0, sizeof(trial));
-        const int64_t grid = fill_xcd_map(&trial, d.bs, d.nh, nt);
+        const int64_t grid = fill_xcd_map(&trial, d.bs, d.nh, nt, d.hd * es);
         const double per_xcd = (double)grid / mxd::kNumXcd;
         const double rounds = ceil(per_xcd / 32.0);
         double slices = 32.0 / (double)(trial.xcd_mode == 2 ? trial.tiles_per_part : nt);  // side by side on an XCD
+        if (trial.xcd_mode == 3) slices /= (double)trial.heads_per_xcd;  // (heads that share their lines fill the L2 as one)
         if (trial.xcd_mode == 1 && slices < (double)trial.heads_per_xcd) slices = (double)trial.heads_per_xcd;
         if (trial.xcd_mode == 0) slices = slices * 8.0 < (double)d.nh ? (double)d.nh : slices * 8.0;
         if (slices < 1.0) slices = 1.0;
@@ -658,7 +679,8 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
         // this form against the general kernel: 2 x 8: 91 / 102 us, 1 x 16: 96 / 123, 4 x 4: 102 / 102, 8 x 2: 120 / 105
         // (152 with one round of workgroups), 16 x 1: 133 / 112 (175), 2 x 6 heads, no pinning: 106 / 94.
         // (four heads, each shared by two XCDs: with the encoder's queries and two batch elements 44.8 against 50.2 us)
-        if (mode < 0 && !((trial.xcd_mode == 1 && trial.heads_per_xcd <= 2) || (trial.xcd_mode == 2 && trial.xcds_per_head <= 2)))
+        if (mode < 0 && !((trial.xcd_mode == 1 && trial.heads_per_xcd <= 2) || (trial.xcd_mode == 2 && trial.xcds_per_head <= 2) ||
+                           (trial.xcd_mode == 3 && trial.xcds_per_head <= 2 * trial.heads_per_xcd)))
             continue;
         double over = ceil(slices) * slice_bytes / (4.0 * 1024 * 1024) - 0.4;
         const double spill = over < 1.0 ? 0.0 : (over > 3.0 ? 2.0 : over - 1.0);
@@ -685,7 +707,7 @@ bool plan_forward_cu(int dtype, const Dims& d, bool fused, int vec, int lpr, int
     p->waves_per_block = mxd::kCuWaves;
     p->iters = (int32_t)((tq / U + mxd::kCuWaves - 1) / mxd::kCuWaves);
     p->tile_q = (int32_t)tq;
-    const int64_t grid = fill_xcd_map(p, d.bs, d.nh, nt);
+    const int64_t grid = fill_xcd_map(p, d.bs, d.nh, nt, d.hd * es);
     if (grid >= (int64_t(1) << 31)) return false;
     p->grid = (uint32_t)grid;
     p->block = (uint32_t)(mxd::kCuWaves * mxd::kWave);
@@ -776,7 +798,7 @@ int make_plan(int backward, int dtype, const Dims& d, int align_bytes, mxd_msda_
     p->tile_q = p->units_per_wave * p->waves_per_block * p->iters / split;
     const int64_t ntiles = (d.nq + p->tile_q - 1) / p->tile_q;
     p->ntiles = (int32_t)ntiles;
-    const int64_t grid = fill_xcd_map(p, d.bs, d.nh, ntiles);
+    const int64_t grid = fill_xcd_map(p, d.bs, d.nh, ntiles, d.hd * es);
     if (grid >= (int64_t(1) << 31)) return fail(MXD_E_SHAPE, "problem needs %lld workgroups, beyond the launch limit", (long long)grid);
     p->grid = (uint32_t)grid;
     p->block = (uint32_t)(p->waves_per_block * mxd::kWave);

@@ -23,7 +23,7 @@
 
 namespace mxd {
 
-constexpr int kNumXcd = 8;
+constexpr int kNumXcd = 8;  // (decode_block takes its logarithm for granted)
 constexpr int kWave = 64;
 constexpr int kMaxLevels = 64;
 constexpr int kChunk = 16;           // samples of a unit staged per pass
@@ -74,6 +74,15 @@ MXD_HD inline bool decode_block(const mxd_msda_plan& p, uint32_t bid, int32_t bs
         const int32_t part = x / nh;
         t = part + p.xcds_per_head * (j % p.tiles_per_part);
         b = j / p.tiles_per_part;
+    } else if (p.xcd_mode == 3) {
+        // (powers of two all, but the tiles)
+        const int32_t x = bid % kNumXcd, j = bid / kNumXcd;
+        const int32_t share = __builtin_ctz((uint32_t)p.heads_per_xcd), groups = 3 - __builtin_ctz((uint32_t)p.xcds_per_head);
+        if (j >= p.tiles_per_part) return false;
+        const int32_t r = (x >> groups) * p.tiles_per_part + j;
+        h = ((x & ((1 << groups) - 1)) << share) + (r & ((1 << share) - 1));
+        b = (r >> share) / p.ntiles;
+        t = (r >> share) - b * p.ntiles;
     } else {
         h = bid % nh;
         const int32_t r = bid / nh;

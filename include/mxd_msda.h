@@ -85,10 +85,12 @@ typedef struct mxd_msda_plan {
                                 backward gives a query of 17 to 32 samples two units, 16 samples each) */
     int32_t ntiles;          /* query tiles per (batch, head)                           */
     int32_t xcd_mode;        /* 0 plain; 1 nh % 8 == 0 (heads pinned to an XCD);
-                                2 8 % nh == 0 (several XCDs share a head)               */
-    int32_t heads_per_xcd;   /* mode 1                                                  */
-    int32_t xcds_per_head;   /* mode 2                                                  */
-    int32_t tiles_per_part;  /* mode 2: tiles each of the XCDs sharing a head takes     */
+                                2 8 % nh == 0 (several XCDs share a head);
+                                3 heads that share 128-byte lines share XCDs            */
+    int32_t heads_per_xcd;   /* modes 1 and 3                                           */
+    int32_t xcds_per_head;   /* modes 2 and 3                                           */
+    int32_t tiles_per_part;  /* mode 2: tiles each of the XCDs sharing a head takes;
+                                mode 3: workgroups of each XCD                          */
     uint32_t grid;           /* workgroups                                              */
     uint32_t block;          /* threads per workgroup                                   */
     uint32_t lds_bytes;      /* dynamic LDS per workgroup                               */

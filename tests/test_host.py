@@ -86,6 +86,31 @@ def test_plan_covers_every_unit_exactly_once(backward, dims):
         assert len(seen) == bs * nh * plan.ntiles
 
 
+@pytest.mark.parametrize("backward", [0, 1])
+@pytest.mark.parametrize("dtype,hd,share", [(1, 32, 2), (2, 16, 4), (0, 16, 2), (1, 24, 2), (1, 33, 1), (0, 32, 1)])
+@pytest.mark.parametrize("bs,nh,nq", [(1, 8, 1), (1, 8, 2300), (3, 4, 130), (6, 8, 77), (5, 2, 33), (2, 16, 65), (2, 12, 65)])
+def test_heads_that_share_lines_share_xcds(backward, dtype, hd, share, bs, nh, nq):
+    """Rows of up to 64 bytes of neighbouring heads lie in one line of 128 bytes: such heads run on the same XCDs, every (batch element,
+    head, tile) once, and every XCD has as many workgroups as any other (but for the last of a part)."""
+    lib = _lib.load()
+    plan = _lib.make_plan(backward, dtype, bs, 500, nh, hd, 2, 2, nq, 4, 16)
+    while nh % share:
+        share //= 2
+    groups = nh // share
+    assert (plan.xcd_mode == 3) == (share > 1 and groups < 8 and 8 % groups == 0)
+    if plan.xcd_mode != 3:
+        return
+    seen, xcds, work = set(), {}, (ctypes.c_int32 * 4)()
+    for bid in range(plan.grid):
+        if lib.mxd_msda_decode_block(ctypes.byref(plan), bid, bs, nh, nq, ctypes.byref(work)):
+            b, h, q0, _ = work
+            assert (b, h, q0) not in seen
+            seen.add((b, h, q0))
+            xcds.setdefault(bid % 8, set()).add(h // share)
+    assert len(seen) == bs * nh * plan.ntiles and all(len(g) == 1 for g in xcds.values())
+    assert plan.grid == 8 * -(-bs * plan.ntiles * share * groups // 8)
+
+
 def test_plan_vector_width_follows_alignment_and_head_dim():
     assert _lib.make_plan(0, 0, 1, 10, 1, 32, 1, 1, 1, 1, 16).vec == 4
     assert _lib.make_plan(0, 0, 1, 10, 1, 32, 1, 1, 1, 1, 8).vec == 2
