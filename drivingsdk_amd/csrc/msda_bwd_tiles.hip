@@ -12,11 +12,10 @@
 //
 //   * The pixels of every level are cut into tiles.  A workgroup (512 threads) owns one tile of
 //     one (batch, head); every thread keeps 32 sums in registers for the whole kernel: a group
-//     of 8 lanes owns 8 consecutive pixels of up to 32 channels (tiles of 512 pixels), 4 pixels
-//     of up to 64 channels (256) or 2 pixels of up to 128 channels (128), lane j holding
-//     channels 4j..4j+3 of every 32-channel block of each -- so that the records are streamed
-//     and the lists built and walked once whatever head_dim is (heads of more than 128
-//     channels take two passes over 128-pixel tiles).
+//     of 4 to 16 lanes owns 2 to 8 consecutive pixels of up to 32 channels (tiles of 512 pixels),
+//     up to 64 (256) or up to 128 (128) -- so that the records are streamed and the lists built
+//     and walked once whatever head_dim is (heads of more than 128 channels take two passes
+//     over 128-pixel tiles).
 //   * The backward's first kernel leaves its samples as pair records {pixel, query, weight,
 //     weight of the pixel to the right}, sorted by tile inside the slab of each of its
 //     workgroups, with a table of run starts.  The owner of a tile streams the runs of its
@@ -39,6 +38,8 @@
 // Which (level, tile, query chunk) a workgroup works on is derived on the device from
 // spatial_shapes / level_start_index, which never leave device memory; the host only needs
 // an upper bound of the number of work items, which follows from nk, nq, nl and np.
+#include <type_traits>
+
 #include "msda_device.h"
 
 namespace mxd {
@@ -122,33 +123,44 @@ __device__ inline void add_levels_without_tiles(const KArgs& a, int b, int h, in
     }
 }
 
-// CHL = channels a lane accumulates per pass, 4 per 32-channel block of the row: 4, 8 or 16, for tiles of 512, 256 or
-// 128 pixels (32 sums per lane either way); heads with more than 8 * CHL channels are done in several passes over the
-// same records.  VEC = elements per load of a grad_out row.
-template <typename T, int CHL, int VEC>
+// LPG lanes (a lane group) read a grad_out row together, VEC elements per load.  A lane accumulates CHL channels per pass: PIECE =
+// max(VEC, 4) consecutive ones of every block of LPG * PIECE channels, of 32 / CHL pixels (32 sums per lane) and of the pixel behind
+// them.  That makes tiles of 512 pixels (LPG 8 and CHL 4, LPG 4 and CHL 8), 256 (8, 8) or 128 (8, 16 and 16, 8); heads with more than
+// LPG * CHL channels are done in several passes over the same records.
+// What a load costs the memory pipeline is its 64 addresses, whatever each of them brings (17 clocks per load of 4, 8 or 16 bytes a lane
+// with every row in L1, and as many when half of the lanes have no row), so 16-bit rows are read 16 bytes a lane like float32 ones
+// (two batch elements of the encoder in bfloat16 168 -> 141 us; 6 x 9675 queries of 32 samples in float16 408 -> 376; 128 channels
+// in bfloat16 182 -> 153).  The pixel behind the group's last one, whose sums the narrowest form alone kept before: 128
+// channels in bfloat16 153 -> 134 us, 37 in float32 228 -> 204 (with one list per trip instead of two, which pays for the registers),
+// whole backward of 72 to 128 channels in float32 0.86 to 1.01 of the time (16 lanes of 8 channels instead of 8 of 16; in the
+// 16-bit types 8 of 16 are up to 5 % faster).
+template <typename T, int LPG, int CHL, int VEC>
 __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const KArgs a, const TileArgs t)
 {
-    static_assert((CHL == 4 || CHL == 8 || CHL == 16) && 4 % VEC == 0, "a lane owns one 4-channel piece of every 32-channel block");
-    constexpr int CH = kLpp * CHL;                      // channels per pass
-    constexpr int NB = CHL / 4;                         // 32-channel blocks per pass
+    constexpr int PIECE = VEC < 4 ? 4 : VEC;            // consecutive channels of a lane
+    static_assert((LPG == 4 || LPG == 8 || LPG == 16) && (CHL == 4 || CHL == 8 || CHL == 16) && CHL % PIECE == 0 && PIECE % VEC == 0, "a lane owns whole pieces");
+    constexpr int CH = LPG * CHL;                       // channels per pass
+    constexpr int NB = CHL / PIECE;                     // pieces per lane and pass, CB channels apart
+    constexpr int NV = PIECE / VEC;                     // loads per piece
+    constexpr int CB = LPG * PIECE;
     constexpr int PPG = 32 / CHL;                       // pixels per lane group
-    constexpr int kTilePx = (kTileThreads / kLpp) * PPG;  // pixels per tile = pixel slots of the workgroup
-    constexpr int kTilePxLog2 = CHL == 4 ? 9 : CHL == 8 ? 8 : 7;
+    constexpr int GPW = kWave / LPG;                    // lane groups per wavefront
+    constexpr int kTilePx = (kTileThreads / LPG) * PPG;  // pixels per tile = pixel slots of the workgroup
+    constexpr int kTilePxLog2 = kTilePx == 512 ? 9 : kTilePx == 256 ? 8 : 7;
     static_assert((1 << kTilePxLog2) == kTilePx, "tile size");
-    // lists a lane group walks together, one entry of each per trip (two trips are in flight: with 16 channels per
-    // lane one list's rows take the registers that two lists' take otherwise)
-    constexpr int kWalk = CHL >= 16 ? 1 : 2;
-    // With 4 channels per lane a lane group also keeps the sums its pairs leave for the pixel behind its last one (the
-    // first pixel of the next group) and hands them over when the rounds are done: a pair is then one list entry wherever
-    // it lies in the tile, instead of two for the one pair in eight that straddles two groups.  (The wider forms have no
-    // registers to spare for it.)
-    constexpr bool kOverlap = CHL == 4;
-    constexpr int kAccPx = PPG + (kOverlap ? 1 : 0);
-    constexpr int kCarryAt = kTileEntCap - 1 - kLpp;    // entries of a wavefront's storage through which its last group hands over
+    // lists a lane group walks together, one entry of each per trip, two trips in flight (tiles of 512 pixels with one list per trip:
+    // encoder float32 165 -> 184 us, bfloat16 142 -> 148, the float16 shape above 376 -> 397; 128 channels with two 153 -> 161)
+    constexpr int kWalk = LPG * CHL >= 64 ? 1 : 2;
+    // A lane group also keeps the sums its pairs leave for the pixel behind its last one (the first pixel of the next group) and
+    // hands them over when the rounds are done: a pair is then one list entry wherever it lies in the tile, instead of two for
+    // the one pair in PPG that straddles two groups.
+    constexpr int kAccPx = PPG + 1;
+    constexpr int kCarryAt = kTileEntCap - 1 - LPG * CHL / 4;  // entries of a wavefront's storage through which its last group hands over
     constexpr int NW = kTileThreads / kWave;            // wavefronts per workgroup
     constexpr uint32_t kDummyOfWave = kTileEntCap - 1;  // last entry slot of every wavefront
-    // (a wavefront transposes the sums of half of its lane groups at a time: 4 groups x 32 sums x 8 lanes = 4 KiB)
-    constexpr int kSlotPxAt = 4 * PPG * CH / 4;         // first entry behind wavefront 0's transposition scratch
+    // (a wavefront transposes the sums of half of its lane groups at a time: 1024 sums, 4 KiB)
+    constexpr int HG = GPW / 2;
+    constexpr int kSlotPxAt = HG * PPG * CH / 4;        // first entry behind wavefront 0's transposition scratch
     static_assert(kSlotPxAt + kTileThreads * 2 / 16 <= kCarryAt, "slot map must fit wavefront 0's entry storage");
     __shared__ uint32_t heads[kTileThreads];            // list head per pixel slot (byte offset of the entry in `ent`)
     // entry: {byte offset of the grad_out row, weight for the list's pixel, weight for the
@@ -182,8 +194,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     }
     if (threadIdx.x < kTileThreads / 2) slot_info[threadIdx.x] = 0;
     // an empty list points at the dummy entry of the wavefront that owns the pixel slot (slot s belongs to lane group
-    // s / PPG, i.e. to wavefront s / (8 PPG); slots past the tile size are never used)
-    heads[threadIdx.x] = ((threadIdx.x / (kLpp * PPG)) % NW * kTileEntCap + kDummyOfWave) * 16u;
+    // s / PPG, i.e. to wavefront s / (GPW PPG); slots past the tile size are never used)
+    heads[threadIdx.x] = ((threadIdx.x / (GPW * PPG)) % NW * kTileEntCap + kDummyOfWave) * 16u;
     if (threadIdx.x == 0) {
         done_count = 0;
         spare_next = 0;
@@ -209,7 +221,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     const int copies_log2 = __builtin_ctz(copies);
     const int nused = copies * npx_pad;              // slots that stand for a pixel of the tile
     const int nspare = kTilePx - nused;              // slots free for extra lists
-    const bool can_split = nspare >= PPG;
+    const bool can_split = nspare >= tile_group_px(kTilePxLog2);
     // (owned && !can_split is what tile_stored_directly() says of this tile)
     const bool direct_t = a.sparse != 0 && a.grad_value_t != nullptr && owned && !can_split;
     typedef uint16_t __attribute__((may_alias)) u16_alias;  // halves of LDS words that are also accessed whole
@@ -248,8 +260,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     auto ent_at = [&](uint32_t off) -> u32x4& { return *reinterpret_cast<u32x4*>(reinterpret_cast<unsigned char*>(ent) + off); };
     if (lane == 0) ent_at(dummy) = u32x4{kInvalidCorner, 0u, 0u, dummy};
 
-    // lane j of group g = tid / 8 keeps channels 32k + 4j .. 32k + 4j + 3 (k < NB) of the pixels g*PPG .. g*PPG + PPG - 1
-    const int grp = tid / kLpp, j = tid % kLpp;
+    // lane j of a group keeps its channels of the pixels grp * PPG .. grp * PPG + PPG - 1
+    const int grp = tid / LPG, j = tid % LPG;
 
     // First channel of the four that a lane loads for channels ch .. ch + 3: its own -- what lies behind a float32 row's
     // end is read and never written, and the range check at the end of the buffer zeroes single dwords.  A dword holds
@@ -264,11 +276,11 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 #pragma unroll
             for (int c = 0; c < CHL; ++c) acc[i][c] = 0.0f;
         // channels past head_dim re-read channel 0; their sums are never written out
-        const int my_ch = cb + j * 4;  // (first channel of this lane in block 0; block k: + 32 k)
+        const int my_ch = cb + j * PIECE;  // (first channel of this lane in block 0; block k: + CB k)
         uint32_t lane_off[NB];
 #pragma unroll
         for (int k = 0; k < NB; ++k)
-            lane_off[k] = ghead_off + (uint32_t)(my_ch + 32 * k < hd ? first_channel(my_ch + 32 * k) : 0) * (uint32_t)sizeof(T);
+            lane_off[k] = ghead_off + (uint32_t)(my_ch + CB * k < hd ? first_channel(my_ch + CB * k) : 0) * (uint32_t)sizeof(T);
         const int nch = (hd - cb) < CH ? (hd - cb) : CH;
 
         // input state of this wavefront (uniform): next group of runs, records of the current
@@ -330,13 +342,9 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 const u32x3 rc = ahead;
                 i0 += kWave;
                 fetch_ahead(i0);
-                // A record is the pair (pixel, pixel + 1).  A pair whose pixels belong to the same
-                // lane group becomes ONE entry in the list of the left pixel (the grad_out row is
-                // fetched once for both); otherwise each pixel gets an entry of its own -- unless the
-                // groups keep sums for the pixel behind their last one (kOverlap), where every pair inside
-                // the tile is one entry (backward at the encoder shape 276.9 -> 269.9 us, float16 286.7 ->
-                // 277.6, BEVFormer shape 1024 -> 1000).  The right pixel of the last pixel of the tile
-                // belongs to the next tile: added with atomics.
+                // A record is the pair (pixel, pixel + 1) and becomes ONE entry in the list of the left pixel (the grad_out row
+                // is fetched once for both).  The right pixel of the last pixel of the tile belongs to the next tile: added
+                // with atomics.
                 int lst[2] = {-1, -1};
                 float w0[2] = {0.f, 0.f}, w1[2] = {0.f, 0.f};
                 uint32_t q = 0;
@@ -353,18 +361,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                     wb = __builtin_bit_cast(float, za);
                     const int copy_off = (int)(q & (uint32_t)(copies - 1)) * npx_pad;
                     const bool in_r = pl + 1 < npx;
-                    const bool pair = in_r && (kOverlap || (pl % PPG) != PPG - 1);
                     lst[0] = pl + copy_off;
                     w0[0] = wa;
-                    w1[0] = pair ? wb : 0.0f;
-                    if (!pair && wb != 0.0f) {
-                        if (in_r) {
-                            lst[1] = pl + 1 + copy_off;
-                            w0[1] = wb;
-                        } else {
-                            spill = true;
-                        }
-                    }
+                    w1[0] = in_r ? wb : 0.0f;
+                    spill = !in_r && wb != 0.0f;
                 }
                 if (can_split && !first_round) {
                     // entries of a pixel with extra lists are dealt to them by query; a pair entry that moves
@@ -388,6 +388,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 const bool count_slots = can_split && first_round;
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
+                    if (k == 1 && (!can_split || first_round)) break;  // (only a pair that moved to an extra list leaves a second entry)
                     const bool push = lst[k] >= 0;
                     const uint64_t mask = __ballot(push);
                     if (mask) {
@@ -443,15 +444,14 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             }
 
             // ---- every group of 8 lanes walks the lists of its PPG pixels ----------------------
-            // The lanes of a group read a 32-channel block of a grad_out row with ONE coalesced load (lane j:
-            // channels 4j..4j+3 of the block): the memory pipeline's cost is per cache line touched by an instruction.
+            // The lanes of a group read a block of a grad_out row with ONE coalesced load.
             // The loop body is branch-free: a list that has ended keeps "reading" the dummy entry.
             // kWalk lists are walked together, one entry of each per trip, and two trips are in flight.
             {
                 // (a row stays as it was loaded until it is used: what is in flight takes half the registers in the 16-bit
                 //  types, and no conversion waits for its row where the row is requested)
                 typedef typename RowIO<T, VEC>::raw_t raw_t;
-                auto fetch = [&](uint32_t& e, raw_t (&g)[NB][4 / VEC], float& wa, float& wb) {
+                auto fetch = [&](uint32_t& e, raw_t (&g)[NB][NV], float& wa, float& wb) {
                     const u32x4 en = ent_at(e);
                     // (a bit cast applied directly to a vector element picks up element 0: copy first)
                     const uint32_t ya = en.y, za = en.z;
@@ -460,8 +460,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 #pragma unroll
                     for (int k = 0; k < NB; ++k)
 #pragma unroll
-                        for (int c = 0; c < 4; c += VEC)
-                            g[k][c / VEC] = RowIO<T, VEC>::load_raw(gres, en.x + lane_off[k] + (uint32_t)(c * sizeof(T)));
+                        for (int v = 0; v < NV; ++v)
+                            g[k][v] = RowIO<T, VEC>::load_raw(gres, en.x + lane_off[k] + (uint32_t)(v * VEC * sizeof(T)));
                     e = en.w;
                 };
 #pragma unroll
@@ -477,21 +477,20 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                     // two sets of rows in flight: the entries and rows of the next trip are requested before the
                     // rows of this trip are used, so that a long list costs its entries' LDS latency per trip
                     // and not the latency of a row load (reads past a list's end land on the dummy entry)
-                    raw_t gA[kWalk][NB][4 / VEC], gB[kWalk][NB][4 / VEC];
+                    raw_t gA[kWalk][NB][NV], gB[kWalk][NB][NV];
                     float uA[kWalk], vA[kWalk], uB[kWalk], vB[kWalk];
-                    auto use = [&](raw_t (&g)[kWalk][NB][4 / VEC], float (&u)[kWalk], float (&v)[kWalk]) {
+                    auto use = [&](raw_t (&g)[kWalk][NB][NV], float (&u)[kWalk], float (&v)[kWalk]) {
 #pragma unroll
                         for (int m = 0; m < kWalk; ++m) {
 #pragma unroll
-                            for (int k = 0; k < NB * (4 / VEC); ++k) {
+                            for (int k = 0; k < NB * NV; ++k) {
                                 float row[VEC];
-                                RowIO<T, VEC>::unpack(g[m][k / (4 / VEC)][k % (4 / VEC)], row);
+                                RowIO<T, VEC>::unpack(g[m][k / NV][k % NV], row);
 #pragma unroll
                                 for (int e = 0; e < VEC; ++e) {
                                     const int c = k * VEC + e;
                                     acc[i + m][c] = __builtin_fmaf(u[m], row[e], acc[i + m][c]);
-                                    if (i + m + 1 < kAccPx)
-                                        acc[(i + m + 1) % kAccPx][c] = __builtin_fmaf(v[m], row[e], acc[(i + m + 1) % kAccPx][c]);
+                                    acc[i + m + 1][c] = __builtin_fmaf(v[m], row[e], acc[i + m + 1][c]);
                                 }
                             }
                         }
@@ -533,25 +532,32 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             if (all_done) break;
         }
 
-        if constexpr (kOverlap) {
+        {
             // what a group collected for the first pixel of the next group: inside a wavefront from lane to lane, from
             // the last group of a wavefront to the first of the next through the entry storage (free now; the last
             // group of the workgroup has nothing to hand over: a pair never starts on the last pixel of a tile)
-            const int gw = lane / kLpp;
-            if (gw == kWave / kLpp - 1)
-                ent[seg + kCarryAt + j] = u32x4{__builtin_bit_cast(uint32_t, acc[PPG][0]), __builtin_bit_cast(uint32_t, acc[PPG][1]),
-                                                __builtin_bit_cast(uint32_t, acc[PPG][2]), __builtin_bit_cast(uint32_t, acc[PPG][3])};
+            const int gw = lane / LPG;
+            if (gw == GPW - 1) {
+#pragma unroll
+                for (int k = 0; k < CHL / 4; ++k)
+                    ent[seg + kCarryAt + k * LPG + j] =
+                        u32x4{__builtin_bit_cast(uint32_t, acc[PPG][4 * k]), __builtin_bit_cast(uint32_t, acc[PPG][4 * k + 1]),
+                              __builtin_bit_cast(uint32_t, acc[PPG][4 * k + 2]), __builtin_bit_cast(uint32_t, acc[PPG][4 * k + 3])};
+            }
             __syncthreads();
             float cin[CHL];
 #pragma unroll
-            for (int c = 0; c < CHL; ++c) cin[c] = __shfl_up(acc[PPG][c], kLpp, kWave);
+            for (int c = 0; c < CHL; ++c) cin[c] = __shfl_up(acc[PPG][c], LPG, kWave);
             if (gw == 0) {
-                const u32x4 o = wave > 0 ? ent[seg - kTileEntCap + kCarryAt + j] : u32x4{0u, 0u, 0u, 0u};
-                const uint32_t o0 = o.x, o1 = o.y, o2 = o.z, o3 = o.w;
-                cin[0] = __builtin_bit_cast(float, o0);
-                cin[1] = __builtin_bit_cast(float, o1);
-                cin[2] = __builtin_bit_cast(float, o2);
-                cin[3] = __builtin_bit_cast(float, o3);
+#pragma unroll
+                for (int k = 0; k < CHL / 4; ++k) {
+                    const u32x4 o = wave > 0 ? ent[seg - kTileEntCap + kCarryAt + k * LPG + j] : u32x4{0u, 0u, 0u, 0u};
+                    const uint32_t o0 = o.x, o1 = o.y, o2 = o.z, o3 = o.w;
+                    cin[4 * k] = __builtin_bit_cast(float, o0);
+                    cin[4 * k + 1] = __builtin_bit_cast(float, o1);
+                    cin[4 * k + 2] = __builtin_bit_cast(float, o2);
+                    cin[4 * k + 3] = __builtin_bit_cast(float, o3);
+                }
             }
 #pragma unroll
             for (int c = 0; c < CHL; ++c) acc[0][c] += cin[c];
@@ -560,7 +566,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             if ((hd & 3) != 0) {  // (uniform)
 #pragma unroll
                 for (int kb = 0; kb < NB; ++kb) {
-                    const int ch = my_ch + 32 * kb;
+                    const int ch = my_ch + CB * kb;
                     const int sh = ch < hd ? ch - first_channel(ch) : 0;
 #pragma unroll
                     for (int i = 0; i < PPG; ++i) {
@@ -594,8 +600,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         if (owned && !split && t.store_vec == 4) {
             // the lanes of a group hold a whole row of each of their pixels: 16-byte stores
 #pragma unroll
-            for (int kb = 0; kb < NB; ++kb) {
-                const int ch_w = my_ch + 32 * kb;
+            for (int c4 = 0; c4 < CHL; c4 += 4) {
+                const int ch_w = my_ch + CB * (c4 / PIECE) + c4 % PIECE;
                 if (ch_w >= hd) continue;
 #pragma unroll
                 for (int i = 0; i < PPG; ++i) {
@@ -603,7 +609,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                     if (px < npx) {
                         f32x4* dst = reinterpret_cast<f32x4*>(gimg + (int64_t)(it.p0 + px) * row_pitch +
                                                               (int64_t)wk.h * hd + ch_w);
-                        f32x4 v = {acc[i][4 * kb + 0], acc[i][4 * kb + 1], acc[i][4 * kb + 2], acc[i][4 * kb + 3]};
+                        f32x4 v = {acc[i][c4], acc[i][c4 + 1], acc[i][c4 + 2], acc[i][c4 + 3]};
                         if (px == 0) {
                             // the first pixel of a tile also receives, through atomics, the right
                             // halves of pairs that start on the last pixel of the previous tile
@@ -632,27 +638,26 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             // Rows shared with other workgroups (tiles split by query range) are added with
             // atomics, which the memory side carries out per 64-byte request: pass the registers
             // through LDS (the entry storage, free after the last round) so that consecutive
-            // lanes hold consecutive floats of a row.  Four lane groups (4 PPG pixel slots, 1024 sums) at a time.
+            // lanes hold consecutive floats of a row.  Half of the wavefront's lane groups (1024 sums) at a time.
             typedef uint32_t __attribute__((may_alias)) u32_alias;
-            static_assert(4 * PPG * CH * 4 <= kTileEntCap * 16, "transposition scratch must fit the entry storage");
             u32x4* tr4 = &ent[seg];
             const u32_alias* tr1 = reinterpret_cast<const u32_alias*>(tr4);
             for (int half = 0; half < 2; ++half) {
                 wave_lds_sync();
-                if (((lane_w / kLpp) >> 2) == half) {
-                    const int gl = (lane_w / kLpp) & 3;
+                if ((lane_w / LPG) / HG == half) {
+                    const int gl = (lane_w / LPG) % HG;
 #pragma unroll
                     for (int i = 0; i < PPG; ++i)
 #pragma unroll
-                        for (int kb = 0; kb < NB; ++kb)
-                            tr4[(gl * PPG + i) * (CH / 4) + 8 * kb + j] =
-                                u32x4{__builtin_bit_cast(uint32_t, acc[i][4 * kb + 0]), __builtin_bit_cast(uint32_t, acc[i][4 * kb + 1]),
-                                      __builtin_bit_cast(uint32_t, acc[i][4 * kb + 2]), __builtin_bit_cast(uint32_t, acc[i][4 * kb + 3])};
+                        for (int c4 = 0; c4 < CHL; c4 += 4)
+                            tr4[(gl * PPG + i) * (CH / 4) + (CB * (c4 / PIECE) + c4 % PIECE + PIECE * j) / 4] =
+                                u32x4{__builtin_bit_cast(uint32_t, acc[i][c4]), __builtin_bit_cast(uint32_t, acc[i][c4 + 1]),
+                                      __builtin_bit_cast(uint32_t, acc[i][c4 + 2]), __builtin_bit_cast(uint32_t, acc[i][c4 + 3])};
                 }
                 wave_lds_sync();
-                const int px_base = wave * (kLpp * PPG) + half * (4 * PPG);
+                const int px_base = wave * (GPW * PPG) + half * (HG * PPG);
 #pragma unroll 4
-                for (int k = 0; k < 4 * PPG * CH / kWave; ++k) {
+                for (int k = 0; k < HG * PPG * CH / kWave; ++k) {
                     const int idx = k * kWave + lane_w;
                     const int pl = idx / CH, c = idx % CH;
                     const int vp = px_base + pl;             // pixel slot of the workgroup
@@ -677,7 +682,11 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             // overwritten by the transposition)
             __syncthreads();
             if (threadIdx.x == 0) done_count = 0;
-            if (lane == 0) ent_at(dummy) = u32x4{kInvalidCorner, 0u, 0u, dummy};
+            // (opaque: the entry would otherwise be kept through the whole pass, in registers that some forms do not have -- and
+            //  memory for spilled ones costs every wavefront time before it starts)
+            uint32_t none = 0u;
+            asm volatile("" : "+v"(none));
+            if (lane == 0) ent_at(dummy) = u32x4{none | kInvalidCorner, none, none, none + dummy};
             __syncthreads();
         }
     }
@@ -686,19 +695,33 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 template <typename T>
 static hipError_t launch_t(const KArgs& a, const TileArgs& t, hipStream_t stream)
 {
-    // an octet of lanes reads a 32-channel block of a grad_out row, 4 channels per lane: one load per lane, whatever the row's
-    // length and alignment (but for 16-bit rows of fewer than 4 channels)
+    // A load brings 16 bytes per lane, or 8 of 16-bit rows that pieces of 16 do not divide; one load per lane and piece whatever the
+    // row's length and alignment (but for 16-bit rows of fewer than 4 channels).
     const dim3 grid(t.grid), block(t.block);
-    if (sizeof(T) == 2 && a.hd < 4) {
-        if (a.tile_px_log2 != kTilePxLog2Max) return hipErrorInvalidConfiguration;
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, sizeof(T) == 2 ? 1 : 4>), grid, block, 0, stream, a, t);
-    } else if (a.tile_px_log2 == 8) {
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 8, 4>), grid, block, 0, stream, a, t);
-    } else if (a.tile_px_log2 == 7) {
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 16, 4>), grid, block, 0, stream, a, t);
-    } else {
-        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, 4, 4>), grid, block, 0, stream, a, t);
+    constexpr bool kHalf = sizeof(T) == 2;
+    auto launch = [&](auto lpg, auto chl, auto vec) {
+        hipLaunchKernelGGL((msda_gradv_tiles_kernel<T, decltype(lpg)::value, decltype(chl)::value, decltype(vec)::value>), grid, block, 0, stream, a, t);
+    };
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 4> four;
+    constexpr std::integral_constant<int, 8> eight;
+    constexpr std::integral_constant<int, 16> sixteen;
+    if constexpr (kHalf) {
+        if (a.hd < 4) {
+            if (a.tile_px_log2 != kTilePxLog2Max) return hipErrorInvalidConfiguration;
+            launch(eight, four, one);
+            return hipGetLastError();
+        }
+        if (a.hd % 8 == 0) {
+            if (a.tile_px_log2 == 8) launch(eight, eight, eight);
+            else if (a.tile_px_log2 == 7) launch(eight, sixteen, eight);
+            else launch(four, eight, eight);
+            return hipGetLastError();
+        }
     }
+    if (a.tile_px_log2 == 8) launch(eight, eight, four);
+    else if (a.tile_px_log2 == 7) launch(sixteen, eight, four);
+    else launch(eight, four, four);
     return hipGetLastError();
 }
 

@@ -100,11 +100,11 @@ __device__ inline i32x4 load_level(const KArgs& a, int l)
 
 // ---- tiles of the grad_value pass, as every kernel of the backward sees them ---------------------------------------
 constexpr int kRecDwords = 3;  // dwords of a pair record
-constexpr int kLpp = 8;        // lanes of a lane group of the tile pass (a group reads a row with one load per 32 channels)
 constexpr int kRowParts = 16;  // pieces a tile's rows are cut into for the zero-fill and the rounding
 
-// Pixels per lane group of the tile pass: 8 for tiles of 512 pixels, 4 for 256, 2 for 128 (64 groups per workgroup).
-__device__ inline int32_t tile_group_px(int32_t tile_px_log2) { return 1 << (tile_px_log2 - 6); }
+// Free pixel slots from which on the tile pass hands out extra lists, a multiple of the pixels of a lane group in every form for the
+// tile size: 8 for tiles of 512 pixels, 4 for 256 and 128.
+__device__ inline int32_t tile_group_px(int32_t tile_px_log2) { return tile_px_log2 == 9 ? 8 : 4; }
 
 // Query chunks the tiles of a level with `nt` tiles are split into by the tile pass (chunk c takes every chunks-th slab of
 // records: see KArgs::run_step).

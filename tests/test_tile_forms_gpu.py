@@ -1,0 +1,28 @@
+"""The grad_value pass in its forms -- 4, 8 and 16 lanes per row, loads of 8 and 16 bytes -- at the edges of their tiles: maps of a few
+pixels more and fewer than a tile and than a tile without a lane group, pairs that straddle groups and tiles, tiles held in copies
+and tiles split by query range; against the oracle."""
+import pytest
+import torch
+
+from drivingsdk_amd import workloads
+from test_msda_gpu import _check_all
+from util import BWD_FP32, FWD_FP32, half_tol
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,hd", [(torch.float16, 8), (torch.bfloat16, 32), (torch.float16, 36), (torch.float16, 40), (torch.bfloat16, 64),
+                                      (torch.float16, 72), (torch.float16, 100), (torch.bfloat16, 128), (torch.float16, 136),
+                                      (torch.float32, 32), (torch.float32, 50), (torch.float32, 70), (torch.float32, 128),
+                                      (torch.float32, 130)])
+@pytest.mark.parametrize("maps,nq", [(((1, 505), (3, 2)), 40), (((21, 24), (8, 16)), 300), (((500, 1), (127, 1)), 300), (((27, 19), (5, 25)), 60),
+                                     (((16, 16), (1, 129)), 2500)], ids=["505+6", "504+128", "500+127", "513+125", "256+129"])
+def test_edges_of_tiles(gpu_device, maps, nq, dtype, hd):
+    g = torch.Generator().manual_seed(hd + nq)
+    shapes, lsi = workloads.level_tensors(maps)
+    bs, nh, nl, npts, nk = 1, 2, len(maps), 3, int(shapes.prod(1).sum())
+    tensors = (torch.randn(bs, nk, nh, hd, generator=g), torch.rand(bs, nq, nh, nl, npts, 2, generator=g) * 1.2 - 0.1,
+               torch.rand(bs, nq, nh, nl, npts, generator=g), torch.randn(bs, nq, nh * hd, generator=g))
+    value, loc, attn, gout = (t.to(dtype) for t in tensors)
+    fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
+    _check_all(workloads.MsdaInputs(value, shapes, lsi, loc, attn, gout), gpu_device, fwd, bwd)
