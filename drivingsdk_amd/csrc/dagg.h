@@ -7,6 +7,7 @@ namespace mxd {
 constexpr int kDaggWaves = 4;        // wavefronts per workgroup of the forward: an anchor each
 constexpr int kDaggBackWaves = 8;    // the same for the backward's first kernel, whose sort is the shorter for it (442 anchors: 52 -> 44 us with 8, 43 with
                                      // 16; 6 x 900 anchors lose 5 % with 16)
+constexpr int kDaggSortWaves = 16;   // the same for the sort as a launch of its own (6 x 900 anchors: 72 us with 8)
 constexpr int kDaggList = 128;       // locations of an anchor that a wavefront looks through before it samples
 constexpr int kDaggSortPx = 4096;    // pixels of a level that a workgroup of the sort counts in LDS
 constexpr int kDaggStrip = 8;        // neighbouring pixels whose gradient rows are formed together
@@ -26,8 +27,10 @@ struct DaggArgs {
     float* image;          // float32 image of grad_feat: grad_feat itself, or in the workspace for 16-bit dtypes
     float* gw_part;        // [G][bs, A][cams, P, scales]: gradients of the weights of one group, locations inside the image only
     float* gl_part;        // [G][bs, A][cams, P][2]: one group's part of the location gradients, summed over the scales
+    f32x2* dots;           // [bs, A][P, cams, scales][upper, lower row][G]: dot products of the row's first pixel and of its right
+                           //   neighbour, in place of the two above; null: the first kernel forms those
     uint32_t* csr;         // [bs][starts]: per level, first record of every pixel, then their number
-    u32x4* rec;            // [bs][nl][2 A P] records sorted by pixel: {anchor << 3 | pixel & 7, index of the weight of group 0 / G,
+    u32x4* rec;            // [bs][nl][2 A P] records sorted by pixel: {anchor << 3 | pixel & 7, row of the sample << 31 | index of the weight of group 0 / G,
                            //   bilinear weight of the pixel, of the pixel to its right}
     int32_t bs, nf, C, G, hd, cams, scales, nl, A, P;
     int32_t nloc;          // P * cams

@@ -389,19 +389,21 @@ struct DaggLevels {
 // into starts, and drops every record at its place.
 struct DaggSort {
     DaggLevels lv;
-    uint32_t wsum[kDaggBackWaves];
+    uint32_t wsum[kDaggSortWaves];
     uint32_t before_s;
     uint32_t cnt[kDaggSortPx];
 };
-template <typename T>
+template <typename T, int WAVES>
 __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned char* smem)
 {
-    constexpr int kThreads = kDaggBackWaves * kWave;
+    constexpr int kThreads = WAVES * kWave;
     DaggSort& sh = *reinterpret_cast<DaggSort*>(smem);
     DaggLevels& lv = sh.lv;
     uint32_t *cnt = sh.cnt, *wsum = sh.wsum, &before_s = sh.before_s;
-    lv.fill(a);
     const int range = block % a.sort_ranges, l = block / a.sort_ranges % a.nl, b = block / a.sort_ranges / a.nl;
+    const i32x4 own = dagg_level(a, l);
+    if (b >= a.bs || (int64_t)own.x * own.y <= (int64_t)range * kDaggSortPx) return;  // (uniform)
+    lv.fill(a);
     const int tid = threadIdx.x;
     const int r0 = range * kDaggSortPx, P = lv.px[l], r1 = P - r0 < kDaggSortPx ? P : r0 + kDaggSortPx;
     if (b >= a.bs || r0 >= P) return;  // (uniform; the launch has a multiple of 8 sort workgroups)
@@ -420,7 +422,7 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
         for (int r = 0; r < 2; ++r) {
             const bool vl = sm.cvalid[2 * r], vr = sm.cvalid[2 * r + 1];
             if (vl || vr)
-                take((vl ? sm.pix[2 * r] : sm.pix[2 * r + 1]) - level.z, vl ? sm.w[2 * r] : sm.w[2 * r + 1], vl && vr ? sm.w[2 * r + 1] : 0.0f);
+                take(r, (vl ? sm.pix[2 * r] : sm.pix[2 * r + 1]) - level.z, vl ? sm.w[2 * r] : sm.w[2 * r + 1], vl && vr ? sm.w[2 * r + 1] : 0.0f);
         }
     };
     // eight points' locations are requested together: one at a time, the two passes are a chain of trips to memory
@@ -434,14 +436,14 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
                 xy[k] = i < points ? load_xy<T>(a.loc, ((int64_t)b * points + i) * a.cams + cam) : f32x2{0.f, 0.f};
             }
             for (int k = 0; k < kTogether; ++k) {
-                each_record(xy[0], [&](int key, float wa, float wb) { take(i0 + k * kThreads, key, wa, wb); });
+                each_record(xy[0], [&](uint32_t r, int key, float wa, float wb) { take(i0 + k * kThreads, r, key, wa, wb); });
 #pragma unroll
                 for (int m = 0; m + 1 < kTogether; ++m) xy[m] = xy[m + 1];
             }
         }
     };
     uint32_t before = 0;  // records of the ranges before this one
-    each_point([&](uint32_t, int key, float, float) {
+    each_point([&](uint32_t, uint32_t, int key, float, float) {
         if (key < r0) ++before;
         else if (key < r1) atomicAdd(&cnt[key - r0], 1u);
     });
@@ -475,10 +477,10 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
     __syncthreads();
 
     u32x4* rec = a.rec + ((size_t)b * a.nl + l) * 2 * points;
-    each_point([&](uint32_t i, int key, float wa, float wb) {
+    each_point([&](uint32_t i, uint32_t r, int key, float wa, float wb) {
         if (key < r0 || key >= r1) return;
         const uint32_t pos = atomicAdd(&cnt[key - r0], 1u);
-        rec[pos] = u32x4{(i / (uint32_t)a.P) << 3 | ((uint32_t)key & 7u), (i * (uint32_t)a.cams + (uint32_t)cam) * (uint32_t)a.scales + (uint32_t)sc,
+        rec[pos] = u32x4{(i / (uint32_t)a.P) << 3 | ((uint32_t)key & 7u), r << 31 | ((i * (uint32_t)a.cams + (uint32_t)cam) * (uint32_t)a.scales + (uint32_t)sc),
                          __builtin_bit_cast(uint32_t, wa), __builtin_bit_cast(uint32_t, wb)};
     });
 }
@@ -517,9 +519,18 @@ __global__ __launch_bounds__(kDaggBackWaves * kWave) void dagg_dots_and_sort_ker
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ i32x4 lvl[kMaxLevels];
-    if (blockIdx.x < sorts) dagg_sort<T>(a, blockIdx.x, smem);
+    if (blockIdx.x < sorts) dagg_sort<T, kDaggBackWaves>(a, blockIdx.x, smem);
     else if (blockIdx.x < sorts + kDaggZeroWgs) dagg_zero(a, blockIdx.x - sorts, smem);
     else dagg_dots<T, VEC>(a, blockIdx.x - sorts - kDaggZeroWgs, smem, lvl);
+}
+
+// The same without dot products, where the kernel behind it forms them.
+template <typename T>
+__global__ __launch_bounds__(kDaggSortWaves * kWave) void dagg_sort_kernel(const DaggArgs a, uint32_t sorts)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x < sorts) dagg_sort<T, kDaggSortWaves>(a, blockIdx.x, smem);
+    else dagg_zero(a, blockIdx.x - sorts, smem);
 }
 
 // ---- gradient of the feature maps --------------------------------------------------------------------------------------------
@@ -542,6 +553,17 @@ __device__ inline void dagg_levels_without_room(const DaggArgs& a, const DaggLev
             const Sample sm = sample_geometry(xy.x, xy.y, i32x4{lv.H[l], lv.W[l], lv.base[l], 0}, a.nf, true);
             const T* w = static_cast<const T*>(a.w) + (li * a.scales + (l - cam * a.scales)) * a.G;
             float* image = a.image + b * a.nf * a.C;
+            if (a.dots != nullptr)
+                for (int g = 0; g < a.G; ++g) {
+                    float d[4] = {0.f, 0.f, 0.f, 0.f};
+                    for (int ch = g * a.hd + (int)lane; ch < (g + 1) * a.hd; ch += kWave)
+                        for (int k = 0; k < 4; ++k)
+                            if (sm.cvalid[k]) d[k] += to_f32(static_cast<const T*>(a.feat)[(b * a.nf + sm.pix[k]) * a.C + ch]) * to_f32(gout[anchor * a.C + ch]);
+                    for (int k = 0; k < 4; ++k) d[k] = group_sum<6>(d[k]);
+                    if (lane == 0)
+                        for (int r = 0; r < 2; ++r)
+                            a.dots[((li * a.scales + (l - cam * a.scales)) * 2 + r) * a.G + g] = f32x2{sm.cvalid[2 * r] ? d[2 * r] : d[2 * r + 1], d[2 * r + 1]};
+                }
             for (int ch = (int)lane; ch < a.C; ch += kWave) {
                 const float g = to_f32(gout[anchor * a.C + ch]) * to_f32(w[ch / a.hd]);
                 for (int k = 0; k < 4; ++k)
@@ -558,16 +580,29 @@ __device__ inline void dagg_levels_without_room(const DaggArgs& a, const DaggLev
 // MIXED: a lane's channels may belong to several groups.
 // WAVE: a unit is a wavefront -- what it reads of records and starts is the same for all lanes and comes through the scalar
 // cache.
-template <typename T, int VEC, bool MIXED, bool WAVE>
-__global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
+// DOTS: forms the samples' dot products with the value rows too.  A record stands for two neighbouring pixels, whose value rows are in
+// registers while the strip is at the first of them; a strip's rows and the one behind them go to LDS with the first records'
+// requests, so that no trip to memory is added, and a record's dots are stored by one lane per group, each taking another record of
+// the batch.  Bound by latency, with 16 wavefronts per CU for their LDS and registers (6 x 900 anchors, 256 channels: 344 us, of
+// which the value rows are 60 and the dots' stores 15; 1.1 GB of rows in and out).  Samples that are shared between strips have their
+// dots from the strip of the first pixel.
+template <typename T, int VEC, bool MIXED, bool WAVE, bool DOTS>
+__global__ __launch_bounds__(256, DOTS ? 4 : 1) void dagg_gradf_kernel(const DaggArgs a)
 {
     // (memory that this kernel does not write, as far as the compiler is concerned: uniform loads become scalar ones)
     typedef const __attribute__((address_space(4))) u32x4* rec_ptr;
     typedef const __attribute__((address_space(4))) uint32_t* csr_ptr;
     __shared__ DaggLevels lv;
-    __shared__ float turn_all[WAVE ? 256 * VEC : 1];
+    __shared__ float turn_all[WAVE && !DOTS ? 256 * VEC : 1];
+    // per wavefront, the strip's value rows and the one behind them
+    static_assert(!DOTS || (WAVE && !MIXED && VEC * sizeof(T) == 16 && sizeof(T) == 4));
+    typedef typename RowIO<T, VEC>::held_t held_t;
+    constexpr int kRows = kDaggStrip + 1;
+    __shared__ __align__(16) held_t values_all[DOTS ? 256 * kRows : 1];
     lv.fill(a);
-    [[maybe_unused]] float* turn = turn_all + (WAVE ? (threadIdx.x & ~63u) * VEC : 0u);
+    [[maybe_unused]] float* turn = turn_all + (WAVE && !DOTS ? (threadIdx.x & ~63u) * VEC : 0u);
+    [[maybe_unused]] held_t* values = values_all + (DOTS ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kWave * kRows : 0);
+    [[maybe_unused]] const int lane = threadIdx.x & (kWave - 1);
     auto scalar = [](int v) { return WAVE ? __builtin_amdgcn_readfirstlane(v) : v; };
     const int lpr = 1 << a.row_lpr_log2, units = 256 >> a.row_lpr_log2;
     const int c = threadIdx.x & (lpr - 1);
@@ -609,9 +644,14 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] = nxt[e] = 0.0f;
         int cur = 0;         // pixel of the strip whose sums are in acc
+        [[maybe_unused]] held_t here = {}, right = {};  // its value row, and its right neighbour's
         auto flush = [&]() { // its row is complete
             const size_t row = ((size_t)b * a.nf + lv.base[l] + p0 + cur) * a.C + ch;
-            if (direct) {
+            if constexpr (DOTS) {
+                // to where its value row was, and from there with the strip's others: stores between the records' loads would be
+                // waited for with those, and the registers of their addresses kept (372 -> 344 us)
+                __builtin_memcpy(&values[cur * kWave + lane], acc, sizeof(acc));
+            } else if (direct) {
                 if (chan_ok) RowIO<T, VEC>::store_global(static_cast<T*>(a.grad_feat) + row, acc);
             } else if constexpr (WAVE) {
                 // through LDS, so that neighbouring lanes add to neighbouring channels: an addition is carried out per 64 bytes that
@@ -638,6 +678,10 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
 #pragma unroll
             for (int e = 0; e < VEC; ++e) acc[e] = nxt[e], nxt[e] = 0.0f;
             ++cur;
+            if constexpr (DOTS) {
+                here = right;
+                right = values[(cur + 1 < kRows ? cur + 1 : cur) * kWave + lane];
+            }
         };
         // (records whose rows are in flight together; the records after them are requested with those rows, or else every
         //  batch would be two trips to memory one after the other)
@@ -647,6 +691,20 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) next[j] = rec[e0 + j < hi ? e0 + j : hi - 1];
         };
+        if constexpr (DOTS)
+            if (lo < hi) {
+                wave_lds_sync();
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // (lgkmcnt(0): the strip before has read its rows)
+                const int32_t row0 = lv.base[l] + p0;
+#pragma unroll
+                for (int i = 0; i < kRows; ++i) {
+                    // (a row behind the tensor's last is nobody's right half)
+                    const int32_t row = row0 + i < a.nf ? row0 + i : a.nf - 1;
+                    const T* from = static_cast<const T*>(a.feat) + ((size_t)b * a.nf + row) * a.C + ch;
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                                     (__attribute__((address_space(3))) void*)(values + i * kWave), 16, 0, 0);
+                }
+            }
         if (lo < hi) request(lo);
         for (uint32_t e0 = lo; e0 < hi; e0 += kAhead) {
             u32x4 rc[kAhead];
@@ -657,7 +715,7 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 row[j] = RowIO<T, VEC>::load_held(grow + (size_t)(rc[j].x >> 3) * a.C);
-                const T* wj = w + (size_t)rc[j].y * a.G;
+                const T* wj = w + (size_t)(rc[j].y & 0x7FFFFFFFu) * a.G;
                 if constexpr (MIXED) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) aw[j][e] = to_f32(wj[(ch + e) / a.hd - ch / a.hd]);
@@ -666,6 +724,17 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
                 }
             }
             if (e0 + kAhead < hi) request(e0 + kAhead);
+            [[maybe_unused]] float d0[kAhead], d1[kAhead];
+            if constexpr (DOTS) {
+                if (e0 == lo) {
+                    __builtin_amdgcn_s_waitcnt(0x0F70);  // (vmcnt(0): the value rows are there)
+                    wave_lds_sync();
+                    here = values[lane];
+                    right = values[kWave + lane];
+                }
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) d0[j] = d1[j] = 0.0f;
+            }
 #pragma unroll
             for (int j = 0; j < kAhead; ++j) {
                 if (e0 + j >= hi) break;
@@ -686,9 +755,62 @@ __global__ __launch_bounds__(256) void dagg_gradf_kernel(const DaggArgs a)
                     acc[e] = __builtin_fmaf(wa, gw, acc[e]);
                     nxt[e] = __builtin_fmaf(wb, gw, nxt[e]);
                 }
+                if constexpr (DOTS) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        d0[j] = __builtin_fmaf(here[e], g[e], d0[j]);
+                        d1[j] = __builtin_fmaf(right[e], g[e], d1[j]);
+                    }
+                }
+            }
+            if constexpr (DOTS) {
+                // over the lanes of a group, which then store a record's each (with the sample's other group's and row's: 64 bytes of 8 groups)
+                auto over = [&](auto lanes, auto sum) {
+                    if (a.lpr_log2 >= decltype(lanes)::value) {
+#pragma unroll
+                        for (int j = 0; j < kAhead; ++j) d0[j] += sum(d0[j]), d1[j] += sum(d1[j]);
+                    }
+                };
+                over(std::integral_constant<int, 1>{}, [](float v) { return dpp_xchg<0xB1>(v); });
+                over(std::integral_constant<int, 2>{}, [](float v) { return dpp_xchg<0x4E>(v); });
+                over(std::integral_constant<int, 3>{}, [](float v) { return dpp_xchg<0x141>(v); });
+                over(std::integral_constant<int, 4>{}, [](float v) { return dpp_xchg<0x140>(v); });
+                over(std::integral_constant<int, 5>{}, [](float v) { return __shfl_xor(v, 16, 64); });
+                over(std::integral_constant<int, 6>{}, [](float v) { return __shfl_xor(v, 32, 64); });
+                f32x2* dots = a.dots + (size_t)b * a.A * per_anchor * 2 * a.G + ((blk * kWave + c) >> a.lpr_log2);
+                const int lanes = 1 << a.lpr_log2;
+                for (int j0 = 0; j0 < kAhead; j0 += lanes) {
+                    const int mine = j0 + (c & (lanes - 1));
+                    uint32_t y = 0;
+                    f32x2 d = {0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < kAhead; ++j) {
+                        y = mine == j ? rc[j].y : y;
+                        d.x = mine == j ? d0[j] : d.x;
+                        d.y = mine == j ? d1[j] : d.y;
+                    }
+                    if (mine < kAhead && e0 + mine < hi && e0 + mine >= s1) dots[((size_t)(y & 0x7FFFFFFFu) * 2 + (y >> 31)) * a.G] = d;
+                }
             }
         }
         while (cur < p1 - p0) flush();
+        if constexpr (DOTS) {
+            const size_t row0 = ((size_t)b * a.nf + lv.base[l] + p0) * a.C;
+            if (direct) {
+#pragma unroll
+                for (int i = 0; i < kDaggStrip; ++i)
+                    if (i < cur) __builtin_nontemporal_store(values[i * kWave + lane], reinterpret_cast<typename RowIO<T, VEC>::mem_t*>(static_cast<T*>(a.grad_feat) + row0 + (size_t)i * a.C + ch));
+            } else {
+                wave_lds_sync();
+                const float* sums = reinterpret_cast<const float*>(values);
+                for (int i = 0; i < cur; ++i)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {  // (neighbouring lanes add to neighbouring channels, as above)
+                        const float v = sums[(i * VEC + e) * kWave + lane];
+                        if (v != 0.0f) unsafeAtomicAdd(a.image + row0 + (size_t)i * a.C + (blk * VEC + e) * kWave + lane, v);
+                    }
+            }
+        }
     }
     if (lv.lost != 0) dagg_levels_without_room<T>(a, lv);
 }
@@ -749,6 +871,50 @@ __global__ __launch_bounds__(256) void dagg_finish_kernel(const DaggArgs a)
         }
 }
 
+// The same from the dot products of whole samples: a lane per (location, group), scale after scale.
+__global__ __launch_bounds__(256) void dagg_finish_dots_kernel(const DaggArgs a)
+{
+    __shared__ i32x4 lvl[kMaxLevels];
+    if ((int)threadIdx.x < a.nl) lvl[threadIdx.x] = dagg_level(a, threadIdx.x);
+    __syncthreads();
+    const int64_t anchor = blockIdx.x, loc0 = anchor * a.nloc;
+    const int g_log2 = 31 - __builtin_clz(a.G);
+    for (int i = threadIdx.x; i < a.nloc << g_log2; i += 256) {
+        const int li = i >> g_log2, g = i & (a.G - 1), cam = li % a.cams;
+        const f32x2 xy = load_xy<float>(a.loc, loc0 + li);
+        const bool in = inside(xy.x, xy.y);
+        float sx = 0.f, sy = 0.f;
+        for (int sc = 0; sc < a.scales; ++sc) {
+            const int64_t sample = (loc0 + li) * a.scales + sc;
+            float ga = 0.f, gx = 0.f, gy = 0.f;
+            if (in) {
+                const Sample sm = sample_geometry(xy.x, xy.y, lvl[cam * a.scales + sc], a.nf, true);
+                if (sm.valid) {
+                    // (a row's dots are those of its first pixel inside and of that one's right neighbour)
+                    const f32x2 up = a.dots[sample * 2 * a.G + g], lo = a.dots[(sample * 2 + 1) * a.G + g];
+                    f32x4 d;
+                    d.x = sm.cvalid[0] ? up.x : 0.0f;
+                    d.y = sm.cvalid[1] ? (sm.cvalid[0] ? up.y : up.x) : 0.0f;
+                    d.z = sm.cvalid[2] ? lo.x : 0.0f;
+                    d.w = sm.cvalid[3] ? (sm.cvalid[2] ? lo.y : lo.x) : 0.0f;
+                    sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, static_cast<const float*>(a.w)[sample * a.G + g], d, ga, gx, gy);
+                }
+            }
+            static_cast<float*>(a.grad_w)[sample * a.G + g] = ga;
+            sx += gx;
+            sy += gy;
+        }
+        for (int d = 1; d < a.G; d <<= 1) {
+            sx += __shfl_xor(sx, d, kWave);
+            sy += __shfl_xor(sy, d, kWave);
+        }
+        if (g == 0) {
+            static_cast<float*>(a.grad_loc)[(loc0 + li) * 2] = sx;
+            static_cast<float*>(a.grad_loc)[(loc0 + li) * 2 + 1] = sy;
+        }
+    }
+}
+
 template <typename F>
 hipError_t by_vec(int es, int vec, F f)
 {
@@ -781,13 +947,17 @@ hipError_t forward_t(const DaggArgs& a, hipStream_t stream)
 template <typename T>
 hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
 {
-    hipError_t e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
+    // (a multiple of 8 sort workgroups: the others keep their places in the XCD mapping)
+    const uint32_t sorts = ((uint32_t)(a.bs * a.nl * a.sort_ranges) + kNumXcd - 1) / kNumXcd * kNumXcd;
+    hipError_t e = hipSuccess;
+    if (a.dots != nullptr) {
+        hipLaunchKernelGGL(dagg_sort_kernel<T>, dim3(sorts + kDaggZeroWgs), dim3(kDaggSortWaves * kWave), sizeof(DaggSort), stream, a, sorts);
+        e = hipGetLastError();
+    } else e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
         constexpr int VEC = decltype(v)::value;
         if constexpr (VEC * sizeof(T) <= 16) {
             size_t lds = kDaggBackWaves * kDotsLds;
             if (lds < sizeof(DaggSort)) lds = sizeof(DaggSort);
-            // (a multiple of 8 sort workgroups: the others keep their places in the XCD mapping)
-            const uint32_t sorts = ((uint32_t)(a.bs * a.nl * a.sort_ranges) + kNumXcd - 1) / kNumXcd * kNumXcd;
             hipLaunchKernelGGL((dagg_dots_and_sort_kernel<T, VEC>), dim3(sorts + kDaggZeroWgs + a.map.grid), dim3(kDaggBackWaves * kWave), lds, stream, a, sorts);
             return hipGetLastError();
         } else {
@@ -806,9 +976,14 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
             int64_t blocks = (a.bs * items * a.row_blocks + units - 1) / units;
             if (blocks > 256 * 32) blocks = 256 * 32;
             const dim3 grid((unsigned)blocks), block(256);
-            if (a.hd % VEC != 0) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true, false>), grid, block, 0, stream, a);
-            else if (a.row_lpr_log2 == 6) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, true>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, false>), grid, block, 0, stream, a);
+            if constexpr (VEC == 4 && sizeof(T) == 4)
+                if (a.dots != nullptr) {
+                    hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, true, true>), grid, block, 0, stream, a);
+                    return hipGetLastError();
+                }
+            if (a.hd % VEC != 0) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, true, false, false>), grid, block, 0, stream, a);
+            else if (a.row_lpr_log2 == 6) hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, true, false>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((dagg_gradf_kernel<T, VEC, false, false, false>), grid, block, 0, stream, a);
             return hipGetLastError();
         } else {
             return hipErrorInvalidConfiguration;
@@ -816,7 +991,8 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
     });
     if (e != hipSuccess) return e;
     const unsigned rounding = sizeof(T) == 2 ? 512u : 0u;
-    hipLaunchKernelGGL(dagg_finish_kernel<T>, dim3((unsigned)(a.bs * a.A) + rounding), dim3(256), (size_t)((a.nloc + 1) & ~1) * 2, stream, a);
+    if (a.dots != nullptr) hipLaunchKernelGGL(dagg_finish_dots_kernel, dim3((unsigned)(a.bs * a.A)), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL(dagg_finish_kernel<T>, dim3((unsigned)(a.bs * a.A) + rounding), dim3(256), (size_t)((a.nloc + 1) & ~1) * 2, stream, a);
     return hipGetLastError();
 }
 

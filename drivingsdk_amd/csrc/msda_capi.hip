@@ -931,7 +931,25 @@ int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
     return MXD_OK;
 }
 
-// Workspace of the backward: {weights' gradients per group, location gradients per group, record starts, records, float32
+// Whether the kernel that forms the rows of grad_feat forms the dot products as well: it has a sample's grad_out row at hand, in the
+// order of the pixels, so that every value row is read once, in order, in place of a gather of four rows per sample and group that
+// misses the L2 in two fifths of them.  In return the sort is no longer hidden behind that gather (68 us), and rows that few samples
+// touch are read whole.  6 x 900 anchors x 13 points, six cameras of four scales (538k pixels), 256 channels of float32: 320 + 224 +
+// 42 us for the three kernels, 68 + 344 + 50 with this.  Which is faster depends on the samples per pixel and on their number
+// (the backward's time that way over this way, locations inside a quarter of the cameras):
+//   3.1 a pixel: 2 / 3 / 4 / 5 / 6 batch elements 0.80 / 0.90 / 1.06 / 1.12 / 1.17, groups of 8 channels with 4 1.43;
+//   2.1 a pixel 0.95 with 6 batch elements, 1.6 0.85, 1.0 0.88 with 12; 12 a pixel 1.04; 512 channels: 2 / 4 batch elements 0.96 / 1.20.
+// Rows of 128 channels, which units of less than a wavefront share, were at 0.87 .. 1.02, 16-bit rows at 0.71 .. 1.05: not for them.
+bool dagg_dots_with_rows(const mxd::DaggArgs& a, int es)
+{
+    const int lanes = a.hd / 4;
+    if (es != 4 || a.C % 256 != 0 || a.hd % 4 != 0 || lanes > mxd::kWave || (lanes & (lanes - 1)) != 0) return false;
+    if (a.G > mxd::kWave || (a.G & (a.G - 1)) != 0) return false;
+    const int64_t samples = (int64_t)a.A * a.P * a.nl;
+    return 4 * samples >= 11 * (int64_t)a.nf && a.bs * samples * (a.C / 256) >= (int64_t(5) << 18);
+}
+
+// Workspace of the backward: {weights' gradients per group, location gradients per group (or the samples' dot products), record starts, records, float32
 // image of grad_mc_ms_feat for 16-bit dtypes}.
 struct DaggSpace {
     size_t gl, csr, rec, image, total;
@@ -940,6 +958,10 @@ struct DaggSpace {
         const size_t locs = (size_t)a.bs * a.A * a.nloc;
         gl = round_up((size_t)a.G * locs * a.scales * 4, 256);
         csr = gl + round_up((size_t)a.G * locs * 8, 256);
+        if (dagg_dots_with_rows(a, es)) {
+            const size_t dots = round_up((size_t)a.G * locs * a.scales * 16, 256);
+            if (csr < dots) csr = dots;
+        }
         rec = csr + round_up((size_t)a.bs * (size_t)a.starts * 4, 256);
         image = rec + (size_t)a.bs * a.nl * 2 * a.A * a.P * 16;
         total = image + (es == 2 ? (size_t)a.bs * a.nf * a.C * 4 : 0);
@@ -1684,6 +1706,8 @@ int mxd_dagg_backward(const void* mc_ms_feat, const int32_t* spatial_shape, cons
     if (reinterpret_cast<uintptr_t>(a.image) & 3u) return fail(MXD_E_SHAPE, "mxd_dagg_backward: grad_mc_ms_feat is not 4-byte aligned");
     a.gw_part = reinterpret_cast<float*>(ws);
     a.gl_part = reinterpret_cast<float*>(ws + space.gl);
+    // (the value rows are copied to LDS 16 bytes a lane)
+    if (dagg_dots_with_rows(a, es) && (reinterpret_cast<uintptr_t>(mc_ms_feat) & 15u) == 0) a.dots = reinterpret_cast<mxd::f32x2*>(ws);
     a.csr = reinterpret_cast<uint32_t*>(ws + space.csr);
     a.rec = reinterpret_cast<mxd::u32x4*>(ws + space.rec);
     const hipError_t e = mxd::launch_dagg_backward(dtype, a, static_cast<hipStream_t>(hip_stream));

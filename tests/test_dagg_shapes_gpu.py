@@ -90,3 +90,18 @@ def test_levels_that_share_rows(gpu_device, cams, maps, starts, nf, C, G, A, P, 
     tol = {torch.float32: BWD_FP32, torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
     for k, (g, r) in enumerate(zip(run_gpu(*inp, gpu_device, dtype=dtype), want)):
         assert rel_err(g, r) <= tol, k
+
+
+@pytest.mark.parametrize("C,G,shared", [(256, 8, False), (256, 1, False), (256, 64, False), (512, 16, False), (256, 8, True), (256, 4, "lost")])
+def test_dots_with_the_rows(gpu_device, C, G, shared):
+    """As many samples as have their dot products formed in the order of the pixels; most lie outside the images."""
+    maps = [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6
+    if shared == "lost":
+        maps = [[(40, 61), (40, 61), (40, 61), (40, 60)]] * 6
+    A = 884 * 256 // C
+    feat, ss, ssi, loc, w, go = make_inputs(2, C, G, A, 31, maps, seed=C + G, pad=True)
+    loc[np.random.default_rng(1).random(loc.shape[:3] + (6,)) < 0.97] += 2.0
+    if shared:  # every camera names the same rows; "lost": more of them than the table of record starts has room for
+        ssi = np.broadcast_to(np.array([0, 17, 5, 60], dtype=np.int32), (6, 4)).copy()
+        feat = np.ascontiguousarray(feat[:, :2460 if shared == "lost" else 150])
+    print(check((feat, ss, ssi, loc, w, go), gpu_device))
