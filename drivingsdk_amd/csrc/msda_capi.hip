@@ -96,8 +96,8 @@ struct Tuning {
                          // (16, 8, 4), 0 = chosen here
     int tile_px_log2;    // MXD_MSDA_TILE_PX_LOG2: log2 of the pixels per tile of the grad_value pass (9, 8, 7), 0 = chosen here
     int gka_slab;        // MXD_MSDA_GKA_SLAB: geometric kernel attention with value in LDS: 0 = never, 1 = wherever it fits, -1 = chosen here
-    int bwd_fixed;       // MXD_MSDA_BWD_FIXED: 0 = the first backward kernel never takes the instantiation with the common launch
-                         // geometry as constants (default 1: where the launch has that geometry)
+    int bwd_fixed;       // MXD_MSDA_BWD_FIXED: 0 = the general first backward kernel also where the launch has a geometry that a kernel
+                         // (one pass, 4 or 8 lanes per row) or an instantiation (256-byte rows) of its own is built for (default 1)
     int bwd_two_pass;    // MXD_MSDA_BWD_TWO_PASS: 1 = the first backward kernel reads rows of 17 to 32 lanes of 16 bytes with 16
                          // lanes in two passes, 0 = with 32 lanes in one
     int bwd_rec_lds;     // MXD_MSDA_BWD_REC_LDS: 0 = workgroups of the first backward kernel that make several passes store
@@ -301,10 +301,9 @@ int backward_lane_bytes(int dtype, const Dims& d)
 {
     const int v = tuning().bwd_lane_bytes;
     if (v == 4 || v == 8 || v == 16) return v;
-    // Rows of 33 to 64 bytes: 8 lanes of 8 bytes per row rather than 4 lanes of 16.  With 16 units per wavefront the
-    // staging strips of a workgroup take 51 KiB of LDS, which leaves 3 wavefronts per SIMD, and a lane stages four
-    // samples of which it keeps two in registers (measured, encoder shape in float16 / bfloat16: backward 322 -> 300 us;
-    // BEVFormer shape in float16 1114 -> 1075 us; with rows of 256 bytes halving the lane width costs 10 %).
+    // Rows of 33 to 64 bytes: 8 lanes of 8 bytes per row rather than 4 lanes of 16 in the general kernel, whose staging strips of 16
+    // units per wavefront take 51 KiB of LDS (encoder shape in float16 / bfloat16: backward 322 -> 300 us; with rows of 256 bytes
+    // halving the lane width costs 10 %).  The kernel of one-pass workgroups takes 4 lanes by itself where it has the workgroups.
     // Rows of up to 32 bytes: 8 lanes of 4 for units that fill a chunk of 16 samples (16 channels in float16, 2 x 13253 queries of 18
     // samples: backward 289 -> 251 us; 3 samples 53 -> 55), with half as many queries per workgroup.
     const int64_t row = d.hd * elem_size(dtype);
