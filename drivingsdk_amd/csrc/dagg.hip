@@ -400,13 +400,16 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
     DaggSort& sh = *reinterpret_cast<DaggSort*>(smem);
     DaggLevels& lv = sh.lv;
     uint32_t *cnt = sh.cnt, *wsum = sh.wsum, &before_s = sh.before_s;
-    const int range = block % a.sort_ranges, l = block / a.sort_ranges % a.nl, b = block / a.sort_ranges / a.nl;
+    // first ranges first, scale by scale: the workgroups that have pixels are neighbours, and so spread over the XCDs (range by range of a
+    // level, 22 apart, they met on four of them: the launch took 68 us with 6 x 900 anchors, 50 like this)
+    const uint32_t maps = (uint32_t)a.bs * (uint32_t)a.cams, i = block % (maps * a.scales);
+    const int range = (int)(block / (maps * a.scales)), b = (int)(i % a.bs), l = (int)(i % maps) / a.bs * a.scales + (int)(i / maps);
     const i32x4 own = dagg_level(a, l);
-    if (b >= a.bs || (int64_t)own.x * own.y <= (int64_t)range * kDaggSortPx) return;  // (uniform)
+    if ((int64_t)own.x * own.y <= (int64_t)range * kDaggSortPx) return;  // (uniform)
     lv.fill(a);
     const int tid = threadIdx.x;
     const int r0 = range * kDaggSortPx, P = lv.px[l], r1 = P - r0 < kDaggSortPx ? P : r0 + kDaggSortPx;
-    if (b >= a.bs || r0 >= P) return;  // (uniform; the launch has a multiple of 8 sort workgroups)
+    if (range >= a.sort_ranges || r0 >= P) return;  // (uniform; the launch has a multiple of 8 sort workgroups)
     for (int i = tid; i < kDaggSortPx; i += kThreads) cnt[i] = 0;
     if (tid == 0) before_s = 0;
     __syncthreads();
@@ -513,7 +516,7 @@ __device__ inline void dagg_zero(const DaggArgs& a, uint32_t block, unsigned cha
 }
 
 // The kernels side by side in one launch: the sort has work for a few workgroups, whose time the others' gathers cover
-// (68 us as a launch of its own for 6 x 900 anchors).
+// (50 us as a launch of its own for 6 x 900 anchors).
 template <typename T, int VEC>
 __global__ __launch_bounds__(kDaggBackWaves * kWave) void dagg_dots_and_sort_kernel(const DaggArgs a, uint32_t sorts)
 {
