@@ -7,7 +7,8 @@ namespace mxd {
 constexpr int kDaggWaves = 4;        // wavefronts per workgroup of the forward: an anchor each
 constexpr int kDaggBackWaves = 8;    // the same for the backward's first kernel, whose sort is the shorter for it (442 anchors: 52 -> 44 us with 8, 43 with
                                      // 16; 6 x 900 anchors lose 5 % with 16)
-constexpr int kDaggSortWaves = 16;   // the same for the sort as a launch of its own (6 x 900 anchors: 72 us with 8)
+constexpr int kDaggSortWaves = 16;   // the same for the sort as a launch of its own (6 x 900 anchors: 72 instead of 68 us with 8, before its
+                                     // points were compacted)
 constexpr int kDaggList = 128;       // locations of an anchor that a wavefront looks through before it samples
 constexpr int kDaggSortPx = 4096;    // pixels of a level that a workgroup of the sort counts in LDS
 constexpr int kDaggStrip = 8;        // neighbouring pixels whose gradient rows are formed together

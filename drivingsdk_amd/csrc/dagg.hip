@@ -387,13 +387,22 @@ struct DaggLevels {
 // ---- sort of the corner pairs by pixel -------------------------------------------------------------------------------------
 // One workgroup per (batch, level, range of kDaggSortPx pixels): counts the records of every pixel in LDS, turns the counts
 // into starts, and drops every record at its place.
-struct DaggSort {
+struct alignas(16) DaggSort {
     DaggLevels lv;
     uint32_t wsum[kDaggSortWaves];
     uint32_t before_s;
     uint32_t cnt[kDaggSortPx];
 };
-template <typename T, int WAVES>
+// What a wavefront keeps of the points that it has requested: those inside the image.
+struct DaggInside {
+    static constexpr int kRounds = 4;
+    f32x2 xy[kRounds * kWave];
+    uint16_t at[kRounds * kWave];  // request << 6 | lane
+};
+// COMPACT: the points inside the image side by side before their geometry is derived, or else a wavefront derives it for all 64
+// wherever one is inside (6 x 900 anchors, a third of the points inside: 50 -> 43 us; the sort beside the dots, which cover it, does
+// without the LDS for it).
+template <typename T, int WAVES, bool COMPACT>
 __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned char* smem)
 {
     constexpr int kThreads = WAVES * kWave;
@@ -431,12 +440,39 @@ __device__ inline void dagg_sort(const DaggArgs& a, uint32_t block, unsigned cha
     // eight points' locations are requested together: one at a time, the two passes are a chain of trips to memory
     constexpr int kTogether = 8;
     auto each_point = [&](auto take) {
-        for (uint32_t i0 = tid; i0 < points; i0 += kTogether * kThreads) {
+        for (uint32_t i0 = tid; COMPACT ? (i0 & ~(uint32_t)(kWave - 1)) < points : i0 < points; i0 += kTogether * kThreads) {
             f32x2 xy[kTogether];
 #pragma unroll
             for (int k = 0; k < kTogether; ++k) {
                 const uint32_t i = i0 + k * kThreads;
                 xy[k] = i < points ? load_xy<T>(a.loc, ((int64_t)b * points + i) * a.cams + cam) : f32x2{0.f, 0.f};
+            }
+            if constexpr (COMPACT) {
+                DaggInside& list = reinterpret_cast<DaggInside*>(smem + sizeof(DaggSort))[tid >> 6];
+                for (int half = 0; half < kTogether; half += DaggInside::kRounds) {
+                    uint32_t n = 0;
+#pragma unroll
+                    for (int k = 0; k < DaggInside::kRounds; ++k) {
+                        const f32x2 p = xy[k];
+                        const bool in = inside(p.x, p.y);
+                        const uint64_t mask = __ballot(in);
+                        if (in) {
+                            const uint32_t pos = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+                            list.xy[pos] = p;
+                            list.at[pos] = (uint16_t)((half + k) << 6 | (tid & (kWave - 1)));
+                        }
+                        n += (uint32_t)__builtin_popcountll(mask);
+                    }
+#pragma unroll
+                    for (int k = 0; k < DaggInside::kRounds; ++k) xy[k] = xy[k + DaggInside::kRounds];
+                    wave_lds_sync();
+                    for (uint32_t e = tid & (kWave - 1); e < n; e += kWave) {
+                        const uint32_t at = list.at[e], i = i0 - (tid & (kWave - 1)) + (at >> 6) * kThreads + (at & (kWave - 1));
+                        each_record(list.xy[e], [&](uint32_t r, int key, float wa, float wb) { take(i, r, key, wa, wb); });
+                    }
+                    wave_lds_sync();
+                }
+                continue;
             }
             for (int k = 0; k < kTogether; ++k) {
                 each_record(xy[0], [&](uint32_t r, int key, float wa, float wb) { take(i0 + k * kThreads, r, key, wa, wb); });
@@ -516,23 +552,27 @@ __device__ inline void dagg_zero(const DaggArgs& a, uint32_t block, unsigned cha
 }
 
 // The kernels side by side in one launch: the sort has work for a few workgroups, whose time the others' gathers cover
-// (50 us as a launch of its own for 6 x 900 anchors).
+// (43 us as a launch of its own for 6 x 900 anchors).
 template <typename T, int VEC>
 __global__ __launch_bounds__(kDaggBackWaves * kWave) void dagg_dots_and_sort_kernel(const DaggArgs a, uint32_t sorts)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ i32x4 lvl[kMaxLevels];
-    if (blockIdx.x < sorts) dagg_sort<T, kDaggBackWaves>(a, blockIdx.x, smem);
+    if (blockIdx.x < sorts) dagg_sort<T, kDaggBackWaves, false>(a, blockIdx.x, smem);
     else if (blockIdx.x < sorts + kDaggZeroWgs) dagg_zero(a, blockIdx.x - sorts, smem);
     else dagg_dots<T, VEC>(a, blockIdx.x - sorts - kDaggZeroWgs, smem, lvl);
 }
+
+static_assert(sizeof(DaggSort) % 16 == 0 && sizeof(DaggInside) % 8 == 0);
+constexpr size_t kDaggSortLds = sizeof(DaggSort) + kDaggSortWaves * sizeof(DaggInside);
+static_assert(kDaggSortLds <= 64 * 1024, "what a launch may take without opting in");
 
 // The same without dot products, where the kernel behind it forms them.
 template <typename T>
 __global__ __launch_bounds__(kDaggSortWaves * kWave) void dagg_sort_kernel(const DaggArgs a, uint32_t sorts)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    if (blockIdx.x < sorts) dagg_sort<T, kDaggSortWaves>(a, blockIdx.x, smem);
+    if (blockIdx.x < sorts) dagg_sort<T, kDaggSortWaves, true>(a, blockIdx.x, smem);
     else dagg_zero(a, blockIdx.x - sorts, smem);
 }
 
@@ -954,7 +994,7 @@ hipError_t backward_t(const DaggArgs& a, hipStream_t stream)
     const uint32_t sorts = ((uint32_t)(a.bs * a.nl * a.sort_ranges) + kNumXcd - 1) / kNumXcd * kNumXcd;
     hipError_t e = hipSuccess;
     if (a.dots != nullptr) {
-        hipLaunchKernelGGL(dagg_sort_kernel<T>, dim3(sorts + kDaggZeroWgs), dim3(kDaggSortWaves * kWave), sizeof(DaggSort), stream, a, sorts);
+        hipLaunchKernelGGL(dagg_sort_kernel<T>, dim3(sorts + kDaggZeroWgs), dim3(kDaggSortWaves * kWave), kDaggSortLds, stream, a, sorts);
         e = hipGetLastError();
     } else e = by_vec(sizeof(T), dagg_vec(sizeof(T), a.hd), [&](auto v) {
         constexpr int VEC = decltype(v)::value;

@@ -932,11 +932,11 @@ int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
 
 // Whether the kernel that forms the rows of grad_feat forms the dot products as well: it has a sample's grad_out row at hand, in the
 // order of the pixels, so that every value row is read once, in order, in place of a gather of four rows per sample and group that
-// misses the L2 in two fifths of them.  In return the sort is no longer hidden behind that gather (68 us), and rows that few samples
+// misses the L2 in two fifths of them.  In return the sort is no longer hidden behind that gather (43 us), and rows that few samples
 // touch are read whole.  6 x 900 anchors x 13 points, six cameras of four scales (538k pixels), 256 channels of float32: 320 + 224 +
-// 42 us for the three kernels, 68 + 344 + 50 with this.  Which is faster depends on the samples per pixel and on their number
+// 42 us for the three kernels, 43 + 344 + 50 with this.  Which is faster depends on the samples per pixel and on their number
 // (the backward's time that way over this way, locations inside a quarter of the cameras):
-//   3.1 a pixel: 2 / 3 / 4 / 5 / 6 batch elements 0.80 / 0.90 / 1.06 / 1.12 / 1.17, groups of 8 channels with 4 1.43;
+//   (with a sort of 68 us)  3.1 a pixel: 2 / 3 / 4 / 5 / 6 batch elements 0.80 / 0.90 / 1.06 / 1.12 / 1.17, groups of 8 channels with 4 1.43;
 //   2.1 a pixel 0.95 with 6 batch elements, 1.6 0.85, 1.0 0.88 with 12; 12 a pixel 1.04; 512 channels: 2 / 4 batch elements 0.96 / 1.20.
 // Rows of 128 channels, which units of less than a wavefront share, were at 0.87 .. 1.02, 16-bit rows at 0.71 .. 1.05: not for them.
 bool dagg_dots_with_rows(const mxd::DaggArgs& a, int es)
