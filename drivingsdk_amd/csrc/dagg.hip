@@ -318,12 +318,12 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
 // ---- the levels as the kernels behind it see them ---------------------------------------------------------------------------
 struct DaggLevels {
     int32_t H[kMaxLevels], W[kMaxLevels], base[kMaxLevels];
-    int32_t px[kMaxLevels];      // pixels inside the feature tensor; 0: the level has no rows (or is one of `lost`)
+    int32_t px[kMaxLevels];      // pixels that the sort has records of, inside the feature tensor; 0: none (no rows, or one of `lost`)
     int32_t csr[kMaxLevels];     // its first entry of DaggArgs::csr
     int32_t chunks[kMaxLevels];  // parts its strips' records are split into
     int32_t first[kMaxLevels + 1];  // work items of the levels before it
     int32_t tiled;               // the levels tile the keys in order: a pixel row belongs to one level
-    uint64_t lost;               // levels, by bit, that found no room in csr: dagg_levels_without_room
+    uint64_t lost;               // levels, by bit, with rows that no record stands for: dagg_levels_without_room
 
     // (a level per lane of the first wavefront: one after the other, 24 levels were 5 us in front of every workgroup)
     __device__ void fill(const DaggArgs& a)
@@ -346,9 +346,10 @@ struct DaggLevels {
             const int32_t end = L.z + P, before = __shfl_up(end, 1, kWave);
             const bool follows = whole && L.z == (lane == 0 ? 0 : before);
             tiled = __ballot(lane < a.nl && !follows) == 0 && __builtin_amdgcn_readlane(end, a.nl - 1) == a.nf;
-            // (levels that overlap far: the ones that find no room in the table of record starts have no records)
+            // (levels without records: the ones that find no room in the table of record starts, where levels overlap far, and one
+            //  that starts before the tensor and reaches into it, whose pixels are not numbered from its first row on)
             int64_t used = P > 0 ? P + 1 : 0, at = prefix(used) - used;
-            bool fits = true;
+            bool fits = !(L.x > 0 && L.y > 0 && L.z < 0 && L.z + p > 0);
             if (__ballot(at + used > a.starts) != 0) {
                 int64_t room = 0;
                 for (int l = 0; l < a.nl; ++l) {
@@ -356,7 +357,7 @@ struct DaggLevels {
                     const bool room_left = room + u <= a.starts;
                     if (lane == l) {
                         at = room;
-                        fits = room_left;
+                        fits = fits && room_left;
                     }
                     if (room_left) room += u;
                 }
@@ -577,9 +578,10 @@ __global__ __launch_bounds__(kDaggSortWaves * kWave) void dagg_sort_kernel(const
 }
 
 // ---- gradient of the feature maps --------------------------------------------------------------------------------------------
-// The samples of levels that found no room in the table of record starts, added to grad_feat's float32 image by atomics: a sample per
-// wavefront, a channel per lane.  Only levels that overlap come here, and then every row has been zeroed and every other level
-// adds with atomics as well.  Slow, and there so that scale_start_index is honoured however it comes.
+// The samples of levels without records (DaggLevels::lost), added to grad_feat's float32 image by atomics, and their dots where the
+// finish kernel takes those from DaggArgs::dots: a sample per wavefront, a channel per lane.  Only levels that overlap or start before
+// the tensor come here, and then every row has been zeroed and every other level adds with atomics as well.  Slow, and there so that
+// scale_start_index is honoured however it comes.
 template <typename T>
 __device__ inline void dagg_levels_without_room(const DaggArgs& a, const DaggLevels& lv)
 {

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import dagg_oracle as dagg
-from test_dagg_gpu import check, make_inputs, run_gpu
+from test_dagg_gpu import _edge_mask, check, make_inputs, run_gpu
 from util import BWD_FP32, FWD_FP32, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -105,3 +105,39 @@ def test_dots_with_the_rows(gpu_device, C, G, shared):
         ssi = np.broadcast_to(np.array([0, 17, 5, 60], dtype=np.int32), (6, 4)).copy()
         feat = np.ascontiguousarray(feat[:, :2460 if shared == "lost" else 150])
     print(check((feat, ss, ssi, loc, w, go), gpu_device))
+
+
+def _around(inp, device, before, after, dtype=torch.float32):
+    """Results on the GPU and the oracle's, which reads rows of zeros where a level reaches out of the tensor."""
+    feat, ss, ssi, loc, w, go = inp
+    rows = np.zeros((feat.shape[0], before + feat.shape[1] + after, feat.shape[2]), dtype=np.float32)
+    rows[:, before:before + feat.shape[1]] = feat
+    args = rows, ss, (ssi + before).astype(np.int32), loc, w
+    want = [dagg.direct_forward(*args), *dagg.direct_backward(*args, go)]
+    want[1] = want[1][:, before:before + feat.shape[1]]
+    del rows
+    torch.full((1 << 27,), float("nan"), device=device)  # (what a workspace finds in its memory)
+    return run_gpu(*inp, device, dtype=dtype), want
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("C,G", [(256, 8), (64, 8), (40, 8)])
+def test_a_level_that_starts_before_the_tensor(gpu_device, C, G, dtype):
+    feat, ss, _, loc, w, go = make_inputs(2, C, G, 33, 5, [[(9, 13), (5, 7)]] * 2, seed=C, pad=True)
+    ssi = np.array([[-20, 97], [-117, 290]], dtype=np.int32)  # (the third lies wholly before it, the last one reaches behind it)
+    inp = [np.asarray(torch.from_numpy(t).to(dtype).float()) if t.dtype == np.float32 else t for t in (feat, ss, ssi, loc, w, go)]
+    tol = {torch.float32: BWD_FP32, torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
+    for k, (g, r) in enumerate(zip(*_around(inp, gpu_device, 117, 40, dtype))):
+        assert rel_err(g, r) <= tol, k
+
+
+def test_a_level_that_starts_before_the_tensor_with_the_rows_dots(gpu_device):
+    """The same where the dot products are formed in the order of the pixels: a level without records has its own from elsewhere."""
+    feat, ss, _, loc, w, go = make_inputs(2, 256, 8, 884, 31, [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6, seed=7, pad=True)
+    loc[np.random.default_rng(1).random(loc.shape[:3] + (6,)) < 0.97] += 2.0
+    ssi = np.cumsum(np.concatenate([[-50], ss.reshape(-1, 2).prod(1)[:-1]])).reshape(6, 4).astype(np.int32)
+    ssi[3, 1] = -30
+    inp = feat, ss, ssi, loc, w, go
+    keep = ~_edge_mask(ss, loc)[..., None]
+    for k, (g, r) in enumerate(zip(*_around(inp, gpu_device, 50, 10))):
+        assert rel_err(*((g * keep, r * keep) if k == 2 else (g, r))) <= (FWD_FP32 if k == 0 else BWD_FP32), k
