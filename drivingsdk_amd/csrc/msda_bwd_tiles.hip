@@ -76,10 +76,11 @@ __device__ inline bool decode_tile_item(const KArgs& a, int32_t item, int lane, 
     return true;
 }
 
-// The samples of levels whose tiles found no room in the run table, added to grad_value one sample per thread with
-// atomics: share `part` of `parts` of the samples of (batch b, head h).  Only levels that overlap can have more tiles
-// between them than the table holds; for such layouts the whole image was zero-filled and every tile adds with atomics
-// as well.  Slow, and there so that level_start_index is honoured however it comes.  Plain operator only.
+// The samples of levels whose tiles found no room in the run table, and of levels that start before the tensor and reach
+// into it (they have no tiles: LevelLanes), added to grad_value one sample per thread with atomics: share `part` of
+// `parts` of the samples of (batch b, head h).  Only levels that overlap can have more tiles between them than the
+// table holds; for such layouts the whole image was zero-filled and every tile adds with atomics as well.  Slow, and
+// there so that level_start_index is honoured however it comes.  Plain operator only.
 // unfit: kMaxLevels flags in LDS, filled here.
 template <typename T>
 __device__ inline void add_levels_without_tiles(const KArgs& a, int b, int h, int part, int parts, int32_t* unfit)
@@ -91,10 +92,11 @@ __device__ inline void add_levels_without_tiles(const KArgs& a, int b, int h, in
             const i32x4 L = load_level(a, l);
             int32_t P;
             const int32_t nt = level_tile_count(L.x, L.y, L.z, a.nk, a.tile_px_log2, &P);
-            const bool fits = first + nt <= a.tbl_stride - 1;
+            const bool before = L.x > 0 && L.y > 0 && L.z < 0 && L.z + (int64_t)L.x * L.y > 0;
+            const bool fits = !before && first + nt <= a.tbl_stride - 1;
             unfit[l] = fits ? 0 : 1;
             if (fits) first += nt;
-            else if (nt > 0) any = 1;
+            else if (before || nt > 0) any = 1;
         }
         any_unfit = any;
     }

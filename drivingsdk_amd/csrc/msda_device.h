@@ -143,7 +143,7 @@ __device__ inline bool tile_stored_directly(int32_t chunks, int32_t npx, int32_t
 struct LevelLanes {
     i32x4 geo;       // this lane's level {H, W, first key, 0}; zeros past the last level
     int32_t px, nt;  // its pixels inside the value tensor, its tiles in the run table
-    int32_t first;   // number of its first tile (tiles are numbered level by level); -1: the table has no room for its tiles
+    int32_t first;   // number of its first tile (tiles are numbered level by level); -1: it has none, or the table has no room for them
     int32_t chunks;  // query chunks per tile
     // Whether the levels tile the keys exactly and in order -- the first level starts at key 0, every other one where the
     // one before it ends, the last one ends at key nk -- and all their tiles fit the run table.  Only then is every row of
@@ -160,7 +160,7 @@ struct LevelLanes {
         const int32_t tiles = level_tile_count(geo.x, geo.y, geo.z, a.nk, a.tile_px_log2, &px), room = a.tbl_stride - 1;
         const int32_t inc = prefix(a, tiles, lane), total = __builtin_amdgcn_readlane(inc, a.nl - 1);
         nt = tiles;
-        first = inc - tiles;
+        first = tiles > 0 ? inc - tiles : -1;  // (a level that starts before the tensor has no tiles, and samples that reach into it)
         if (total > room) {
             // levels that overlap: one whose tiles find no room is left out, a later one may still fit
             nt = 0;
@@ -168,7 +168,7 @@ struct LevelLanes {
             int32_t at = 0;
             for (int l = 0; l < a.nl; ++l) {
                 const int32_t n = __builtin_amdgcn_readlane(tiles, l);
-                if (at + n > room) continue;
+                if (n == 0 || at + n > room) continue;
                 if (lane == l) nt = n, first = at;
                 at += n;
             }

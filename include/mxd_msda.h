@@ -189,8 +189,9 @@ size_t mxd_msda_backward_workspace_bytes(int dtype, int64_t bs, int64_t nk, int6
                                 (op_kernel/multi_scale_deformable_attn_grad.cpp:181-186).  One case is slow by default:
                                 levels that overlap so far that they have more than num_keys/T + num_levels tiles of
                                 T pixels between them (T = 512 for heads of up to 32 channels, 256 for up to 64, 128
-                                beyond) -- mxd_msda_backward then adds the levels beyond that sample by sample.  The
-                                fused form and the sibling operators have no such fallback: there the default form
+                                beyond), and levels whose start is negative -- mxd_msda_backward then adds the levels
+                                without tiles sample by sample.  The fused form and the sibling operators have no such
+                                fallback (but mxd_dagg_backward, which has its own): there the default form
                                 leaves those levels out of grad_value, and this flag (or MXD_MSDA_BWD_ATOMIC=1 in the
                                 environment) asks for the form that does not care */
 
