@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     __shared__ uint32_t run_src_all[NW * kWave];
     __shared__ uint32_t run_pre_all[NW * kWave];
     __shared__ int32_t lv_unfit[kMaxLevels];
-    __shared__ int done_count;
+    __shared__ int done_count, nan_seen;
     // Pixels that collect far more entries than the others (inputs that pile samples on a few pixels) get extra
     // lists in the slots of the workgroup that no pixel of the tile uses -- when there are such slots.  The first
     // round counts entries per slot (two 16-bit counters per word); after it the same array holds, per slot,
@@ -200,6 +200,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     heads[threadIdx.x] = ((threadIdx.x / (GPW * PPG)) % NW * kTileEntCap + kDummyOfWave) * 16u;
     if (threadIdx.x == 0) {
         done_count = 0;
+        nan_seen = 0;
         spare_next = 0;
         round1_total = 0;
     }
@@ -270,6 +271,21 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     // two 16-bit elements, so there the last lane of a row whose length is no multiple of 4 reads the row's last four
     // and moves its sums to their places when the rounds are done.
     auto first_channel = [&](int ch) { return sizeof(T) == 2 && VEC == 4 ? piece_start<4>(ch, hd) : ch; };
+
+    // the next channel pass starts from a clean state (the dummy entry may have been overwritten by the transposition)
+    auto clean_state = [&]() {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            done_count = 0;
+            nan_seen = 0;
+        }
+        // (opaque: the entry would otherwise be kept through the whole pass, in registers that some forms do not have -- and
+        //  memory for spilled ones costs every wavefront time before it starts)
+        uint32_t none = 0u;
+        asm volatile("" : "+v"(none));
+        if (lane == 0) ent_at(dummy) = u32x4{none | kInvalidCorner, none, none, none + dummy};
+        __syncthreads();
+    };
 
     for (int cb = 0; cb < hd; cb += CH) {
         float acc[kAccPx][CHL];
@@ -535,6 +551,12 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         }
 
         {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < kAccPx; ++i)
+#pragma unroll
+                for (int c = 0; c < CHL; ++c) bad |= acc[i][c] != acc[i][c];
+            if (bad) nan_seen = 1;
             // what a group collected for the first pixel of the next group: inside a wavefront from lane to lane, from
             // the last group of a wavefront to the first of the next through the entry storage (free now; the last
             // group of the workgroup has nothing to hand over: a pair never starts on the last pixel of a tile)
@@ -547,6 +569,61 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                               __builtin_bit_cast(uint32_t, acc[PPG][4 * k + 2]), __builtin_bit_cast(uint32_t, acc[PPG][4 * k + 3])};
             }
             __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(nan_seen) != 0) {
+                // The walk adds a row of grad_out to the pixel of an entry and, times the entry's other weight, to the pixel behind it,
+                // also where that weight is zero because there is no such pixel: an infinite row leaves NaN there.  Sums that hold
+                // NaN are formed again here, by a wavefront for an eighth of the pixels, in LDS, from what is there only: record by
+                // record, ten times as long, and only for tiles that have such rows.  (With a mask in the walk the forms of two
+                // lists per trip take 3 to 4 % longer: two batch elements of the encoder in float32 166 -> 171 us, 6 x 9675 queries
+                // of 32 samples in float16 378 -> 394.)
+                typedef float __attribute__((may_alias)) f32_alias;
+                f32_alias* sums = reinterpret_cast<f32_alias*>(ent);
+                static_assert(kTilePx * CH * sizeof(float) <= sizeof(ent), "a tile's sums fit the entry storage");
+                constexpr int kOwn = kTilePx / NW;
+                const int own0 = wave * kOwn, own1 = own0 + kOwn < npx ? own0 + kOwn : npx;
+                __syncthreads();  // (the handed-over sums are not needed)
+                for (int k = lane; k < kOwn * CH; k += kWave) sums[own0 * CH + k] = 0.0f;
+                wave_lds_sync();
+                for (int r = 0; r < item_runs && own0 < npx; ++r) {
+                    const uint32_t w = (uint32_t)(it.c0 + it.cstep * r) * a.run_step % (uint32_t)a.nwg;
+                    const uint32_t* row = tbl + (size_t)w * a.tbl_stride;
+                    const uint32_t first = row[0], n = row[1] - first;
+                    for (uint32_t i0 = 0; i0 < n; i0 += kWave) {
+                        const uint32_t i = i0 + lane;
+                        u32x3 rc = {0u, 0u, 0u};
+                        if (i < n) rc = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rres, (w * (uint32_t)a.rec_cap + first + i) * (kRecDwords * 4u), 0, 0));
+                        const uint32_t key = rc.x, ya = rc.y, za = rc.z;
+                        const int pl = (int)(key & (uint32_t)(kTilePx - 1));
+                        uint64_t mask = __ballot(i < n && pl < npx && (key >> kTilePxLog2) < (uint32_t)a.nq && pl + 1 >= own0 && pl < own1);
+                        while (mask) {
+                            const int from = __builtin_ctzll(mask);
+                            mask &= mask - 1;
+                            const uint32_t k = __builtin_amdgcn_readlane(key, from);
+                            const float wa = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ya, from));
+                            const float wb = __builtin_bit_cast(float, __builtin_amdgcn_readlane(za, from));
+                            const int p = (int)(k & (uint32_t)(kTilePx - 1));
+                            const T* grow = gout + ((int64_t)wk.b * a.nq + (k >> kTilePxLog2)) * row_pitch + (int64_t)wk.h * hd + cb;
+                            for (int c = lane; c < nch; c += kWave) {
+                                const float g = to_f32(grow[c]);
+                                if (p >= own0) sums[p * CH + c] = __builtin_fmaf(wa, g, sums[p * CH + c]);
+                                if (p + 1 < own1 && wb != 0.0f) sums[(p + 1) * CH + c] = __builtin_fmaf(wb, g, sums[(p + 1) * CH + c]);
+                            }
+                        }
+                    }
+                }
+                wave_lds_sync();
+                for (int k = lane; k < (own1 - own0) * CH; k += kWave) {
+                    const int px = own0 + k / CH, c = k % CH;
+                    if (c >= nch) continue;
+                    const int64_t at = (int64_t)(it.p0 + px) * row_pitch + (int64_t)wk.h * hd + cb + c;
+                    const float v = sums[px * CH + c];
+                    if (!owned || px == 0) unsafeAtomicAdd(gimg + at, v);
+                    else if (sizeof(T) == 2 && direct_t) static_cast<T*>(a.grad_value_t)[(size_t)wk.b * (a.gbatch_bytes / 4) + at] = from_f32<T>(v);
+                    else gimg[at] = t.accumulate ? gimg[at] + v : v;
+                }
+                clean_state();
+                continue;
+            }
             float cin[CHL];
 #pragma unroll
             for (int c = 0; c < CHL; ++c) cin[c] = __shfl_up(acc[PPG][c], LPG, kWave);
@@ -679,18 +756,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             }
             wave_lds_sync();
         }
-        if (cb + CH < hd) {
-            // next channel pass starts from a clean state (the dummy entry may have been
-            // overwritten by the transposition)
-            __syncthreads();
-            if (threadIdx.x == 0) done_count = 0;
-            // (opaque: the entry would otherwise be kept through the whole pass, in registers that some forms do not have -- and
-            //  memory for spilled ones costs every wavefront time before it starts)
-            uint32_t none = 0u;
-            asm volatile("" : "+v"(none));
-            if (lane == 0) ent_at(dummy) = u32x4{none | kInvalidCorner, none, none, none + dummy};
-            __syncthreads();
-        }
+        if (cb + CH < hd) clean_state();
     }
 }
 
