@@ -690,7 +690,17 @@ __global__ __launch_bounds__(256, DOTS ? 4 : 1) void dagg_gradf_kernel(const Dag
         for (int e = 0; e < VEC; ++e) acc[e] = nxt[e] = 0.0f;
         int cur = 0;         // pixel of the strip whose sums are in acc
         [[maybe_unused]] held_t here = {}, right = {};  // its value row, and its right neighbour's
+        uint32_t nan_px = 0; // pixels of the strip whose sums hold NaN
         auto flush = [&]() { // its row is complete
+            bool bad = false;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) bad |= acc[e] != acc[e];
+            if (__ballot(bad) != 0) {
+                if (bad) nan_px |= 1u << cur;
+                // (added below; a row that is stored whole is stored again)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) acc[e] = bad ? 0.0f : acc[e];
+            }
             const size_t row = ((size_t)b * a.nf + lv.base[l] + p0 + cur) * a.C + ch;
             if constexpr (DOTS) {
                 // to where its value row was, and from there with the strip's others: stores between the records' loads would be
@@ -839,6 +849,40 @@ __global__ __launch_bounds__(256, DOTS ? 4 : 1) void dagg_gradf_kernel(const Dag
             }
         }
         while (cur < p1 - p0) flush();
+        // A record's row is multiplied by both weights, also where there is no pixel to the right (or, for the records of the pixel
+        // before the strip, none to the left): an infinite row of grad_out leaves NaN there.  Sums that hold NaN are formed again from
+        // what there is, record by record.  (This costs the form with dots 346 -> 351 us at the size above; tests among the
+        // products, as branches or as selections, 364 to 390.)
+        if (__ballot(nan_px != 0) != 0) {
+            for (int i = 0; i < p1 - p0; ++i) {
+                if (((nan_px >> i) & 1u) == 0) continue;
+                float sum[VEC];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) sum[e] = 0.0f;
+                for (uint32_t k = lo; k < hi; ++k) {
+                    const u32x4 rc = rec[k];
+                    const int px = k < s1 ? -1 : (int)(rc.x & 7u);
+                    const uint32_t z = px == i ? rc.z : rc.w;
+                    if (px != i && (px + 1 != i || z << 1 == 0)) continue;
+                    float g[VEC];
+                    RowIO<T, VEC>::load_global(grow + (size_t)(rc.x >> 3) * a.C, g);
+                    const T* wk = w + (size_t)(rc.y & 0x7FFFFFFFu) * a.G;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        sum[e] = __builtin_fmaf(__builtin_bit_cast(float, z), g[e] * to_f32(wk[MIXED ? (ch + e) / a.hd - ch / a.hd : 0]), sum[e]);
+                }
+                const size_t row = ((size_t)b * a.nf + lv.base[l] + p0 + i) * a.C + ch;
+                if constexpr (DOTS) {
+                    __builtin_memcpy(&values[i * kWave + lane], sum, sizeof(sum));
+                } else if (chan_ok && direct) {
+                    RowIO<T, VEC>::store_global(static_cast<T*>(a.grad_feat) + row, sum);
+                } else if (chan_ok) {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e)
+                        if (ch + e >= chn) unsafeAtomicAdd(a.image + row + e, sum[e]);
+                }
+            }
+        }
         if constexpr (DOTS) {
             const size_t row0 = ((size_t)b * a.nf + lv.base[l] + p0) * a.C;
             if (direct) {

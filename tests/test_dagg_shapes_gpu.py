@@ -141,3 +141,51 @@ def test_a_level_that_starts_before_the_tensor_with_the_rows_dots(gpu_device):
     keep = ~_edge_mask(ss, loc)[..., None]
     for k, (g, r) in enumerate(zip(*_around(inp, gpu_device, 50, 10))):
         assert rel_err(*((g * keep, r * keep) if k == 2 else (g, r))) <= (FWD_FP32 if k == 0 else BWD_FP32), k
+
+
+def _whole_strips(C, G, seed):
+    """Samples enough for the dots in the order of the pixels, spread so evenly that most strips of 8 pixels have one wavefront (3 054 of
+    them, of up to 986 records if every location were inside), the last ones of a level partly filled; the levels of 17 pixels are split."""
+    inp = make_inputs(2, C, G, 884 * 256 // C, 31, [[(20, 25), (23, 22), (5, 101), (1, 17)]] * 6, seed=seed, pad=True)
+    loc = inp[3]
+    keep = np.array([0.3, 0.03, 0.03, 0.03, 0.01, 0.0])
+    loc[np.random.default_rng(1).random(loc.shape[:4]) >= keep] += 2.0
+    return inp
+
+
+@pytest.mark.parametrize("C,G", [(256, 8), (256, 1), (256, 64), (512, 16)])
+def test_dots_with_rows_that_are_stored_whole(gpu_device, C, G):
+    print(check(_whole_strips(C, G, C + G), gpu_device))
+
+
+@pytest.mark.parametrize("C,G,dtype", [(256, 8, torch.float32), (64, 8, torch.float32), (40, 8, torch.float32), (6, 2, torch.float32),
+                                       (512, 8, torch.float16), (256, 8, torch.bfloat16), (36, 2, torch.float16), ("dots", 8, torch.float32)])
+def test_an_infinite_gradient_stays_with_the_rows_it_reaches(gpu_device, C, G, dtype):
+    """Rows of the maps' gradient that samples of the anchor have as a corner, in the channels of the group; the pixel to the right of a
+    map's last column and the second pixel of the strip to the right of a sample do not."""
+    if C == "dots":
+        C, inp = 256, _whole_strips(256, G, 3)
+        feat, ss, ssi, loc, w, go = inp
+        loc[1, 5, :, :2] = np.random.default_rng(2).random(loc[1, 5, :, :2].shape)
+    else:
+        feat, ss, ssi, loc, w, go = make_inputs(2, C, G, 33, 9, [[(9, 13), (21, 24), (1, 1)]] * 2, seed=C, pad=True)
+    loc[1, 5, 0, 0], loc[1, 5, 1, 0] = 0.99, 0.01
+    feat, loc, w, go = (np.asarray(torch.from_numpy(t).to(dtype).float()) for t in (feat, loc, w, go))
+    hd = C // G
+    go[1, 5, :hd] = 0
+    want = dagg.direct_backward(feat, ss, ssi, loc, w, go)[0].reshape(2, -1, G, hd)
+    go[1, 5, :hd] = np.inf
+    hit = np.zeros(want.shape[:3], dtype=bool)
+    for cam in range(ss.shape[0]):
+        x, y = loc[1, 5, :, cam].astype(np.float64).T
+        ok = (x > 0) & (x < 1) & (y > 0) & (y < 1)
+        for sc in range(ss.shape[1]):
+            h, wd = ss[cam, sc]
+            x0, y0 = np.floor(x[ok] * wd - 0.5).astype(int), np.floor(y[ok] * h - 0.5).astype(int)
+            for yy, xx in ((y0, x0), (y0, x0 + 1), (y0 + 1, x0), (y0 + 1, x0 + 1)):
+                m = (yy >= 0) & (yy < h) & (xx >= 0) & (xx < wd)
+                hit[1, ssi[cam, sc] + (yy * wd + xx)[m], 0] = True
+    got = run_gpu(feat, ss, ssi, loc, w, go, gpu_device, dtype=dtype)[1].reshape(want.shape)
+    assert 0 < hit.sum() < hit[1, :, 0].size
+    assert np.array_equal(~np.isfinite(got).all(-1), hit) and not np.isfinite(got[hit]).any()
+    assert rel_err(got[~hit], want[~hit]) <= {torch.float32: BWD_FP32, torch.float16: 2e-3, torch.bfloat16: 2.0 ** -7}[dtype]
