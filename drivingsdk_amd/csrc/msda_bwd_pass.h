@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
                 if constexpr (kDot2) {
                     uint32_t words[kPairs];
                     __builtin_memcpy(words, &raw[k], sizeof(words));
-                    // (4 lanes: the sums of 8 lanes of 8 bytes, in their order)
+                    // (4 lanes: the sums of 8 lanes of 8 bytes, in their order, where pieces of 16 bytes divide the row)
                     constexpr int kPart = LPR == 4 ? kPairs / 2 : kPairs;
 #pragma unroll
                     for (int e = 0; e < kPart; ++e) dk = dot2_acc<T>(words[e], gpk[e], dk);

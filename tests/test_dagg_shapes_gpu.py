@@ -94,7 +94,8 @@ def test_levels_that_share_rows(gpu_device, cams, maps, starts, nf, C, G, A, P, 
 
 @pytest.mark.parametrize("C,G,shared", [(256, 8, False), (256, 1, False), (256, 64, False), (512, 16, False), (256, 8, True), (256, 4, "lost")])
 def test_dots_with_the_rows(gpu_device, C, G, shared):
-    """As many samples as have their dot products formed in the order of the pixels; most lie outside the images."""
+    """As many samples as have their dot products formed in the order of the pixels; most lie outside the images.  (Every strip is split
+    here, or its level overlaps others: its rows are added to zeros.)"""
     maps = [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6
     if shared == "lost":
         maps = [[(40, 61), (40, 61), (40, 61), (40, 60)]] * 6
