@@ -934,10 +934,14 @@ int dagg_plan(mxd::DaggArgs* a, int es, bool backward)
 // order of the pixels, so that every value row is read once, in order, in place of a gather of four rows per sample and group that
 // misses the L2 in two fifths of them.  In return the sort is no longer hidden behind that gather (43 us), and rows that few samples
 // touch are read whole.  6 x 900 anchors x 13 points, six cameras of four scales (538k pixels), 256 channels of float32: 320 + 224 +
-// 42 us for the three kernels, 43 + 344 + 50 with this.  Which is faster depends on the samples per pixel and on their number
-// (the backward's time that way over this way, locations inside a quarter of the cameras):
-//   (with a sort of 68 us)  3.1 a pixel: 2 / 3 / 4 / 5 / 6 batch elements 0.80 / 0.90 / 1.06 / 1.12 / 1.17, groups of 8 channels with 4 1.43;
-//   2.1 a pixel 0.95 with 6 batch elements, 1.6 0.85, 1.0 0.88 with 12; 12 a pixel 1.04; 512 channels: 2 / 4 batch elements 0.96 / 1.20.
+// 42 us for the three kernels, 43 + 351 + 50 with this.  Which is faster is a matter of that gather: a
+// wavefront of it per anchor and group costs as much as 40 locations and the locations that it looks at, times the 128-byte lines of
+// a group's row; where the maps fit the caches it takes half of that.  The backward's time that way over this way (256 channels in
+// groups of 32, two fifths of the locations inside):
+//   900 anchors x 13 points, maps of 92 MB: 1 / 2 / 3 / 4 / 6 batch elements (0.85 M each by that count) 0.82 / 0.91 / 1.18 / 1.27 / 1.36; groups
+//   of 8 channels (3.4 M) 1.01 / 1.38 / 1.56 / 1.69 / 1.81; 512 channels (1.7 M) 0.97 / 1.21 / 1.32 / 1.37 / 1.39; maps of 23 MB 0.77 / 1.01 / 0.98 /
+//   0.95 / 1.13; 600 anchors (0.57 M): 2 / 3 / 4 / 6 / 8 0.80 / 0.87 / 1.06 / 1.21 / 1.27; 300 (0.28 M): 4 / 6 / 8 / 12 0.85 / 0.95 / 1.02 / 1.02.
+// Over 473 problems of all sizes this line is 1.7 % from the faster way on average (never this way: 11 %, always: 7 %).
 // Rows of 128 channels, which units of less than a wavefront share, were at 0.87 .. 1.02, 16-bit rows at 0.71 .. 1.05: not for them.
 bool dagg_dots_with_rows(const mxd::DaggArgs& a, int es)
 {
@@ -945,7 +949,8 @@ bool dagg_dots_with_rows(const mxd::DaggArgs& a, int es)
     if (es != 4 || a.C % 256 != 0 || a.hd % 4 != 0 || lanes > mxd::kWave || (lanes & (lanes - 1)) != 0) return false;
     if (a.G > mxd::kWave || (a.G & (a.G - 1)) != 0) return false;
     const int64_t samples = (int64_t)a.A * a.P * a.nl;
-    return 4 * samples >= 11 * (int64_t)a.nf && a.bs * samples * (a.C / 256) >= (int64_t(5) << 18);
+    const int64_t gather = a.bs * (int64_t)a.A * a.G * (a.nloc + 40) * (a.hd > 32 ? a.hd / 32 : 1);
+    return samples >= a.nf && gather >= ((int64_t)a.bs * a.nf * a.C * 4 >= (int64_t(64) << 20) ? 2400000 : 4800000);
 }
 
 // Workspace of the backward: {weights' gradients per group, location gradients per group (or the samples' dot products), record starts, records, float32

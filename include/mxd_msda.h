@@ -241,7 +241,8 @@ int mxd_dagg_forward(const void* mc_ms_feat, const int32_t* spatial_shape, const
 
 /* Bytes of scratch mxd_dagg_backward needs (0 if the sizes are invalid): the hand-over between the two
  * backward kernels (records sorted by pixel and where each pixel's begin), the fp32 image of grad_mc_ms_feat for
- * 16-bit dtypes, and one float32 partial image of grad_sampling_location and of grad_weights per group. */
+ * 16-bit dtypes, and per group either one float32 partial image of grad_sampling_location and of grad_weights (4 bytes a
+ * sample and 8 a location) or, for large float32 problems, the samples' dot products (16 bytes a sample). */
 size_t mxd_dagg_backward_workspace_bytes(int dtype, int64_t bs, int64_t num_feat, int64_t num_embeds, int64_t num_cams,
                                          int64_t num_scale, int64_t num_anchors, int64_t num_pts, int64_t num_groups);
 

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from drivingsdk_amd import _lib
 from oracle import dagg_oracle as dagg
 from test_dagg_gpu import _edge_mask, check, make_inputs, run_gpu
 from util import BWD_FP32, FWD_FP32, rel_err
@@ -92,6 +93,16 @@ def test_levels_that_share_rows(gpu_device, cams, maps, starts, nf, C, G, A, P, 
         assert rel_err(g, r) <= tol, k
 
 
+def _dots_with_rows(inp):
+    """Whether the backward forms the dots in the order of the pixels: its workspace has room for them, 16 bytes per sample and group beside
+    32 bytes of records per sample."""
+    feat, ss, _, loc, w, _ = inp
+    (bs, nf, C), (cams, scales), (_, A, P), G = feat.shape, ss.shape[:2], loc.shape[:3], w.shape[-1]
+    samples = w.size // G
+    need = _lib.load().mxd_dagg_backward_workspace_bytes(0, bs, nf, C, cams, scales, A, P, G)
+    return need >= 32 * samples + 16 * G * samples
+
+
 @pytest.mark.parametrize("C,G,shared", [(256, 8, False), (256, 1, False), (256, 64, False), (512, 16, False), (256, 8, True), (256, 4, "lost")])
 def test_dots_with_the_rows(gpu_device, C, G, shared):
     """As many samples as have their dot products formed in the order of the pixels; most lie outside the images.  (Every strip is split
@@ -99,12 +110,13 @@ def test_dots_with_the_rows(gpu_device, C, G, shared):
     maps = [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6
     if shared == "lost":
         maps = [[(40, 61), (40, 61), (40, 61), (40, 60)]] * 6
-    A = 884 * 256 // C
+    A = 1440 * 256 // C
     feat, ss, ssi, loc, w, go = make_inputs(2, C, G, A, 31, maps, seed=C + G, pad=True)
     loc[np.random.default_rng(1).random(loc.shape[:3] + (6,)) < 0.97] += 2.0
     if shared:  # every camera names the same rows; "lost": more of them than the table of record starts has room for
         ssi = np.broadcast_to(np.array([0, 17, 5, 60], dtype=np.int32), (6, 4)).copy()
         feat = np.ascontiguousarray(feat[:, :2460 if shared == "lost" else 150])
+    assert _dots_with_rows((feat, ss, ssi, loc, w, go))
     print(check((feat, ss, ssi, loc, w, go), gpu_device))
 
 
@@ -134,23 +146,26 @@ def test_a_level_that_starts_before_the_tensor(gpu_device, C, G, dtype):
 
 def test_a_level_that_starts_before_the_tensor_with_the_rows_dots(gpu_device):
     """The same where the dot products are formed in the order of the pixels: a level without records has its own from elsewhere."""
-    feat, ss, _, loc, w, go = make_inputs(2, 256, 8, 884, 31, [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6, seed=7, pad=True)
+    feat, ss, _, loc, w, go = make_inputs(2, 256, 8, 1440, 31, [[(9, 13), (5, 7), (1, 17), (1, 1)]] * 6, seed=7, pad=True)
     loc[np.random.default_rng(1).random(loc.shape[:3] + (6,)) < 0.97] += 2.0
     ssi = np.cumsum(np.concatenate([[-50], ss.reshape(-1, 2).prod(1)[:-1]])).reshape(6, 4).astype(np.int32)
     ssi[3, 1] = -30
     inp = feat, ss, ssi, loc, w, go
+    assert _dots_with_rows(inp)
     keep = ~_edge_mask(ss, loc)[..., None]
     for k, (g, r) in enumerate(zip(*_around(inp, gpu_device, 50, 10))):
         assert rel_err(*((g * keep, r * keep) if k == 2 else (g, r))) <= (FWD_FP32 if k == 0 else BWD_FP32), k
 
 
 def _whole_strips(C, G, seed):
-    """Samples enough for the dots in the order of the pixels, spread so evenly that most strips of 8 pixels have one wavefront (3 054 of
-    them, of up to 986 records if every location were inside), the last ones of a level partly filled; the levels of 17 pixels are split."""
-    inp = make_inputs(2, C, G, 884 * 256 // C, 31, [[(20, 25), (23, 22), (5, 101), (1, 17)]] * 6, seed=seed, pad=True)
+    """Samples enough for the dots in the order of the pixels, spread so evenly that most strips of 8 pixels have one wavefront (4 200 of
+    them, of up to 884 records if every location were inside), the last ones of a level partly filled; the levels of 17
+    pixels are split."""
+    inp = make_inputs(2, C, G, 1440 * 256 // C, 31, [[(37, 25), (23, 40), (9, 101), (1, 17)]] * 6, seed=seed, pad=True)
     loc = inp[3]
     keep = np.array([0.3, 0.03, 0.03, 0.03, 0.01, 0.0])
     loc[np.random.default_rng(1).random(loc.shape[:4]) >= keep] += 2.0
+    assert _dots_with_rows(inp)
     return inp
 
 
