@@ -295,11 +295,9 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
             if (act) {
                 float ga = 0.f;
                 if (sm.valid) {
-                    const f32x4 dd = dots[lane];
-                    const float hw = 1.0f - sm.lw, hh = 1.0f - sm.lh;
-                    ga = sm.w[0] * dd[0] + sm.w[1] * dd[1] + sm.w[2] * dd[2] + sm.w[3] * dd[3];
-                    g.x = sm.Wf * aw * (hh * (dd[1] - dd[0]) + sm.lh * (dd[3] - dd[2]));
-                    g.y = sm.Hf * aw * (hw * (dd[2] - dd[0]) + sm.lw * (dd[3] - dd[1]));
+                    float gx, gy;
+                    sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, aw, dots[lane], ga, gx, gy);
+                    g = f32x2{gx, gy};
                 }
                 gw[(int)(fj >> 16) * a.scales + ts] = ga;
             }

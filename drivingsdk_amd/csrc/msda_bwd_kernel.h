@@ -267,12 +267,8 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                 // the records these samples will leave, merged exactly as where they are written
                 bool have[2], keep[2];
                 int32_t key[2];
-                float za[2] = {0.f, 0.f}, zb[2] = {0.f, 0.f};
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    have[r] = active && (sm.cvalid[2 * r] || sm.cvalid[2 * r + 1]) && tile_first[l] >= 0;
-                    key[r] = sm.cvalid[2 * r] ? sm.pix[2 * r] : sm.pix[2 * r + 1];
-                }
+                float za[2], zb[2];
+                pair_records(sm, 0.0f, active && tile_first[l] >= 0, have, key, za, zb);
                 merge_pair_records_in_quad(have, key, za, zb, keep);
 #pragma unroll
                 for (int r = 0; r < 2; ++r)
@@ -325,6 +321,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             Sample sm;
             sm.cvalid[0] = sm.cvalid[1] = sm.cvalid[2] = sm.cvalid[3] = false;
             sm.pix[0] = sm.pix[1] = sm.pix[2] = sm.pix[3] = 0;
+            sm.w[0] = sm.w[1] = sm.w[2] = sm.w[3] = 0.0f;
             if (act) {
                 const SampleRef sr = sample_ref<SRC>(a, wk.b, wk.q_begin + qr, wk.h, s);
                 l = sr.l;
@@ -336,34 +333,15 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             }
             bool have[2], keep[2];
             int32_t key[2];
-            float za[2] = {0.f, 0.f}, zb[2] = {0.f, 0.f};
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                have[r] = act && (sm.cvalid[2 * r] || sm.cvalid[2 * r + 1]) && tile_first[l] >= 0;
-                key[r] = sm.cvalid[2 * r] ? sm.pix[2 * r] : sm.pix[2 * r + 1];
-            }
+            float za[2], zb[2];
+            pair_records(sm, 0.0f, act && tile_first[l] >= 0, have, key, za, zb);
             merge_pair_records_in_quad(have, key, za, zb, keep);
 #pragma unroll
             for (int r = 0; r < 2; ++r)
                 if (keep[r]) atomicAdd(&cursor[tile_first[l] + ((key[r] - lvl[l].z) >> a.tile_px_log2)], 1);
         }
         __syncthreads();
-        if (wave == 0) {
-            // exclusive prefix over the counts, 64 at a time
-            int32_t carry = 0;
-            for (int base = 0; base < a.tbl_stride; base += kWave) {
-                const int i = base + lane;
-                const int32_t v = i < a.tbl_stride ? cursor[i] : 0;
-                int32_t inc = v;
-#pragma unroll
-                for (int d = 1; d < kWave; d <<= 1) {
-                    const int32_t o = __shfl_up(inc, d, kWave);
-                    if (lane >= d) inc += o;
-                }
-                if (i < a.tbl_stride) cursor[i] = carry + inc - v;
-                carry += __builtin_amdgcn_readlane(inc, kWave - 1);
-            }
-        }
+        if (wave == 0) scan_counters(cursor, a.tbl_stride, lane, [&](int i, int32_t start) { cursor[i] = start; });
         __syncthreads();
         uint32_t* row = a.tbl + wg_row * a.tbl_stride;
         for (int i = threadIdx.x; i < a.tbl_stride; i += blockDim.x) row[i] = (uint32_t)cursor[i];
@@ -406,7 +384,6 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
     // is small collects its records, 12 bytes each, in a buffer of its own behind the counters and writes the slab in
     // whole lines when it is done: a pass adds a few records to every run, and stored one by one those pieces -- the
     // shorter, the smaller the tiles of the grad_value pass are -- reach memory as partial lines.
-    typedef uint32_t __attribute__((may_alias)) u32_alias;
     u32_alias* recbuf = nullptr;
     if constexpr (RECBUF) {
         if (!rec_in_lds && a.rec_lds_bytes != 0)
@@ -612,42 +589,12 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                     float ga = 0.f, gx = 0.f, gy = 0.f;
                     if (sm.valid) sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, aw, dd, ga, gx, gy);
                     if constexpr (FUSED) {
-                        // chain rule through the softmax and through location = reference + offset * scale
                         gattn[sr.w_e] = from_f32<T>(aw * (ga - unit_stats(u)[2]));
-                        float r2 = 0.0f, r3 = 0.0f;  // boxes: gradient of (w, h)
-                        if (a.ref_dim == 2) {
-                            gloc[2 * sr.loc_e] = from_f32<T>(gx / (float)lvl[l].y);
-                            gloc[2 * sr.loc_e + 1] = from_f32<T>(gy / (float)lvl[l].x);
-                        } else {
-                            gloc[2 * sr.loc_e] = from_f32<T>(gx / (float)a.np * to_f32(rp[2]) * 0.5f);
-                            gloc[2 * sr.loc_e + 1] = from_f32<T>(gy / (float)a.np * to_f32(rp[3]) * 0.5f);
-                            r2 = gx * (ox / (float)a.np * 0.5f);
-                            r3 = gy * (oy / (float)a.np * 0.5f);
-                        }
+                        const f32x4 gr = offset_gradient(a, rp, sm.Wf, sm.Hf, gx, gy, gloc + 2 * sr.loc_e,
+                                                         [&](int k) { return k == 0 ? ox : oy; });
                         if (a.grad_ref != nullptr) {
-                            // the points of a level share the reference point: sum over them here, per head
-                            // into a float32 partial image that a small kernel adds up over the heads
-                            float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + q) * (a.nl * a.ref_dim) +
-                                          l * a.ref_dim;
-                            if (a.np_pow2) {
-                                for (int d = 1; d < a.np; d <<= 1) {
-                                    gx += __shfl_xor(gx, d, kWave);
-                                    gy += __shfl_xor(gy, d, kWave);
-                                    r2 += __shfl_xor(r2, d, kWave);
-                                    r3 += __shfl_xor(r3, d, kWave);
-                                }
-                                if ((s & (a.np - 1)) == 0) {
-                                    part[0] = gx;
-                                    part[1] = gy;
-                                    if (a.ref_dim == 4) {
-                                        part[2] = r2;
-                                        part[3] = r3;
-                                    }
-                                }
-                            } else {
-                                // (any other number of points: summed below, from the place of the dots)
-                                dots[u * kChunk + sl] = f32x4{gx, gy, r2, r3};
-                            }
+                            if (a.np_pow2) store_reference_sum(a, reference_part(a, wk.b, wk.h, q, l), s, gr);
+                            else dots[u * kChunk + sl] = gr;  // (any other number of points: summed below, from the place of the dots)
                         }
                     } else if constexpr (SRC != kSrcGrid) __builtin_nontemporal_store(from_f32<T>(ga), gattn + sr.w_e);
                     if constexpr (FUSED) {
@@ -704,7 +651,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
                         if (q >= wk.q_end || s0 >= s1) continue;
                         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
                         for (int s = s0; s < s1; ++s) sum += dots[((u << sp) + ((s - c0) >> 4)) * kChunk + ((s - c0) & (kChunk - 1))];
-                        float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + q) * (a.nl * a.ref_dim) + l * a.ref_dim;
+                        float* part = reference_part(a, wk.b, wk.h, q, l);
                         const bool whole = s0 == l0 && s1 == l1;  // (a level that lies in two chunks is added up in memory)
                         for (int k = 0; k < a.ref_dim; ++k) {
                             const float v = k == 0 ? sum[0] : k == 1 ? sum[1] : k == 2 ? sum[2] : sum[3];
@@ -721,30 +668,12 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
             }
         }
 
-        // slots of levels that attention_weights carries beyond spatial_shapes: zero gradients
-        const int extra = a.S_full - a.S;
-        if (extra > 0) {
-            for (int i = lane; i < (U >> sp) * extra; i += kWave) {
-                const int u = i / extra, s = a.S + i % extra, q = q0 + u;
-                if (q < wk.q_end) {
-                    const int64_t e = (((int64_t)wk.b * a.nq + q) * a.nh + wk.h) * a.S_full + s;
-                    gattn[e] = from_f32<T>(0.f);
-                    gloc[2 * e] = from_f32<T>(0.f);
-                    gloc[2 * e + 1] = from_f32<T>(0.f);
-                }
-            }
-        }
+        zero_extra_slots<T>(a, wk.b, wk.h, q0, wk.q_end, U >> sp, lane, gattn, gloc);
     }
     if constexpr (RECBUF) {
         if (recbuf != nullptr) {  // (uniform over the workgroup; every wavefront leaves the loop above)
             __syncthreads();
-            // the slab as it lies in the buffer: 16 bytes per lane, then the odd words
-            const int words = 3 * cursor[a.tbl_stride - 1], quads = words >> 2;
-            for (int i = threadIdx.x; i < quads; i += blockDim.x)
-                __builtin_amdgcn_raw_buffer_store_b128(u32x4{recbuf[4 * i], recbuf[4 * i + 1], recbuf[4 * i + 2], recbuf[4 * i + 3]}, sres,
-                                                       (uint32_t)i * 16u, 0, 2);
-            for (int i = 4 * quads + threadIdx.x; i < words; i += blockDim.x)
-                __builtin_amdgcn_raw_buffer_store_b32(recbuf[i], sres, (uint32_t)i * 4u, 0, 2);
+            store_slab(recbuf, kRecDwords * cursor[a.tbl_stride - 1], sres, (int)threadIdx.x, (int)blockDim.x);
         }
     }
 }

@@ -19,7 +19,7 @@
 #pragma once
 #include <type_traits>
 
-#include "msda_device.h"
+#include "msda_bwd_parts.h"
 
 namespace mxd {
 
@@ -47,7 +47,6 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
     constexpr bool OVER = LPR == 4;  // strips in the records' place
     static_assert(kChunkStride * 4 <= kPassRecWords, "strips fit the records' place");
     typedef typename RowIO<T, VEC>::raw_t raw_t;
-    typedef uint32_t __attribute__((may_alias)) u32_alias;
 
     extern __shared__ __align__(16) unsigned char smem[];
     {
@@ -204,14 +203,7 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         bool have[2], keep[2];
         int32_t key[2];
         float wa[2], wb[2];
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const bool vl = sm.cvalid[2 * r], vr = sm.cvalid[2 * r + 1];
-            have[r] = p.active && (vl || vr) && L.w >= 0;
-            key[r] = vl ? sm.pix[2 * r] : sm.pix[2 * r + 1];
-            wa[r] = (vl ? sm.w[2 * r] : sm.w[2 * r + 1]) * aw[k];
-            wb[r] = (vl && vr) ? sm.w[2 * r + 1] * aw[k] : 0.0f;
-        }
+        pair_records(sm, aw[k], p.active && L.w >= 0, have, key, wa, wb);
         merge_pair_records_in_quad<true>(have, key, wa, wb, keep);
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
@@ -242,24 +234,11 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         total = __builtin_amdgcn_readlane(inc, a.tbl_stride - 1);  // (the entry behind the last tile counts nothing)
         if (wave == 0 && lane < a.tbl_stride) tbl[lane] = (uint32_t)starts;
     } else {
-        if (wave == 0) {
-            int32_t carry = 0;
-            for (int base = 0; base < a.tbl_stride; base += kWave) {
-                const int i = base + lane;
-                const int32_t v = i < a.tbl_stride ? cursor[i] : 0;
-                int32_t inc = v;
-#pragma unroll
-                for (int d = 1; d < kWave; d <<= 1) {
-                    const int32_t o = __shfl_up(inc, d, kWave);
-                    if (lane >= d) inc += o;
-                }
-                if (i < a.tbl_stride) {
-                    cursor[i] = carry + inc - v;
-                    tbl[i] = (uint32_t)(carry + inc - v);
-                }
-                carry += __builtin_amdgcn_readlane(inc, kWave - 1);
-            }
-        }
+        if (wave == 0)
+            scan_counters(cursor, a.tbl_stride, lane, [&](int i, int32_t start) {
+                cursor[i] = start;
+                tbl[i] = (uint32_t)start;
+            });
         __syncthreads();
         total = cursor[a.tbl_stride - 1];  // (no record has this number: the entry behind the last tile holds the sum)
     }
@@ -278,15 +257,8 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         }
     __syncthreads();  // the records are whole (and nobody reads the counters any more)
     {
-        // the slab as it lies in LDS: 16 bytes per lane, then the odd words.  (Non-temporal: the records are read by the next
-        // kernel and should not push value rows out of L2)
         const __amdgpu_buffer_rsrc_t sres = make_rsrc(a.rec + wg_row * a.rec_cap * kRecDwords, (uint32_t)a.rec_cap * (kRecDwords * 4u));
-        const int words = kRecDwords * total, quads = words >> 2;
-        for (int i = tid; i < quads; i += kThreads)
-            __builtin_amdgcn_raw_buffer_store_b128(u32x4{recs[4 * i], recs[4 * i + 1], recs[4 * i + 2], recs[4 * i + 3]}, sres, (uint32_t)i * 16u,
-                                                   0, 2);
-        const int i = 4 * quads + tid;
-        if (i < words) __builtin_amdgcn_raw_buffer_store_b32(recs[i], sres, (uint32_t)i * 4u, 0, 2);
+        store_slab(recs, kRecDwords * total, sres, tid, kThreads);
     }
     if constexpr (OVER) {
         __syncthreads();  // the slab is on its way
@@ -384,42 +356,13 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         T* la = gattn + e0;
         T* ll = gloc + 2 * e0;
         if constexpr (FUSED) {
-            // chain rule through the softmax and through location = reference + offset * scale
-            const T* rp = ref + ((bq + p.q) * a.nl + l) * a.ref_dim;
+            const T* off = static_cast<const T*>(a.loc) + 2 * e0;
             la[p.e] = from_f32<T>(aw[k] * (ga - stats[4 * p.u + 2]));
-            float r2 = 0.0f, r3 = 0.0f;  // boxes: gradient of (w, h)
-            if (a.ref_dim == 2) {
-                ll[2 * p.e] = from_f32<T>(gx / Wf);
-                ll[2 * p.e + 1] = from_f32<T>(gy / Hf);
-            } else {
-                ll[2 * p.e] = from_f32<T>(gx / (float)a.np * to_f32(rp[2]) * 0.5f);
-                ll[2 * p.e + 1] = from_f32<T>(gy / (float)a.np * to_f32(rp[3]) * 0.5f);
-                r2 = gx * (to_f32((static_cast<const T*>(a.loc) + 2 * e0)[2 * p.e]) / (float)a.np * 0.5f);
-                r3 = gy * (to_f32((static_cast<const T*>(a.loc) + 2 * e0)[2 * p.e + 1]) / (float)a.np * 0.5f);
-            }
+            const f32x4 gr = offset_gradient(a, ref + ((bq + p.q) * a.nl + l) * a.ref_dim, Wf, Hf, gx, gy, ll + 2 * p.e,
+                                             [&](int j) { return to_f32(off[2 * p.e + j]); });
             if (a.grad_ref != nullptr) {
-                // the points of a level share the reference point: sum over them here, per head
-                // into a float32 partial image that a small kernel adds up over the heads
-                float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + p.q) * (a.nl * a.ref_dim) + l * a.ref_dim;
-                if (a.np_pow2) {
-                    for (int d = 1; d < a.np; d <<= 1) {
-                        gx += __shfl_xor(gx, d, kWave);
-                        gy += __shfl_xor(gy, d, kWave);
-                        r2 += __shfl_xor(r2, d, kWave);
-                        r3 += __shfl_xor(r3, d, kWave);
-                    }
-                    if ((p.sn & (a.np - 1)) == 0) {
-                        part[0] = gx;
-                        part[1] = gy;
-                        if (a.ref_dim == 4) {
-                            part[2] = r2;
-                            part[3] = r3;
-                        }
-                    }
-                } else {
-                    // (any other number of points: summed below, from the place of the dots)
-                    strip[p.u * kChunkStride + p.sn] = __builtin_bit_cast(u32x4, f32x4{gx, gy, r2, r3});
-                }
+                if (a.np_pow2) store_reference_sum(a, reference_part(a, wk.b, wk.h, p.q, l), p.sn, gr);
+                else strip[p.u * kChunkStride + p.sn] = __builtin_bit_cast(u32x4, gr);  // (any other number of points: summed below, from the place of the dots)
             }
         } else {
             // (streamed out like the records)
@@ -437,7 +380,7 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
                 if (q >= wk.q_end) continue;
                 f32x4 sum = {0.f, 0.f, 0.f, 0.f};
                 for (int t = 0; t < a.np; ++t) sum += __builtin_bit_cast(f32x4, strip[u * kChunkStride + l * a.np + t]);
-                float* part = a.grad_ref + (((int64_t)wk.h * a.bs + wk.b) * a.nq + q) * (a.nl * a.ref_dim) + l * a.ref_dim;
+                float* part = reference_part(a, wk.b, wk.h, q, l);
                 part[0] = sum[0];
                 part[1] = sum[1];
                 if (a.ref_dim == 4) {
@@ -448,19 +391,7 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         }
     }
 
-    // slots of levels that attention_weights carries beyond spatial_shapes: zero gradients
-    const int extra = a.S_full - a.S;
-    if (extra > 0) {
-        for (int i = lane; i < (U >> SP) * extra; i += kWave) {
-            const int u = i / extra, q = q0 + u;
-            if (q < wk.q_end) {
-                const int64_t e = ((bq + q) * a.nh + wk.h) * a.S_full + a.S + i % extra;
-                gattn[e] = from_f32<T>(0.f);
-                gloc[2 * e] = from_f32<T>(0.f);
-                gloc[2 * e + 1] = from_f32<T>(0.f);
-            }
-        }
-    }
+    zero_extra_slots<T>(a, wk.b, wk.h, q0, wk.q_end, U >> SP, lane, gattn, gloc);
 }
 
 }  // namespace mxd
