@@ -21,9 +21,10 @@
 //     the grad_out rows of its records -- those of a batch element stay in L2 -- and stored once, whole.
 //
 // Measured (6 x 900 anchors x 13 points, 6 cameras x 4 scales, 256 channels in 8 groups, float32), one unit of lanes per anchor and
-// group and the tile pass -> these: forward 395 -> 270 us (float16, one batch element 140 -> 25), forward and backward 1969 ->
-// 855.  Of the 585 us of the backward the dots with the sort beside them take 318, the gradient of the maps 221, the caller's
-// layouts 40 (kernel times one at a time; rows from HBM bound all but the last).
+// group and the tile pass -> these: forward 395 -> 270 us (float16, one batch element 140 -> 25), forward and backward 1969 -> 855
+// with the dots formed by the anchors' wavefronts -- 318 us with the sort beside them, the gradient of the maps 221, the caller's
+// layouts 40 -- and 700 with the dots formed beside the maps' gradient: sort 43, rows and dots 351, layouts 51 (kernel times one at
+// a time; rows from HBM bound all but the sort and the layouts).
 #include "dagg.h"
 
 namespace mxd {
@@ -626,7 +627,7 @@ __device__ inline void dagg_levels_without_room(const DaggArgs& a, const DaggLev
 // DOTS: forms the samples' dot products with the value rows too.  A record stands for two neighbouring pixels, whose value rows are in
 // registers while the strip is at the first of them; a strip's rows and the one behind them go to LDS with the first records'
 // requests, so that no trip to memory is added, and a record's dots are stored by one lane per group, each taking another record of
-// the batch.  Bound by latency, with 16 wavefronts per CU for their LDS and registers (6 x 900 anchors, 256 channels: 344 us, of
+// the batch.  Bound by latency, with 16 wavefronts per CU for their LDS and registers (6 x 900 anchors, 256 channels: 351 us, of
 // which the value rows are 60 and the dots' stores 15; 1.1 GB of rows in and out).  Samples that are shared between strips have their
 // dots from the strip of the first pixel.
 template <typename T, int VEC, bool MIXED, bool WAVE, bool DOTS>

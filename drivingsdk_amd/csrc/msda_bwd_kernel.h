@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void msda_bwd_kernel(const KArgs a)
         // this workgroup's share of the zero-fill of the image (every workgroup of the launch takes one, also those
         // without work): the stores ride along with this kernel instead of taking a launch of their own
         const LevelLanes lv(a, (int)threadIdx.x & (kWave - 1));
-        // the levels and their first tiles (-1: a level that does not fit the run table is left out of grad_value)
+        // the levels and their first tiles (-1: a level without tiles in the run table leaves no records)
         if ((int)threadIdx.x < a.nl) {
             lvl[threadIdx.x] = lv.geo;
             tile_first[threadIdx.x] = lv.first;

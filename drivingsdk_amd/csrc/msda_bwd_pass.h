@@ -9,8 +9,9 @@
 //     to memory;
 //   * run starts are a scan that every wavefront makes for itself (up to 64 tiles): three barriers per slab;
 //   * the dots replace the row offsets that they were gathered by, in place;
-//   * rows of 33 to 64 bytes are read by 4 lanes of 16 bytes (where there are enough of them: launch_pass): a row of 64 bytes costs the L1 a line of 128 however it is read, but half
-//     of the instructions of 8 lanes of 8 bytes (181 -> 117 million at the second shape below).
+//   * rows of 33 to 64 bytes are read by 4 lanes of 16 bytes (where there are enough of them: launch_pass): a row of 64 bytes costs the
+//     L1 a line of 128 however it is read, but half of the instructions of 8 lanes of 8 bytes (181 -> 117 million at the last shape
+//     below).
 // Measured, this kernel against the instantiations of the general one that it replaces (two batch elements of the encoder in float32 /
 // the same in bfloat16, fused / 6 x 9675 queries of 32 samples over 30 825 keys in float16): 142 -> 132, 185 -> 132, 399 -> 379 us.
 // A workgroup goes through one slab: with a loop over several, shared out evenly, the last case took 430 to 490 us (values kept across
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
     const int tid = (int)threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    i32x4* lvl = reinterpret_cast<i32x4*>(smem);  // {H, W, first key, first tile (-1: no room in the run table)}
+    i32x4* lvl = reinterpret_cast<i32x4*>(smem);  // {H, W, first key, first tile (-1: none in the run table)}
     float* stats = reinterpret_cast<float*>(smem + (size_t)a.nl * sizeof(i32x4));  // fused form: per unit {max logit, sum of exponentials, D}
     u32x4* strips = reinterpret_cast<u32x4*>(stats + (FUSED ? 4 * kPassUnits : 0));
     u32_alias* recs = reinterpret_cast<u32_alias*>(strips + (OVER ? 0 : kPassUnits * kChunkStride));

@@ -461,7 +461,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 first_round = false;
             }
 
-            // ---- every group of 8 lanes walks the lists of its PPG pixels ----------------------
+            // ---- every group of LPG lanes walks the lists of its PPG pixels --------------------
             // The lanes of a group read a block of a grad_out row with ONE coalesced load.
             // The loop body is branch-free: a list that has ended keeps "reading" the dummy entry.
             // kWalk lists are walked together, one entry of each per trip, and two trips are in flight.

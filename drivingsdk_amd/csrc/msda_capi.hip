@@ -399,7 +399,7 @@ BwdLayout bwd_layout_for(int dtype, const Dims& d, int tile_px_log2, bool early_
     L.nwg = (d.nq + L.tile_q - 1) / L.tile_q;
     L.rec_cap = 2 * L.tile_q * d.nl * d.np;
     // tiles per (batch, head) when the levels do not overlap: sum of ceil(pixels / tile) <= nk / tile + nl
-    // (the kernels leave out levels that would not fit, which can only happen for overlapping levels)
+    // (levels that would not fit, which can only happen for overlapping ones, leave no records: add_levels_without_tiles)
     L.tbl_stride = (d.nk >> tile_px_log2) + d.nl + 1;
     const int64_t tbl = d.bs * d.nh * L.nwg * L.tbl_stride * 4;
     // dynamic LDS of the first kernel with the most units per wavefront the row can have (16-byte aligned pointers)

@@ -35,8 +35,9 @@ constexpr int kCuWaves = 16;         // wavefronts of its workgroups
 constexpr int kCuTableBytes = 2 * (kMaxLevels + 1) * 16 + 32;  // its two level tables ahead of the cached rows (multiple of 64)
 
 constexpr int kTileThreads = 512;    // threads of the workgroups of the grad_value pass
-// Pixels per tile of the grad_value pass: every thread of a workgroup keeps 32 sums (16-bit rows of whole 16-byte pieces: 64, at
-// half the lanes per row), so a workgroup holds 512 pixels of up to 32 channels, 256 of up to 64 or 128 of up to 128 (heads of more channels take two passes over 128-pixel tiles).
+// Pixels per tile of the grad_value pass: every thread of a workgroup keeps 32 sums (and those of the pixel behind its last one), so a
+// workgroup holds 512 pixels of up to 32 channels, 256 of up to 64 or 128 of up to 128 (heads of more channels take two passes
+// over 128-pixel tiles).
 // The launcher picks the size from head_dim (KArgs::tile_px_log2: 9, 8 or 7); the first backward kernel sorts its
 // records by tiles of that size.
 constexpr int kTilePxLog2Max = 9;
