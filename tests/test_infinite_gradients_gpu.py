@@ -22,7 +22,8 @@ def _touched(maps, starts, nk, loc):
 
 
 @pytest.mark.parametrize("dtype,hd", [(torch.float32, 9), (torch.float32, 32), (torch.float32, 50), (torch.float32, 128), (torch.float16, 2),
-                                      (torch.float16, 32), (torch.float16, 36), (torch.float16, 64), (torch.bfloat16, 100), (torch.bfloat16, 128)])
+                                      (torch.float16, 32), (torch.float16, 36), (torch.float16, 64), (torch.bfloat16, 100), (torch.bfloat16, 128),
+                                      (torch.float32, 130), (torch.float16, 136)])
 @pytest.mark.parametrize("maps,nq", [(((1, 505), (3, 2)), 40), (((21, 24), (8, 16), (1, 1)), 300), (((60, 1), (27, 19)), 40), (((5, 6), (1, 9)), 2500)])
 def test_gradient_of_the_maps(gpu_device, maps, nq, dtype, hd):
     g = torch.Generator().manual_seed(hd + nq)
