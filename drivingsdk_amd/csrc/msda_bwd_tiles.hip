@@ -28,9 +28,8 @@
 //     read-modify-write of shared accumulators.  The walk is pipelined by hand: the entries and
 //     rows of the next trip are requested before the rows of the current trip are used.
 //   * At the end plain 16-byte stores for tiles a single workgroup owns; tiles of hot (coarse)
-//     levels are split over several workgroups by query range and tiles much smaller than the
-//     workgroup are held in several copies: those pass their registers through LDS and add
-//     whole rows with a few atomics per workgroup.
+//     levels are split over several workgroups by query range, which add their rows with atomics.
+//     Tiles much smaller than the workgroup are held in several copies, which are added up in LDS.
 //   * Slots of the workgroup that stand for no pixel take extra lists of pixels that collect
 //     far more entries than the others (decided from the counts of a work item's first round),
 //     so that a hot pixel's entries are walked by several lane groups side by side.
@@ -160,14 +159,11 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     constexpr int kCarryAt = kTileEntCap - 1 - LPG * CHL / 4;  // entries of a wavefront's storage through which its last group hands over
     constexpr int NW = kTileThreads / kWave;            // wavefronts per workgroup
     constexpr uint32_t kDummyOfWave = kTileEntCap - 1;  // last entry slot of every wavefront
-    // (a wavefront transposes the sums of half of its lane groups at a time: 1024 sums, 4 KiB)
-    constexpr int HG = GPW / 2;
-    constexpr int kSlotPxAt = HG * PPG * CH / 4;        // first entry behind wavefront 0's transposition scratch
-    static_assert(kSlotPxAt + kTileThreads * 2 / 16 <= kCarryAt, "slot map must fit wavefront 0's entry storage");
     __shared__ uint32_t heads[kTileThreads];            // list head per pixel slot (byte offset of the entry in `ent`)
     // entry: {byte offset of the grad_out row, weight for the list's pixel, weight for the
     // next pixel, next entry of the same list}
     __shared__ u32x4 ent[NW * kTileEntCap];
+    static_assert(kTilePx * CH * sizeof(float) <= sizeof(ent), "a tile's sums fit the entry storage");
     // up to 64 runs of records per wavefront at a time: first record, records before the run
     __shared__ uint32_t run_src_all[NW * kWave];
     __shared__ uint32_t run_pre_all[NW * kWave];
@@ -216,17 +212,16 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int npx = it.p1 - it.p0;
     // A tile much smaller than the workgroup is held in several copies (lists and registers),
-    // each taking the samples of some queries; the copies meet in the image through atomics.
+    // each taking the samples of some queries; the copies are added up at the end.
     const int npx_pad = (npx + PPG - 1) / PPG * PPG;
     int copies = 1;
     while (copies < 8 && 2 * copies * npx_pad <= kTilePx) copies *= 2;
-    const bool owned = it.exclusive && copies == 1;  // plain stores are enough
+    const bool owned = it.exclusive != 0;            // plain stores are enough (this is what tile_stored_directly() says of the tile)
     const int copies_log2 = __builtin_ctz(copies);
     const int nused = copies * npx_pad;              // slots that stand for a pixel of the tile
     const int nspare = kTilePx - nused;              // slots free for extra lists
     const bool can_split = nspare >= tile_group_px(kTilePxLog2);
-    // (owned && !can_split is what tile_stored_directly() says of this tile)
-    const bool direct_t = a.sparse != 0 && a.grad_value_t != nullptr && owned && !can_split;
+    const bool direct_t = a.sparse != 0 && a.grad_value_t != nullptr && owned;
     typedef uint16_t __attribute__((may_alias)) u16_alias;  // halves of LDS words that are also accessed whole
     u16_alias* slot_info16 = reinterpret_cast<u16_alias*>(slot_info);
     bool first_round = true;                         // (of the first channel pass)
@@ -578,7 +573,6 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 // of 32 samples in float16 378 -> 394.)
                 typedef float __attribute__((may_alias)) f32_alias;
                 f32_alias* sums = reinterpret_cast<f32_alias*>(ent);
-                static_assert(kTilePx * CH * sizeof(float) <= sizeof(ent), "a tile's sums fit the entry storage");
                 constexpr int kOwn = kTilePx / NW;
                 const int own0 = wave * kOwn, own1 = own0 + kOwn < npx ? own0 + kOwn : npx;
                 __syncthreads();  // (the handed-over sums are not needed)
@@ -662,21 +656,40 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
         // occupying registers during the rounds)
         int grp_w = grp, lane_w = lane;
         asm volatile("" : "+v"(grp_w), "+v"(lane_w));
-        // extra lists were handed out: their slots add to their pixels' rows through the atomics below; the map
-        // from extra slot to pixel goes into wavefront 0's entry storage, behind its transposition scratch
-        const bool split = spare_next != 0;  // (uniform; written before the barrier that ended the first round)
-        u16_alias* slot_px = reinterpret_cast<u16_alias*>(&ent[kSlotPxAt]);
-        if (split) {
-            slot_px[tid] = 0xFFFFu;
-            __syncthreads();
-            if (tid < nused) {
-                const uint32_t o = slot_info16[tid];
-                for (uint32_t r = 0; r < (o >> 9); ++r)
-                    if ((o & 511u) + r < (uint32_t)nspare) slot_px[(o & 511u) + r] = (uint16_t)(tid - (tid / npx_pad) * npx_pad);
+        const bool split = __builtin_amdgcn_readfirstlane((int)spare_next) != 0;  // extra lists were handed out
+        // A row of the image, in four-byte steps of the caller's channel, and what becomes of four sums of it.
+        auto put = [&](int px, int ch, f32x4 v) {
+            float* dst = gimg + (int64_t)(it.p0 + px) * row_pitch + (int64_t)wk.h * hd + ch;
+            if (px == 0) {
+                // the first pixel of a tile also receives, through atomics, the right
+                // halves of pairs that start on the last pixel of the previous tile
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (ch + c < hd) unsafeAtomicAdd(dst + c, v[c]);
+            } else if (sizeof(T) == 2 && direct_t) {
+                // 16-bit dtypes: nobody else adds to this row, so it goes to the caller's tensor at once
+                // (the fp32 image keeps only the rows that receive atomic additions)
+                typedef T t4 __attribute__((ext_vector_type(4)));
+                const t4 r = {from_f32<T>(v[0]), from_f32<T>(v[1]), from_f32<T>(v[2]), from_f32<T>(v[3])};
+                __builtin_nontemporal_store(r, reinterpret_cast<t4*>(static_cast<T*>(a.grad_value_t) + (size_t)wk.b * (a.gbatch_bytes / 4) +
+                                                                     (dst - gimg)));
+            } else if (t.store_vec == 4) {
+                if (t.accumulate) v += *reinterpret_cast<f32x4*>(dst);
+                // (non-temporal: nothing reads these rows again before the kernel ends; backward 283.8 ->
+                //  281.3 us at the encoder shape)
+                __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(dst));
+            } else {
+                typedef f32x4 __attribute__((aligned(4))) any4;  // (rows start anywhere)
+                if (t.accumulate) {
+                    for (int c = 0; c < 4 && ch + c < hd; ++c) dst[c] += v[c];
+                } else if (ch + 4 <= hd) {
+                    *reinterpret_cast<any4*>(dst) = v;
+                } else {
+                    for (int c = 0; c < 4 && ch + c < hd; ++c) dst[c] = v[c];
+                }
             }
-            __syncthreads();
-        }
-        if (owned && !split && t.store_vec == 4) {
+        };
+        if (owned && copies == 1 && !split && t.store_vec == 4) {
             // the lanes of a group hold a whole row of each of their pixels: 16-byte stores
 #pragma unroll
             for (int c4 = 0; c4 < CHL; c4 += 4) {
@@ -685,76 +698,60 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
 #pragma unroll
                 for (int i = 0; i < PPG; ++i) {
                     const int px = grp_w * PPG + i;
-                    if (px < npx) {
-                        f32x4* dst = reinterpret_cast<f32x4*>(gimg + (int64_t)(it.p0 + px) * row_pitch +
-                                                              (int64_t)wk.h * hd + ch_w);
-                        f32x4 v = {acc[i][c4], acc[i][c4 + 1], acc[i][c4 + 2], acc[i][c4 + 3]};
-                        if (px == 0) {
-                            // the first pixel of a tile also receives, through atomics, the right
-                            // halves of pairs that start on the last pixel of the previous tile
-                            float* d1 = reinterpret_cast<float*>(dst);
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) unsafeAtomicAdd(d1 + c, v[c]);
-                        } else if (sizeof(T) == 2 && direct_t) {
-                            // 16-bit dtypes: nobody else adds to this row, so it goes to the caller's tensor at once
-                            // (the fp32 image keeps only the rows that receive atomic additions)
-                            typedef T t4 __attribute__((ext_vector_type(4)));
-                            const t4 r = {from_f32<T>(v[0]), from_f32<T>(v[1]), from_f32<T>(v[2]), from_f32<T>(v[3])};
-                            __builtin_nontemporal_store(r, reinterpret_cast<t4*>(static_cast<T*>(a.grad_value_t) +
-                                                                                 (size_t)wk.b * (a.gbatch_bytes / 4) +
-                                                                                 (int64_t)(it.p0 + px) * row_pitch +
-                                                                                 (int64_t)wk.h * hd + ch_w));
-                        } else {
-                            if (t.accumulate) v += *dst;
-                            // (non-temporal: nothing reads these rows again before the kernel ends; backward 283.8 ->
-                            //  281.3 us at the encoder shape)
-                            __builtin_nontemporal_store(v, dst);
-                        }
-                    }
+                    if (px < npx) put(px, ch_w, f32x4{acc[i][c4], acc[i][c4 + 1], acc[i][c4 + 2], acc[i][c4 + 3]});
                 }
             }
         } else {
-            // Rows shared with other workgroups (tiles split by query range) are added with
-            // atomics, which the memory side carries out per 64-byte request: pass the registers
-            // through LDS (the entry storage, free after the last round) so that consecutive
-            // lanes hold consecutive floats of a row.  Half of the wavefront's lane groups (1024 sums) at a time.
-            typedef uint32_t __attribute__((may_alias)) u32_alias;
-            u32x4* tr4 = &ent[seg];
-            const u32_alias* tr1 = reinterpret_cast<const u32_alias*>(tr4);
-            for (int half = 0; half < 2; ++half) {
-                wave_lds_sync();
-                if ((lane_w / LPG) / HG == half) {
-                    const int gl = (lane_w / LPG) % HG;
+            // Through LDS (the entry storage, free after the last round): the copies of a small tile and the extra lists of
+            // hot pixels are added up there, so that a tile that no other workgroup touches is stored like any other and one
+            // that several share costs one atomic addition per row and not one per copy.  (Atomics are what the write-out waits for, 64
+            // bytes in some 22 clocks of a CU: with one per copy a tile of 152 pixels in two took 9.5 of its item's 19 us, the last of the
+            // launch -- 2 x 900 queries of 16 samples in float32 31.6 -> 25.8 us.)  They are carried out per 64-byte request, so
+            // consecutive lanes hold consecutive floats there.
+            typedef f32x4 __attribute__((may_alias)) f32x4_alias;
+            typedef float __attribute__((may_alias)) f32_alias;
+            f32x4_alias* sums4 = reinterpret_cast<f32x4_alias*>(ent);
+            const f32_alias* sums1 = reinterpret_cast<const f32_alias*>(ent);
+            constexpr int QR = CH / 4;  // quads of a row
+            __syncthreads();            // (the sums handed over have been read)
 #pragma unroll
-                    for (int i = 0; i < PPG; ++i)
+            for (int i = 0; i < PPG; ++i)
 #pragma unroll
-                        for (int c4 = 0; c4 < CHL; c4 += 4)
-                            tr4[(gl * PPG + i) * (CH / 4) + (CB * (c4 / PIECE) + c4 % PIECE + PIECE * j) / 4] =
-                                u32x4{__builtin_bit_cast(uint32_t, acc[i][c4]), __builtin_bit_cast(uint32_t, acc[i][c4 + 1]),
-                                      __builtin_bit_cast(uint32_t, acc[i][c4 + 2]), __builtin_bit_cast(uint32_t, acc[i][c4 + 3])};
-                }
-                wave_lds_sync();
-                const int px_base = wave * (GPW * PPG) + half * (HG * PPG);
-#pragma unroll 4
-                for (int k = 0; k < HG * PPG * CH / kWave; ++k) {
-                    const int idx = k * kWave + lane_w;
-                    const int pl = idx / CH, c = idx % CH;
-                    const int vp = px_base + pl;             // pixel slot of the workgroup
-                    int px = vp - (vp / npx_pad) * npx_pad;  // pixel of the tile (any copy)
-                    if (vp >= nused) px = split ? (int)slot_px[vp - nused] : npx;  // (0xFFFF: slot without a pixel)
-                    if (px < npx && c < nch) {
-                        const float v = __builtin_bit_cast(float, (uint32_t)tr1[idx]);
-                        float* dst = gimg + (int64_t)(it.p0 + px) * row_pitch + (int64_t)wk.h * hd + cb + c;
-                        if (!owned || split || px == 0)
-                            unsafeAtomicAdd(dst, v);
-                        else if (t.accumulate)
-                            *dst += v;
-                        else
-                            __builtin_nontemporal_store(v, dst);
+                for (int c4 = 0; c4 < CHL; c4 += 4)
+                    sums4[(grp_w * PPG + i) * QR + (CB * (c4 / PIECE) + c4 % PIECE + PIECE * j) / 4] =
+                        f32x4{acc[i][c4], acc[i][c4 + 1], acc[i][c4 + 2], acc[i][c4 + 3]};
+            __syncthreads();
+            const int tid_w = wave * kWave + lane_w;
+            // every slot that stands for pixel px of the tile
+            auto each_slot = [&](int px, auto take) {
+                for (int c = 0, slot = px; c < copies; ++c, slot += npx_pad) {
+                    take(slot);
+                    if (split) {
+                        const uint32_t o = slot_info16[slot];
+                        for (uint32_t r = 0; r < (o >> 9); ++r)
+                            if ((o & 511u) + r < (uint32_t)nspare) take(nused + (int)((o & 511u) + r));
                     }
                 }
+            };
+            if (owned) {
+                for (int i = tid_w; i < npx * QR; i += kTileThreads) {
+                    const int px = i / QR, q4 = i % QR;
+                    if (4 * q4 >= nch) continue;
+                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                    each_slot(px, [&](int slot) { v += sums4[slot * QR + q4]; });
+                    put(px, cb + 4 * q4, v);
+                }
+            } else {
+#pragma unroll 2
+                for (int i = tid_w; i < npx * CH; i += kTileThreads) {
+                    const int px = i / CH, c = i % CH;
+                    if (c >= nch) continue;
+                    float v = 0.0f;
+                    each_slot(px, [&](int slot) { v += sums1[slot * CH + c]; });
+                    unsafeAtomicAdd(gimg + (int64_t)(it.p0 + px) * row_pitch + (int64_t)wk.h * hd + cb + c, v);
+                }
             }
-            wave_lds_sync();
+            __syncthreads();
         }
         if (cb + CH < hd) clean_state();
     }

@@ -127,15 +127,10 @@ __device__ inline int32_t level_tile_chunks(const KArgs& a, int32_t nt)
     return (int32_t)chunks;
 }
 
-// A tile of `npx` pixels whose rows its one workgroup of the tile pass stores directly: no other workgroup adds to
-// them (the tile is not split by query range and is too full to be held in copies or to have slots left for extra
-// lists), except to the tile's first pixel, which also receives the right halves of pairs that start on the last
-// pixel of the tile before it.
-__device__ inline bool tile_stored_directly(int32_t chunks, int32_t npx, int32_t tile_px_log2)
-{
-    const int32_t g = tile_group_px(tile_px_log2);
-    return chunks == 1 && (1 << tile_px_log2) - ((npx + g - 1) / g * g) < g;
-}
+// A tile whose rows its one workgroup of the tile pass stores directly: no other workgroup adds to them (the tile is not split by query
+// range), except to the tile's first pixel, which also receives the right halves of pairs that start on the last pixel of the tile
+// before it.
+__device__ inline bool tile_stored_directly(int32_t chunks) { return chunks == 1; }
 
 // What the kernels of the backward need to know of the levels, one level per lane of a wavefront.  Every workgroup goes through this
 // before it starts: walked through one level after the other it is a chain of memory and LDS latencies that short work items wait
@@ -202,7 +197,7 @@ struct LevelLanes {
         const int32_t ti = tile - __builtin_amdgcn_readlane(first, l), tile_px = 1 << a.tile_px_log2, P = __builtin_amdgcn_readlane(px, l);
         const int32_t p0 = base(l) + ti * tile_px;
         const int32_t npx = (P - ti * tile_px) < tile_px ? (P - ti * tile_px) : tile_px;
-        if (tile_stored_directly(__builtin_amdgcn_readlane(chunks, l), npx, a.tile_px_log2)) {
+        if (tile_stored_directly(__builtin_amdgcn_readlane(chunks, l))) {
             *r0 = p0;
             *r1 = part == 0 ? p0 + 1 : p0;
         } else {

@@ -6,7 +6,7 @@ import torch
 
 from drivingsdk_amd import workloads
 from test_msda_gpu import _check_all
-from util import BWD_FP32, FWD_FP32, half_tol
+from util import BWD_FP32, FWD_FP32, half_tol, set_tuning
 
 pytestmark = pytest.mark.gpu
 
@@ -23,6 +23,25 @@ def test_edges_of_tiles(gpu_device, maps, nq, dtype, hd):
     bs, nh, nl, npts, nk = 1, 2, len(maps), 3, int(shapes.prod(1).sum())
     tensors = (torch.randn(bs, nk, nh, hd, generator=g), torch.rand(bs, nq, nh, nl, npts, 2, generator=g) * 1.2 - 0.1,
                torch.rand(bs, nq, nh, nl, npts, generator=g), torch.randn(bs, nq, nh * hd, generator=g))
+    value, loc, attn, gout = (t.to(dtype) for t in tensors)
+    fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
+    _check_all(workloads.MsdaInputs(value, shapes, lsi, loc, attn, gout), gpu_device, fwd, bwd)
+
+
+@pytest.mark.parametrize("dtype,hd", [(torch.float32, 32), (torch.float32, 37), (torch.float32, 70), (torch.bfloat16, 32), (torch.float16, 130)])
+@pytest.mark.parametrize("target", [128, 100000], ids=["shared", "owned"])
+@pytest.mark.parametrize("maps", [((15, 25),), ((10, 10), (1, 3)), ((7, 18), (21, 24))], ids=["375", "100+3", "126+504"])
+def test_copies_and_extra_lists_are_added_up(gpu_device, monkeypatch, maps, target, dtype, hd):
+    """More records than a round holds, three quarters of them on a few pixels: tiles in copies with extra lists for the hot pixels, of
+    one workgroup that stores them and of several that add to them."""
+    set_tuning(monkeypatch, MXD_MSDA_TILE_TARGET=target)
+    g = torch.Generator().manual_seed(hd + len(maps))
+    shapes, lsi = workloads.level_tensors(maps)
+    bs, nh, nl, npts, nq, nk = 1, 2, len(maps), 4, 2500, int(shapes.prod(1).sum())
+    loc = torch.rand(bs, nq, nh, nl, npts, 2, generator=g)
+    loc[:, :, :, :, 1:] = 0.4 + 0.05 * loc[:, :, :, :, 1:]
+    tensors = (torch.randn(bs, nk, nh, hd, generator=g), loc, torch.rand(bs, nq, nh, nl, npts, generator=g),
+               torch.randn(bs, nq, nh * hd, generator=g))
     value, loc, attn, gout = (t.to(dtype) for t in tensors)
     fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
     _check_all(workloads.MsdaInputs(value, shapes, lsi, loc, attn, gout), gpu_device, fwd, bwd)
