@@ -255,7 +255,7 @@ __device__ inline SampleRef sample_ref(const KArgs& a, int b, int q, int h, int 
 }
 
 // Launch description of the tile-ownership grad_value kernel.
-constexpr int kTileEntCap = 576;  // list entries (16 bytes) per wavefront and round
+constexpr int kTileEntCap = 560;  // list entries (16 bytes) per wavefront and round
 struct TileArgs {
     mxd_msda_plan map;     // only the XCD mapping fields are used: one "query" per work item
     int32_t target;        // pair records per work item aimed at when a hot tile is split by query range

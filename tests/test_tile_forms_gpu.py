@@ -45,3 +45,23 @@ def test_copies_and_extra_lists_are_added_up(gpu_device, monkeypatch, maps, targ
     value, loc, attn, gout = (t.to(dtype) for t in tensors)
     fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
     _check_all(workloads.MsdaInputs(value, shapes, lsi, loc, attn, gout), gpu_device, fwd, bwd)
+
+
+@pytest.mark.parametrize("nq", [31, 33, 700, 17000])
+@pytest.mark.parametrize("order", ["sorted", "random"])
+@pytest.mark.parametrize("dtype,hd", [(torch.float32, 8), (torch.float16, 32)])
+def test_runs_of_records(gpu_device, dtype, hd, order, nq):
+    """Runs of no, few and many records of a tile: queries in the order of the map, which leave most tiles no record of most slabs, and in
+    no order; fewer runs than a wavefront looks through at a time and more, batches and windows of records that end within and between runs."""
+    g = torch.Generator().manual_seed(nq)
+    maps = ((40, 41), (9, 7))
+    shapes, lsi = workloads.level_tensors(maps)
+    bs, nh, nl, npts, nk = 1, 1, 2, 2, int(shapes.prod(1).sum())
+    loc = torch.rand(bs, nq, 1, 1, 1, 2, generator=g).expand(bs, nq, nh, nl, npts, 2) + 0.01 * torch.randn(bs, nq, nh, nl, npts, 2, generator=g)
+    if order == "sorted":
+        loc = loc[:, loc[0, :, 0, 0, 0, 1].argsort()]
+    tensors = (torch.randn(bs, nk, nh, hd, generator=g), loc.contiguous(), torch.rand(bs, nq, nh, nl, npts, generator=g),
+               torch.randn(bs, nq, nh * hd, generator=g))
+    value, loc, attn, gout = (t.to(dtype) for t in tensors)
+    fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
+    _check_all(workloads.MsdaInputs(value, shapes, lsi, loc, attn, gout), gpu_device, fwd, bwd)
