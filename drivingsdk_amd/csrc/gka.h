@@ -4,7 +4,8 @@
 
 namespace mxd {
 
-constexpr int kGkaSamples = 8;   // samples of a tile of queries that a thread of the scatter keeps in registers while they are sorted
+// Samples of a tile of queries that a thread of the scatter keeps in registers while they are sorted, beside the sums of `px` pixels.
+constexpr int gka_samples(int px, bool quad) { return quad && px > 8 ? 6 : 8; }
 constexpr int kGkaPixels = 16;   // pixels whose sums a lane group of the scatter keeps in registers, at most
 constexpr int kGkaLevelBytes = kMaxLevels * 16;
 
@@ -33,6 +34,8 @@ struct GkaArgs {
     // grad_value: the same, queries per tile, lanes of 4 channels that share a row, pixels per lane group
     int32_t sc_splits, sc_split_q, sc_block, sc_tile_q, sc_lanes_log2, sc_px;
     uint32_t sc_lds;
+    int32_t sc_direct;     // rows of grad_out are 16-byte aligned: they go straight to LDS
+    int32_t sc_dots;       // the gradient of the weights is formed there too, else by a kernel of its own
 };
 
 hipError_t raise_gka_lds();

@@ -7,18 +7,21 @@
 // [24, 7156 queries, 4 heads, 15 points].  From L1 and L2 they come at 18 TB/s (the general kernels: forward 147 us, dots of the
 // backward 279 us with their records); LDS gives 128 bytes per clock and CU, 78 TB/s.  So
 //
-//   * forward and the dots of the backward (gradient of the weights) put the (batch, head)'s slab of value into LDS once per
-//     workgroup and gather there.  What bounds them: reading locations and weights and writing the result (300 MB), and LDS.
+//   * the forward (and the dots of the backward where lane pairs share a row) puts the (batch, head)'s slab of value into LDS once per
+//     workgroup and gathers there.  What bounds them: reading locations and weights and writing the result (300 MB), and LDS.
 //   * grad_value is summed by pixel: a workgroup takes tiles of queries, puts their grad_out rows into LDS, sorts the tile's
 //     samples by pixel (integer LDS counters) and lets lane groups that own pixels add the rows of their samples to registers.
-//     Clamping piles samples on the border pixels (16 times the average on the corners): pixels are dealt to the groups in turn.
 //     The query ranges of a slab leave float32 images of it, which a last kernel adds up and rounds.
-//     What bounds it: LDS again, and half of what it reads there is for groups whose lists have ended (a tile of 192 queries has 7
-//     samples per pixel).  Smaller tiles lose (64 queries: 356 against 286 us for the backward), so do larger ones that a CU holds one
-//     workgroup of (307), and so does sharing long lists among the groups of a wavefront (327).
+//   * The dots of the backward (gradient of the weights) are formed on the way, with the pixel's row of value in registers: a sample's
+//     grad_out row is read once for both.  (As a kernel of their own, gathering rows of value from the slab: 112 us at the size above.)
+//     What bounds it: the vector ALU of the walk (60 instructions for four samples of each of a wavefront's groups) and, with clamping that
+//     piles samples on the border pixels (16 times the average on the corners), groups whose lists have ended: a tile of 192 queries has 7
+//     samples per pixel.  Smaller tiles lose (64 queries: 356 against 286 us for the backward), so do larger ones that a CU holds one
+//     workgroup of (307), and so does sharing long lists among the groups of a wavefront (327; hot pixels in two to four parts: 226 against 207).  (The weights go round a quad by moves: folded into the multiply-adds by inline
+//     assembly, whose operands' wait states the compiler does not see, they were read too early.)
 //
-// Measured at that size, float32: forward 147 -> 82 us, dots 279 -> 112, grad_value 370 -> 183 + 9; float16 forward and backward
-// 65 and 220 us.
+// Measured at that size, float32: forward 147 -> 82 us, dots and grad_value 649 -> 295 (112 + 183) -> 207, sum of the images 9; float16
+// forward and backward 65 and 220 -> 190 us.
 #include "gka.h"
 
 namespace mxd {
@@ -214,100 +217,169 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
     }
 }
 
-// grad_value, or one query range's part of it: PX pixels per lane group.
-template <typename T, int PX>
+// Inclusive sum over the lanes of a wavefront.
+__device__ inline uint32_t wave_scan(uint32_t v)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr 1, 2, 4, 8
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast 15, 31
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
+    return v;
+}
+
+// grad_value, or one query range's part of it, and the gradient of the weights: PX pixels per lane group.
+// QUAD: four lanes and more share a row (GkaArgs::sc_dots); without, the gradient of the weights is left to gka_slab_kernel.
+template <typename T, int PX, bool QUAD>
 __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
 {
     typedef RowIO<T, 4> Row;
+    constexpr int NS = gka_samples(PX, QUAD), HS = PX > 12 ? 2 : NS / 2;  // samples of a tile per thread, and those requested together
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ uint32_t wave_sum[16];
-    const int tid = (int)threadIdx.x, block = (int)blockDim.x, lane = tid & (kWave - 1);
+    const int tid = (int)threadIdx.x, block = (int)blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row_bytes = a.part_ch * (int)sizeof(T);
     i32x4* lvl = reinterpret_cast<i32x4*>(smem);
     u32x2* ent = reinterpret_cast<u32x2*>(smem + kGkaLevelBytes);                    // sorted samples: {row in `rows`, weight}
     unsigned char* rows = reinterpret_cast<unsigned char*>(ent) + (((size_t)a.sc_tile_q * a.S * 8 + 15) & ~(size_t)15);
-    uint32_t* count = reinterpret_cast<uint32_t*>(rows + (size_t)a.sc_tile_q * row_bytes);  // [nk]
+    const uint32_t zero_row = (uint32_t)a.sc_tile_q * (uint32_t)row_bytes;           // (behind the tile's rows, one of zeros)
+    uint32_t* count = reinterpret_cast<uint32_t*>(rows + zero_row + row_bytes);      // [nk]
     uint32_t* start = count + a.nk;                                                  // [nk + 1]
+    uint32_t* ranks = start + a.nk + 1;                                              // [kWave]
+    uint16_t* pixel_of = reinterpret_cast<uint16_t*>(ranks + kWave);                 // QUAD: [PX][groups] the groups' pixels, nk: none
     uint32_t wg = xcd_order(blockIdx.x, gridDim.x);
     const int h = (int)(wg % (uint32_t)a.nh);
     wg /= (uint32_t)a.nh;
-    const int ch = h * a.hd + (int)(wg % (uint32_t)a.parts) * a.part_ch;  // first channel of the rows
+    const int cpart = (int)(wg % (uint32_t)a.parts), ch = h * a.hd + cpart * a.part_ch;  // first channel of the rows
     wg /= (uint32_t)a.parts;
     const int split = (int)(wg % (uint32_t)a.sc_splits), b = (int)(wg / (uint32_t)a.sc_splits);
     const int q_begin = split * a.sc_split_q, q_end = q_begin + a.sc_split_q < a.nq ? q_begin + a.sc_split_q : a.nq;
     const T* attn = static_cast<const T*>(a.attn);
     const T* gout = static_cast<const T*>(a.grad_out) + (int64_t)b * a.nq * a.nh * a.hd + ch;
-    const int64_t pitch = (int64_t)a.nh * a.hd;
+    const int pitch = a.nh * a.hd;
+    const int groups_log2 = __builtin_ctz(block) - a.sc_lanes_log2, groups = 1 << groups_log2;
     load_levels(a, lvl);
     for (int i = tid; i < a.nk; i += block) count[i] = 0;
+    if constexpr (QUAD)
+        for (int i = tid; i < PX << groups_log2; i += block) pixel_of[i] = (uint16_t)(i < a.nk ? i : a.nk);
+    if (tid < kWave) ranks[tid] = 0;
+    for (int i = tid; i < row_bytes / 4; i += block) reinterpret_cast<uint32_t*>(rows + zero_row)[i] = 0;
     float acc[PX][4];
 #pragma unroll
     for (int i = 0; i < PX; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[i][e] = 0.0f;
-    const int groups = block >> a.sc_lanes_log2, grp = tid >> a.sc_lanes_log2, j = tid & ((1 << a.sc_lanes_log2) - 1);
-    constexpr int kTogether = 4;                       // rows of a pixel that are read side by side
     const int per = (a.nk + block - 1) / block;        // counters of a thread in the prefix sum
     const int piece_log2 = a.lpr_log2;                 // 16-byte pieces of a row
     __syncthreads();
     for (int q0 = q_begin; q0 < q_end; q0 += a.sc_tile_q) {
         const int nq = q0 + a.sc_tile_q < q_end ? a.sc_tile_q : q_end - q0, n = nq * a.S;
         // ---- samples of the tile: pixel, weight, place among the samples of the pixel; rows of the tile into LDS ----------
-        uint32_t place[kGkaSamples];  // pixel | place << 16, ~0: none
-        T w[kGkaSamples];
+        uint32_t place[NS];  // pixel (nk: none) | place << 16
+        T w[NS];
         int t0 = tid;
         asm volatile("" : "+v"(t0));  // (what follows from it is not to be kept across the tiles)
-#pragma unroll
-        for (int half = 0; half < kGkaSamples; half += 4) {
-            f32x2 xy[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = t0 + (half + k) * block;
-                if (i < n) {
-                    const int q = (int)(((uint32_t)i * a.s_magic) >> 20), s = i - q * a.S;
-                    const int64_t at = (((int64_t)b * a.nq + q0 + q) * a.nh + h) * a.S + s;
-                    xy[k] = load_xy(a.loc, at);
-                    w[half + k] = attn[at];
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = t0 + (half + k) * block;
-                place[half + k] = ~0u;
-                if (i < n) {
-                    const int q = (int)(((uint32_t)i * a.s_magic) >> 20), s = i - q * a.S;
-                    const int32_t px = sample_pixel(a, lvl, s, xy[k]);
-                    if (px >= 0) place[half + k] = (uint32_t)px | atomicAdd(&count[px], 1u) << 16;
-                }
+        typedef RowIO<T, 16 / (int)sizeof(T)> Wide;
+        const int pieces = nq << piece_log2;
+        // (the tile's parts of the tensors, from where 32-bit offsets reach: gka_plan_parts)
+        const int64_t first = (((int64_t)b * a.nq + q0) * a.nh + h) * a.S;
+        const float* tile_loc = a.loc + 2 * first;
+        const T *tile_attn = attn + first, *tile_rows = gout + (int64_t)q0 * pitch;
+        const uint32_t per_q = (uint32_t)(a.nh * a.S);
+        if (a.sc_direct) {
+            // (straight into LDS, while the samples are on their way too)
+            for (int i0 = wave * kWave; i0 < pieces; i0 += block) {
+                const int i = i0 + (t0 & (kWave - 1)), q = i >> piece_log2, p = i & ((1 << piece_log2) - 1);
+                if (i < pieces)
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(tile_rows + (uint32_t)(q * pitch + p * (16 / (int)sizeof(T)))),
+                                                     (__attribute__((address_space(3))) void*)(rows + i0 * 16), 16, 0, 0);
             }
         }
-        typedef RowIO<T, 16 / (int)sizeof(T)> Wide;
-        for (int i0 = t0; i0 < nq << piece_log2; i0 += 4 * block) {
+#pragma unroll
+        for (int half = 0; half < NS; half += HS) {
+            f32x2 xy[HS];
+#pragma unroll
+            for (int k = 0; k < HS; ++k) {
+                const uint32_t i = t0 + (half + k) * block < n ? t0 + (half + k) * block : 0, q = (i * a.s_magic) >> 20, at = q * per_q + (i - q * (uint32_t)a.S);
+                xy[k] = load_xy(tile_loc, at);
+                w[half + k] = tile_attn[at];
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);  // (requested together)
+#pragma unroll
+            for (int k = 0; k < HS; ++k) {
+                const int i = t0 + (half + k) * block, q = (int)(((uint32_t)i * a.s_magic) >> 20);
+                const int32_t px = sample_pixel(a, lvl, i < n ? i - q * a.S : 0, xy[k]);
+                place[half + k] = (uint32_t)(i < n && px >= 0 ? px : a.nk);
+            }
+            uint32_t before[HS];
+#pragma unroll
+            for (int k = 0; k < HS; ++k) before[k] = atomicAdd(&count[place[half + k]], 1u);  // (samples without a pixel: start[0], not yet in use)
+#pragma unroll
+            for (int k = 0; k < HS; ++k) place[half + k] |= before[k] << 16;
+        }
+        if (a.sc_direct) {
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // (vmcnt(0))
+        } else for (int i0 = t0; i0 < pieces; i0 += 4 * block) {
             typename Wide::vec_t v[4];
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const int i = i0 + m * block, q = i >> piece_log2, p = i & ((1 << piece_log2) - 1);
-                if (q < nq) v[m] = *reinterpret_cast<const typename Wide::mem_t*>(gout + (q0 + q) * pitch + p * (16 / (int)sizeof(T)));
+                if (q < nq) v[m] = *reinterpret_cast<const typename Wide::mem_t*>(tile_rows + (uint32_t)(q * pitch + p * (16 / (int)sizeof(T))));
             }
 #pragma unroll
             for (int m = 0; m < 4; ++m)
                 if ((i0 + m * block) >> piece_log2 < nq) reinterpret_cast<typename Wide::vec_t*>(rows)[i0 + m * block] = v[m];
         }
         __syncthreads();
+        if (QUAD && q0 == q_begin && q_end - q_begin > a.sc_tile_q) {
+            // Pixels are dealt to the groups by the samples they have in the first tile, most first: the groups of a wavefront walk
+            // pixels of about the same number of samples side by side.  The wavefront that has the most of the first row -- the corners
+            // -- and the one beside it on its SIMD have the least of the other rows.  (Four buckets per power of two of the number over
+            // the average.  Workgroups of one tile have nothing to learn from it, and where lane pairs walk a pixel it gains nothing.)
+            auto bucket = [&](uint32_t c) {
+                const uint32_t v = __builtin_bit_cast(uint32_t, (float)c * (float)a.nk / (float)n) >> 21;
+                const uint32_t k = v < ((127u - 4u) << 2) ? 0u : v - ((127u - 4u) << 2);
+                return kWave - 1 - (k < kWave ? k : kWave - 1);
+            };
+            int t = tid;
+            asm volatile("" : "+v"(t));
+#pragma unroll 1
+            for (int i = t; i < a.nk; i += block) atomicAdd(&ranks[bucket(count[i])], 1u);
+            __syncthreads();
+            if (tid < kWave) {
+                const uint32_t v = ranks[tid];
+                ranks[tid] = wave_scan(v) - v;
+            }
+            __syncthreads();
+            const int per_wave_log2 = 6 - a.sc_lanes_log2, waves = block / kWave;
+#pragma unroll 1
+            for (int i = t; i < PX << groups_log2; i += block) {
+                const int rank = i < a.nk ? (int)atomicAdd(&ranks[bucket(count[i])], 1u) : i, row = rank >> groups_log2;
+                int at = rank & (groups - 1);
+                if (row > 0) {
+                    const int v = at >> per_wave_log2, to = v < waves - 2 ? (v < 3 ? v + 1 : v + 2) : v == waves - 2 ? 4 : 0;
+                    at = (at & ((1 << per_wave_log2) - 1)) | to << per_wave_log2;
+                }
+                pixel_of[(row << groups_log2) + at] = (uint16_t)(i < a.nk ? i : a.nk);
+            }
+        }
         // ---- first sample of every pixel ------------------------------------------------------------------------------------
         uint32_t sum = 0;
-        const int c0 = tid * per;
+        int t2 = tid;
+        asm volatile("" : "+v"(t2));
+        const int c0 = t2 * per;
         for (int i = c0; i < c0 + per && i < a.nk; ++i) sum += count[i];
-        uint32_t inc = sum;
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-            const uint32_t o = __shfl_up(inc, d, kWave);
-            if (lane >= d) inc += o;
-        }
-        if (lane == kWave - 1) wave_sum[tid >> 6] = inc;
+        const uint32_t inc = wave_scan(sum);
+        if ((t2 & (kWave - 1)) == kWave - 1) wave_sum[wave] = inc;
         __syncthreads();
         uint32_t at = inc - sum;
-        for (int v = 0; v < tid >> 6; ++v) at += wave_sum[v];
+        for (int v = 0; v < wave; ++v) at += wave_sum[v];
         for (int i = c0; i < c0 + per && i < a.nk; ++i) {
             start[i] = at;
             at += count[i];
@@ -315,56 +387,148 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
             if (i == a.nk - 1) start[a.nk] = at;
         }
         __syncthreads();
+        uint32_t at2[NS / 2];  // entries of the samples, two per word, 0xFFFF: none
 #pragma unroll
-        for (int k = 0; k < kGkaSamples; ++k) {
-            if (place[k] != ~0u) {
+        for (int k = 0; k < NS; ++k) {
+            uint32_t e = 0xFFFFu;
+            if ((place[k] & 0xFFFFu) < (uint32_t)a.nk) {
                 const uint32_t q = ((uint32_t)(t0 + k * block) * a.s_magic) >> 20;
-                ent[start[place[k] & 0xFFFFu] + (place[k] >> 16)] = u32x2{q * (uint32_t)row_bytes, __builtin_bit_cast(uint32_t, to_f32(w[k]))};
+                e = start[place[k] & 0xFFFFu] + (place[k] >> 16);
+                ent[e] = u32x2{q * (uint32_t)row_bytes, __builtin_bit_cast(uint32_t, to_f32(w[k]))};
             }
+            at2[k / 2] = k % 2 == 0 ? e : at2[k / 2] | e << 16;
         }
         __syncthreads();
         // ---- the groups add the rows of their pixels' samples ---------------------------------------------------------------
-        int g0 = grp;
-#pragma unroll
-        for (int i = 0; i < PX; ++i) {
-            asm volatile("" : "+v"(g0));
-            const int p = i * groups + g0;
-            uint32_t k = 0, end = 0;
+        int t3 = tid;
+        asm volatile("" : "+v"(t3));
+        int g0 = t3 >> a.sc_lanes_log2;
+        const int j = t3 & ((1 << a.sc_lanes_log2) - 1);
+        auto samples_of = [&](int p, uint32_t& k, uint32_t& end) {
             if (p < a.nk) {
                 k = start[p];
                 end = start[p + 1];
             }
-            while (k < end) {
-                typename Row::held_t row[kTogether];
-                float wt[kTogether];
+        };
+        if constexpr (QUAD) {
+            // A lane looks up one entry of four, and a quad hands them round: what the walk reads from LDS, which binds it, is rows.
+            // An entry's weight gives way to its dot product with the pixel's row of value.
+            const T* value = static_cast<const T*>(a.value) + (int64_t)b * a.nk * a.nh * a.hd + ch + j * 4;
+            const uint32_t mine = (uint32_t)(j & 3), turned = mine ^ ((j >> 2) & 1 ? 3u : 0u);  // (the mirrors below turn a quad round)
+            const bool odd = (turned & 1u) != 0, upper = (turned & 2u) != 0;
+            const unsigned char* my_rows = rows + j * 4 * (int)sizeof(T);
+            auto fetch = [&](int p) { return Row::load_held(value + (uint32_t)((p < a.nk ? p : 0) * pitch)); };
+            int p = pixel_of[g0];
+            typename Row::held_t vnext = fetch(p);
 #pragma unroll
-                for (int m = 0; m < kTogether; ++m) {
-                    const u32x2 en = ent[k + m < end ? k + m : end - 1];
-                    const uint32_t ow = en.y;
-                    wt[m] = __builtin_bit_cast(float, ow);
-                    row[m] = *reinterpret_cast<const typename Row::vec_t*>(rows + en.x + j * 4 * (int)sizeof(T));
+            for (int i = 0; i < PX; ++i) {
+                asm volatile("" : "+v"(g0));
+                uint32_t k = 0, end = 0;
+                samples_of(p, k, end);
+                const typename Row::held_t vrow = vnext;
+                if (i + 1 < PX) {
+                    p = pixel_of[((i + 1) << groups_log2) + g0];
+                    vnext = fetch(p);
                 }
+                while (k < end) {
+                    const bool ok = k + mine < end;
+                    const u32x2 en = ent[ok ? k + mine : k];
+                    const uint32_t ox = en.x, oy = en.y;
+                    const int off = (int)(ok ? ox : zero_row);
+                    const float wt = ok ? __builtin_bit_cast(float, oy) : 0.0f;
+                    typename Row::held_t row[4];
+                    row[0] = *reinterpret_cast<const typename Row::vec_t*>(my_rows + (uint32_t)__builtin_amdgcn_update_dpp(0, off, 0x00, 0xF, 0xF, true));
+                    row[1] = *reinterpret_cast<const typename Row::vec_t*>(my_rows + (uint32_t)__builtin_amdgcn_update_dpp(0, off, 0x55, 0xF, 0xF, true));
+                    row[2] = *reinterpret_cast<const typename Row::vec_t*>(my_rows + (uint32_t)__builtin_amdgcn_update_dpp(0, off, 0xAA, 0xF, 0xF, true));
+                    row[3] = *reinterpret_cast<const typename Row::vec_t*>(my_rows + (uint32_t)__builtin_amdgcn_update_dpp(0, off, 0xFF, 0xF, 0xF, true));
+                    float d[4];
+                    auto use = [&](auto lane_of_quad) {
+                        constexpr int m = decltype(lane_of_quad)::value;
+                        if constexpr (sizeof(T) == 2) {
+                            typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+                            const u32x2_t vv = __builtin_bit_cast(u32x2_t, vrow), gg = __builtin_bit_cast(u32x2_t, row[m]);
+                            const uint32_t v0 = vv.x, v1 = vv.y, g0 = gg.x, g1 = gg.y;
+                            d[m] = dot2_acc<T>(v1, g1, dot2_acc<T>(v0, g0, 0.0f));
+                        } else {
+                            d[m] = vrow[0] * row[m][0];
 #pragma unroll
-                for (int m = 0; m < kTogether; ++m) {
-                    float v[4];
-                    Row::unpack_held(row[m], v);
-                    if (k + m < end) {
+                            for (int e = 1; e < 4; ++e) d[m] = __builtin_fmaf(vrow[e], row[m][e], d[m]);
+                        }
+                        float g[4];
+                        Row::unpack_held(row[m], g);
+                        const float w1 = dpp_xchg<m * 0x55>(wt);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(wt[m], v[e], acc[i][e]);
+                        for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(w1, g[e], acc[i][e]);
+                    };
+                    use(std::integral_constant<int, 0>{});
+                    use(std::integral_constant<int, 1>{});
+                    use(std::integral_constant<int, 2>{});
+                    use(std::integral_constant<int, 3>{});
+                    // over the lanes of the group, four sums at a time: every step halves what a lane keeps
+                    const float d01 = (odd ? d[1] : d[0]) + dpp_xchg<0xB1>(odd ? d[0] : d[1]);
+                    const float d23 = (odd ? d[3] : d[2]) + dpp_xchg<0xB1>(odd ? d[2] : d[3]);
+                    float dot = (upper ? d23 : d01) + dpp_xchg<0x4E>(upper ? d01 : d23);
+                    if (a.sc_lanes_log2 >= 3) dot += dpp_xchg<0x141>(dot);
+                    if (a.sc_lanes_log2 >= 4) dot += dpp_xchg<0x140>(dot);
+                    if (a.sc_lanes_log2 >= 5) dot += __shfl_xor(dot, 16, 64);
+                    if (a.sc_lanes_log2 >= 6) dot += __shfl_xor(dot, 32, 64);
+                    if (ok && j < 4) reinterpret_cast<float*>(ent)[2 * (k + mine) + 1] = dot;
+                    k += 4;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PX; ++i) {
+                asm volatile("" : "+v"(g0));
+                uint32_t k = 0, end = 0;
+                samples_of((i << groups_log2) + g0, k, end);
+                for (; k < end; k += 4) {
+                    typename Row::held_t row[4];
+                    float wt[4];
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        const u32x2 en = ent[k + m < end ? k + m : end - 1];
+                        const uint32_t ow = en.y;
+                        wt[m] = __builtin_bit_cast(float, ow);
+                        row[m] = *reinterpret_cast<const typename Row::vec_t*>(rows + en.x + j * 4 * (int)sizeof(T));
+                    }
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        float v[4];
+                        Row::unpack_held(row[m], v);
+                        if (k + m < end) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(wt[m], v[e], acc[i][e]);
+                        }
                     }
                 }
-                k += kTogether;
             }
         }
         __syncthreads();
+        if constexpr (QUAD) {
+            T* dst = static_cast<T*>(a.grad_attn) + first;
+            float* dots = a.dots + (int64_t)cpart * a.bs * a.nq * a.nh * a.S + first;
+            int t1 = tid;
+            asm volatile("" : "+v"(t1));
+#pragma unroll
+            for (int k = 0; k < NS; ++k) {
+                const int i = t1 + k * block;
+                if (i >= n) break;
+                const uint32_t e = at2[k / 2] >> (k % 2 * 16) & 0xFFFFu;
+                const float d = e != 0xFFFFu ? reinterpret_cast<const float*>(ent)[2 * e + 1] : 0.0f;
+                const uint32_t q = ((uint32_t)i * a.s_magic) >> 20, at = q * per_q + ((uint32_t)i - q * (uint32_t)a.S);
+                if (a.parts == 1) dst[at] = from_f32<T>(d);
+                else dots[at] = d;
+            }
+        }
     }
-    float* part = a.part + ((int64_t)split * a.bs + b) * a.nk * a.nh * a.hd + ch + j * 4;
-    int g0 = grp;
+    int g0 = tid >> a.sc_lanes_log2;
+    float* part = a.part + ((int64_t)split * a.bs + b) * a.nk * a.nh * a.hd + ch + (tid & ((1 << a.sc_lanes_log2) - 1)) * 4;
 #pragma unroll
     for (int i = 0; i < PX; ++i) {
         asm volatile("" : "+v"(g0));
-        const int p = i * groups + g0;
-        if (p < a.nk) *reinterpret_cast<f32x4*>(part + p * pitch) = f32x4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+        const int p = QUAD ? pixel_of[(i << groups_log2) + g0] : (i << groups_log2) + g0;
+        if (p < a.nk) *reinterpret_cast<f32x4*>(part + (int64_t)p * pitch) = f32x4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
     }
 }
 
@@ -404,12 +568,18 @@ hipError_t by_lanes(int lpr_log2, F f)
 }
 
 template <typename T, typename F>
-hipError_t by_pixels(int px, F f)
+hipError_t by_pixels(int px, int lanes_log2, F f)
 {
-    if (px <= 4) return f(&gka_scatter_kernel<T, 4>);
-    if (px <= 8) return f(&gka_scatter_kernel<T, 8>);
-    if (px <= 12) return f(&gka_scatter_kernel<T, 12>);
-    if (px <= kGkaPixels) return f(&gka_scatter_kernel<T, kGkaPixels>);
+    if constexpr (sizeof(T) == 4)  // (16-bit rows are shared by four lanes at least)
+        if (lanes_log2 < 2) {
+            if (px <= 8) return f(&gka_scatter_kernel<T, 8, false>);
+            if (px <= 12) return f(&gka_scatter_kernel<T, 12, false>);
+            return px <= kGkaPixels ? f(&gka_scatter_kernel<T, kGkaPixels, false>) : hipErrorInvalidConfiguration;
+        }
+    if (px <= 4) return f(&gka_scatter_kernel<T, 4, true>);
+    if (px <= 8) return f(&gka_scatter_kernel<T, 8, true>);
+    if (px <= 12) return f(&gka_scatter_kernel<T, 12, true>);
+    if (px <= kGkaPixels) return f(&gka_scatter_kernel<T, kGkaPixels, true>);
     return hipErrorInvalidConfiguration;
 }
 
@@ -425,7 +595,8 @@ hipError_t raise_t()
         if (e == hipSuccess) e = by_lanes<T, true>(l, raise);
     }
     for (int px = 4; px <= kGkaPixels; px += 4)
-        if (e == hipSuccess) e = by_pixels<T>(px, raise);
+        for (int lanes_log2 : {1, 2})
+            if (e == hipSuccess) e = by_pixels<T>(px, lanes_log2, raise);
     return e;
 }
 
@@ -441,9 +612,9 @@ hipError_t slab_t(const GkaArgs& a, hipStream_t stream)
 template <typename T>
 hipError_t backward_t(const GkaArgs& a, hipStream_t stream)
 {
-    hipError_t e = slab_t<T, true>(a, stream);
+    hipError_t e = a.sc_dots ? hipSuccess : slab_t<T, true>(a, stream);
     if (e != hipSuccess) return e;
-    e = by_pixels<T>(a.sc_px, [&](auto* kernel) {
+    e = by_pixels<T>(a.sc_px, a.sc_lanes_log2, [&](auto* kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.sc_splits)), dim3(a.sc_block), a.sc_lds, stream, a);
         return hipGetLastError();
     });

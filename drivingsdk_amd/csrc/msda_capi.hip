@@ -1027,11 +1027,16 @@ bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
     a->sc_block = ceil_div(d.nk, 512 / sc_lanes) <= mxd::kGkaPixels ? 512 : 1024;
     a->sc_px = (int32_t)ceil_div(d.nk, a->sc_block / sc_lanes);
     if (a->sc_px > mxd::kGkaPixels) return false;
-    const int64_t room = (a->sc_block == 512 ? lim / 2 : lim) - mxd::kGkaLevelBytes - (2 * d.nk + 1) * 4 - 32;
+    // (places for pixels in the lane groups: as many as the kernel is built for)
+    const int64_t places = sc_lanes < 4 ? 0 : ceil_div(a->sc_px, 4) * 4 * (a->sc_block / sc_lanes);
+    const int64_t tables = row + (2 * d.nk + 1 + mxd::kWave) * 4 + places * 2;
+    const int64_t room = (a->sc_block == 512 ? lim / 2 : lim) - mxd::kGkaLevelBytes - tables - 32;
     int64_t tile = room / (row + S * 8);
-    if (tile > mxd::kGkaSamples * a->sc_block / S) tile = mxd::kGkaSamples * a->sc_block / S;
+    if (tile > mxd::gka_samples(a->sc_px, sc_lanes >= 4) * a->sc_block / S) tile = mxd::gka_samples(a->sc_px, sc_lanes >= 4) * a->sc_block / S;
     if (tile * S * S >= (1 << 20)) tile = (1 << 20) / (S * S) - 1;
     if (tile > 4088) tile = 4088;  // (32-bit products of the division by S)
+    const int64_t reach = (int64_t(1) << 31) / (d.nh * (S * 8 > d.hd * es ? S * 8 : d.hd * es));  // (32-bit offsets of locations and rows)
+    if (tile > reach) tile = reach;
     if (tile > d.nq) tile = d.nq;
     if (tile >= 8) tile &= ~(int64_t)7;
     if (tile < 8 && tile < d.nq) return false;
@@ -1039,7 +1044,9 @@ bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
     s = gka_splits(slabs, d.nq, a->sc_block == 512 ? 512 : 256, (double)tile, tile);
     a->sc_split_q = (int32_t)ceil_div(d.nq, s);
     a->sc_splits = (int32_t)ceil_div(d.nq, a->sc_split_q);
-    a->sc_lds = (uint32_t)(mxd::kGkaLevelBytes + ((tile * S * 8 + 15) & ~15) + tile * row + (2 * d.nk + 1) * 4);
+    // The scatter forms the dots from the rows that it reads anyway; lane pairs (8 channels in float32) cannot.
+    a->sc_dots = sc_lanes >= 4;
+    a->sc_lds = (uint32_t)(mxd::kGkaLevelBytes + ((tile * S * 8 + 15) & ~15) + tile * row + tables);
     return true;
 }
 
@@ -1612,6 +1619,7 @@ int mxd_gka_backward(const void* value, const int32_t* spatial_shapes, const int
     a.grad_attn = grad_attn_weights;
     a.part = static_cast<float*>(workspace);
     a.dots = reinterpret_cast<float*>(static_cast<char*>(workspace) + gka_image_bytes(a));
+    a.sc_direct = (reinterpret_cast<uintptr_t>(grad_output) & 15u) == 0;
     const hipError_t e = mxd::launch_gka_backward(code, a, static_cast<hipStream_t>(hip_stream));
     if (e != hipSuccess) return fail(MXD_E_LAUNCH, "mxd_gka_backward: launch failed: %s", hipGetErrorString(e));
     return MXD_OK;

@@ -4,6 +4,8 @@ on one pixel, channels in two parts, maps just inside and outside of what fits, 
 import pytest
 import torch
 
+import mx_driving
+
 from oracle import gka_oracle as gka
 from test_gka_gpu import make_inputs, run_gpu
 from util import BWD_FP32, FWD_FP32, HALF, rel_err, set_tuning
@@ -54,3 +56,32 @@ def test_all_samples_on_one_pixel_and_nan_locations(gpu_device):
 def test_levels_that_overlap(gpu_device):
     value, sh, lsi, loc, attn, go = make_inputs([2, 200, 16, 2, 2, 5], (9, 13), seed=4)
     compare((value, sh, torch.tensor([0, 40]), loc, attn, go), gpu_device)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd", [8, 16, 32, 64])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_many_tiles_with_border_pixels_of_many_samples(gpu_device, hd, dtype, offset):
+    """Workgroups of several tiles, which deal the pixels by their samples in the first one, an infinite row of grad_out and rows of it that
+    start on any element: 2500 queries sampling far beyond the border, then none of them inside it."""
+    value, sh, lsi, loc, attn, go = make_inputs([1, 2500, hd, 2, 1, 5], (13, 22), seed=hd)
+    loc[:, 1700:] = loc[:, 1700:] * 0 - 5.0                     # all on the first pixel
+    v, a, g = (t.to(dtype).double() for t in (value, attn, go))
+    want = gka.backward(v, sh, lsi, loc, a, g)
+    dev = gpu_device
+    dv, da = value.to(dev, dtype).requires_grad_(), attn.to(dev, dtype).requires_grad_()
+    buf = torch.empty(go.numel() + offset, device=dev, dtype=dtype)[offset:].view(go.shape)
+    buf.copy_(go.to(dev, dtype))
+    out = mx_driving.geometric_kernel_attention(dv, sh.to(dev), lsi.to(dev), loc.to(dev), da)
+    got = torch.autograd.grad(out, (dv, da), buf, retain_graph=True)
+    tol = {torch.float32: BWD_FP32, torch.float16: HALF, torch.bfloat16: 2.0 ** -8}[dtype]
+    for name, g_, w_ in zip(("grad_value", "grad_attn_weights"), got, want):
+        assert rel_err(g_.double().cpu().numpy(), w_) <= tol, name
+    buf[0, 7] = float("inf")                                    # pixels that query 7 does not sample stay finite
+    gv, ga = torch.autograd.grad(out, (dv, da), buf)
+    px = (loc[0, 7, :, 0, :, 1].clamp(0, 12) * 22 + loc[0, 7, :, 0, :, 0].clamp(0, 21)).long()
+    for h in range(2):
+        hit = torch.zeros(13 * 22, dtype=torch.bool)
+        hit[px[h]] = True
+        assert torch.isfinite(gv[0, ~hit.to(dev), h]).all() and not torch.isfinite(gv[0, hit.to(dev), h]).any()
+    assert torch.isfinite(ga[0, torch.arange(2500, device=dev) != 7]).all()
