@@ -21,10 +21,11 @@
 //     the grad_out rows of its records -- those of a batch element stay in L2 -- and stored once, whole.
 //
 // Measured (6 x 900 anchors x 13 points, 6 cameras x 4 scales, 256 channels in 8 groups, float32), one unit of lanes per anchor and
-// group and the tile pass -> these: forward 395 -> 270 us (float16, one batch element 140 -> 25), forward and backward 1969 -> 855
+// group and the tile pass -> these: forward 395 -> 237 us (float16, one batch element 140 -> 25), forward and backward 1969 -> 820
 // with the dots formed by the anchors' wavefronts -- 318 us with the sort beside them, the gradient of the maps 221, the caller's
-// layouts 40 -- and 700 with the dots formed beside the maps' gradient: sort 43, rows and dots 351, layouts 51 (kernel times one at
-// a time; rows from HBM bound all but the sort and the layouts).
+// layouts 40 -- and 670 with the dots formed beside the maps' gradient: sort 43, rows and dots 351, layouts 51 (kernel times one at
+// a time; rows that the L2 does not hold bound all but the sort and the layouts: with six cameras that name the same maps the forward
+// takes 131 us).
 #include "dagg.h"
 
 namespace mxd {
@@ -83,6 +84,17 @@ __device__ inline int find_locations(const DaggArgs& a, int64_t anchor, int firs
     return n;
 }
 
+// Which of a group's samples a lane stands for: scale by scale, the locations side by side.  (Neighbouring lane groups then gather
+// from the same map at a time, where an anchor's points are close to each other: 6 x 900 anchors in float32, forward, 272 us with the
+// scales of a location side by side, 237 like this.)
+__device__ inline bool sample_of_lane(int lane, int locs, int scales, int& scale, int& loc)
+{
+    // (a quotient of small numbers: half a step away from a whole one at least, which is more than the reciprocal's error)
+    scale = scales == 1 ? (lane < locs ? 0 : 1) : (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)locs));
+    loc = lane - scale * locs;
+    return scale < scales;
+}
+
 // ---- forward -------------------------------------------------------------------------------------------------------------
 // ONE: a row piece is the channels of one group (its weight is multiplied into the corner weights once); otherwise 128
 // bytes of several groups' channels, whose weights wait in LDS.
@@ -117,10 +129,7 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
     const __amdgpu_buffer_rsrc_t vres =
         make_rsrc(static_cast<const char*>(a.feat) + (size_t)wk.b * a.batch_bytes, a.batch_bytes);
 
-    // lane t of a group of samples: scale t % scales of its location t / scales
-    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
     const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);  // locations per group of samples
-    const bool tl_ok = tl < step;
 
     float acc[VEC];
 #pragma unroll
@@ -129,9 +138,10 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
         const int n = find_locations<T>(a, anchor, first, found, lane);
         wave_lds_sync();
         for (int v0 = 0; v0 < n; v0 += step) {
-            const int vi = v0 + tl;
-            const bool act = tl_ok && vi < n;
-            const Found f = found[act ? vi : 0];
+            const int locs = n - v0 < step ? n - v0 : step;
+            int ts, tl;
+            const bool act = sample_of_lane(lane, locs, a.scales, ts, tl);
+            const Found f = found[act ? v0 + tl : 0];
             const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
             const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
                                               a.nf, act);
@@ -150,7 +160,6 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
             off[lane] = o;
             wts[lane] = cw;
             wave_lds_sync();
-            const int locs = n - v0 < step ? n - v0 : step;
             const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);  // (uniform; samples that do not exist read zeros)
 #pragma unroll 2
             for (int t = 0; t < trips; ++t) {
@@ -232,16 +241,15 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
         for (int e = 0; e < kPairs; ++e) gpk[e] = __builtin_bit_cast(uint32_t, t2{from_f32<T>(gv[2 * e]), from_f32<T>(gv[2 * e + 1])});
     }
 
-    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
     const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);
-    const bool tl_ok = tl < step;
     for (int first = 0; first < a.nloc; first += kDaggList) {
         const int n = find_locations<T>(a, anchor, first, found, lane);
         wave_lds_sync();
         for (int v0 = 0; v0 < n; v0 += step) {
-            const int vi = v0 + tl;
-            const bool act = tl_ok && vi < n;
-            const Found f = found[act ? vi : 0];
+            const int locs = n - v0 < step ? n - v0 : step;
+            int ts, tl;
+            const bool act = sample_of_lane(lane, locs, a.scales, ts, tl);
+            const Found f = found[act ? v0 + tl : 0];
             const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
             const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
                                               a.nf, act);
@@ -251,7 +259,6 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
             for (int k = 0; k < 4; ++k) o[k] = sm.cvalid[k] ? (uint32_t)sm.pix[k] * a.pitch_bytes : kInvalidCorner;
             off[lane] = o;
             wave_lds_sync();
-            const int locs = n - v0 < step ? n - v0 : step;
             const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);
             auto gather = [&](auto lg) {
                 constexpr int LG = decltype(lg)::value;
@@ -306,7 +313,7 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
             wave_lds_sync();
             if (act && ts == 0) {
                 // the scales of a location share it
-                for (int k = 1; k < a.scales; ++k) g += gxy[lane + k];
+                for (int k = 1; k < a.scales; ++k) g += gxy[lane + k * locs];
                 gl[fj >> 16] = g;
             }
             wave_lds_sync();
