@@ -45,3 +45,15 @@ def test_short_rows(gpu_device, nl, npts, dtype, hd):
 def test_narrow_16_bit_rows_with_a_forced_tile_size(gpu_device, monkeypatch, dtype, hd):
     set_tuning(monkeypatch, MXD_MSDA_TILE_PX_LOG2=7)
     _check_all(_inputs(_MAPS, 4, 131, 4, hd, dtype, hd), gpu_device, half_tol(dtype), half_tol(dtype))
+
+
+@pytest.mark.parametrize("dtype,hd", [(torch.float32, 32), (torch.float32, 13), (torch.float16, 32), (torch.bfloat16, 24), (torch.float16, 64), (torch.bfloat16, 33)])
+@pytest.mark.parametrize("nl,npts", [(1, 8), (2, 8), (3, 8), (1, 16), (1, 10), (3, 10), (1, 24), (1, 30)])
+def test_eight_points_side_by_side(gpu_device, monkeypatch, nl, npts, dtype, hd):
+    """Levels of eight points and more, with one unit per query and with two, whole and cut off at their last queries; rows of 4 lanes and
+    of 8 (the former need a line of the launch moved)."""
+    fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
+    for nq in (1, 67, 10000):
+        if nq == 10000 and (npts, hd) not in ((8, 32), (8, 13)):
+            continue
+        _check_all(_inputs(_MAPS[:nl], npts, nq, 3, hd, dtype, 10 * nl + npts), gpu_device, fwd, bwd)
