@@ -25,9 +25,15 @@ struct GridArgs {
     // gradient of the grid: channels per workgroup, of which so many planes are staged at a time, chunks per image, ranges of
     // output pixels, output pixels per thread, workgroups
     int32_t gg_channels, gg_planes, gg_chunks, gg_ranges, gg_px, gg_wgs;
+    // both gradients by the same workgroups (gb_wgs > 0): channels per workgroup, chunks per image, output pixels per thread
+    int32_t gb_channels, gb_chunks, gb_px, gb_wgs;
+    int32_t sum_chunks;  // images of sums in `part` that the sum kernel adds up (0, 1: none)
     int32_t block;
     uint32_t lds;
 };
+
+// Bytes of a plane's float64 sums in LDS, what lies behind them on a 16-byte boundary.
+__host__ __device__ inline uint32_t grid_sums_bytes(int64_t px) { return (uint32_t)((px * 8 + 15) & ~int64_t(15)); }
 
 hipError_t raise_grid_lds();
 hipError_t launch_grid_planes_forward(int dtype, const GridArgs& a, hipStream_t stream);

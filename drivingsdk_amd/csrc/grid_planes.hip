@@ -13,10 +13,11 @@
 // The gradient of the grid is a sum over the channels: a workgroup takes a range of output pixels and a chunk of the channels,
 // stages the planes one after another (several at a time where they are small) and keeps the sums of its pixels in registers;
 // chunks are added up by a kernel of its own.  The gradient of the maps needs all output pixels of a plane and the gradient of the
-// grid many channels of a pixel: two kinds of workgroups of one launch, which read grad_out twice (a fifth of what moves).
+// grid many channels of a pixel: two kinds of workgroups of one launch, which read grad_out twice (a fifth of what moves) -- or, where
+// a plane with its sums leaves a CU room for one workgroup anyway, one kind that does both plane by plane.
 //
-// Measured at that size: forward 43 us (190 MB, 4.4 TB/s: the rate of a copy), gradient of the maps 77, of the grid 69, both in one
-// launch 134 us (380 MB, 2.8 TB/s); in float16 29 and 118 us.  Small calls ([24, 128, 16, 20] -> 12 x 20) take 5 and 11 us.
+// Measured at that size: forward 49 us (190 MB, 3.9 TB/s), both gradients by two kinds of workgroups 122 us (400 MB, 3.3 TB/s), by
+// one 88; in float16 109 and 77 us.  Small calls ([24, 128, 16, 20] -> 12 x 20) take 5 and 9 us.
 #include "grid_planes.h"
 
 namespace mxd {
@@ -30,13 +31,13 @@ struct Piece {
     typedef vec_t mem_t __attribute__((aligned(sizeof(T))));  // a plane of odd size starts anywhere
 };
 
-// Consecutive elements on their way to LDS: request() asks for a thread's first four 16-byte pieces, place() stores them, and the
-// rest of a stretch that is longer than four pieces per thread.
-template <typename T>
+// Consecutive elements on their way to LDS: request() asks for a thread's first four (kAhead) 16-byte pieces, place() stores them,
+// and the rest of a stretch that is longer than that.
+template <typename T, int kAhead = 4>
 struct Stage {
     typedef typename Piece<T>::vec_t vec_t;
     typedef typename Piece<T>::mem_t mem_t;
-    static constexpr int kE = Piece<T>::kElems, kAhead = 4;
+    static constexpr int kE = Piece<T>::kElems;
     vec_t v[kAhead];
 
     __device__ inline void request(const T* src, int elems, int i0)
@@ -200,6 +201,21 @@ __device__ inline void grad_maps(const GridArgs& a, uint32_t wg, unsigned char* 
     if ((elems & 1) && threadIdx.x == 0) dst[elems - 1] = from_f64<T>(acc[elems - 1]);
 }
 
+// A pixel's sums over the channels of a chunk: into the chunk's image of sums, or, where there is one chunk, to grad_grid.
+template <typename T>
+__device__ inline void store_points(const GridArgs& a, int chunks, int chunk, int img, int p, float sx, float sy)
+{
+    const int64_t at = (int64_t)img * a.outs + p;
+    if (chunks > 1) {
+        reinterpret_cast<f32x2*>(a.part)[(int64_t)chunk * a.n * a.outs + at] = f32x2{sx, sy};
+        return;
+    }
+    const Sample s = grid_sample(a, load_xy(static_cast<const T*>(a.grid), at));  // for d(pixel)/d(grid)
+    T* dst = static_cast<T*>(a.grad_grid) + 2 * at;
+    dst[0] = from_f32<T>(sx * s.Wf);
+    dst[1] = from_f32<T>(sy * s.Hf);
+}
+
 // Gradient of the grid: PX output pixels per thread, their sums over the channels of a chunk in registers.
 template <typename T, int PX>
 __device__ inline void grad_points(const GridArgs& a, uint32_t wg, unsigned char* smem)
@@ -282,16 +298,7 @@ __device__ inline void grad_points(const GridArgs& a, uint32_t wg, unsigned char
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
         const int p = first + k * step;
-        if (k >= a.gg_px || p >= a.outs) continue;
-        const int64_t at = (int64_t)img * a.outs + p;
-        if (a.gg_chunks > 1) {
-            reinterpret_cast<f32x2*>(a.part)[(int64_t)chunk * a.n * a.outs + at] = f32x2{sx[k], sy[k]};
-        } else {
-            const Sample s = grid_sample(a, load_xy(grid, p));  // for d(pixel)/d(grid)
-            T* dst = static_cast<T*>(a.grad_grid) + 2 * at;
-            dst[0] = from_f32<T>(sx[k] * s.Wf);
-            dst[1] = from_f32<T>(sy[k] * s.Hf);
-        }
+        if (k < a.gg_px && p < a.outs) store_points<T>(a, a.gg_chunks, chunk, img, p, sx[k], sy[k]);
     }
 }
 
@@ -302,6 +309,151 @@ __global__ __launch_bounds__(1024) void grid_planes_bwd_kernel(const GridArgs a)
     // (the workgroups that read much come first: the others fill up behind them)
     if ((int)blockIdx.x < a.gg_wgs) grad_points<T, PX>(a, xcd_order(blockIdx.x, (uint32_t)a.gg_wgs), smem);
     else grad_maps<T>(a, xcd_order(blockIdx.x - (uint32_t)a.gg_wgs, (uint32_t)a.gx_wgs), smem);
+}
+
+// Both gradients, of planes whose sums leave a CU room for one workgroup: a workgroup takes a chunk of an image's channels, a plane
+// at a time, whose pixels and float64 sums lie in LDS side by side.  The geometry of its output pixels and the sums of the grid's
+// gradient stay in registers from plane to plane; the next plane and its grad_out travel while the one at hand is worked on, and
+// its sums go out, and are cleared, in the step that puts the next plane in place: two barriers per plane, grad_out read once.
+// What bounds it is LDS, at work for 3.9 of some 6 us per plane of 64 x 176 and 24 x 176 output pixels; 1.2 us are the step between.
+// (No VGPR may spill here: with 28 of them on the stack, in float32 with nine pixels per thread, the compiler saved one inside the
+//  masked end of place() and the lanes masked off there read rubbish.  Hence grad_out kept once, and reloaded pixel by pixel.)
+template <typename T, int PX>
+__global__ __launch_bounds__(1024) void grid_planes_both_kernel(const GridArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    double* sums = reinterpret_cast<double*>(smem);
+    const int px = a.h * a.w, first = (int)threadIdx.x;
+    constexpr int step = 2 * kGridThreads;
+    // (a corner outside the plane is read where it would lie, up to w + 1 elements before or behind: in the sums or in the room left
+    //  behind the plane; it is added to a word that nobody reads, one per lane)
+    T* plane = reinterpret_cast<T*>(smem + grid_sums_bytes(px));
+    double* nowhere = reinterpret_cast<double*>(smem + a.lds - kWave * sizeof(double)) + (first & (kWave - 1));
+    int wave_first = __builtin_amdgcn_readfirstlane(first & ~(kWave - 1));
+    const uint32_t wg = xcd_order(blockIdx.x, gridDim.x);
+    const int img = (int)(wg / (uint32_t)a.gb_chunks), chunk = (int)(wg % (uint32_t)a.gb_chunks);
+    const int c_begin = chunk * a.gb_channels, c_end = c_begin + a.gb_channels < a.c ? c_begin + a.gb_channels : a.c;
+    const T* grid = static_cast<const T*>(a.grid) + (int64_t)img * a.outs * 2;
+    const T* grad = static_cast<const T*>(a.grad_out) + ((int64_t)img * a.c + c_begin) * a.outs;
+    const T* src = static_cast<const T*>(a.x) + ((int64_t)img * a.c + c_begin) * px;
+    T* dst = static_cast<T*>(a.grad_x) + ((int64_t)img * a.c + c_begin) * px;
+
+    // (past the last output pixel: zero, from the buffer's bounds check)
+    T g[PX];
+    auto load_grad = [&](int k) {
+        const int left = a.outs - k * step;
+        const __amdgpu_buffer_rsrc_t row = make_rsrc(grad + k * step, left > 0 ? (uint32_t)left * (uint32_t)sizeof(T) : 0u);
+        const int at = first * (int)sizeof(T);
+        if constexpr (sizeof(T) == 4) g[k] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(row, at, 0, 0));
+        else g[k] = __builtin_bit_cast(T, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(row, at, 0, 0));
+    };
+    Stage<T, (int)sizeof(T)> st;  // (the largest plane that fits, in one go)
+    st.request(src, px);
+#pragma unroll
+    for (int k = 0; k < PX; ++k) load_grad(k);
+    // a pixel as {upper left corner + w + 1, which corners exist << 28} (the corner may lie a row and a pixel before the plane)
+    uint32_t corner[PX];
+    float lw[PX], lh[PX], sx[PX], sy[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        corner[k] = 0;
+        lw[k] = lh[k] = sx[k] = sy[k] = 0.0f;
+        if (first + k * step < a.outs) {
+            const Sample s = grid_sample(a, load_xy(grid, first + k * step));
+            uint32_t mask = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
+            if (mask) {
+                corner[k] = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
+                lw[k] = s.lw;
+                lh[k] = s.lh;
+            }
+        }
+    }
+    for (int i = first; i < (px + 1) / 2; i += step) reinterpret_cast<u32x4*>(sums)[i] = u32x4{0u, 0u, 0u, 0u};
+    st.place(src, plane, px);
+    __syncthreads();
+    for (int c = c_begin + 1;; ++c) {
+        if (c < c_end) {
+            src += px;
+            grad += a.outs;
+            st.request(src, px);
+        }
+        T r[2][4];
+        int at[2];
+        auto read = [&](int k) {
+            // (opaque: what follows from it would otherwise be kept for all pixels across the channels, which does not fit)
+            asm volatile("" : "+v"(corner[k]), "+v"(lw[k]), "+v"(lh[k]));
+            at[k & 1] = (int)(corner[k] & 0x0FFFFFFFu) - a.w - 1;
+            const T *r0 = plane + at[k & 1], *r1 = r0 + a.w;
+            r[k & 1][0] = r0[0];
+            r[k & 1][1] = r0[1];
+            r[k & 1][2] = r1[0];
+            r[k & 1][3] = r1[1];
+        };
+        asm volatile("" : "+s"(wave_first));  // (opaque: one comparison per pixel, not nine kept)
+        read(0);
+#pragma unroll
+        for (int k = 0; k < PX; ++k) {
+            if (k + 1 < PX) read(k + 1);
+            if (k * step + wave_first >= a.outs) break;
+            const int m = (int)corner[k], p = at[k & 1];
+            const float gc = to_f32(g[k]);
+            bool in[4];
+            float v[4], wt[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                in[j] = (m & (int)(1u << (28 + j))) != 0;
+                v[j] = in[j] ? to_f32(r[k & 1][j]) : 0.0f;
+            }
+            const float dx = __builtin_fmaf(lh[k], v[3] - v[2], (1.0f - lh[k]) * (v[1] - v[0]));
+            const float dy = __builtin_fmaf(lw[k], v[3] - v[1], (1.0f - lw[k]) * (v[2] - v[0]));
+            sx[k] = __builtin_fmaf(gc, dx, sx[k]);
+            sy[k] = __builtin_fmaf(gc, dy, sy[k]);
+            // (opaque: the sums would otherwise be formed behind the last pixel, from the rows of all pixels kept in registers)
+            asm volatile("" : "+v"(sx[k]), "+v"(sy[k]));
+            bilinear_weights(lw[k], lh[k], wt);
+            const int to[4] = {p, p + 1, p + a.w, p + a.w + 1};
+            // (no branches: behind one, the wait for a pixel's four values is one for the additions of the pixel before it as well,
+            //  110 us instead of 93 at the size above before the registers were trimmed)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                __hip_atomic_fetch_add(in[j] ? sums + to[j] : nowhere, (double)(wt[j] * gc), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (c < c_end) load_grad(k);  // (of the next channel)
+            __builtin_amdgcn_sched_barrier(0);  // (one pixel ahead, no more: the registers are full)
+        }
+        __syncthreads();
+        if (c < c_end) {
+            // (waited for here, and not behind the stores that come next: loads and stores return in order)
+#pragma unroll
+            for (int k = 0; k < PX; ++k) asm volatile("" ::"v"(g[k]));
+            st.place(src, plane, px);
+        }
+        // (two sums per lane: LDS gives those without bank conflicts)
+        typedef T pair_t __attribute__((ext_vector_type(2)));
+        typedef pair_t mem_t __attribute__((aligned(sizeof(T))));
+        typedef double f64x2 __attribute__((ext_vector_type(2)));
+        for (int i = first; i < px / 2; i += step) {
+            const f64x2 v = reinterpret_cast<const f64x2*>(sums)[i];
+            reinterpret_cast<f64x2*>(sums)[i] = f64x2{0.0, 0.0};
+            *reinterpret_cast<mem_t*>(dst + 2 * (int64_t)i) = pair_t{from_f64<T>(v.x), from_f64<T>(v.y)};
+        }
+        if ((px & 1) && first == 0) {
+            dst[px - 1] = from_f64<T>(sums[px - 1]);
+            sums[px - 1] = 0.0;
+        }
+        if (c >= c_end) break;
+        dst += px;
+        __syncthreads();
+    }
+    int mine = first;
+    asm volatile("" : "+v"(mine));  // (opaque: as above)
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        const int p = mine + k * step;
+        if (p < a.outs) store_points<T>(a, a.gb_chunks, chunk, img, p, sx[k], sy[k]);
+    }
 }
 
 // Sum over the channel chunks: 32 output pixels per workgroup, 8 threads that share the chunks of each.
@@ -315,7 +467,7 @@ __global__ __launch_bounds__(256) void grid_planes_sum_kernel(const GridArgs a)
     if (i < total) {
         const f32x2* part = reinterpret_cast<const f32x2*>(a.part) + i;
 #pragma unroll 4
-        for (int c = row; c < a.gg_chunks; c += 8) sum += part[c * total];
+        for (int c = row; c < a.sum_chunks; c += 8) sum += part[c * total];
     }
     sums[row][threadIdx.x & 31] = sum;
     __syncthreads();
@@ -346,8 +498,12 @@ hipError_t raise_t()
     for (int px : {1, 3, 6, kGridMaxPx})
         if (e == hipSuccess)
             e = by_pixels(px, [](auto p) {
-                return hipFuncSetAttribute(reinterpret_cast<const void*>(&grid_planes_bwd_kernel<T, decltype(p)::value>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes);
+                hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void*>(&grid_planes_bwd_kernel<T, decltype(p)::value>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes);
+                if (r == hipSuccess)
+                    r = hipFuncSetAttribute(reinterpret_cast<const void*>(&grid_planes_both_kernel<T, decltype(p)::value>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes);
+                return r;
             });
     return e;
 }
@@ -362,12 +518,20 @@ hipError_t forward_t(const GridArgs& a, hipStream_t stream)
 template <typename T>
 hipError_t backward_t(const GridArgs& a, hipStream_t stream)
 {
-    const dim3 wgs((unsigned)(a.gx_wgs + a.gg_wgs));
-    hipError_t e = by_pixels(a.gg_px, [&](auto p) {
-        hipLaunchKernelGGL((grid_planes_bwd_kernel<T, decltype(p)::value>), wgs, dim3(a.block), a.lds, stream, a);
-        return hipGetLastError();
-    });
-    if (e != hipSuccess || a.gg_wgs == 0 || a.gg_chunks == 1) return e;
+    hipError_t e;
+    if (a.gb_wgs) {
+        e = by_pixels(a.gb_px, [&](auto p) {
+            hipLaunchKernelGGL((grid_planes_both_kernel<T, decltype(p)::value>), dim3((unsigned)a.gb_wgs), dim3(a.block), a.lds, stream, a);
+            return hipGetLastError();
+        });
+    } else {
+        e = by_pixels(a.gg_px, [&](auto p) {
+            hipLaunchKernelGGL((grid_planes_bwd_kernel<T, decltype(p)::value>), dim3((unsigned)(a.gx_wgs + a.gg_wgs)), dim3(a.block), a.lds,
+                               stream, a);
+            return hipGetLastError();
+        });
+    }
+    if (e != hipSuccess || a.sum_chunks <= 1) return e;
     const int64_t total = (int64_t)a.n * a.outs;
     hipLaunchKernelGGL(grid_planes_sum_kernel<T>, dim3((unsigned)((total + 31) / 32)), dim3(256), 0, stream, a);
     return hipGetLastError();

@@ -37,6 +37,19 @@ def test_planes(gpu_device, input_shape, grid_shape, dtype):
         assert got.dtype == dtype and rel_err(got.double().cpu().numpy(), ref.numpy()) <= tol
 
 
+# (planes of more than 10240 pixels, 256 and more of them: both gradients by the same workgroups.  One and many chunks of the channels, the
+#  last of them short; one, two, three, six and nine output pixels per thread, full and partly so; the largest float32 plane)
+LARGE = [([257, 1, 97, 107], [257, 3, 5, 2]), ([2, 129, 103, 101], [2, 32, 32, 2]), ([1, 256, 64, 161], [1, 25, 41, 2]),
+         ([5, 70, 80, 168], [5, 37, 83, 2]), ([3, 100, 75, 140], [3, 48, 128, 2]), ([3, 100, 75, 140], [3, 96, 96, 2]),
+         ([3, 100, 75, 140], [3, 97, 96, 2])]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("input_shape,grid_shape", LARGE)
+def test_large_planes(gpu_device, input_shape, grid_shape, dtype):
+    test_planes(gpu_device, input_shape, grid_shape, dtype)
+
+
 def test_single_gradients_and_the_python_function(gpu_device):
     x, grid, go = [t.to(gpu_device) for t in make_inputs([2, 20, 30, 40], [2, 25, 35, 2], seed=2)]
 
@@ -53,9 +66,10 @@ def test_single_gradients_and_the_python_function(gpu_device):
             assert torch.allclose(torch.autograd.grad(o, t, go, retain_graph=True)[0], both[k], rtol=1e-5, atol=1e-5)
 
 
-def test_infinite_pixels_outside_the_samples(gpu_device):
+@pytest.mark.parametrize("input_shape", [[1, 4, 8, 8], [2, 128, 80, 130]])
+def test_infinite_pixels_outside_the_samples(gpu_device, input_shape):
     """A pixel that no sample reaches must not enter a result, whatever it holds (corners outside the image read some pixel)."""
-    x, grid, go = make_inputs([1, 4, 8, 8], [1, 6, 6, 2], seed=6)
+    x, grid, go = make_inputs(input_shape, [input_shape[0], 6, 6, 2], seed=6)
     grid = grid * 0.05 + torch.tensor([1.0, 1.0])   # around the lower right corner, part of it outside
     x[:, :, 0, 0] = float("inf")
     xd, gd = x.to(gpu_device).requires_grad_(), grid.to(gpu_device).requires_grad_()
