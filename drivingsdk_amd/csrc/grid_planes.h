@@ -20,6 +20,7 @@ struct GridArgs {
     int32_t mode;          // 1 + padding mode (0 zeros, 1 border) + 2 * align_corners
     // forward: planes per workgroup, chunks of them per image, splits of the output pixels
     int32_t planes, chunks, splits, split_px;
+    int32_t run_px;  // > 0: a workgroup's planes one after the other, so many output pixels per thread
     // gradient of the maps: planes per workgroup, chunks per image, bands of a large plane and their pixels, workgroups
     int32_t gx_planes, gx_chunks, gx_bands, gx_band_px, gx_wgs;
     // gradient of the grid: channels per workgroup, of which so many planes are staged at a time, chunks per image, ranges of
@@ -34,6 +35,12 @@ struct GridArgs {
 
 // Bytes of a plane's float64 sums in LDS, what lies behind them on a 16-byte boundary.
 __host__ __device__ inline uint32_t grid_sums_bytes(int64_t px) { return (uint32_t)((px * 8 + 15) & ~int64_t(15)); }
+
+// Output pixels per thread up to which two workgroups of 1024 threads fit the registers of a CU (forward, planes one after the other).
+__host__ __device__ constexpr int grid_run_px(int es) { return es == 4 ? 6 : 3; }
+
+// Elements before a plane in LDS that a corner a row and a pixel before it can reach, in whole 16-byte pieces.
+__host__ __device__ inline int grid_margin(int es, int w) { return (w + 16 / es) / (16 / es) * (16 / es); }
 
 hipError_t raise_grid_lds();
 hipError_t launch_grid_planes_forward(int dtype, const GridArgs& a, hipStream_t stream);

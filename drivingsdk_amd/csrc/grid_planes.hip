@@ -16,7 +16,7 @@
 // grid many channels of a pixel: two kinds of workgroups of one launch, which read grad_out twice (a fifth of what moves) -- or, where
 // a plane with its sums leaves a CU room for one workgroup anyway, one kind that does both plane by plane.
 //
-// Measured at that size: forward 49 us (190 MB, 3.9 TB/s), both gradients by two kinds of workgroups 122 us (400 MB, 3.3 TB/s), by
+// Measured at that size: forward 39 us (190 MB, 4.9 TB/s: the rate of a copy), both gradients by two kinds of workgroups 122 us (400 MB, 3.3 TB/s), by
 // one 88; in float16 109 and 77 us.  Small calls ([24, 128, 16, 20] -> 12 x 20) take 5 and 9 us.
 #include "grid_planes.h"
 
@@ -127,6 +127,73 @@ __global__ __launch_bounds__(1024) void grid_planes_fwd_kernel(const GridArgs a)
             }
             *o = from_f32<T>(acc);
         }
+    }
+}
+
+// Forward of many planes of an image, one after the other: the geometry of the workgroup's output pixels stays in registers, and the next
+// plane travels while the one at hand is sampled.  Bound by memory: 24 x 128 planes of 64 x 176, 24 x 176 samples, float32, 39 us (190 MB,
+// 4.9 TB/s, a copy's rate) where a workgroup per plane took 51, half of its time in geometry.
+template <typename T, int PX>
+__global__ __launch_bounds__(1024, PX <= grid_run_px((int)sizeof(T)) ? 8 : 4) void grid_planes_fwd_run_kernel(const GridArgs a)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int step = 2 * kGridThreads;
+    const int px = a.h * a.w, first = (int)threadIdx.x;
+    // (a corner outside the plane is read where it would lie, in the room left before and behind the plane)
+    T* plane = reinterpret_cast<T*>(smem) + grid_margin((int)sizeof(T), a.w);
+    const uint32_t wg = xcd_order(blockIdx.x, gridDim.x);
+    const int img = (int)(wg / (uint32_t)a.chunks), c_begin = (int)(wg % (uint32_t)a.chunks) * a.planes;
+    const int c_end = c_begin + a.planes < a.c ? c_begin + a.planes : a.c;
+    const T* grid = static_cast<const T*>(a.grid) + (int64_t)img * a.outs * 2;
+    const T* src = static_cast<const T*>(a.x) + ((int64_t)img * a.c + c_begin) * px;
+    T* out = static_cast<T*>(a.out) + ((int64_t)img * a.c + c_begin) * a.outs;
+    int wave_first = __builtin_amdgcn_readfirstlane(first & ~(kWave - 1));
+    Stage<T, (int)sizeof(T) == 4 ? 3 : 2> st;
+    st.request(src, px);
+    // a pixel as {upper left corner + w + 1, which corners exist << 28} (the corner may lie a row and a pixel before the plane)
+    uint32_t corner[PX];
+    float lw[PX], lh[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        corner[k] = 0;
+        lw[k] = lh[k] = 0.0f;
+        if (first + k * step < a.outs) {
+            const Sample s = grid_sample(a, load_xy(grid, first + k * step));
+            uint32_t mask = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
+            if (mask) {
+                corner[k] = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
+                lw[k] = s.lw;
+                lh[k] = s.lh;
+            }
+        }
+    }
+    st.place(src, plane, px);
+    __syncthreads();
+    for (int c = c_begin + 1;; ++c, out += a.outs) {
+        if (c < c_end) {
+            src += px;
+            st.request(src, px);
+        }
+        asm volatile("" : "+s"(wave_first));  // (opaque: one comparison per pixel, not nine kept)
+#pragma unroll
+        for (int k = 0; k < PX; ++k) {
+            if (k * step + wave_first >= a.outs) break;
+            asm volatile("" : "+v"(corner[k]), "+v"(lw[k]), "+v"(lh[k]));
+            const int m = (int)corner[k];
+            const T *r0 = plane + ((m & 0x0FFFFFFF) - a.w - 1), *r1 = r0 + a.w;
+            const T r[4] = {r0[0], r0[1], r1[0], r1[1]};
+            float wt[4], acc = 0.0f;
+            bilinear_weights(lw[k], lh[k], wt);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(wt[j], m & (int)(1u << (28 + j)) ? to_f32(r[j]) : 0.0f, acc);
+            if (k * step + first < a.outs) (out + k * step)[(uint32_t)first] = from_f32<T>(acc);
+        }
+        if (c >= c_end) break;
+        __syncthreads();  // (the plane has been read)
+        st.place(src, plane, px);
+        __syncthreads();
     }
 }
 
@@ -503,6 +570,9 @@ hipError_t raise_t()
                 if (r == hipSuccess)
                     r = hipFuncSetAttribute(reinterpret_cast<const void*>(&grid_planes_both_kernel<T, decltype(p)::value>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes);
+                if (r == hipSuccess)
+                    r = hipFuncSetAttribute(reinterpret_cast<const void*>(&grid_planes_fwd_run_kernel<T, decltype(p)::value>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes);
                 return r;
             });
     return e;
@@ -511,6 +581,12 @@ hipError_t raise_t()
 template <typename T>
 hipError_t forward_t(const GridArgs& a, hipStream_t stream)
 {
+    if (a.run_px)
+        return by_pixels(a.run_px, [&](auto p) {
+            hipLaunchKernelGGL((grid_planes_fwd_run_kernel<T, decltype(p)::value>), dim3((unsigned)a.n * a.chunks), dim3(a.block), a.lds,
+                               stream, a);
+            return hipGetLastError();
+        });
     hipLaunchKernelGGL(grid_planes_fwd_kernel<T>, dim3((unsigned)a.n * a.chunks * a.splits), dim3(a.block), a.lds, stream, a);
     return hipGetLastError();
 }

@@ -1120,8 +1120,38 @@ int64_t grid_planes_together(int64_t bytes, int64_t c, int64_t n)
 
 int grid_block(int64_t lds) { return 2 * lds > mxd::kCuLdsBytes ? 2 * mxd::kGridThreads : mxd::kGridThreads; }
 
+// Planes one after the other, the geometry kept: for planes of 20 KB and more (below, several share a workgroup and its geometry already:
+// 60 x 128 of 40 x 100, float32, 62 -> 53 us for 60 x 70 samples but 29 -> 33 for 20 x 30; 24 x 128 of 64 x 88, float16, 26 -> 30) and for runs
+// at least twice as long as what would share (24 x 64 of 64 x 88 in float32, three a run: 14.0 -> 14.5; 24 x 128 of them 23 -> 21).
+// 24 x 128 planes of 64 x 176 and 24 x 176 samples: 51 -> 39 us, float16 29.0 -> 26.2; 24 x 80 of 80 x 160 and 90 x 100 samples 58 -> 42.
+// The run's length: the least of rounds of workgroups times planes, and one more for a run's start.
+bool grid_planes_run_plan(int es, mxd::GridArgs* a)
+{
+    const int64_t px = (int64_t)a->h * a->w, block = 2 * mxd::kGridThreads, each = ceil_div(a->outs, block);
+    const int64_t lds = ((mxd::grid_margin(es, a->w) + px + a->w + 1) * es + 15) & ~int64_t(15);
+    const int64_t slots = 2 * lds <= mxd::kCuLdsBytes && each <= mxd::grid_run_px(es) ? kGridFill : kGridFill / 2;
+    if (px * es < 20 * 1024 || lds > mxd::kCuLdsBytes || each > mxd::kGridMaxPx || (int64_t)a->n * a->c < 2 * slots) return false;
+    int64_t best = INT64_MAX, run = 0;
+    for (int64_t planes = a->c; planes >= 2; --planes) {
+        const int64_t cost = ceil_div(a->n * ceil_div(a->c, planes), slots) * (planes + 1);
+        if (cost < best || (cost == best && ceil_div(a->c, planes) == ceil_div(a->c, run))) {
+            best = cost;
+            run = planes;
+        }
+    }
+    if (run <= 2 * (mxd::kGridStageBytes / (px * es))) return false;
+    a->planes = (int32_t)run;
+    a->chunks = (int32_t)ceil_div(a->c, run);
+    a->run_px = (int32_t)each;
+    a->splits = 1;
+    a->block = (int32_t)block;
+    a->lds = (uint32_t)lds;
+    return true;
+}
+
 int grid_planes_forward_plan(int es, mxd::GridArgs* a)
 {
+    if (grid_planes_run_plan(es, a)) return MXD_OK;
     const int64_t bytes = (int64_t)a->h * a->w * es;
     a->planes = (int32_t)grid_planes_together(bytes, a->c, a->n);
     a->chunks = (int32_t)ceil_div(a->c, a->planes);
