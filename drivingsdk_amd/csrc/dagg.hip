@@ -84,16 +84,12 @@ __device__ inline int find_locations(const DaggArgs& a, int64_t anchor, int firs
     return n;
 }
 
-// Which of a group's samples a lane stands for: scale by scale, the locations side by side.  (Neighbouring lane groups then gather
-// from the same map at a time, where an anchor's points are close to each other: 6 x 900 anchors in float32, forward, 272 us with the
-// scales of a location side by side, 237 like this.)
-__device__ inline bool sample_of_lane(int lane, int locs, int scales, int& scale, int& loc)
-{
-    // (a quotient of small numbers: half a step away from a whole one at least, which is more than the reciprocal's error)
-    scale = scales == 1 ? (lane < locs ? 0 : 1) : (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)locs));
-    loc = lane - scale * locs;
-    return scale < scales;
-}
+// A group of samples is staged location by location (lane t: scale t % scales of its location t / scales, so that the weights of a
+// location's scales are read side by side) and gathered scale by scale: the place in LDS of the sample that a lane stages.
+// (Neighbouring lane groups then gather from the same map at a time, where an anchor's points are close to each other: 6 x 900 anchors in
+// float32, forward, 272 us with the scales of a location side by side, 235 like this.  With lanes standing for the samples in the
+// order of the gather small calls lose 2 to 5 %: 6 x 296 anchors, 8 groups of 4 channels in float16 11.1 -> 11.6.)
+__device__ inline int sample_place(int lane, bool act, int locs, int scale, int loc) { return act ? scale * locs + loc : lane; }
 
 // ---- forward -------------------------------------------------------------------------------------------------------------
 // ONE: a row piece is the channels of one group (its weight is multiplied into the corner weights once); otherwise 128
@@ -130,6 +126,7 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
         make_rsrc(static_cast<const char*>(a.feat) + (size_t)wk.b * a.batch_bytes, a.batch_bytes);
 
     const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);  // locations per group of samples
+    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
 
     float acc[VEC];
 #pragma unroll
@@ -139,8 +136,8 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
         wave_lds_sync();
         for (int v0 = 0; v0 < n; v0 += step) {
             const int locs = n - v0 < step ? n - v0 : step;
-            int ts, tl;
-            const bool act = sample_of_lane(lane, locs, a.scales, ts, tl);
+            const bool act = tl < locs;
+            const int place = sample_place(lane, act, locs, ts, tl);
             const Found f = found[act ? v0 + tl : 0];
             const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
             const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
@@ -151,14 +148,14 @@ __global__ __launch_bounds__(kDaggWaves * kWave) void dagg_fwd_kernel(const Dagg
             float aw = 1.0f;
             if constexpr (ONE) aw = act ? to_f32(*gw) : 0.0f;
             else
-                for (int k = 0; k < heads; ++k) gws[lane * a.piece_heads + k] = act ? to_f32(gw[k]) : 0.0f;
+                for (int k = 0; k < heads; ++k) gws[place * a.piece_heads + k] = act ? to_f32(gw[k]) : 0.0f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 o[k] = sm.cvalid[k] ? (uint32_t)sm.pix[k] * a.pitch_bytes : kInvalidCorner;
                 cw[k] = sm.valid ? sm.w[k] * aw : 0.0f;
             }
-            off[lane] = o;
-            wts[lane] = cw;
+            off[place] = o;
+            wts[place] = cw;
             wave_lds_sync();
             const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);  // (uniform; samples that do not exist read zeros)
 #pragma unroll 2
@@ -242,13 +239,14 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
     }
 
     const int step = (int)(((uint32_t)kWave * a.sc_magic) >> 20);
+    const int tl = (int)(((uint32_t)lane * a.sc_magic) >> 20), ts = lane - tl * a.scales;
     for (int first = 0; first < a.nloc; first += kDaggList) {
         const int n = find_locations<T>(a, anchor, first, found, lane);
         wave_lds_sync();
         for (int v0 = 0; v0 < n; v0 += step) {
             const int locs = n - v0 < step ? n - v0 : step;
-            int ts, tl;
-            const bool act = sample_of_lane(lane, locs, a.scales, ts, tl);
+            const bool act = tl < locs;
+            const int place = sample_place(lane, act, locs, ts, tl);
             const Found f = found[act ? v0 + tl : 0];
             const uint32_t fx = f.x, fy = f.y, fj = f.z, fc = f.w;
             const Sample sm = sample_geometry(__builtin_bit_cast(float, fx), __builtin_bit_cast(float, fy), lvl[act ? (int)fc * a.scales + ts : 0],
@@ -257,7 +255,7 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
             u32x4 o;
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = sm.cvalid[k] ? (uint32_t)sm.pix[k] * a.pitch_bytes : kInvalidCorner;
-            off[lane] = o;
+            off[place] = o;
             wave_lds_sync();
             const int trips = (locs * a.scales + U - 1) >> (6 - a.lpr_log2);
             auto gather = [&](auto lg) {
@@ -304,7 +302,7 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
                 float ga = 0.f;
                 if (sm.valid) {
                     float gx, gy;
-                    sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, aw, dots[lane], ga, gx, gy);
+                    sample_gradients(sm.lw, sm.lh, sm.Wf, sm.Hf, aw, dots[place], ga, gx, gy);
                     g = f32x2{gx, gy};
                 }
                 gw[(int)(fj >> 16) * a.scales + ts] = ga;
@@ -313,7 +311,7 @@ __device__ inline void dagg_dots(const DaggArgs& a, uint32_t block, unsigned cha
             wave_lds_sync();
             if (act && ts == 0) {
                 // the scales of a location share it
-                for (int k = 1; k < a.scales; ++k) g += gxy[lane + k * locs];
+                for (int k = 1; k < a.scales; ++k) g += gxy[lane + k];
                 gl[fj >> 16] = g;
             }
             wave_lds_sync();
