@@ -1171,14 +1171,35 @@ int grid_planes_forward_plan(int es, mxd::GridArgs* a)
 // plane; at least one plane per CU, and no more output pixels than the registers of a workgroup hold.  24 x 128 planes of 64 x 176:
 // 122 -> 88 us, 2 x 128 of 70 x 150 12.7 -> 11.2, 300 x 8 of 80 x 160 in float16 with the sum over chunks 88 -> 80.  Below the line it
 // gains or loses: 23 x 128 planes of 70 x 110 104 -> 95, 10 x 64 of them 28.6 -> 29.2, 300 x 8 of 75 x 95 52 -> 61, 24 x 64 of 32 x 88 30 -> 33.
-// One round of workgroups; never more chunks than the two kinds would make, whose sums size the workspace.
+//
+// Chunks per image: what costs least of rounds of workgroups times planes, a plane and a half more for a workgroup's start and, from two
+// chunks on, the sum over them (some 4.5 us, and 4 more for 128 images of 24 x 176 output pixels; a plane takes some 6).  From one round of workgroups
+// to four; never more chunks than the two kinds would make, whose sums size the workspace.  (One round alone leaves half of the chip idle
+// where the images are not many fewer than the CUs: 130 x 64 planes of 64 x 176 388 us in one chunk, 274 + 12 in three, two kinds of
+// workgroups 322 + 12; 300 x 64 767, in two 590 + 24, two kinds 710 + 25.)
 bool grid_planes_both_plan(int es, mxd::GridArgs* a)
 {
-    const int64_t px = (int64_t)a->h * a->w, block = 2 * mxd::kGridThreads, cus = kGridFill / 2;
+    const int64_t px = (int64_t)a->h * a->w, block = 2 * mxd::kGridThreads, cus = kGridFill / 2, n = a->n;
     const int64_t lds = mxd::grid_sums_bytes(px) + (((px + a->w + 1) * es + 15) & ~int64_t(15)) + mxd::kWave * 8;
-    if (2 * px * 8 <= mxd::kCuLdsBytes || lds > mxd::kCuLdsBytes || a->outs > block * mxd::kGridMaxPx || (int64_t)a->n * a->c < cus) return false;
-    int64_t chunks = cus / a->n < 1 ? 1 : cus / a->n;
-    if (chunks > a->gg_chunks) chunks = a->gg_chunks;
+    if (2 * px * 8 <= mxd::kCuLdsBytes || lds > mxd::kCuLdsBytes || a->outs > block * mxd::kGridMaxPx || n * a->c < cus) return false;
+    int64_t chunks = 1;
+    double best = 0.0;
+    auto consider = [&](int64_t k) {
+        const int64_t planes = ceil_div(a->c, k), wgs = n * ceil_div(a->c, planes);
+        const double cost = (double)ceil_div(wgs, cus) * ((double)planes + 1.5) + (k > 1 ? 0.75 + (double)n / 128.0 : 0.0);
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            chunks = k;
+        }
+    };
+    consider(1);
+    for (int64_t k = cus / n < 2 ? 2 : cus / n; k <= a->gg_chunks && n * k <= 4 * cus + n; ++k) consider(k);
+    // Where the two kinds make one chunk too (one channel, or two images per CU and more) nothing is summed either way, and an image count just
+    // beyond a whole number of rounds leaves theirs the faster ones (their time in planes, fitted to these): 300 x 1 planes 21.9 / 23.4 us,
+    // 400 x 1 27.2 / 25.0, 513 x 3 68.6 / 73.9, 520 x 16 328 / 310; 300 x 1 of 70 x 150 with 96 x 96 output pixels 38 / 43, 400 x 1 48 / 46.  With one output
+    // pixel per thread the step between planes is most of it: 257 x 1 of 75 x 160, 12 x 20, float16, 9.2 / 7.9.
+    const double rounds = (double)ceil_div(n, cus);
+    if (a->gg_chunks == 1 && a->outs > block && rounds * ((double)a->c + 1.0) > (double)n * ((double)a->c + 0.5) / 168.0 + 0.95) return false;
     a->gb_channels = (int32_t)ceil_div(a->c, chunks);
     a->gb_chunks = (int32_t)ceil_div(a->c, a->gb_channels);
     a->gb_px = (int32_t)ceil_div(a->outs, block);
