@@ -1140,6 +1140,15 @@ bool grid_planes_run_plan(int es, mxd::GridArgs* a)
         }
     }
     if (run <= 2 * (mxd::kGridStageBytes / (px * es))) return false;
+    // How much of their rounds the runs must fill, and how long they may be, by the output pixels per thread, whose geometry is what a run saves.  (A
+    // workgroup per plane leaves no round empty and has more planes on their way at a time.)  That form / this one over 590 sizes:
+    // from 1.8 pixels per thread on 0.97 to 1.51 with two workgroups per CU, whatever the fill, with one 1.00 to 1.66 from 0.6 full on (0.81 to 1.11
+    // at 0.5), but planes of 20 to 23 KB from 0.9 on (0.89 to 1.05 below).  Fewer pixels: 0.67 to 1.14 at 0.5 to 0.68; from 0.7 on, above one
+    // pixel, 0.98 to 1.28 in runs of up to ten planes, 0.83 to 1.16 in longer ones, up to one pixel 0.97 to 1.21 in runs of up to five, 0.83 to 1.12 in longer ones.
+    const bool two = slots == kGridFill, few = 5 * (int64_t)a->outs < 9 * block;
+    const double fill = (double)((int64_t)a->n * a->c) / (double)(slots * run * ceil_div(a->n * ceil_div(a->c, run), slots));
+    if (fill < (few ? 0.7 : two ? 0.0 : px * es < 24 * 1024 ? 0.9 : 0.6)) return false;
+    if (few && run > (each > 1 && two ? 10 : 5)) return false;
     a->planes = (int32_t)run;
     a->chunks = (int32_t)ceil_div(a->c, run);
     a->run_px = (int32_t)each;

@@ -53,10 +53,11 @@ def test_large_planes(gpu_device, input_shape, grid_shape, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("input_shape,grid_shape", [([8, 130, 79, 157], [8, 3, 5, 2]), ([8, 131, 79, 157], [8, 41, 50, 2]),
                                                     ([6, 176, 79, 157], [6, 48, 128, 2]), ([4, 131, 79, 157], [4, 97, 95, 2]),
-                                                    ([513, 3, 67, 97], [513, 9, 7, 2]), ([5, 128, 160, 255], [5, 9, 7, 2])])
+                                                    ([513, 3, 67, 97], [513, 9, 7, 2]), ([5, 128, 160, 255], [5, 9, 7, 2]),
+                                                    ([8, 190, 79, 157], [8, 3, 5, 2]), ([3, 255, 160, 252], [3, 9, 7, 2])])
 def test_runs_of_planes(gpu_device, input_shape, grid_shape, dtype):
     """Many planes per workgroup, one after the other (the last run short; one, three, six and nine output pixels per thread; planes of
-    odd size; a plane that takes a CU's LDS whole): the same bits as few planes, which get a workgroup each."""
+    odd size; a plane that takes a CU's LDS whole), and sizes just outside of that form: the same bits as few planes, which get a workgroup each."""
     g = torch.Generator().manual_seed(7)
     grid = ((2 * torch.rand(grid_shape, generator=g) - 1) * 1.2).to(gpu_device, dtype)
     x = torch.rand(input_shape[1:], generator=g).to(gpu_device, dtype) + torch.arange(input_shape[0], device=gpu_device, dtype=dtype).view(-1, 1, 1, 1)
