@@ -302,6 +302,14 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
         }
 #pragma unroll
         for (int half = 0; half < NS; half += HS) {
+            // (A wavefront beyond the tile's samples, whose lanes would all count on the same word, one addition after the other: 6 x 900 queries x 4
+            //  heads x 4 points on 15 x 25 pixels, backward in float32 8 channels 33.5 -> 29.8 us, 64 channels 30.9 -> 27.6, on 60 x 66 in float16 16
+            //  channels 41.6 -> 33.7.  Not where the branch costs 34 spilled registers more: 24 x 7156 x 4 x 15 on 30 x 30 pixels 0.88 of the speed.)
+            if (!(QUAD && sizeof(T) == 4 && PX > 12) && half * block + wave * kWave >= n) {
+#pragma unroll
+                for (int k = 0; k < HS; ++k) place[half + k] = (uint32_t)a.nk;
+                continue;
+            }
             f32x2 xy[HS];
 #pragma unroll
             for (int k = 0; k < HS; ++k) {
@@ -572,6 +580,7 @@ hipError_t by_pixels(int px, int lanes_log2, F f)
 {
     if constexpr (sizeof(T) == 4)  // (16-bit rows are shared by four lanes at least)
         if (lanes_log2 < 2) {
+            if (px <= 4) return f(&gka_scatter_kernel<T, 4, false>);
             if (px <= 8) return f(&gka_scatter_kernel<T, 8, false>);
             if (px <= 12) return f(&gka_scatter_kernel<T, 12, false>);
             return px <= kGkaPixels ? f(&gka_scatter_kernel<T, kGkaPixels, false>) : hipErrorInvalidConfiguration;
