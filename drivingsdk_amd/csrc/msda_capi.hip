@@ -991,8 +991,9 @@ int64_t gka_splits(int64_t slabs, int64_t nq, int64_t slots, double fixed, int64
 }
 
 // Geometric kernel attention with the (batch, head)'s slab of value in LDS (gka.hip), `parts` of its channels at a time: whether the
-// part's slab, in the dtype for the gather and as float32 sums in registers for grad_value, fits, and the launch geometry.
-bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
+// part's slab, in the dtype for the gather and as float32 sums in registers for grad_value, fits, and the launch geometry.  Without
+// `gather` the slab in LDS is not asked for where the scatter forms the dots, which then is the backward's only kernel over the samples.
+bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, bool gather, mxd::GkaArgs* a)
 {
     memset(a, 0, sizeof(*a));
     const int es = elem_size(dtype);
@@ -1017,7 +1018,7 @@ bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
     const bool two = 2 * lds2 <= lim || lds1 > lim;
     a->block = two ? 512 : 1024;
     a->lds = (uint32_t)(two ? lds2 : lds1);
-    if ((two ? lds2 : lds1) > lim) return false;
+    if ((two ? lds2 : lds1) > lim && (gather || sc_lanes < 4)) return false;
     const int64_t slabs = d.bs * d.nh * parts;
     int64_t s = gka_splits(slabs, d.nq, 2 * (int64_t)a->lds <= lim ? 512 : 256, (double)d.nk / 2, 64 / lanes * (a->block / 64));
     a->split_q = (int32_t)ceil_div(d.nq, s);
@@ -1058,7 +1059,11 @@ bool gka_plan_parts(int dtype, const Dims& d, int64_t parts, mxd::GkaArgs* a)
 // three at 1.0 million; in float32 three of four at half a million).  16-bit units of fewer than 4 samples stay with the general
 // kernel (1 to 3 samples: 0.9 to 1.2 of its time), with fewer than 8 slabs those of fewer than 12 (four slabs: 1 sample 1.5, 4 samples 1.1
 // to 1.3, 8 samples 1.0 to 1.2, 12 samples 0.9 to 1.0).  Backward: wherever the slab fits, whole or in two parts (48 x 24 pixels, 64 channels, float32,
-// two parts: 180 -> 112 us; in four parts 64 x 46 pixels of 32 channels went from 80 to 107 us).
+// two parts: 180 -> 112 us; in four parts 64 x 46 pixels of 32 channels went from 80 to 107 us).  Maps whose slab does not fit, float32, go to
+// the scatter whole where it takes them (its rows of value stay in registers) if two parts would leave rows of 8 channels to lane pairs, whose dots
+// are a gather of their own -- 60 x 43 and 45 x 60 pixels of 16 channels, 26 sizes: 1.2 to 2.0 times as fast as in parts -- and from 1.5 million
+// samples on, 16 to 128 channels: 1.06 to 2.7 times as fast as in two parts, which sort the samples twice, or as the general kernels.  Fewer fill the chip
+// better in two parts: 1.3 million samples 0.95 to 1.4, 0.6 0.89 to 1.4, 0.3 0.7 to 0.9.
 bool gka_plan(int dtype, const Dims& d, bool backward, mxd::GkaArgs* a)
 {
     const int mode = tuning().gka_slab;
@@ -1066,9 +1071,14 @@ bool gka_plan(int dtype, const Dims& d, bool backward, mxd::GkaArgs* a)
     if (!backward) {
         const bool half = elem_size(dtype) == 2, pays = d.bs * d.nh * d.nq * d.nl * d.np >= (half ? int64_t(7) << 17 : int64_t(1) << 19) &&
                                                         (!half || d.nl * d.np >= (d.bs * d.nh < 8 ? 12 : 4));
-        return (mode > 0 || pays) && gka_plan_parts(dtype, d, 1, a);
+        return (mode > 0 || pays) && gka_plan_parts(dtype, d, 1, true, a);
     }
-    return gka_plan_parts(dtype, d, 1, a) || gka_plan_parts(dtype, d, 2, a);
+    if (gka_plan_parts(dtype, d, 1, true, a)) return true;
+    mxd::GkaArgs two;
+    const bool parts = gka_plan_parts(dtype, d, 2, true, &two), many = mode > 0 || d.bs * d.nh * d.nq * d.nl * d.np >= int64_t(3) << 19;
+    if ((many || (parts && !two.sc_dots)) && gka_plan_parts(dtype, d, 1, false, a)) return true;
+    if (parts) *a = two;
+    return parts;
 }
 
 // Workspace of its backward: images of grad_value, dots of the channel parts.

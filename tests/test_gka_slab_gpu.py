@@ -34,7 +34,9 @@ def compare(inp, device, dtype=torch.float32):
     ([2, 700, 8, 2, 1, 7], (9, 13)), ([1, 1, 16, 2, 1, 4], (8, 12)), ([2, 333, 16, 3, 1, 20], (40, 60)), ([1, 911, 32, 2, 2, 9], (17, 19)),
     ([3, 257, 64, 4, 1, 16], (24, 25)), ([1, 130, 128, 2, 1, 5], (10, 20)), ([1, 5000, 32, 1, 1, 1], (3, 5)), ([2, 90, 64, 1, 3, 17], (7, 11)),
     ([1, 300, 16, 2, 1, 17], (60, 68)), ([1, 300, 64, 2, 1, 6], (25, 26)), ([1, 300, 64, 2, 1, 6], (31, 33)), ([2, 257, 64, 2, 1, 18], (24, 48)),
-    ([1, 40, 16, 2, 1, 6], (64, 74))])
+    ([1, 40, 16, 2, 1, 6], (64, 74)),
+    # maps whose slab does not fit the LDS but whose scatter does, up to the most pixels it takes
+    ([1, 2100, 16, 2, 1, 17], (60, 43)), ([1, 1900, 64, 1, 1, 6], (32, 32)), ([1, 700, 32, 2, 1, 9], (32, 64)), ([1, 300, 16, 1, 2, 9], (32, 64))])
 def test_sizes(gpu_device, shape, hw, dtype):
     compare(make_inputs(shape, hw, seed=shape[1]), gpu_device, dtype)
 

@@ -412,6 +412,16 @@ def test_geometric_kernel_attention_keeps_a_small_map_in_one_tile(monkeypatch, c
         _lib.reload_tuning()
 
 
+@pytest.mark.parametrize("nk,hd,bs,nq,nh,npts,parts", [
+    (375, 64, 1, 400, 8, 6, 1), (2580, 16, 1, 400, 8, 6, 1), (2580, 16, 24, 7156, 4, 15, 1), (900, 64, 24, 7156, 4, 15, 1), (900, 64, 2, 2500, 8, 8, 2),
+    (2048, 32, 12, 7156, 4, 15, 1), (2048, 32, 6, 900, 4, 4, 2), (1152, 64, 24, 7156, 4, 15, 2)])
+def test_geometric_kernel_attention_takes_channels_whole_where_that_measured_faster(nk, hd, bs, nq, nh, npts, parts):
+    """float32, backward: maps whose slab of value exceeds the LDS (the workspace holds the dots of the parts where there are several)."""
+    size = _lib.load().mxd_gka_backward_workspace_bytes(0, bs, nk, nh, hd, 1, nq, npts)
+    image, dots = bs * nk * nh * hd * 4, parts * bs * nq * nh * npts * 4 if parts > 1 else 0
+    assert any(size == (splits * image + 255) // 256 * 256 + dots for splits in range(1, 65))
+
+
 @pytest.mark.parametrize("code,hd,honoured", [(1, 3, False), (2, 1, False), (1, 4, True), (0, 3, True)])
 def test_tile_sizes_that_no_kernel_is_built_for_are_not_taken(monkeypatch, code, hd, honoured):
     """16-bit rows of fewer than 4 channels have the grad_value pass for tiles of 512 pixels alone: there MXD_MSDA_TILE_PX_LOG2
