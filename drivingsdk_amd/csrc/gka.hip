@@ -55,11 +55,12 @@ __device__ inline int32_t sample_pixel(const GkaArgs& a, const i32x4* lvl, int s
     return sm.cvalid[0] ? sm.pix[0] : -1;
 }
 
-// Forward (DOTS = false) or gradient of the weights (DOTS = true); LPR lanes of 16 bytes share a row.
+// Forward (DOTS = false) or, of rows of 8 channels in float32, gradient of the weights (DOTS = true); LPR lanes of 16 bytes share a row.
 template <typename T, int LPR_LOG2, bool DOTS>
 __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
 {
     constexpr int LPR = 1 << LPR_LOG2, U = kWave / LPR, VEC = 16 / (int)sizeof(T);
+    static_assert(!DOTS || sizeof(T) == 4);
     constexpr int K = LPR < kChunk ? kChunk / LPR : 1;  // staged samples (and dots) per lane
     typedef RowIO<T, VEC> Row;
     struct Staged {
@@ -134,16 +135,10 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
     const Staged* mine = stage + g * kChunkStride;
     for (; q0 < q_end; q0 += nw * U) {
         float acc[VEC], gv[VEC];
-        uint32_t gp[VEC / 2];
-        typedef T t2 __attribute__((ext_vector_type(2)));
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] = 0.0f;
         if constexpr (DOTS) {
             Row::unpack_held(next_row, gv);
-            if constexpr (sizeof(T) == 2) {
-#pragma unroll
-                for (int e = 0; e < VEC / 2; ++e) gp[e] = __builtin_bit_cast(uint32_t, t2{next_row[2 * e], next_row[2 * e + 1]});
-            }
             next_row = fetch_row(q0 + nw * U);
         }
         for (int c0 = 0; c0 < a.S; c0 += kChunk) {
@@ -179,20 +174,10 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
                     // (four samples side by side; what is staged behind the last one is the row of zeros)
 #pragma unroll
                     for (int s = s4; s < s4 + 4; ++s) {
-                        const u32x4 raw = *reinterpret_cast<const u32x4*>(slab + mine[s].row + c * 16);
-                        float p = 0.0f;
-                        if constexpr (sizeof(T) == 2) {
+                        float v[VEC], p = 0.0f;
+                        Row::unpack(*reinterpret_cast<const typename Row::raw_t*>(slab + mine[s].row + c * 16), v);
 #pragma unroll
-                            for (int e = 0; e < VEC / 2; ++e) {
-                                const uint32_t pair = raw[e];
-                                p = dot2_acc<T>(pair, gp[e], p);
-                            }
-                        } else {
-                            float v[VEC];
-                            Row::unpack(raw, v);
-#pragma unroll
-                            for (int e = 0; e < VEC; ++e) p = __builtin_fmaf(v[e], gv[e], p);
-                        }
+                        for (int e = 0; e < VEC; ++e) p = __builtin_fmaf(v[e], gv[e], p);
                         p = group_sum<LPR_LOG2>(p);
                         if (c == (s & (LPR - 1))) dot[s >> LPR_LOG2 < K ? s >> LPR_LOG2 : 0] = p;
                     }
@@ -562,15 +547,15 @@ __global__ __launch_bounds__(256) void gka_sum_kernel(const GkaArgs a, uint32_t 
     RowIO<T, 4>::store_global(static_cast<T*>(a.grad_value) + 4 * i, v);
 }
 
-template <typename T, bool DOTS, typename F>
+template <typename T, typename F>
 hipError_t by_lanes(int lpr_log2, F f)
 {
     switch (lpr_log2) {
-        case 1: return f(&gka_slab_kernel<T, 1, DOTS>);
-        case 2: return f(&gka_slab_kernel<T, 2, DOTS>);
-        case 3: return f(&gka_slab_kernel<T, 3, DOTS>);
-        case 4: return f(&gka_slab_kernel<T, 4, DOTS>);
-        case 5: return f(&gka_slab_kernel<T, 5, DOTS>);
+        case 1: return f(&gka_slab_kernel<T, 1, false>);
+        case 2: return f(&gka_slab_kernel<T, 2, false>);
+        case 3: return f(&gka_slab_kernel<T, 3, false>);
+        case 4: return f(&gka_slab_kernel<T, 4, false>);
+        case 5: return f(&gka_slab_kernel<T, 5, false>);
         default: return hipErrorInvalidConfiguration;
     }
 }
@@ -599,29 +584,30 @@ hipError_t raise_t()
         return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kCuLdsBytes - 256);
     };
     hipError_t e = hipSuccess;
-    for (int l = 1; l <= 5; ++l) {
-        if (e == hipSuccess) e = by_lanes<T, false>(l, raise);
-        if (e == hipSuccess) e = by_lanes<T, true>(l, raise);
-    }
+    for (int l = 1; l <= 5; ++l)
+        if (e == hipSuccess) e = by_lanes<T>(l, raise);
+    if constexpr (sizeof(T) == 4)
+        if (e == hipSuccess) e = raise(&gka_slab_kernel<T, 1, true>);
     for (int px = 4; px <= kGkaPixels; px += 4)
         for (int lanes_log2 : {1, 2})
             if (e == hipSuccess) e = by_pixels<T>(px, lanes_log2, raise);
     return e;
 }
 
-template <typename T, bool DOTS>
-hipError_t slab_t(const GkaArgs& a, hipStream_t stream)
+hipError_t launch_slab(void (*kernel)(const GkaArgs), const GkaArgs& a, hipStream_t stream)
 {
-    return by_lanes<T, DOTS>(a.lpr_log2, [&](auto* kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.splits)), dim3(a.block), a.lds, stream, a);
-        return hipGetLastError();
-    });
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.splits)), dim3(a.block), a.lds, stream, a);
+    return hipGetLastError();
 }
 
 template <typename T>
 hipError_t backward_t(const GkaArgs& a, hipStream_t stream)
 {
-    hipError_t e = a.sc_dots ? hipSuccess : slab_t<T, true>(a, stream);
+    hipError_t e = hipSuccess;
+    if (!a.sc_dots) {  // (lane pairs share a row: 8 channels in float32)
+        if constexpr (sizeof(T) == 4) e = a.lpr_log2 == 1 ? launch_slab(&gka_slab_kernel<T, 1, true>, a, stream) : hipErrorInvalidConfiguration;
+        else e = hipErrorInvalidConfiguration;
+    }
     if (e != hipSuccess) return e;
     e = by_pixels<T>(a.sc_px, a.sc_lanes_log2, [&](auto* kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(a.bs * a.nh * a.parts * a.sc_splits)), dim3(a.sc_block), a.sc_lds, stream, a);
@@ -648,9 +634,9 @@ hipError_t raise_gka_lds()
 hipError_t launch_gka_forward(int dtype, const GkaArgs& a, hipStream_t stream)
 {
     switch (dtype) {
-        case MXD_DTYPE_F32: return slab_t<float, false>(a, stream);
-        case MXD_DTYPE_F16: return slab_t<f16_t, false>(a, stream);
-        case MXD_DTYPE_BF16: return slab_t<bf16_t, false>(a, stream);
+        case MXD_DTYPE_F32: return by_lanes<float>(a.lpr_log2, [&](auto* kernel) { return launch_slab(kernel, a, stream); });
+        case MXD_DTYPE_F16: return by_lanes<f16_t>(a.lpr_log2, [&](auto* kernel) { return launch_slab(kernel, a, stream); });
+        case MXD_DTYPE_BF16: return by_lanes<bf16_t>(a.lpr_log2, [&](auto* kernel) { return launch_slab(kernel, a, stream); });
         default: return hipErrorInvalidValue;
     }
 }

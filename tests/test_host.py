@@ -491,3 +491,15 @@ def test_two_units_for_17_samples_never_cost_a_problem_its_form_or_the_static_ar
         assert rows * (nk // 512 + nl + 1) * 4 <= 1 << 28 < 2 * rows * (nk // 512 + nl + 1) * 4
         total = lib.mxd_msda_backward_workspace_bytes(1, 6, nk, 8, 32, nl, nl, nq, 5)
         assert total > 48 * nq * 20 * 2 * 12                 # the hand-over is there: not the form with global atomics
+
+
+def test_the_gather_of_dots_is_built_for_lane_pairs_alone():
+    """Rows of four lanes and more have their dots formed by the scatter: of the kernels that gather them one can be launched."""
+    import shutil
+    import subprocess
+    nm = shutil.which("nm")
+    if nm is None:
+        pytest.skip("no nm")
+    names = subprocess.run([nm, "-C", _lib.LIB_PATH], check=True, capture_output=True, text=True).stdout
+    gathers = {n for n in names.split("\n") if "__device_stub__gka_slab_kernel" in n and "true>" in n}
+    assert len(gathers) == 1 and "float, 1, true" in gathers.pop()
