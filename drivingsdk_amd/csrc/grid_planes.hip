@@ -32,8 +32,8 @@ struct Piece {
 };
 
 // Consecutive elements on their way to LDS: request() asks for a thread's first four (kAhead) 16-byte pieces, place() stores them,
-// and the rest of a stretch that is longer than that.
-template <typename T, int kAhead = 4>
+// and the rest of a stretch that is longer than that (kWhole: there is none).
+template <typename T, int kAhead = 4, bool kWhole = false>
 struct Stage {
     typedef typename Piece<T>::vec_t vec_t;
     typedef typename Piece<T>::mem_t mem_t;
@@ -56,10 +56,16 @@ struct Stage {
             for (int j = 0; j < kAhead; ++j)
                 if (i0 + j * step < pieces) *reinterpret_cast<vec_t*>(lds + (i0 + j * step) * kE) = v[j];
             i0 += kAhead * step;
-            if (i0 >= pieces) break;
+            if (kWhole || i0 >= pieces) break;
             request(src, elems, i0);
         }
-        for (int i = pieces * kE + (int)threadIdx.x; i < elems; i += step) lds[i] = src[i];
+        if constexpr (kWhole) {
+            // (fewer than a piece is left: no loop, which the compiler unrolls for lengths that do not occur)
+            const int i = pieces * kE + (int)threadIdx.x;
+            if (i < elems) lds[i] = src[i];
+        } else {
+            for (int i = pieces * kE + (int)threadIdx.x; i < elems; i += step) lds[i] = src[i];
+        }
     }
 };
 
@@ -383,8 +389,11 @@ __global__ __launch_bounds__(1024) void grid_planes_bwd_kernel(const GridArgs a)
 // gradient stay in registers from plane to plane; the next plane and its grad_out travel while the one at hand is worked on, and
 // its sums go out, and are cleared, in the step that puts the next plane in place: two barriers per plane, grad_out read once.
 // What bounds it is LDS, at work for 3.9 of some 6 us per plane of 64 x 176 and 24 x 176 output pixels; 1.2 us are the step between.
-// (No VGPR may spill here: with 28 of them on the stack, in float32 with nine pixels per thread, the compiler saved one inside the
-//  masked end of place() and the lanes masked off there read rubbish.  Hence grad_out kept once, and reloaded pixel by pixel.)
+// (No VGPR may spill here, nor in the forward's runs: the build checks it.  A build of this kernel that spilled 28, in float32 with nine pixels per
+//  thread, gave wrong sums; its listing had a store to the stack inside the masked end of place(), where lanes that are masked off leave theirs
+//  unsaved.  Most of the registers went to place(): the loop over what does not occur here -- pieces beyond the first ones, elements behind
+//  the last piece, eight at a time -- took 8 to 20 of them.  Without it: 24 x 128 planes of 64 x 176 in float32 87 -> 82 us.  grad_out is
+//  kept once, and reloaded pixel by pixel.)
 template <typename T, int PX>
 __global__ __launch_bounds__(1024) void grid_planes_both_kernel(const GridArgs a)
 {
@@ -414,7 +423,8 @@ __global__ __launch_bounds__(1024) void grid_planes_both_kernel(const GridArgs a
         if constexpr (sizeof(T) == 4) g[k] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(row, at, 0, 0));
         else g[k] = __builtin_bit_cast(T, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(row, at, 0, 0));
     };
-    Stage<T, (int)sizeof(T)> st;  // (the largest plane that fits, in one go)
+    Stage<T, (int)sizeof(T), true> st;  // (the largest plane that fits, in one go)
+    static_assert(kCuLdsBytes / (8 + (int)sizeof(T)) <= (int)sizeof(T) * step * Piece<T>::kElems);
     st.request(src, px);
 #pragma unroll
     for (int k = 0; k < PX; ++k) load_grad(k);

@@ -38,10 +38,10 @@ def test_planes(gpu_device, input_shape, grid_shape, dtype):
 
 
 # (planes of more than 10240 pixels, 256 and more of them: both gradients by the same workgroups.  One and many chunks of the channels, the
-#  last of them short; one, two, three, six and nine output pixels per thread, full and partly so; the largest float32 plane)
+#  last of them short; one, two, three, six and nine output pixels per thread, full and partly so; the largest plane in float32 and in 16 bits)
 LARGE = [([257, 1, 97, 107], [257, 3, 5, 2]), ([131, 22, 97, 107], [131, 5, 7, 2]), ([2, 129, 103, 101], [2, 32, 32, 2]), ([1, 256, 64, 161], [1, 25, 41, 2]),
          ([5, 70, 80, 168], [5, 37, 83, 2]), ([3, 100, 75, 140], [3, 48, 128, 2]), ([3, 100, 75, 140], [3, 96, 96, 2]),
-         ([3, 100, 75, 140], [3, 97, 96, 2])]
+         ([3, 100, 75, 140], [3, 97, 96, 2]), ([2, 130, 120, 135], [2, 9, 7, 2])]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])

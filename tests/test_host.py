@@ -503,3 +503,28 @@ def test_the_gather_of_dots_is_built_for_lane_pairs_alone():
     names = subprocess.run([nm, "-C", _lib.LIB_PATH], check=True, capture_output=True, text=True).stdout
     gathers = {n for n in names.split("\n") if "__device_stub__gka_slab_kernel" in n and "true>" in n}
     assert len(gathers) == 1 and "float, 1, true" in gathers.pop()
+
+
+@pytest.mark.parametrize("kernel,report,builds", [
+    ("grid_planes_both_kernel", "VGPRs Spill: 0", True), ("grid_planes_both_kernel", "VGPRs Spill: 6", False),
+    ("grid_planes_fwd_run_kernel", "VGPRs Spill: 10", False), ("grid_planes_fwd_run_kernel", "", False), ("grid_planes_bwd_kernel", "VGPRs Spill: 2", False)])
+def test_the_build_refuses_spilled_registers_where_they_were_lost(tmp_path, kernel, report, builds):
+    """The Makefile's rule, with a compiler that reports what it is told to (and with nothing said of the kernels in question)."""
+    import shutil
+    import subprocess
+    if shutil.which("make") is None or shutil.which("awk") is None:
+        pytest.skip("no make or awk")
+    src = os.path.join(ROOT, "drivingsdk_amd", "csrc")
+    for name in os.listdir(src):
+        if name == "Makefile" or name.endswith((".hip", ".h")):
+            os.makedirs(tmp_path / "a" / "csrc", exist_ok=True)
+            shutil.copy(os.path.join(src, name), tmp_path / "a" / "csrc")
+    os.makedirs(tmp_path / "include")
+    shutil.copy(os.path.join(ROOT, "include", "mxd_msda.h"), tmp_path / "include")
+    cc = tmp_path / "cc"
+    cc.write_text("#!/bin/sh\nfor a; do last=$a; done\ntouch $last\n"
+                  f"echo 'x.hip:1:0: remark: Function Name: _ZN3mxd23{kernel}IfLi9EEEv [-Rpass-analysis=kernel-resource-usage]' >&2\n"
+                  f"echo 'x.hip:1:0: remark:     SGPRs Spill: 5 [-Rpass]' >&2\necho 'x.hip:1:0: remark:     {report} [-Rpass]' >&2\n")
+    cc.chmod(0o755)
+    res = subprocess.run(["make", "-C", str(tmp_path / "a" / "csrc"), "PYTHON=true", f"HIPCC={cc}", "grid_planes.o"], capture_output=True, text=True)
+    assert (res.returncode == 0) == builds and (tmp_path / "a" / "csrc" / "grid_planes.o").exists() == builds, res.stderr
