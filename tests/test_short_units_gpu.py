@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from drivingsdk_amd import workloads
+from test_first_pass_gpu import _takes_4_lanes
 from test_msda_gpu import _check_all
 from util import BWD_FP32, FWD_FP32, half_tol, set_tuning
 
@@ -49,11 +50,13 @@ def test_narrow_16_bit_rows_with_a_forced_tile_size(gpu_device, monkeypatch, dty
 
 @pytest.mark.parametrize("dtype,hd", [(torch.float32, 32), (torch.float32, 13), (torch.float16, 32), (torch.bfloat16, 24), (torch.float16, 64), (torch.bfloat16, 33)])
 @pytest.mark.parametrize("nl,npts", [(1, 8), (2, 8), (3, 8), (1, 16), (1, 10), (3, 10), (1, 24), (1, 30)])
-def test_eight_points_side_by_side(gpu_device, monkeypatch, nl, npts, dtype, hd):
-    """Levels of eight points and more, with one unit per query and with two, whole and cut off at their last queries; rows of 4 lanes and
-    of 8 (the former need a line of the launch moved)."""
+def test_eight_points_side_by_side(gpu_device, nl, npts, dtype, hd):
+    """Levels of eight points and more, with one unit per query and with two, whole and cut off at their last queries; rows of 8 lanes, and
+    of 4 where a launch has workgroups enough for them."""
     fwd, bwd = (FWD_FP32, BWD_FP32) if dtype == torch.float32 else (half_tol(dtype),) * 2
-    for nq in (1, 67, 10000):
-        if nq == 10000 and (npts, hd) not in ((8, 32), (8, 13)):
-            continue
+    nqs = (1, 67)
+    if 32 < hd * (torch.finfo(dtype).bits // 8) <= 64:
+        nqs += (10003,)
+        assert _takes_4_lanes(2, sum(h * w for h, w in _MAPS[:nl]), 3, hd, nl, nqs[-1], npts, dtype)
+    for nq in nqs:
         _check_all(_inputs(_MAPS[:nl], npts, nq, 3, hd, dtype, 10 * nl + npts), gpu_device, fwd, bwd)
