@@ -202,21 +202,6 @@ __global__ __launch_bounds__(1024) void gka_slab_kernel(const GkaArgs a)
     }
 }
 
-// Inclusive sum over the lanes of a wavefront.
-__device__ inline uint32_t wave_scan(uint32_t v)
-{
-    auto step = [&](auto ctrl, auto rows) {
-        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-    };
-    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr 1, 2, 4, 8
-    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
-    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
-    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
-    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast 15, 31
-    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
-    return v;
-}
-
 // grad_value, or one query range's part of it, and the gradient of the weights: PX pixels per lane group.
 // QUAD: four lanes and more share a row (GkaArgs::sc_dots); without, the gradient of the weights is left to gka_slab_kernel.
 template <typename T, int PX, bool QUAD>
@@ -228,6 +213,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
     __shared__ uint32_t wave_sum[16];
     const int tid = (int)threadIdx.x, block = (int)blockDim.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto add = [](uint32_t x, uint32_t y) { return x + y; };
     const int row_bytes = a.part_ch * (int)sizeof(T);
     i32x4* lvl = reinterpret_cast<i32x4*>(smem);
     u32x2* ent = reinterpret_cast<u32x2*>(smem + kGkaLevelBytes);                    // sorted samples: {row in `rows`, weight}
@@ -347,7 +333,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
             __syncthreads();
             if (tid < kWave) {
                 const uint32_t v = ranks[tid];
-                ranks[tid] = wave_scan(v) - v;
+                ranks[tid] = wave_scan(v, add) - v;
             }
             __syncthreads();
             const int per_wave_log2 = 6 - a.sc_lanes_log2, waves = block / kWave;
@@ -368,7 +354,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
         asm volatile("" : "+v"(t2));
         const int c0 = t2 * per;
         for (int i = c0; i < c0 + per && i < a.nk; ++i) sum += count[i];
-        const uint32_t inc = wave_scan(sum);
+        const uint32_t inc = wave_scan(sum, add);
         if ((t2 & (kWave - 1)) == kWave - 1) wave_sum[wave] = inc;
         __syncthreads();
         uint32_t at = inc - sum;

@@ -83,6 +83,26 @@ __device__ inline Sample grid_sample(const GridArgs& a, f32x2 xy)
     return grid_geometry(xy.x, xy.y, i32x4{a.h, a.w, 0, 0}, a.h * a.w, true, a.mode);
 }
 
+// What the planes of an image share of an output pixel: {upper left corner + w + 1, which corners exist << 28} (the corner may lie a
+// row and a pixel before the plane) and its place in the cell; zeros for one without a corner, and where there is no pixel (`there`).
+template <typename T>
+__device__ inline void pixel_geometry(const GridArgs& a, const T* grid, int at, bool there, uint32_t& corner, float& lw, float& lh)
+{
+    corner = 0;
+    lw = lh = 0.0f;
+    if (there) {
+        const Sample s = grid_sample(a, load_xy(grid, at));
+        uint32_t mask = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
+        if (mask) {
+            corner = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
+            lw = s.lw;
+            lh = s.lh;
+        }
+    }
+}
+
 // Work items in the order of their numbers on every XCD (workgroups are dealt to the XCDs in turn): the splits and ranges that read
 // the same planes follow each other in one L2.
 __device__ inline uint32_t xcd_order(uint32_t wg, uint32_t total)
@@ -156,25 +176,10 @@ __global__ __launch_bounds__(1024, PX <= grid_run_px((int)sizeof(T)) ? 8 : 4) vo
     int wave_first = __builtin_amdgcn_readfirstlane(first & ~(kWave - 1));
     Stage<T, (int)sizeof(T) == 4 ? 3 : 2> st;
     st.request(src, px);
-    // a pixel as {upper left corner + w + 1, which corners exist << 28} (the corner may lie a row and a pixel before the plane)
     uint32_t corner[PX];
     float lw[PX], lh[PX];
 #pragma unroll
-    for (int k = 0; k < PX; ++k) {
-        corner[k] = 0;
-        lw[k] = lh[k] = 0.0f;
-        if (first + k * step < a.outs) {
-            const Sample s = grid_sample(a, load_xy(grid, first + k * step));
-            uint32_t mask = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
-            if (mask) {
-                corner[k] = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
-                lw[k] = s.lw;
-                lh[k] = s.lh;
-            }
-        }
-    }
+    for (int k = 0; k < PX; ++k) pixel_geometry(a, grid, first + k * step, first + k * step < a.outs, corner[k], lw[k], lh[k]);
     st.place(src, plane, px);
     __syncthreads();
     for (int c = c_begin + 1;; ++c, out += a.outs) {
@@ -302,7 +307,6 @@ __device__ inline void grad_points(const GridArgs& a, uint32_t wg, unsigned char
     const T* grid = static_cast<const T*>(a.grid) + (int64_t)img * a.outs * 2;
     const T* grad = static_cast<const T*>(a.grad_out) + (int64_t)img * a.c * a.outs;
 
-    // a pixel as {upper left corner + w + 1, which corners exist << 28} (the corner may lie a row and a pixel before the plane)
     uint32_t corner[PX];
     float lw[PX], lh[PX], sx[PX], sy[PX];
     T g[PX];
@@ -316,19 +320,8 @@ __device__ inline void grad_points(const GridArgs& a, uint32_t wg, unsigned char
     };
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
-        corner[k] = 0;
-        lw[k] = lh[k] = sx[k] = sy[k] = 0.0f;
-        if (k < a.gg_px && first + k * step < a.outs) {
-            const Sample s = grid_sample(a, load_xy(grid, first + k * step));
-            uint32_t mask = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
-            if (mask) {
-                corner[k] = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
-                lw[k] = s.lw;
-                lh[k] = s.lh;
-            }
-        }
+        sx[k] = sy[k] = 0.0f;
+        pixel_geometry(a, grid, first + k * step, k < a.gg_px && first + k * step < a.outs, corner[k], lw[k], lh[k]);
     }
     // (the next planes are requested before the ones at hand are used)
     const T* src = static_cast<const T*>(a.x) + ((int64_t)img * a.c + c_begin) * px;
@@ -428,24 +421,12 @@ __global__ __launch_bounds__(1024) void grid_planes_both_kernel(const GridArgs a
     st.request(src, px);
 #pragma unroll
     for (int k = 0; k < PX; ++k) load_grad(k);
-    // a pixel as {upper left corner + w + 1, which corners exist << 28} (the corner may lie a row and a pixel before the plane)
     uint32_t corner[PX];
     float lw[PX], lh[PX], sx[PX], sy[PX];
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
-        corner[k] = 0;
-        lw[k] = lh[k] = sx[k] = sy[k] = 0.0f;
-        if (first + k * step < a.outs) {
-            const Sample s = grid_sample(a, load_xy(grid, first + k * step));
-            uint32_t mask = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mask |= s.cvalid[j] ? 1u << j : 0u;
-            if (mask) {
-                corner[k] = (uint32_t)(s.pix[0] + a.w + 1) | mask << 28;
-                lw[k] = s.lw;
-                lh[k] = s.lh;
-            }
-        }
+        sx[k] = sy[k] = 0.0f;
+        pixel_geometry(a, grid, first + k * step, first + k * step < a.outs, corner[k], lw[k], lh[k]);
     }
     for (int i = first; i < (px + 1) / 2; i += step) reinterpret_cast<u32x4*>(sums)[i] = u32x4{0u, 0u, 0u, 0u};
     st.place(src, plane, px);

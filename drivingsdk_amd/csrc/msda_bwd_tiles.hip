@@ -321,18 +321,8 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
             const uint32_t m = run_of4[lane];
             auto larger = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
             const uint32_t m0 = m & 255u, m1 = larger(m0, (m >> 8) & 255u), m2 = larger(m1, (m >> 16) & 255u), m3 = larger(m2, m >> 24);
-            int32_t up = (int32_t)m3;  // largest mark so far, over the lanes before this one
-            auto step = [&](auto ctrl, auto rows) {
-                const int32_t o = __builtin_amdgcn_update_dpp(0, up, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
-                up = up > o ? up : o;
-            };
-            step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr 1, 2, 4, 8
-            step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
-            step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
-            step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
-            step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast 15, 31
-            step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
-            const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, up, 0x138, 0xF, 0xF, false);  // wave_shr 1
+            const uint32_t up = wave_scan(m3, larger);  // largest mark so far
+            const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)up, 0x138, 0xF, 0xF, false);  // wave_shr 1
             run_of4[lane] = larger(m0, before) | larger(m1, before) << 8 | larger(m2, before) << 16 | larger(m3, before) << 24;
             wave_lds_sync();
         };

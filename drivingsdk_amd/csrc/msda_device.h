@@ -632,6 +632,22 @@ __device__ inline float dpp_xchg(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// Inclusive scan over the lanes of a wavefront, of an operation that zero leaves alone.
+template <typename Op>
+__device__ inline uint32_t wave_scan(uint32_t v, Op op)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr 1, 2, 4, 8
+    step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast 15, 31
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
+    return v;
+}
+
 template <int LANES_LOG2>
 __device__ inline float group_sum(float v)
 {
