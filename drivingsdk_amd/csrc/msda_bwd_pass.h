@@ -332,10 +332,13 @@ __global__ __launch_bounds__(kPassUnits* LPR, LPR == 8 ? 6 : 4) void msda_bwd_pa
         raw_t ra[4], rb[4];
         // Eight points and more per level: a trip takes eight of a unit side by side (rows of 4 lanes: of two units, and unit after unit before
         // the next eight; rows of 8 lanes: a unit's other eight next).  They touch the same rows on the coarse levels, which have left
-        // the L1 when a sample of every unit at a time comes to the unit's next point.  Backward of 2 x 12000 queries in no order, 4 levels
-        // x 8 points, float16 325 -> 301 us, float32 416 -> 398; in the raster order of the maps, where neighbouring queries' points
-        // are close to each other, 557 -> 558 and 772 -> 759; 6 x 9675 queries over four levels, float16, this kernel 360 -> 317.  Four points
-        // per level gain 1 to 3 % in no order and lose up to 2.5 % in raster order; so do rows of 8 lanes with one unit per query.
+        // the L1 when a sample of every unit at a time comes to the unit's next point.  This kernel at 2 x 12000 queries in no order, 8
+        // heads of 32 channels, 4 levels x 8 points: float16 128 -> 104 us, float32 168 -> 148; at 2 x 19947 in the raster order of the maps, where
+        // neighbouring queries' points are close to each other: 191 -> 190 and 284 -> 268; 6 x 9675 queries over four levels, float16,
+        // 360 -> 317.  Fewer points per level gain where there is no order and mostly lose in raster order (of the
+        // time before, in no order / in raster order): seven 0.87 / 1.03 in float16, 0.92 / 0.98 in float32, six 0.92 / 1.02 and 0.94 / 0.99, five
+        // 0.95 / 1.02 and 0.96 / 1.03, four in float16 0.90 / 1.05: they stay as they were.  So do rows of 8 lanes with one unit per query
+        // (four points in float32, raster order: 150 -> 158 us).
         if (eight) {
             // Units of 16 samples (or of 8): the trip's part of their rows of grad_out comes from LDS.
             constexpr int kWords = kDot2 ? kPairs : VEC;

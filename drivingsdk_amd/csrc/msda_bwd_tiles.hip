@@ -331,8 +331,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void msda_gradv_tiles_kernel(const
                 window = first & ~(kWindow - 1);
                 open_window((uint32_t)window);
             }
-            // (one 12-byte load, non-temporal: the records are read once.  Unconditional, beyond the buffer where there is no record: behind
-            //  a branch around a load the compiler can only wait for every load there is)
+            // (one 12-byte load, non-temporal: a record is read once, but for the two batches ahead that a walk drops and the next round asks for
+            //  again, up to 128 of some 500 records: 3 to 17 % more bytes than with one batch ahead where items have many rounds.
+            //  Unconditional, beyond the buffer where there is no record: behind a branch around a load the compiler can only wait for
+            //  every load there is)
             const int i = first + lane;
             const uint32_t at = i < N ? (run_at[run_of[i & (kWindow - 1)]] + (uint32_t)i) * (kRecDwords * 4u) : ~0u;
             to = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rres, at, 0, 2));

@@ -214,8 +214,8 @@ struct LevelLanes {
 __device__ inline void zero_fill(const KArgs& a, const LevelLanes& lv)
 {
     if (a.fill_n4 != 0 && a.sparse != 0 && lv.canonical) {
-        // only the rows that receive atomic additions in the tile pass (tiles split by query range, small tiles,
-        // and the first pixel of every other tile); a row of the image is nh*hd floats, a multiple of 16 bytes here
+        // only the rows that receive atomic additions in the tile pass (tiles split by query range and the first
+        // pixel of every other tile); a row of the image is nh*hd floats, a multiple of 16 bytes here
         const int32_t tiles = a.tbl_stride - 1;  // (bound: pieces of tiles that do not exist are skipped)
         const int64_t pieces = (int64_t)a.bs * tiles * kRowParts;
         const uint32_t row4 = (uint32_t)(a.nh * a.hd) / 4;
