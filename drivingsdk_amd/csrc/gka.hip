@@ -208,6 +208,7 @@ template <typename T, int PX, bool QUAD>
 __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
 {
     typedef RowIO<T, 4> Row;
+    constexpr bool kLeaveOut = !(QUAD && sizeof(T) == 4 && PX > 12);
     constexpr int NS = gka_samples(PX, QUAD), HS = PX > 12 ? 2 : NS / 2;  // samples of a tile per thread, and those requested together
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ uint32_t wave_sum[16];
@@ -245,6 +246,7 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
     for (int i = 0; i < PX; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[i][e] = 0.0f;
+    const uint32_t spare = min((uint32_t)(tid & (kWave - 1)), (uint32_t)a.nk);  // (of the words from count[nk] on, start[0] to start[nk])
     const int per = (a.nk + block - 1) / block;        // counters of a thread in the prefix sum
     const int piece_log2 = a.lpr_log2;                 // 16-byte pieces of a row
     __syncthreads();
@@ -275,8 +277,9 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
         for (int half = 0; half < NS; half += HS) {
             // (A wavefront beyond the tile's samples, whose lanes would all count on the same word, one addition after the other: 6 x 900 queries x 4
             //  heads x 4 points on 15 x 25 pixels, backward in float32 8 channels 33.5 -> 29.8 us, 64 channels 30.9 -> 27.6, on 60 x 66 in float16 16
-            //  channels 41.6 -> 33.7.  Not where the branch costs 34 spilled registers more: 24 x 7156 x 4 x 15 on 30 x 30 pixels 0.88 of the speed.)
-            if (!(QUAD && sizeof(T) == 4 && PX > 12) && half * block + wave * kWave >= n) {
+            //  channels 41.6 -> 33.7.  Not where the branch costs 34 spilled registers more: 24 x 7156 x 4 x 15 on 30 x 30 pixels 0.88 of the speed.
+            //  There, and in float32's other forms, the lanes without a sample count on words of their own: 30 x 30 pixels, 6 x 900 x 4 x 4, 1.07.)
+            if (kLeaveOut && half * block + wave * kWave >= n) {
 #pragma unroll
                 for (int k = 0; k < HS; ++k) place[half + k] = (uint32_t)a.nk;
                 continue;
@@ -298,7 +301,11 @@ __global__ __launch_bounds__(1024) void gka_scatter_kernel(const GkaArgs a)
             }
             uint32_t before[HS];
 #pragma unroll
-            for (int k = 0; k < HS; ++k) before[k] = atomicAdd(&count[place[half + k]], 1u);  // (samples without a pixel: start[0], not yet in use)
+            for (int k = 0; k < HS; ++k) {  // (samples without a pixel: `start`, not yet in use)
+                uint32_t at = place[half + k];
+                if (QUAD && sizeof(T) == 4 && at == (uint32_t)a.nk) at += spare;
+                before[k] = atomicAdd(&count[at], 1u);
+            }
 #pragma unroll
             for (int k = 0; k < HS; ++k) place[half + k] |= before[k] << 16;
         }
