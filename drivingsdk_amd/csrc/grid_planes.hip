@@ -16,8 +16,8 @@
 // grid many channels of a pixel: two kinds of workgroups of one launch, which read grad_out twice (a fifth of what moves) -- or, where
 // a plane with its sums leaves a CU room for one workgroup anyway, one kind that does both plane by plane.
 //
-// Measured at that size: forward 39 us (190 MB, 4.9 TB/s: the rate of a copy), both gradients by two kinds of workgroups 122 us (400 MB, 3.3 TB/s), by
-// one 88; in float16 109 and 77 us.  Small calls ([24, 128, 16, 20] -> 12 x 20) take 5 and 9 us.
+// Measured at that size: forward 39 us (190 MB, 4.9 TB/s: the rate of a copy), both gradients by two kinds of workgroups 122 us (400 MB,
+// 3.3 TB/s), by one 82; in float16 109 and 70 us.  Small calls ([24, 128, 16, 20] -> 12 x 20) take 5 and 9 us.
 #include "grid_planes.h"
 
 namespace mxd {

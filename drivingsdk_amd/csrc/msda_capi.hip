@@ -1188,7 +1188,7 @@ int grid_planes_forward_plan(int es, mxd::GridArgs* a)
 // Both gradients by the same workgroups, each a chunk of an image's channels, plane by plane: for planes whose float64 sums take
 // more than half of a CU's LDS, so that the two kinds of workgroups get one at a time onto a CU, and which fit it together with the
 // plane; at least one plane per CU, and no more output pixels than the registers of a workgroup hold.  24 x 128 planes of 64 x 176:
-// 122 -> 88 us, 2 x 128 of 70 x 150 12.7 -> 11.2, 300 x 8 of 80 x 160 in float16 with the sum over chunks 88 -> 80.  Below the line it
+// 122 -> 82 us, 2 x 128 of 70 x 150 12.7 -> 11.2, 300 x 8 of 80 x 160 in float16 with the sum over chunks 88 -> 73.  Below the line it
 // gains or loses: 23 x 128 planes of 70 x 110 104 -> 95, 10 x 64 of them 28.6 -> 29.2, 300 x 8 of 75 x 95 52 -> 61, 24 x 64 of 32 x 88 30 -> 33.
 //
 // Chunks per image: what costs least of rounds of workgroups times planes, a plane and a half more for a workgroup's start and, from two
